@@ -18,7 +18,7 @@ import sys
 import numpy as np
 import torch
 
-sys.path.insert(0, os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "snntc-2023_amd"))
+sys.path.insert(0, os.path.join(os.getcwd(), "snntc-2023_amd"))       # imported from the root of the tree that is measured
 import snntc_amd as snn  # noqa: E402
 from snntc_amd import networks, train  # noqa: E402
 
