@@ -3,9 +3,14 @@
 The library is looked up next to the HIP sources (``snntc-2023_amd/csrc/libsnntc_hip.so``, built
 in-tree by ``make -C snntc-2023_amd/csrc``) or at ``$SNNTC_HIP_LIB``.  There is no CPU fallback:
 if the library is missing, loading raises ``SnntcLibraryError``.
+
+The package's own calls go through ``_binding.so`` (csrc/binding.cpp, built by the same make), which
+calls that same library; the ctypes handle serves the side outputs and callers of the C ABI.
 """
 import ctypes
 import os
+
+import numpy as np
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC_DIR = os.path.normpath(os.path.join(_HERE, "..", "csrc"))
@@ -49,6 +54,15 @@ class SnntcError(RuntimeError):
 
 
 _lib = None
+_native = None
+
+
+def params_array(params, n):
+    """Any sequence of n numbers as a contiguous float32 vector."""
+    p = np.ascontiguousarray(np.asarray(params, dtype=np.float32).reshape(-1))
+    if p.size != n:
+        raise ValueError(f"Params must hold {n} float32 values, got {p.size}")
+    return p
 
 
 def lib_path():
@@ -116,6 +130,21 @@ def load():
     lib.snntc_static_scratch_bytes.restype = sz
     _lib = lib
     return lib
+
+
+def native():
+    """The native host path (csrc/binding.cpp), bound to the library on first use."""
+    global _native
+    if _native is None:
+        load()
+        try:
+            from . import _binding
+        except ImportError as e:
+            raise SnntcLibraryError(f"snntc_amd/_binding.so is missing or cannot be loaded ({e}): build it with "
+                                    f"`make -C {CSRC_DIR}`. There is no CPU fallback for the SNN-TC ops.") from e
+        _binding.bind(lib_path(), SnntcLibraryError, SnntcError, params_array)
+        _native = _binding
+    return _native
 
 
 def check(status):

@@ -8,14 +8,15 @@ and the loss run gfx950 kernels and, like the four ops, take float32 tensors on 
 is no host fallback.  ``SNN_avgpool2d`` and ``SNN_LRN`` are compositions of stock PyTorch ops, as they are
 stock TF ops in the reference.
 """
+import functools
 import math
 
 import numpy as np
 import torch
 import torch.nn.functional as F
 
-from ._lib import SnntcLibraryError
-from .ops import SnnCvSame, SnnCvTimes, SnnFcTimes, SnnMinPool, SnnPadTime, SoftmaxTimeLoss
+from ._lib import SnntcLibraryError, native
+from .ops import SnnCvSame, SnnCvTimes, SnnMinPool, SnnPadTime, SoftmaxTimeLoss
 
 # Mirrors the reference's module-level switch (SNN_TC_Modules.py:11): when True the layers keep
 # the largest batch and element count they have seen in ``maxD`` (every tensor must stay below
@@ -44,6 +45,17 @@ def _same_pad(size, kernel, stride):
     return before, total - before
 
 
+@functools.lru_cache(maxsize=1024)
+def _same_pads(H, W, kh, kw, sh, sw):
+    """(top, bottom, left, right) of the SAME padding of an H x W image (a negative total is refused: tf.pad
+    would fail there and the reference never reaches that case)."""
+    top, bottom = _same_pad(H, kh, sh)
+    left, right = _same_pad(W, kw, sw)
+    if min(top, bottom, left, right) < 0:
+        raise ValueError("negative SAME padding: kernel smaller than stride is not supported")
+    return top, bottom, left, right
+
+
 def _require_device(t, what):
     """The kernels behind these layers exist for float32 NHWC tensors on a ROCm device only."""
     if not isinstance(t, torch.Tensor):
@@ -55,16 +67,11 @@ def _require_device(t, what):
 
 
 def _pad_hw(x, kh, kw, sh, sw, value):
-    """Pads NHWC ``x`` for SAME mode with ``value`` in one kernel pass (a negative total is refused: tf.pad
-    would fail there and the reference never reaches that case)."""
+    """Pads NHWC ``x`` for SAME mode with ``value`` in one kernel pass."""
     _require_device(x, "input")
     if x.dim() != 4:
         raise ValueError(f"input must be [B,H,W,C], got shape {tuple(x.shape)}")
-    H, W = x.shape[1], x.shape[2]
-    top, bottom = _same_pad(H, kh, sh)
-    left, right = _same_pad(W, kw, sw)
-    if min(top, bottom, left, right) < 0:
-        raise ValueError("negative SAME padding: kernel smaller than stride is not supported")
+    top, bottom, left, right = _same_pads(x.shape[1], x.shape[2], kh, kw, sh, sw)
     if top or bottom or left or right:
         return SnnPadTime.apply(x.contiguous(), top, bottom, left, right, float(value))
     return x
@@ -106,11 +113,10 @@ class SNN_dense(torch.nn.Module, _CostsMixin):
         self.weight = torch.nn.Parameter(torch.from_numpy(weight))
 
     def forward(self, X):
-        B = X.shape[0]
         if Check_Dim:
-            self.maxD[0] = max(self.maxD[0], int(B))
-            self.maxD[1] = max(self.maxD[1], int(B) * int(X.shape[1]))
-        return SnnFcTimes.apply(X, self.weight, self.Params)      # Y[:B] of the [2B,J] op output
+            self.maxD[0] = max(self.maxD[0], int(X.shape[0]))
+            self.maxD[1] = max(self.maxD[1], int(X.shape[0]) * int(X.shape[1]))
+        return native().fc_layer(X, self.weight, self.Params, True)      # Y[:B] of the [2B,J] op output
 
 
 class SNN_conv(torch.nn.Module, _CostsMixin):
@@ -158,11 +164,7 @@ class SNN_conv(torch.nn.Module, _CostsMixin):
 
     def same_pads(self, H, W):
         """(top, bottom, left, right) of the SAME padding of an H x W image."""
-        top, bottom = _same_pad(H, self.Kh, self.Sh)
-        left, right = _same_pad(W, self.Kw, self.Sw)
-        if min(top, bottom, left, right) < 0:
-            raise ValueError("negative SAME padding: kernel smaller than stride is not supported")
-        return top, bottom, left, right
+        return _same_pads(H, W, self.Kh, self.Kw, self.Sh, self.Sw)
 
     def padded_input_buffer(self, B, H, W, device):
         """The layer's own padded input for B images of H x W (SAME mode): a tensor [B,Hp,Wp,C] that lives as
@@ -173,7 +175,7 @@ class SNN_conv(torch.nn.Module, _CostsMixin):
         layer keeps the buffers of the MAX_PADDED_BUFFERS input shapes used last; release_buffers() drops
         them all."""
         top, bottom, left, right = self.same_pads(H, W)
-        key = (B, H, W, str(device))
+        key = (B, H, W, device)
         buf = self._padded.pop(key, None)
         if buf is None:
             buf = torch.full((B, top + H + bottom, left + W + right, self.C), float(self.Params[0]),
@@ -253,10 +255,7 @@ class _Pool2d(torch.nn.Module):
     def _padded_nchw(self, input):
         """Stock-op padding (any device), for the layers that are stock ops in the reference too."""
         if self.padding == 'SAME':
-            top, bottom = _same_pad(input.shape[1], self.Kh, self.Sh)
-            left, right = _same_pad(input.shape[2], self.Kw, self.Sw)
-            if min(top, bottom, left, right) < 0:
-                raise ValueError("negative SAME padding: kernel smaller than stride is not supported")
+            top, bottom, left, right = _same_pads(input.shape[1], input.shape[2], self.Kh, self.Kw, self.Sh, self.Sw)
             input = F.pad(input, (0, 0, left, right, top, bottom), mode="constant", value=float(self.padvalue))
         return input.permute(0, 3, 1, 2)
 
@@ -273,10 +272,7 @@ class SNN_maxpool2d(_Pool2d):
         H, W = input.shape[1], input.shape[2]
         top = bottom = left = right = 0
         if self.padding == 'SAME':
-            top, bottom = _same_pad(H, self.Kh, self.Sh)
-            left, right = _same_pad(W, self.Kw, self.Sw)
-            if min(top, bottom, left, right) < 0:
-                raise ValueError("negative SAME padding: kernel smaller than stride is not supported")
+            top, bottom, left, right = _same_pads(H, W, self.Kh, self.Kw, self.Sh, self.Sw)
         nh = (H + top + bottom - self.Kh) // self.Sh + 1
         nw = (W + left + right - self.Kw) // self.Sw + 1
         next_xpad, next_offset = None, (0, 0)
