@@ -271,6 +271,35 @@ SNNTC_API int snntc_sgd_update(float* const* w, const float* const* dw, const in
                      void* stream);
 
 /* ---------------------------------------------------------------------------------------------
+ * Glue of the example training recipe (snntc-mnist.py:55-96).
+ *   snntc_encode_time        z[e] = exp(1 - image[e]) for e in [0, n)
+ *   snntc_label_loss         the loss above for integer labels[B] (int64): sample_loss[B], dtimes[B,J] (may be
+ *                            NULL) and correct[B] = 1 where the earliest output (the lowest index of equal ones)
+ *                            is the label.  A label outside [0, J) leaves NaN in its loss and gradient.
+ *   snntc_weight_cost_*      K * sum_l mean_j max(0, 1 - sum_i w_ij) + K2 * sum_l mean(w^2) over `count` weight
+ *                            tensors w[l][rows[l], cols[l]]: _sums reads the weights into the workspace, _grad
+ *                            writes (accumulate = 0) or adds (1) upstream * d cost / d w[l] into grad[l] (a NULL
+ *                            grad[l] is skipped; upstream: a device scalar, NULL = 1), both one launch per 24 tensors.
+ *   snntc_recipe_total       total = mean(sample_loss) + cost (sample_loss may be NULL: the cost alone) and, where
+ *                            correct is given, n_correct = the sum of it; after _sums, same workspace.
+ * w, grad, rows and cols are HOST arrays of `count` entries, read before the call returns; total and n_correct are
+ * device scalars.  Errors: a negative size, rows or cols < 1, a NULL required pointer -> BAD_ARGUMENT; sizes beyond
+ * INT32_MAX elements -> TOO_LARGE; a workspace below _workspace_bytes -> WORKSPACE.
+ * ------------------------------------------------------------------------------------------- */
+SNNTC_API int snntc_encode_time(const float* image, float* z, int64_t n, void* stream);
+SNNTC_API int snntc_label_loss(const float* times, const int64_t* labels, float* sample_loss, float* dtimes, int32_t* correct,
+                     int64_t B, int64_t J, void* stream);
+SNNTC_API int snntc_weight_cost_workspace_bytes(const int64_t* rows, const int64_t* cols, int64_t count, size_t* bytes);
+SNNTC_API int snntc_weight_cost_sums(const float* const* w, const int64_t* rows, const int64_t* cols, int64_t count,
+                           void* workspace, size_t workspace_bytes, void* stream);
+SNNTC_API int snntc_weight_cost_grad(const float* const* w, float* const* grad, const int64_t* rows, const int64_t* cols,
+                           int64_t count, float k, float k2, const float* upstream, int accumulate, void* workspace,
+                           size_t workspace_bytes, void* stream);
+SNNTC_API int snntc_recipe_total(const int64_t* rows, const int64_t* cols, int64_t count, float k, float k2,
+                       const float* sample_loss, const int32_t* correct, int64_t B, float* total, int64_t* n_correct,
+                       void* workspace, size_t workspace_bytes, void* stream);
+
+/* ---------------------------------------------------------------------------------------------
  * Health of the bounded wait described at snntc_fc_forward (no counterpart in the reference, whose scan
  * has one thread per neuron and nothing to wait for).
  *   snntc_scan_status(&giveups, stream)  number of wavefronts, on the current device since the process

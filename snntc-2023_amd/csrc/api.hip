@@ -466,6 +466,83 @@ int snntc_sgd_update(float* const* w, const float* const* dw, const int64_t* n, 
     return launch_sgd_update(w, dw, n, (int)count, lr, static_cast<hipStream_t>(stream));
 }
 
+int snntc_encode_time(const float* image, float* z, int64_t n, void* stream) {
+    if (n < 0) return fail(SNNTC_ERR_BAD_ARGUMENT, "snntc_encode_time: negative size");
+    if (n > 0 && (!image || !z)) return fail(SNNTC_ERR_BAD_ARGUMENT, "snntc_encode_time: null pointer");
+    return launch_encode_time(image, z, n, static_cast<hipStream_t>(stream));
+}
+
+int snntc_label_loss(const float* times, const int64_t* labels, float* sample_loss, float* dtimes, int32_t* correct,
+                     int64_t B, int64_t J, void* stream) {
+    if (B < 0 || J < 0) return fail(SNNTC_ERR_BAD_ARGUMENT, "snntc_label_loss: negative size");
+    if (B > INT32_MAX || J > INT32_MAX || B * J > INT32_MAX)
+        return fail(SNNTC_ERR_TOO_LARGE, "snntc_label_loss: more than INT32_MAX elements");
+    if (B > 0 && J > 0 && (!times || !labels || !sample_loss || !correct))
+        return fail(SNNTC_ERR_BAD_ARGUMENT, "snntc_label_loss: null pointer");
+    return launch_label_loss(times, labels, sample_loss, dtimes, correct, B, J, static_cast<hipStream_t>(stream));
+}
+
+// Checks shared by the weight-cost entry points.
+static int cost_check(const int64_t* rows, const int64_t* cols, int64_t count, const char* who) {
+    if (count < 0 || count > INT32_MAX || (count > 0 && (!rows || !cols)))
+        return fail(SNNTC_ERR_BAD_ARGUMENT, "%s: bad tensor count or null array", who);
+    for (int64_t t = 0; t < count; ++t) {
+        if (rows[t] < 1 || cols[t] < 1)
+            return fail(SNNTC_ERR_BAD_ARGUMENT, "%s: tensor %lld has no elements", who, (long long)t);
+        if (rows[t] > kInt32Max || cols[t] > kInt32Max || rows[t] * cols[t] > kInt32Max)
+            return fail(SNNTC_ERR_TOO_LARGE, "%s: tensor %lld has more than INT32_MAX elements", who, (long long)t);
+    }
+    return SNNTC_OK;
+}
+
+static int cost_workspace(const int64_t* rows, const int64_t* cols, int64_t count, const void* ws, size_t have) {
+    return check_workspace(ws, have, weight_cost_workspace_floats(rows, cols, (int)count) * sizeof(float));
+}
+
+int snntc_weight_cost_workspace_bytes(const int64_t* rows, const int64_t* cols, int64_t count, size_t* bytes) {
+    const int rc = cost_check(rows, cols, count, "snntc_weight_cost_workspace_bytes");
+    if (rc) return rc;
+    if (!bytes) return fail(SNNTC_ERR_BAD_ARGUMENT, "snntc_weight_cost_workspace_bytes: bytes is NULL");
+    *bytes = weight_cost_workspace_floats(rows, cols, (int)count) * sizeof(float);
+    return SNNTC_OK;
+}
+
+int snntc_weight_cost_sums(const float* const* w, const int64_t* rows, const int64_t* cols, int64_t count, void* workspace,
+                           size_t workspace_bytes, void* stream) {
+    int rc = cost_check(rows, cols, count, "snntc_weight_cost_sums");
+    if (!rc) rc = cost_workspace(rows, cols, count, workspace, workspace_bytes);
+    if (rc || count == 0) return rc;
+    if (!w) return fail(SNNTC_ERR_BAD_ARGUMENT, "snntc_weight_cost_sums: null array");
+    for (int64_t t = 0; t < count; ++t)
+        if (!w[t]) return fail(SNNTC_ERR_BAD_ARGUMENT, "snntc_weight_cost_sums: tensor %lld is a null pointer", (long long)t);
+    return launch_weight_cost_sums(w, rows, cols, (int)count, static_cast<float*>(workspace), static_cast<hipStream_t>(stream));
+}
+
+int snntc_weight_cost_grad(const float* const* w, float* const* grad, const int64_t* rows, const int64_t* cols, int64_t count,
+                           float k, float k2, const float* upstream, int accumulate, void* workspace, size_t workspace_bytes,
+                           void* stream) {
+    int rc = cost_check(rows, cols, count, "snntc_weight_cost_grad");
+    if (!rc) rc = cost_workspace(rows, cols, count, workspace, workspace_bytes);
+    if (rc || count == 0) return rc;
+    if (!w || !grad) return fail(SNNTC_ERR_BAD_ARGUMENT, "snntc_weight_cost_grad: null array");
+    for (int64_t t = 0; t < count; ++t)
+        if (!w[t]) return fail(SNNTC_ERR_BAD_ARGUMENT, "snntc_weight_cost_grad: tensor %lld is a null pointer", (long long)t);
+    return launch_weight_cost_grad(w, grad, rows, cols, (int)count, k, k2, upstream, accumulate != 0,
+                                   static_cast<float*>(workspace), static_cast<hipStream_t>(stream));
+}
+
+int snntc_recipe_total(const int64_t* rows, const int64_t* cols, int64_t count, float k, float k2, const float* sample_loss,
+                       const int32_t* correct, int64_t B, float* total, int64_t* n_correct, void* workspace,
+                       size_t workspace_bytes, void* stream) {
+    int rc = cost_check(rows, cols, count, "snntc_recipe_total");
+    if (!rc) rc = cost_workspace(rows, cols, count, workspace, workspace_bytes);
+    if (rc) return rc;
+    if (B < 0 || B > INT32_MAX || !total || (correct && (!n_correct || !sample_loss)))
+        return fail(SNNTC_ERR_BAD_ARGUMENT, "snntc_recipe_total: bad argument");
+    return launch_recipe_total(rows, cols, (int)count, k, k2, sample_loss, correct, B, total, n_correct,
+                               static_cast<float*>(workspace), static_cast<hipStream_t>(stream));
+}
+
 int snntc_scan_status(int64_t* giveups, void* stream) {
     if (!giveups) return fail(SNNTC_ERR_BAD_ARGUMENT, "snntc_scan_status: giveups is NULL");
     return read_scan_giveups(giveups, static_cast<hipStream_t>(stream));

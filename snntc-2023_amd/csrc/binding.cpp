@@ -19,6 +19,7 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/autograd.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -46,7 +47,8 @@ using torch::autograd::variable_list;
     F(snntc_cv_forward_chained) F(snntc_cv_forward_workspace_bytes) F(snntc_cv_backward_cropped)                   \
     F(snntc_cv_backward_workspace_bytes) F(snntc_softmax_time_loss) F(snntc_sgd_update)                            \
     F(snntc_min_pool_forward) F(snntc_min_pool_forward_chained) F(snntc_min_pool_backward)                         \
-    F(snntc_pad_time_forward) F(snntc_pad_time_backward)
+    F(snntc_pad_time_forward) F(snntc_pad_time_backward) F(snntc_encode_time) F(snntc_label_loss)                  \
+    F(snntc_weight_cost_workspace_bytes) F(snntc_weight_cost_sums) F(snntc_weight_cost_grad) F(snntc_recipe_total)
 
 struct Library {
 #define SNNTC_FIELD(f) decltype(&::f) f = nullptr;
@@ -510,6 +512,144 @@ void sgd_update(const std::vector<Tensor>& ws, const std::vector<Tensor>& gs, fl
     check(lib.snntc_sgd_update(wp.data(), gp.data(), n.data(), (int64_t)n.size(), lr, stream_of(ws[0])));
 }
 
+// ---- the example training recipe -------------------------------------------------------------------------------------
+
+Tensor encode_time(const Tensor& image) {
+    const Tensor x = image.contiguous();
+    const c10::DeviceGuard guard(x.device());
+    const Tensor z = empty(x, x.sizes());
+    check(lib.snntc_encode_time(f32(x), f32(z), x.numel(), stream_of(x)));
+    return z;
+}
+
+// Host arrays of the weight tensors the constraint cost runs over, and its device scratch.
+struct CostArgs {
+    std::vector<const float*> w;
+    std::vector<int64_t> rows, cols;
+    Tensor ws;
+    explicit CostArgs(const std::vector<Tensor>& weights) {
+        for (const Tensor& t : weights) {
+            w.push_back(f32(t));
+            rows.push_back(t.size(0));
+            cols.push_back(t.size(1));
+        }
+    }
+    int64_t count() const { return (int64_t)w.size(); }
+    void sums(const Tensor& like, void* stream) {
+        size_t need = 0;
+        check(lib.snntc_weight_cost_workspace_bytes(rows.data(), cols.data(), count(), &need));
+        ws = scratch(like, need);
+        check(lib.snntc_weight_cost_sums(w.data(), rows.data(), cols.data(), count(), ws.data_ptr(), ws.numel(), stream));
+    }
+    void grad(float* const* g, float k, float k2, const float* upstream, bool accumulate, void* stream) {
+        check(lib.snntc_weight_cost_grad(w.data(), g, rows.data(), cols.data(), count(), k, k2, upstream, accumulate, ws.data_ptr(),
+                                         ws.numel(), stream));
+    }
+};
+
+struct CostNode : public Node {
+    std::vector<SavedVariable> weights;
+    Tensor ws;
+    float k, k2;
+    std::string name() const override { return "ConstraintCostBackward"; }
+    void release_variables() override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        for (SavedVariable& w : weights) w.reset_data();
+        ws.reset();
+    }
+    variable_list apply(variable_list&& grads) override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        variable_list out(weights.size());
+        if (!grads[0].defined()) return out;
+        std::vector<Tensor> w;
+        for (SavedVariable& s : weights) w.push_back(s.unpack());
+        at::AutoGradMode no_grad(false);
+        const Tensor up = grads[0].contiguous();
+        const c10::DeviceGuard guard(up.device());
+        CostArgs args(w);
+        args.ws = ws;
+        std::vector<float*> g;
+        for (size_t i = 0; i < w.size(); ++i) {
+            if (task_should_compute_output(i)) out[i] = empty(w[i], w[i].sizes());
+            g.push_back(f32(out[i]));
+        }
+        args.grad(g.data(), k, k2, f32(up), false, stream_of(up));
+        return out;
+    }
+};
+
+// The weight-constraint cost of contiguous float32 weight matrices on one device, differentiable.
+Tensor constraint_cost(const std::vector<Tensor>& weights, float k, float k2) {
+    const c10::DeviceGuard guard(weights[0].device());
+    void* stream = stream_of(weights[0]);
+    CostArgs args(weights);
+    Tensor total;
+    bool grad = false;
+    {
+        at::AutoGradMode no_grad(false);
+        args.sums(weights[0], stream);
+        total = empty(weights[0], {});
+        check(lib.snntc_recipe_total(args.rows.data(), args.cols.data(), args.count(), k, k2, nullptr, nullptr, 0, f32(total), nullptr,
+                                     args.ws.data_ptr(), args.ws.numel(), stream));
+    }
+    for (const Tensor& w : weights) grad = grad || wants_grad(w);
+    if (!grad) return total;
+    std::shared_ptr<CostNode> node(new CostNode(), torch::autograd::deleteNode);
+    torch::autograd::edge_list edges;
+    for (const Tensor& w : weights) {
+        edges.push_back(torch::autograd::impl::gradient_edge(w));
+        node->weights.emplace_back(w, false);
+    }
+    node->set_next_edges(std::move(edges));
+    node->ws = args.ws; node->k = k; node->k2 = k2;
+    return with_history(total, node);
+}
+
+// Loss, cost, count of correct samples and -- with `train` -- every gradient of one step: the data gradients
+// through the engine from the loss kernel's dtimes, then the cost's added into each weight's .grad.
+LossOut recipe_step(const Tensor& pred_in, const Tensor& labels_in, const std::vector<Tensor>& weights, float k, float k2, bool train) {
+    const Tensor pred = dev_f32(pred_in, "predictions", 2);
+    const int64_t B = pred.size(0), J = pred.size(1);
+    const c10::DeviceGuard guard(pred.device());
+    void* stream = stream_of(pred);
+    Tensor sample_loss, dtimes, correct, total, n_correct;
+    CostArgs args(weights);
+    {
+        at::AutoGradMode no_grad(false);
+        const Tensor labels = labels_in.contiguous();
+        sample_loss = empty(pred, {B});
+        correct = at::empty({B}, pred.options().dtype(at::kInt));
+        if (train) dtimes = empty(pred, pred.sizes());
+        check(lib.snntc_label_loss(f32(pred), static_cast<int64_t*>(labels.data_ptr()), f32(sample_loss), f32(dtimes),
+                                   static_cast<int32_t*>(correct.data_ptr()), B, J, stream));
+    }
+    if (train) torch::autograd::backward({pred}, {dtimes});
+    at::AutoGradMode no_grad(false);
+    args.sums(pred, stream);
+    total = empty(pred, {});
+    n_correct = at::empty({}, pred.options().dtype(at::kLong));
+    check(lib.snntc_recipe_total(args.rows.data(), args.cols.data(), args.count(), k, k2, f32(sample_loss),
+                                 static_cast<int32_t*>(correct.data_ptr()), B, f32(total), static_cast<int64_t*>(n_correct.data_ptr()),
+                                 args.ws.data_ptr(), args.ws.numel(), stream));
+    if (train) {
+        std::vector<float*> g;
+        std::vector<Tensor> keep;
+        for (const Tensor& w : weights) {
+            Tensor& wg = w.mutable_grad();
+            if (!w.requires_grad()) { g.push_back(nullptr); continue; }
+            if (!wg.defined()) {
+                wg = at::zeros_like(w);
+            } else if (!(wg.is_cuda() && wg.scalar_type() == at::kFloat && wg.is_contiguous() && wg.sizes() == w.sizes())) {
+                wg = wg.to(w.options()).contiguous();
+            }
+            written_behind_autograd(wg);
+            g.push_back(f32(wg));
+        }
+        args.grad(g.data(), k, k2, nullptr, true, stream);
+    }
+    return LossOut{total, n_correct};
+}
+
 // ---- Python arguments ----------------------------------------------------------------------------------------------
 
 const Tensor& tensor_arg(PyObject* o, const char* name) {
@@ -829,6 +969,60 @@ SNNTC_METHOD(py_sgd_update) {
     END_HANDLE_TH_ERRORS
 }
 
+std::vector<Tensor> tensor_list(PyObject* o, const char* name) {
+    TORCH_CHECK_TYPE(PyList_Check(o), name, " must be a list");
+    std::vector<Tensor> v;
+    for (Py_ssize_t i = 0; i < PyList_GET_SIZE(o); ++i) v.push_back(tensor_arg(PyList_GET_ITEM(o, i), name));
+    return v;
+}
+
+// encode_time(image) -> exp(1 - image) for a float32 device tensor
+SNNTC_METHOD(py_encode_time) {
+    HANDLE_TH_ERRORS
+    arity(n, 1, "encode_time");
+    const Tensor x = tensor_arg(a[0], "image");
+    Tensor z;
+    {
+        NoGil nogil;
+        at::AutoGradMode no_grad(false);
+        z = encode_time(x);
+    }
+    return wrap(z);
+    END_HANDLE_TH_ERRORS
+}
+
+// constraint_cost(weights, k, k2) -> scalar, differentiable
+SNNTC_METHOD(py_constraint_cost) {
+    HANDLE_TH_ERRORS
+    arity(n, 3, "constraint_cost");
+    const std::vector<Tensor> w = tensor_list(a[0], "weights");
+    const float k = float_arg(a[1]), k2 = float_arg(a[2]);
+    Tensor out;
+    {
+        NoGil nogil;
+        out = constraint_cost(w, k, k2);
+    }
+    return wrap(out);
+    END_HANDLE_TH_ERRORS
+}
+
+// recipe_step(predictions, labels, weights, k, k2, train) -> (loss, number of correct samples)
+SNNTC_METHOD(py_recipe_step) {
+    HANDLE_TH_ERRORS
+    arity(n, 6, "recipe_step");
+    const Tensor p = tensor_arg(a[0], "predictions"), l = tensor_arg(a[1], "labels");
+    const std::vector<Tensor> w = tensor_list(a[2], "weights");
+    const float k = float_arg(a[3]), k2 = float_arg(a[4]);
+    const bool train = bool_arg(a[5]);
+    LossOut r;
+    {
+        NoGil nogil;
+        r = recipe_step(p, l, w, k, k2, train);
+    }
+    return wrap2(r.loss, r.grad);
+    END_HANDLE_TH_ERRORS
+}
+
 // bind(path, SnntcLibraryError, SnntcError, params_array): looks the C ABI up in the library loaded from `path`
 SNNTC_METHOD(py_bind) {
     HANDLE_TH_ERRORS
@@ -855,7 +1049,8 @@ SNNTC_METHOD(py_bind) {
 PyMethodDef g_methods[] = {SNNTC_ENTRY(bind), SNNTC_ENTRY(fc_forward), SNNTC_ENTRY(fc_layer), SNNTC_ENTRY(fc_backward),
                            SNNTC_ENTRY(cv_forward), SNNTC_ENTRY(cv_layer), SNNTC_ENTRY(cv_same), SNNTC_ENTRY(cv_backward),
                            SNNTC_ENTRY(min_pool), SNNTC_ENTRY(min_pool_layer), SNNTC_ENTRY(pad_layer), SNNTC_ENTRY(time_loss),
-                           SNNTC_ENTRY(loss_layer), SNNTC_ENTRY(sgd_update), {nullptr, nullptr, 0, nullptr}};
+                           SNNTC_ENTRY(loss_layer), SNNTC_ENTRY(sgd_update), SNNTC_ENTRY(encode_time), SNNTC_ENTRY(constraint_cost),
+                           SNNTC_ENTRY(recipe_step), {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_binding", "Native host path of the SNN-TC ops.", -1, g_methods,
                         nullptr, nullptr, nullptr, nullptr};

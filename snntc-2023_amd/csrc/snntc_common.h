@@ -244,4 +244,16 @@ int launch_sgd_update(float* const* w, const float* const* dw, const int64_t* n,
 int launch_softmax_time_loss(const float* times, const float* label, float* sample_loss, float* dtimes,
                              int64_t B, int64_t J, hipStream_t stream);
 
+// Glue of the example training recipe (recipe.hip).
+int launch_encode_time(const float* image, float* z, int64_t n, hipStream_t stream);
+int launch_label_loss(const float* times, const int64_t* labels, float* sample_loss, float* dtimes, int32_t* correct,
+                      int64_t B, int64_t J, hipStream_t stream);
+size_t weight_cost_workspace_floats(const int64_t* rows, const int64_t* cols, int count);
+int launch_weight_cost_sums(const float* const* w, const int64_t* rows, const int64_t* cols, int count, float* ws,
+                            hipStream_t stream);
+int launch_weight_cost_grad(const float* const* w, float* const* grad, const int64_t* rows, const int64_t* cols, int count,
+                            float k, float k2, const float* upstream, bool accumulate, float* ws, hipStream_t stream);
+int launch_recipe_total(const int64_t* rows, const int64_t* cols, int count, float k, float k2, const float* sample_loss,
+                        const int32_t* correct, int64_t B, float* total, int64_t* n_correct, float* ws, hipStream_t stream);
+
 }  // namespace snntc

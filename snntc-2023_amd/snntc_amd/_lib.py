@@ -36,6 +36,8 @@ EXPORTS = (
     "snntc_softmax_time_loss", "snntc_sgd_update",
     "snntc_min_pool_forward", "snntc_min_pool_backward",
     "snntc_pad_time_forward", "snntc_pad_time_backward",
+    "snntc_encode_time", "snntc_label_loss", "snntc_weight_cost_workspace_bytes", "snntc_weight_cost_sums",
+    "snntc_weight_cost_grad", "snntc_recipe_total",
     "snntc_scan_status", "snntc_debug_set_scan_wait_polls",
     "snntc_profile_enable", "snntc_profile_collect", "snntc_profile_entry",
 )
@@ -119,6 +121,14 @@ def load():
     lib.snntc_min_pool_backward.argtypes = [vp, vp, vp] + [i64] * 12 + [vp]
     lib.snntc_pad_time_forward.argtypes = [vp, vp] + [i64] * 8 + [c.c_float, vp]
     lib.snntc_pad_time_backward.argtypes = [vp, vp] + [i64] * 8 + [vp]
+    pi64 = c.POINTER(i64)
+    lib.snntc_encode_time.argtypes = [vp, vp, i64, vp]
+    lib.snntc_label_loss.argtypes = [vp, vp, vp, vp, vp, i64, i64, vp]
+    lib.snntc_weight_cost_workspace_bytes.argtypes = [pi64, pi64, i64, c.POINTER(sz)]
+    lib.snntc_weight_cost_sums.argtypes = [c.POINTER(vp), pi64, pi64, i64, vp, sz, vp]
+    lib.snntc_weight_cost_grad.argtypes = [c.POINTER(vp), c.POINTER(vp), pi64, pi64, i64, c.c_float, c.c_float, vp, c.c_int,
+                                           vp, sz, vp]
+    lib.snntc_recipe_total.argtypes = [pi64, pi64, i64, c.c_float, c.c_float, vp, vp, i64, vp, vp, vp, sz, vp]
     lib.snntc_scan_status.argtypes = [c.POINTER(i64), vp]
     lib.snntc_debug_set_scan_wait_polls.argtypes = [c.c_int]
     lib.snntc_profile_enable.argtypes = [c.c_int]
