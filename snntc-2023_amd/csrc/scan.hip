@@ -8,11 +8,9 @@
 // |ysum| > x*|wsum| with the product rounded on its own, and y = ysum * (1/wsum).
 //
 // Kernels, by launch size (launch_scan_lds picks):
-//   scan_filter_kernel     large and mid-sized launches: weight slice in LDS, one or two neurons per
-//                          lane, and the tests of a step skipped wherever a margin test on a whole
-//                          chunk of eight inputs proves that none of them can close the set;
-//   scan_lds_kernel        small launches (a couple of wavefronts per SIMD): weight slice in LDS, every
-//                          step with its tests, written for latency;
+//   scan_filter_kernel     weight slice in LDS, one, two or four neurons per lane, and the tests of a step skipped
+//                          wherever a margin test on a whole chunk of eight inputs proves that none of
+//                          them can close the set;
 //   scan_lds_split_kernel  fewer work items than CUs: one item per workgroup, its weights gathered
 //                          into LDS in scan order first, then one wavefront accumulating and the
 //                          others sharing the item's tests;
@@ -148,10 +146,8 @@ constexpr int LDS_SCAN_THREADS = 1024;
 constexpr int LDS_SCAN_BYTES = 160 * 1024;
 // The widest slice that fits is taken: the register budget allows one 16-wave workgroup per CU anyway,
 // and fewer slices re-read the sorted rows less often.
-// Behind the slice: 64 bytes for a reduction and room for the chunk buffers of at least four
-// wavefronts (scan_filter_kernel: 64 bytes per segment of a wavefront, at most 8 segments).
-constexpr int FILTER_XBUF_SEG_BYTES = 2 * CHUNK * (int)sizeof(float);
-constexpr int LDS_SCAN_TARGET = 160 * 1024 - 64 - 4 * 8 * FILTER_XBUF_SEG_BYTES;
+constexpr int FILTER_RED_BYTES = 64;                       // behind the slice: one float per wavefront for a reduction
+constexpr int LDS_SCAN_TARGET = LDS_SCAN_BYTES - FILTER_RED_BYTES;
 
 struct Chunk {
     float x[CHUNK];
@@ -162,6 +158,7 @@ struct Chunk {
 // scalar chunk offset and a per-lane byte offset that never changes during a scan.  No per-lane
 // address arithmetic is left, so issuing the next loads never has to wait for those in flight.
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
 struct RowSource {
     __amdgpu_buffer_rsrc_t xs, pr;
@@ -184,18 +181,6 @@ __device__ __forceinline__ void load_chunk_flat(Chunk& c, const float* __restric
     c.x[4] = b.x; c.x[5] = b.y; c.x[6] = b.z; c.x[7] = b.w;
     c.p[0] = pa.x; c.p[1] = pa.y; c.p[2] = pa.z; c.p[3] = pa.w;
     c.p[4] = pb.x; c.p[5] = pb.y; c.p[6] = pb.z; c.p[7] = pb.w;
-}
-
-__device__ __forceinline__ void load_chunk(Chunk& c, const RowSource& src, int lane_bytes, int k) {
-    const u32x4 a = __builtin_amdgcn_raw_buffer_load_b128(src.xs, lane_bytes, k * 4, 0);
-    const u32x4 b = __builtin_amdgcn_raw_buffer_load_b128(src.xs, lane_bytes + 16, k * 4, 0);
-    const u32x4 pa = __builtin_amdgcn_raw_buffer_load_b128(src.pr, lane_bytes, k * 4, 0);
-    const u32x4 pb = __builtin_amdgcn_raw_buffer_load_b128(src.pr, lane_bytes + 16, k * 4, 0);
-    c.x[0] = __uint_as_float(a.x); c.x[1] = __uint_as_float(a.y); c.x[2] = __uint_as_float(a.z);
-    c.x[3] = __uint_as_float(a.w); c.x[4] = __uint_as_float(b.x); c.x[5] = __uint_as_float(b.y);
-    c.x[6] = __uint_as_float(b.z); c.x[7] = __uint_as_float(b.w);
-    c.p[0] = (int)pa.x; c.p[1] = (int)pa.y; c.p[2] = (int)pa.z; c.p[3] = (int)pa.w;
-    c.p[4] = (int)pb.x; c.p[5] = (int)pb.y; c.p[6] = (int)pb.z; c.p[7] = (int)pb.w;
 }
 
 #define SNNTC_SCAN_COUNT "v_add_u32_e32 %[kcnt], 1, %[kcnt]\n"
@@ -255,6 +240,59 @@ __device__ __forceinline__ void scan_chunk_vector(float& wsum, float& ysum, floa
                      SNNTC_VSCAN_STEP(3) SNNTC_VSCAN_STEP(4) SNNTC_VSCAN_STEP(5) SNNTC_VSCAN_STEP(6)
                      SNNTC_VSCAN_STEP(7) SNNTC_VSCAN_EPILOGUE
                      : SNNTC_VSCAN_STATE : SNNTC_VSCAN_INPUTS : "vcc", "scc");
+}
+
+// The same for scans known to be in the plain state with ysum - x*wsum above `slack` (many roundings of the sums
+// of a chunk): at five instructions per input.  A lane leaves where ysum - x*wsum falls to slack, before it
+// consumes x.  If its weight sum is positive then, it has fired (the value before x was above slack), and
+// the reference closes it there exactly if ysum <= x*wsum, with x = x_exit; in every other case the caller
+// steps the chunk through with all tests.  A lane that stays keeps the plain state: a negative weight sum with
+// ysum - x*wsum > 0 has not fired.
+#define SNNTC_CLOSE_STEP(U)                                                  \
+    "v_mov_b32_e32 %[xe], %[x" #U "]\n"                                      \
+    "v_fma_f32 %[t], %[x" #U "], %[wsum], %[slack]\n"                        \
+    "v_cmpx_gt_f32_e32 vcc, %[ysum], %[t]\n"                                \
+    "v_add_f32_e32 %[wsum], %[wsum], %[w" #U "]\n"                          \
+    "v_fmac_f32_e32 %[ysum], %[x" #U "], %[w" #U "]\n"
+#define SNNTC_CLOSE_EPILOGUE                         \
+    "v_mov_b32_e32 %[stays], 1\n"                    \
+    "s_mov_b64 exec, %[save]\n"
+// Returns the lanes that left.  (As a vector flag turned into a mask: a statement with vector and scalar results
+// has only divergent values for the compiler, and the masks would move to vector registers.)
+template <bool COUNT>
+__device__ __forceinline__ uint64_t close_chunk_vector(float& wsum, float& ysum, int& kcnt, float& x_exit, uint64_t run,
+                                                       const float (&x)[CHUNK], const float (&w)[CHUNK], float slack) {
+    uint64_t saved_exec;
+    float t;
+    int stays = 0;
+    x_exit = 0.0f;
+    if (COUNT)
+        asm volatile(SNNTC_VSCAN_PROLOGUE SNNTC_CLOSE_STEP(0) SNNTC_SCAN_COUNT SNNTC_CLOSE_STEP(1) SNNTC_SCAN_COUNT
+                     SNNTC_CLOSE_STEP(2) SNNTC_SCAN_COUNT SNNTC_CLOSE_STEP(3) SNNTC_SCAN_COUNT SNNTC_CLOSE_STEP(4)
+                     SNNTC_SCAN_COUNT SNNTC_CLOSE_STEP(5) SNNTC_SCAN_COUNT SNNTC_CLOSE_STEP(6) SNNTC_SCAN_COUNT
+                     SNNTC_CLOSE_STEP(7) SNNTC_SCAN_COUNT SNNTC_CLOSE_EPILOGUE
+                     : [wsum] "+v"(wsum), [ysum] "+v"(ysum), [kcnt] "+v"(kcnt), [xe] "+v"(x_exit), [stays] "+v"(stays),
+                       [save] "=&s"(saved_exec), [t] "=&v"(t)
+                     : SNNTC_SCAN_INPUTS("v", x), [slack] "v"(slack) : "vcc", "scc");
+    else
+        asm volatile(SNNTC_VSCAN_PROLOGUE SNNTC_CLOSE_STEP(0) SNNTC_CLOSE_STEP(1) SNNTC_CLOSE_STEP(2) SNNTC_CLOSE_STEP(3)
+                     SNNTC_CLOSE_STEP(4) SNNTC_CLOSE_STEP(5) SNNTC_CLOSE_STEP(6) SNNTC_CLOSE_STEP(7) SNNTC_CLOSE_EPILOGUE
+                     : [wsum] "+v"(wsum), [ysum] "+v"(ysum), [xe] "+v"(x_exit), [stays] "+v"(stays),
+                       [save] "=&s"(saved_exec), [t] "=&v"(t)
+                     : SNNTC_SCAN_INPUTS("v", x), [slack] "v"(slack) : "vcc", "scc");
+    return run & __builtin_amdgcn_ballot_w64(stays == 0);
+}
+
+// One step with all tests (an input behind the full chunks of a row).
+__device__ __forceinline__ void scan_step_vector(float& wsum, float& ysum, float& ya, float& yg, int& kcnt, uint64_t run,
+                                                 float x, float w) {
+    uint64_t saved_exec;
+    float t;
+    const float inf = INFINITY;
+    asm volatile(SNNTC_VSCAN_PROLOGUE SNNTC_VSCAN_STEP(0) SNNTC_SCAN_COUNT "s_mov_b64 exec, %[save]\n"
+                 : [wsum] "+v"(wsum), [ysum] "+v"(ysum), [ya] "+v"(ya), [yg] "+v"(yg), [kcnt] "+v"(kcnt),
+                   [save] "=&s"(saved_exec), [t] "=&v"(t)
+                 : [run] "s"(run), [inf] "v"(inf), [x0] "v"(x), [w0] "v"(w) : "vcc", "scc");
 }
 
 // Eight inputs added to the running sums of the lanes in `run`, no tests: what a wavefront does for
@@ -357,118 +395,6 @@ __device__ __forceinline__ float fill_weight_slice(float* __restrict__ wl, const
         }
     }
     return amax;
-}
-
-// Launches with at most a couple of wavefronts per SIMD, where nothing hides a stall: workgroups of
-// at most four wavefronts (so that the work spreads over the chip), one neuron per lane, seven chunks
-// of (x, row) in flight through buffer loads, and the step-by-step block for every chunk (the
-// filtered kernel below pays a fixed price per work item that such small launches do not win back).
-constexpr int LOW_LATENCY_THREADS = 256;
-
-template <int COLS, bool WANT_K>
-__global__ void __launch_bounds__(LOW_LATENCY_THREADS)
-scan_lds_kernel(const float* __restrict__ sorted, const int32_t* __restrict__ perm,
-                const int32_t* __restrict__ n_real, const float* __restrict__ w, float* __restrict__ y_out,
-                float* __restrict__ rcp_out, int32_t* __restrict__ k_out, int S, int I, int stride, int J,
-                int n_slices, int n_groups, NeuronParams np, TimeCopy copy) {
-    extern __shared__ __align__(16) float wl[];                          // [I + bias][COLS]
-    constexpr int SEGS = kWave / COLS;                     // segments per wavefront
-    const int WAVES = blockDim.x / kWave;                  // 1..4, chosen by the launcher
-    // slice-major over XCD-contiguous ids: the workgroups of one XCD share a few weight slices
-    const int block = xcd_contiguous(blockIdx.x, gridDim.x);
-    const int slice = block / n_groups;
-    const int group = block - slice * n_groups;
-    const int j0 = slice * COLS;
-    const int rows = I + np.bias;
-
-    fill_weight_slice<COLS>(wl, w, rows, J, j0);
-    __syncthreads();
-
-    const int lane = threadIdx.x % kWave;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int sub = lane / COLS, col = lane - sub * COLS;
-    const int j = j0 + col;
-    const float* __restrict__ wcol = wl + col;
-    const int last_chunk = stride - CHUNK;                 // start of the last readable chunk of a row
-
-    for (int item = group * WAVES + wave; item * SEGS < S; item += n_groups * WAVES) {
-        const int seg_raw = item * SEGS + sub;
-        const bool live = seg_raw < S && j < J;
-        const int seg = seg_raw < S ? seg_raw : S - 1;      // idle lanes shadow a valid segment
-        const float* __restrict__ xs = sorted + (size_t)seg * stride;
-        const int32_t* __restrict__ pr = perm + (size_t)seg * stride;
-        const int seg0 = __builtin_amdgcn_readfirstlane(item * SEGS);
-        const int n_segs = S - seg0 < SEGS ? S - seg0 : SEGS;
-        const RowSource rows_of_item = make_row_source(sorted + (size_t)seg0 * stride, perm + (size_t)seg0 * stride,
-                                                       n_segs * stride * (int)sizeof(float));
-        const int lane_bytes = (seg - seg0) * stride * (int)sizeof(float);
-        const int n = live ? n_real[seg] : 0;
-        const int n_full = n & ~(CHUNK - 1);
-
-        float wsum = -np.theta, ysum = 0.0f, ya = 0.0f;
-        bool fired0 = false;
-        if (np.bias) {
-            const float wb = wcol[I * COLS];
-            wsum += wb;
-            ysum = np.biasvolt * wb;
-            ya = wsum < 0.0f ? -ysum : ysum;
-            fired0 = ya > fabsf(wsum) * np.biasvolt;
-        }
-        uint64_t closed = 0;
-        int kcnt = 0;
-        float yg = fired0 ? ya : INFINITY;                  // gate value of the step block
-
-        // NBUF chunks of (x, row) are held: c is consumed, c+1 feeds the LDS reads, up to c+NBUF-1
-        // are being fetched.  The phase loop is unrolled so that buffer indices are compile-time.
-        constexpr int NBUF = 8, AHEAD = NBUF - 1;
-        Chunk xp[NBUF];
-        float wv[2][CHUNK];
-#pragma unroll
-        for (int b = 0; b < AHEAD; ++b) load_chunk(xp[b], rows_of_item, lane_bytes, b * CHUNK <= last_chunk ? b * CHUNK : 0);
-#pragma unroll
-        for (int u = 0; u < CHUNK; ++u) wv[0][u] = wcol[xp[0].p[u] * COLS];
-
-        // The body is one straight block per NBUF chunks (no exit between phases: a phase whose lanes
-        // are all done runs with an empty EXEC), which lets the compiler keep all seven chunks in flight.
-        for (int k0 = 0;; k0 += NBUF * CHUNK) {
-#pragma unroll
-            for (int ph = 0; ph < NBUF; ++ph) {
-                __builtin_amdgcn_sched_barrier(0);          // keep each phase's loads and reads in it
-                const int k = k0 + ph * CHUNK;
-                const uint64_t run = __ballot(k < n_full) & ~closed;
-                const int kn = k + AHEAD * CHUNK;
-                load_chunk(xp[(ph + AHEAD) % NBUF], rows_of_item, lane_bytes, kn <= last_chunk ? kn : 0);
-#pragma unroll
-                for (int u = 0; u < CHUNK; ++u) wv[(ph + 1) % 2][u] = wcol[xp[(ph + 1) % NBUF].p[u] * COLS];
-                scan_chunk_vector<WANT_K>(wsum, ysum, ya, yg, kcnt, closed, run, xp[ph % NBUF].x, wv[ph % 2]);
-            }
-            if ((__ballot(k0 + NBUF * CHUNK < n_full) & ~closed) == 0) break;
-        }
-
-        // per-lane epilogue: up to CHUNK-1 trailing inputs, then the output
-        if (live) {
-            LaneState s;
-            s.wsum = wsum; s.ysum = ysum; s.wa = fabsf(wsum); s.ya = ya;
-            const bool was_closed = (closed >> lane) & 1;
-            s.fired = was_closed || yg < INFINITY;
-            bool open = !was_closed;
-            for (int k = n_full; k < n && open; ++k) {
-                open = scan_step(s, xs[k], wcol[pr[k] * COLS]);
-                if (WANT_K && open) ++kcnt;
-            }
-            float y = np.max_time, r = 0.0f;
-            if (s.fired) {
-                r = 1.0f / s.wsum;
-                y = s.ysum * r;
-                if (y >= np.max_time) { y = np.max_time; r = 0.0f; }
-            }
-            const size_t o = (size_t)seg * J + j;
-            y_out[o] = y;
-            rcp_out[o] = r;
-            if (copy.dst) copy.dst[time_copy_pixel(copy, seg) * J + j] = y;
-            if (WANT_K) k_out[o] = (s.fired && r != 0.0f) ? kcnt : -1;
-        }
-    }
 }
 
 // Launches of a few dozen work items (the 10-wide head of a classifier): one item per workgroup,
@@ -808,14 +734,18 @@ __device__ __forceinline__ void read_columns(const float* p, float (&out)[CH]) {
 }
 // The same through a pointer that is known to point into LDS.
 typedef float lds_float2 __attribute__((ext_vector_type(2)));
+typedef float lds_float4 __attribute__((ext_vector_type(4)));
 template <int CH>
 __device__ __forceinline__ void read_columns(__attribute__((address_space(3))) const float* p, float (&out)[CH]) {
-    static_assert(CH == 1 || CH == 2, "one or two columns per lane");
+    static_assert(CH == 1 || CH == 2 || CH == 4, "one, two or four columns per lane");
     if constexpr (CH == 1) {
         out[0] = *p;
-    } else {
+    } else if constexpr (CH == 2) {
         const lds_float2 v = *reinterpret_cast<__attribute__((address_space(3))) const lds_float2*>(p);
         out[0] = v.x; out[1] = v.y;
+    } else {
+        const lds_float4 v = *reinterpret_cast<__attribute__((address_space(3))) const lds_float4*>(p);
+        out[0] = v.x; out[1] = v.y; out[2] = v.z; out[3] = v.w;
     }
 }
 
@@ -849,49 +779,45 @@ __device__ __forceinline__ void read_columns(__attribute__((address_space(3))) c
 // all but contrived cases, and otherwise walks on step by step.  NaN sums never pass a
 // reference test and never close; a NaN bound or threshold fails the fast test.
 //
-// CH (1 or 2) adjacent neurons per lane: one row address and one 4- or 8-byte LDS read serve CH
-// scans, and a wavefront covers 64*CH/COLS segments.  Workgroups, slices and items are laid out as
-// in scan_lds_kernel, with up to 16 wavefronts per workgroup.
+// CH (1, 2 or 4) adjacent neurons per lane: one row address, one input time and one 4-, 8- or 16-byte LDS read
+// serve CH scans, and a wavefront covers 64*CH/COLS segments.  What bounds the loop is vector issue (127
+// instructions per chunk of 4 x 64 neurons) and, under it, the power limit: the same instruction stream runs
+// 16 % slower on random weights than on zeros.  Per 64 neuron-steps, 16 wavefronts per CU: 21.2 / 15.7 / 12.7
+// clocks with one, two and four neurons per lane (17.8 for the two-neuron form that tracked the smallest
+// weight sum of a chunk and passed the input times through LDS).  3x3 patches of 64 channels to 64 neurons,
+// 65 536 segments: 310 -> 238 us; 128 -> 128 channels on 28x28, 32 images: 472 -> 416; 256 -> 256 on 14x14: 555 -> 440;
+// dense 784 -> 800 at 4096 rows: 379 -> 302.
 // ---------------------------------------------------------------------------------------------
-constexpr float FILTER_REL = 0x1p-22f;                    // 4u
-constexpr float FILTER_W = 9.0f * 0x1p-22f;               // 36u, times max|w| of the slice
 // The fast loop does not evaluate the eight t of a chunk: it bounds them from the last one.  With the
 // sums as computed, D_u = ysum_u - x_u*wsum_u obeys  D_{u-1} = D_u + (x_u - x_{u-1})*wsum_{u-1} - e_u,
 // |e_u| <= u*(|ysum_u| + x_u*|wsum_u|) (the roundings of the two sums), hence for every u of the chunk
 //     D_u >= D_7 + (x_7 - x_0) * min(0, wsum_0 .. wsum_7) - 7 * max|e|:
 // D only falls while the weight sum is positive, and where the sum is negative it can have been lower
-// earlier by at most that much.  The lane keeps the smallest weight sum of the chunk (one three-way
-// minimum per two inputs, started at zero), evaluates t_7 and accepts the chunk if
-//     fma(x_7 - x_0, min, t_7)  >  thr + 12u * 1.01 * (|ysum_7| + x_7*|wsum_7| + 14*x_7*max|w|)
-// (the second term covers the seven e_u, the roundings of t_u, t_7, x_7 - x_0 and of the bound itself;
-// sums inside the chunk differ from the final ones by at most seven inputs).  Every t_u then exceeds
-// thr, which is the condition above.  With a weight sum that stays positive the bound is t_7 itself, so
-// a chunk fails exactly where it failed before, give or take the wider margin (a few 10^-6 of the sums).
-// Two additions, one half of a minimum per input instead of three and a half instructions.
-constexpr float FILTER_END_Y = 0x1p-19f;                  // 32u >= 4u + 12.2u, times |ysum_7|
-constexpr float FILTER_END_XW = 0x1p-20f;                 // 16u >= 12.2u, times x_7 * |wsum_7|
-constexpr float FILTER_END_W = 0x1p-16f;                  // 256u >= 36u + 170u, times x_7 * max|w| of the slice
+// earlier by at most that much.  The smallest weight sum of the chunk is not tracked but bounded from its
+// two ends: none of the eight sums lies more than four weights below both, so with W = max|w| of the slice
+//     min(0, wsum_0 .. wsum_7) >= min(wsum_start, wsum_7, 4W) - 4W
+// (up to four roundings of a sum).  The lane evaluates t_7 and accepts the chunk if
+//     fma(x_7 - x_0, min(wsum_start, wsum_7, 4W), t_7)  >  thr + (x_7 - x_0)*4W
+//                                                         + 17u * 1.01 * (|ysum_7| + x_7*|wsum_7| + 18*x_7*W)
+// (the last term covers the seven e_u, the roundings of the weight sums, of t_u, t_7, x_7 - x_0 and of the
+// bound itself; sums inside the chunk differ from the final ones by at most seven inputs).  Every t_u then
+// exceeds thr, which is the condition above.  With weight sums that stay above 4W the bound is t_7 itself;
+// below, a chunk may fail although none of its inputs closes the set, by (x_7 - x_0)*4W at most.
+// Two additions per input and ten instructions per chunk and neuron.
+constexpr float FILTER_END_Y = 0x1p-19f;                  // 32u >= 4u + 17.2u, times |ysum_7|
+constexpr float FILTER_END_XW = 0x1p-19f;                 // 32u >= 17.2u, times x_7 * |wsum_7|
+constexpr float FILTER_END_W = 0x1p-15f;                  // 512u >= 36u + 310u, times x_7 * max|w| of the slice
 
-// Eight inputs for one scan of every lane.  Lanes in the mask `open` that pass the test keep the new
-// sums; open lanes that fail keep the old ones, take the chunk's first index as kflag and leave
-// `open`.  The arithmetic does not depend on EXEC or branches (lanes that are not open compute along
-// and discard), so the compiler is free to interleave it with the LDS traffic of the next chunk; the
-// decision works on lane masks in scalar registers: one compare, three mask operations, three selects.
-// dx = x[7] - x[0], x7s = FILTER_END_XW * x[7], thrx = FILTER_END_W * max|w| * x[7].
-__device__ __forceinline__ void filter_chunk(float& wsum, float& ysum, int& kflag, uint64_t& open, int k, float thrx,
-                                             float dx, float x7s, const float (&x)[CHUNK], const float (&w)[CHUNK]) {
-    float wb = wsum, yb = ysum, m = 0.0f;
-#pragma unroll
-    for (int u = 0; u < CHUNK; u += 2) {
-        wb += w[u];
-        yb = __fmaf_rn(x[u], w[u], yb);
-        const float w0 = wb;
-        wb += w[u + 1];
-        yb = __fmaf_rn(x[u + 1], w[u + 1], yb);
-        m = fminf(fminf(m, w0), wb);
-    }
-    const float t7 = __fmaf_rn(-x[CHUNK - 1], wb, yb);
-    const float bound = __fmaf_rn(dx, m, t7);
+// The test of a chunk for one scan of every lane: wb, yb are the sums behind it.  Lanes in the mask `open`
+// that pass take them over; open lanes that fail keep the sums from before the chunk, take the chunk's
+// first index as kcur and leave `open`.  The arithmetic does not depend on EXEC or branches (lanes that
+// are not open compute along and discard), so the compiler is free to interleave it with the LDS traffic
+// of the next chunk; the decision works on lane masks in scalar registers.
+// dx = x[7] - x[0], x7s = FILTER_END_XW * x[7], thrx = FILTER_END_W * W * x[7] + dx * w4, w4 = 4W.
+__device__ __forceinline__ void filter_test(float& wsum, float& ysum, int& kcur, uint64_t& open, int k, float wb, float yb,
+                                            float x7, float thrx, float dx, float x7s, float w4) {
+    const float t7 = __fmaf_rn(-x7, wb, yb);
+    const float bound = __fmaf_rn(dx, fminf(fminf(wsum, wb), w4), t7);
     const float thr = __fmaf_rn(FILTER_END_Y, fabsf(yb), __fmaf_rn(x7s, fabsf(wb), thrx));
     uint64_t stop;
     // (two statements: the first has scalar results only, so the masks stay uniform values for the compiler
@@ -905,8 +831,60 @@ __device__ __forceinline__ void filter_chunk(float& wsum, float& ysum, int& kfla
     asm("v_cndmask_b32_e64 %[ws], %[ws], %[wb], %[open]\n"
         "v_cndmask_b32_e64 %[ys], %[ys], %[yb], %[open]\n"
         "v_cndmask_b32_e64 %[kf], %[kf], %[vk], %[stop]\n"
-        : [ws] "+v"(wsum), [ys] "+v"(ysum), [kf] "+v"(kflag)
+        : [ws] "+v"(wsum), [ys] "+v"(ysum), [kf] "+v"(kcur)
         : [open] "s"(open), [stop] "s"(stop), [wb] "v"(wb), [yb] "v"(yb), [vk] "v"(k));
+}
+
+// Whether a scan that has consumed k > 0 inputs, with a positive weight sum ws and not fired, is certain never to
+// fire on the inputs [k, n) of its row.  Called by the whole wavefront with uniform
+// arguments; wcol is the scan's column of the slice.  depth = ysum - x*ws behind the last input consumed.
+// While the weight sum stays positive, ysum - x*wsum only falls, up to the roundings of the two sums, and the
+// reference's `fired` test is false as long as it is negative.  The running weight sums are formed here in
+// another order (64 inputs at a time by a wavefront scan), so they and the depth have to keep a margin.  With
+// m = n - k, M the largest and T the sum of absolute values of the weights seen, u = 2^-24:
+//   the reference's weight sums differ from the true ones by at most m*u*M', M' their largest absolute value, and
+//   those formed here by at most u*(6T + (m/64 + 1)*M');
+//   every step moves ysum - x*wsum by at most u*(|ysum| + x*|wsum|) more than it should, and
+//   |ysum| <= |depth| + 2*x_last*M'.
+// (Factors rounded up generously: the margins are of the order of 1e-3.)
+template <int COLS>
+__device__ bool never_fires(const float* __restrict__ xs, const int32_t* __restrict__ pr, const float* __restrict__ wcol, int k,
+                            int n, float ws, float ys, int lane) {
+    const float depth = __fmaf_rn(-xs[k - 1], ws, ys);
+    constexpr int BATCH = 4;                                        // wavefronts of inputs whose rows are requested together
+    float carry = ws, low = ws, high = ws, total = 0.0f;
+    for (int base = k; base < n; base += BATCH * kWave) {
+        float wt[BATCH];
+        int row[BATCH];
+#pragma unroll
+        for (int b = 0; b < BATCH; ++b) row[b] = base + b * kWave + lane < n ? pr[base + b * kWave + lane] : -1;
+#pragma unroll
+        for (int b = 0; b < BATCH; ++b) wt[b] = row[b] >= 0 ? wcol[row[b] * COLS] : 0.0f;
+#pragma unroll
+        for (int b = 0; b < BATCH; ++b) {
+            float s = wt[b];
+            total += fabsf(s);
+#pragma unroll
+            for (int d = 1; d < kWave; d <<= 1) {
+                const float up = __shfl_up(s, d, kWave);
+                s += lane >= d ? up : 0.0f;
+            }
+            s += carry;
+            low = fminf(low, s);
+            high = fmaxf(high, s);
+            carry = __shfl(s, kWave - 1, kWave);
+        }
+    }
+#pragma unroll
+    for (int d = kWave / 2; d > 0; d >>= 1) {
+        low = fminf(low, __shfl_xor(low, d, kWave));
+        high = fmaxf(high, __shfl_xor(high, d, kWave));
+        total += __shfl_xor(total, d, kWave);
+    }
+    const float u = 0x1p-24f * 1.1f, m = (float)(n - k + 64), x_last = xs[n - 1];
+    const float low_margin = u * (1.02f * m * high + 8.0f * total);
+    const float depth_margin = u * m * (3.0f * x_last * high + fabsf(depth)) * 1.1f;
+    return low > low_margin && depth < -depth_margin && total < INFINITY;
 }
 
 // Largest of the threads' `m` over the workgroup, the same value in every thread.  `red` is room for
@@ -923,30 +901,34 @@ __device__ __forceinline__ float block_max(float m, float* __restrict__ red) {
     return r;
 }
 
-constexpr int FILTER_RED_BYTES = 64;                       // one float per wavefront behind the slice
-
 // Value of `v` in lane 4*(lane/4) + q: a quad broadcast, which the hardware applies as an operand
 // modifier (DPP) of the move or of the VOP2 instruction that consumes it.
 template <int Q>
-__device__ __forceinline__ int quad_broadcast(int v) {
-    return __builtin_amdgcn_mov_dpp(v, Q * 0x55, 0xf, 0xf, true);
+__device__ __forceinline__ float quad_broadcast(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), Q * 0x55, 0xf, 0xf, true));
 }
 
-// a[q] = base + (value of `row` in lane q of the quad << SHIFT), q = 0..3: the LDS addresses of four
-// weight rows from the row indices the quad's lanes hold.  One shift, then four adds that take the
-// broadcast as an operand modifier (the two idle cycles between them are what a DPP read of a
-// register written by the instruction before it needs).
-template <int SHIFT>
-__device__ __forceinline__ void quad_row_addresses(int row, unsigned base, unsigned (&a)[4]) {
-    int t;
-    asm("v_lshlrev_b32_e32 %[t], %[sh], %[row]\n"
-        "s_nop 1\n"
-        "v_add_u32_dpp %[a0], %[t], %[base] quad_perm:[0,0,0,0] row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
-        "v_add_u32_dpp %[a1], %[t], %[base] quad_perm:[1,1,1,1] row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
-        "v_add_u32_dpp %[a2], %[t], %[base] quad_perm:[2,2,2,2] row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
-        "v_add_u32_dpp %[a3], %[t], %[base] quad_perm:[3,3,3,3] row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
-        : [t] "=&v"(t), [a0] "=&v"(a[0]), [a1] "=&v"(a[1]), [a2] "=&v"(a[2]), [a3] "=&v"(a[3])
-        : [row] "v"(row), [base] "v"(base), [sh] "n"(SHIFT));
+// LDS addresses of the four weight rows whose (shifted) indices lanes 2*HALF and 2*HALF + 1 of the quad
+// hold, two each: adds that take the broadcast as an operand modifier.  (The two idle cycles are what a
+// DPP read of a register written by the instruction before it needs.)
+template <int HALF>
+__device__ __forceinline__ void quad_row_addresses(int even, int odd, unsigned base, unsigned (&a)[4]) {
+    if constexpr (HALF == 0)
+        asm("s_nop 1\n"
+            "v_add_u32_dpp %[a0], %[e], %[base] quad_perm:[0,0,0,0] row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+            "v_add_u32_dpp %[a1], %[o], %[base] quad_perm:[0,0,0,0] row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+            "v_add_u32_dpp %[a2], %[e], %[base] quad_perm:[1,1,1,1] row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+            "v_add_u32_dpp %[a3], %[o], %[base] quad_perm:[1,1,1,1] row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+            : [a0] "=&v"(a[0]), [a1] "=&v"(a[1]), [a2] "=&v"(a[2]), [a3] "=&v"(a[3])
+            : [e] "v"(even), [o] "v"(odd), [base] "v"(base));
+    else
+        asm("s_nop 1\n"
+            "v_add_u32_dpp %[a0], %[e], %[base] quad_perm:[2,2,2,2] row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+            "v_add_u32_dpp %[a1], %[o], %[base] quad_perm:[2,2,2,2] row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+            "v_add_u32_dpp %[a2], %[e], %[base] quad_perm:[3,3,3,3] row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+            "v_add_u32_dpp %[a3], %[o], %[base] quad_perm:[3,3,3,3] row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+            : [a0] "=&v"(a[0]), [a1] "=&v"(a[1]), [a2] "=&v"(a[2]), [a3] "=&v"(a[3])
+            : [e] "v"(even), [o] "v"(odd), [base] "v"(base));
 }
 
 typedef __attribute__((address_space(3))) const float lds_cfloat;
@@ -962,14 +944,39 @@ __device__ __forceinline__ bool for_each_phase(F&& f) {
     return for_each_phase_impl(f, std::make_integer_sequence<int, N>{});
 }
 
-// Segments a wavefront of the filter kernel works on, and whether their input times go through
-// LDS: they do unless every quad has a segment of its own (then the quad broadcast is all there is
-// to share, and the buffers of 16 segments per wavefront would not fit beside the slice).
-constexpr int filter_segments(int cols, int ch) { return kWave / (cols / ch); }
-constexpr bool filter_stages_times(int cols, int ch) { return filter_segments(cols, ch) <= 8; }
-// dynamic LDS of a workgroup of `waves` wavefronts behind its slice
-constexpr size_t filter_extra_lds(int cols, int ch, int waves) {
-    return FILTER_RED_BYTES + (filter_stages_times(cols, ch) ? (size_t)waves * filter_segments(cols, ch) * FILTER_XBUF_SEG_BYTES : 0);
+// The lane's CH columns of an output row, `left` of which exist; one wide store where rows keep the alignment.
+template <int CH>
+__device__ __forceinline__ void store_columns(float* __restrict__ p, const float (&v)[CH], int left, int pitch) {
+    if constexpr (CH == 4) {
+        if ((pitch & 3) == 0 && (reinterpret_cast<uintptr_t>(p) & 15) == 0) {
+            if (left > 0) *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
+            return;
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < CH; ++c)
+        if (c < left) p[c] = v[c];
+}
+
+__device__ __forceinline__ uint64_t ballot(bool b) { return __builtin_amdgcn_ballot_w64(b); }
+// Whether the lane's bit is set in a lane mask.
+__device__ __forceinline__ bool in_mask(uint64_t m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
+
+// Value v of lane N of the lane's row of sixteen, in every lane of the row.
+template <int N>
+__device__ __forceinline__ float row_broadcast(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x150 + N, 0xf, 0xf, true));
+}
+// LDS addresses of the four weight rows whose shifted indices lanes N and N + 1 of the row of sixteen hold.
+template <int N>
+__device__ __forceinline__ void row_row_addresses(int even, int odd, unsigned base, unsigned (&a)[4]) {
+    asm("s_nop 1\n"
+        "v_add_u32_dpp %[a0], %[e], %[base] row_newbcast:%[n0] row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+        "v_add_u32_dpp %[a1], %[o], %[base] row_newbcast:%[n0] row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+        "v_add_u32_dpp %[a2], %[e], %[base] row_newbcast:%[n1] row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+        "v_add_u32_dpp %[a3], %[o], %[base] row_newbcast:%[n1] row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+        : [a0] "=&v"(a[0]), [a1] "=&v"(a[1]), [a2] "=&v"(a[2]), [a3] "=&v"(a[3])
+        : [e] "v"(even), [o] "v"(odd), [base] "v"(base), [n0] "n"(N), [n1] "n"(N + 1));
 }
 
 template <int COLS, int CH, bool WANT_K>
@@ -977,14 +984,15 @@ __global__ void __launch_bounds__(LDS_SCAN_THREADS)
 scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__ perm,
                    const int32_t* __restrict__ n_real, const float* __restrict__ w, float* __restrict__ y_out,
                    float* __restrict__ rcp_out, int32_t* __restrict__ k_out, int S, int I, int stride, int J,
-                   int n_slices, int n_groups, NeuronParams np, TimeCopy copy) {
+                   int n_slices, int n_groups, int waves, NeuronParams np, TimeCopy copy) {
     extern __shared__ __align__(16) float wl[];                          // [I + bias][COLS], then `red`
     constexpr int LANES = COLS / CH;                       // lanes per segment
     constexpr int SEGS = kWave / LANES;                    // segments per wavefront
     static_assert(LANES % 4 == 0, "the four lanes of a quad belong to one segment");
-    // Input times reach the lanes through LDS where several quads share a segment (see the fast loop)
-    constexpr bool XLDS = filter_stages_times(COLS, CH);
-    const int WAVES = blockDim.x / kWave;
+    // How a segment's (x, row) entries reach its lanes (see the fast loop): through rows of sixteen lanes where
+    // a segment has at least that many, else through quads
+    constexpr bool BY_ROW = LANES % 16 == 0;
+    constexpr int ROUND = 4;                               // chunks per round of the fast loop
     const int block = xcd_contiguous(blockIdx.x, gridDim.x);
     const int slice = block / n_groups;
     const int group = block - slice * n_groups;
@@ -992,27 +1000,21 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
     const int rows = I + np.bias;
     // the slice, and the largest |w| in it (the threads' shares of the copy, then the workgroup's)
     const float w_max = block_max(fill_weight_slice<COLS>(wl, w, rows, J, j0), wl + rows * COLS);
-    const float thr_w = FILTER_W * w_max;                   // margin of the accumulate-only rounds below
     const float end_w = FILTER_END_W * w_max;               // margin of the fast loop
+    const float w4 = 4.0f * 1.00001f * w_max;               // 4W of its bound on the weight sums
 
     const int lane = threadIdx.x % kWave;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int sub = lane / LANES, cg = lane - sub * LANES;
     const int j = j0 + CH * cg;                            // first of the lane's columns
     const float* __restrict__ wcol = wl + CH * cg;
-    const int last_chunk = stride - CHUNK;
-
-    const int quad_lane = lane & 3;
     const unsigned wbase = (unsigned)(uintptr_t)(lds_cfloat*)wcol;          // LDS byte address of the lane's columns
-    // [wave][buffer][segment of the wavefront][CHUNK] input times, behind the slice and `red`
-    float* __restrict__ xbuf = wl + rows * COLS + FILTER_RED_BYTES / (int)sizeof(float) +
-                               (size_t)wave * 2 * SEGS * CHUNK + sub * CHUNK;
-    const bool x_writer = cg < 4;                          // the first quad of every segment
     constexpr int NONE = 0x7fffffff;
     constexpr int ROW_SHIFT = COLS == 64 ? 8 : COLS == 32 ? 7 : COLS == 16 ? 6 : 5;      // a weight row is COLS * 4 bytes
     static_assert(COLS == 64 || COLS == 32 || COLS == 16 || COLS == 8, "slice width");
 
-    for (int item = group * WAVES + wave; item * SEGS < S; item += n_groups * WAVES) {
+    // `waves` wavefronts of the workgroup work on items; the others have only helped to copy the slice
+    for (int item = group * waves + wave; wave < waves && item * SEGS < S; item += n_groups * waves) {
         const int seg_raw = item * SEGS + sub;
         const int seg = seg_raw < S ? seg_raw : S - 1;      // idle lanes shadow a valid segment
         const float* __restrict__ xs = sorted + (size_t)seg * stride;
@@ -1021,327 +1023,396 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
         const int n_segs = S - seg0 < SEGS ? S - seg0 : SEGS;
         const RowSource rows_of_item = make_row_source(sorted + (size_t)seg0 * stride, perm + (size_t)seg0 * stride,
                                                        n_segs * stride * (int)sizeof(float));
-        const int lane_bytes = ((seg - seg0) * stride + quad_lane) * (int)sizeof(float);
+        const int lane_bytes = ((seg - seg0) * stride + 2 * (lane & (BY_ROW ? 15 : 3))) * (int)sizeof(float);
         const int n_seg = n_real[seg];
         const float first_x = xs[0];
-        // The ring of (x, row) entries the fast loop below consumes (see there).  Its first round is requested
-        // here, next to the two loads above and before anything waits for them: practically every item
-        // starts its first pass at input 0, and the round trips would otherwise follow one another.
-        constexpr int RING = 8;                             // chunks of entries held or on their way
-        float rxl[RING], rxh[RING];
-        int rpl[RING], rph[RING];
-        auto request = [&](int slot, int k) {
-            const int kb = (k <= last_chunk ? k : 0) * (int)sizeof(float);
-            rxl[slot] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rows_of_item.xs, lane_bytes, kb, 0));
-            rxh[slot] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rows_of_item.xs, lane_bytes + 16, kb, 0));
-            rpl[slot] = (int)__builtin_amdgcn_raw_buffer_load_b32(rows_of_item.pr, lane_bytes, kb, 0);
-            rph[slot] = (int)__builtin_amdgcn_raw_buffer_load_b32(rows_of_item.pr, lane_bytes + 16, kb, 0);
+        // The (x, row) stream of a segment is the same for all its lanes.  If every lane fetched the eight
+        // entries of a chunk itself, a wavefront would move four kilobytes per chunk through the vector
+        // memory path, which then bounds the kernel.  Instead a lane fetches two entries of both arrays with
+        // two 8-byte buffer loads that need no address arithmetic, and a value reaches the other lanes as a DPP
+        // broadcast: free for the row offsets, which enter the LDS address through an add that takes the
+        // broadcast as an operand modifier, one move per input time (shared by the lane's CH scans).  Sixteen
+        // lanes of one segment hold a whole round of four chunks, so a round takes one pair of loads; a quad
+        // holds one chunk, and every chunk takes one.  (Requests past the end of a row return the next row of
+        // the item, past the last one zeros: the buffer descriptor ends with the item.  Nothing uses them.)
+        //
+        // held: rows: block b holds the round b rounds ahead of the current one; quads: a ring of chunks.
+        // The first entries are requested here, next to the two loads above and before anything waits for
+        // them: practically every item starts its first pass at input 0.
+        constexpr int BLOCKS = BY_ROW ? (CH == 4 ? 2 : 3) : ROUND;
+        constexpr int BLOCK_INPUTS = BY_ROW ? ROUND * CHUNK : CHUNK;
+        u32x2 rx[BLOCKS], rp[BLOCKS];
+        auto request = [&](int b, int k) {
+            rx[b] = __builtin_amdgcn_raw_buffer_load_b64(rows_of_item.xs, lane_bytes, k * (int)sizeof(float), 0);
+            rp[b] = __builtin_amdgcn_raw_buffer_load_b64(rows_of_item.pr, lane_bytes, k * (int)sizeof(float), 0);
         };
+        auto request_first = [&](int k) {
 #pragma unroll
-        for (int b = 0; b < RING - 1; ++b) request(b, b * CHUNK);
-        bool ring_at_zero = true;                           // the ring holds the entries from input 0 on
+            for (int b = 0; b < BLOCKS - 1; ++b) request(b, k + b * BLOCK_INPUTS);
+        };
+        request_first(0);
         const int n_full = n_seg & ~(CHUNK - 1);
+        int n_full_max = 0;                                 // of the longest of the wavefront's rows
+#pragma unroll
+        for (int q = 0; q < SEGS; ++q) n_full_max = max(n_full_max, __builtin_amdgcn_readlane(n_full, q * LANES));
 
-        // Per scan: the running sums, the number of inputs they hold (kcur), and where the scan stands:
+        // Per scan: the running sums, the number of inputs they hold (kcur), and where it stands, as lane masks (in
+        // scalar registers: per-lane flags cost four-neuron lanes the registers the fast loop needs)
         //   armed    waits to run the fast loop from kcur (no reference test can close before kcur)
-        //   kflag    first index of a chunk that failed the fast test and has to be stepped through (or -1)
-        //   fin      closed; sums, fired state and count are final
+        //   step     has to be stepped through from kcur
+        //   fin      done: sums, fired state and count are final
+        //   fired    the fired state that goes with the sums
         float wsum[CH], ysum[CH];
-        int kcur[CH], kflag[CH];
-        bool live[CH], armed[CH], fin[CH], fired_cur[CH];   // fired_cur: the fired state that goes with the sums
+        int kcur[CH];
+        uint64_t armed[CH], step[CH], fin[CH], fired[CH], any_armed = 0;
         float wb[CH];
         if (np.bias) read_columns<CH>(wcol + I * COLS, wb);
 #pragma unroll
         for (int c = 0; c < CH; ++c) {
-            live[c] = seg_raw < S && j + c < J;
+            const bool live = seg_raw < S && j + c < J;
+            bool fired0 = false;
             wsum[c] = -np.theta; ysum[c] = 0.0f;
-            fired_cur[c] = false;
             if (np.bias) {
                 wsum[c] += wb[c];
                 ysum[c] = np.biasvolt * wb[c];
                 const float ya0 = wsum[c] < 0.0f ? -ysum[c] : ysum[c];
-                fired_cur[c] = ya0 > fabsf(wsum[c]) * np.biasvolt;
+                fired0 = ya0 > fabsf(wsum[c]) * np.biasvolt;
             }
             kcur[c] = 0;
-            fin[c] = false;
             // The fast loop takes scans whose fired state is what their sums imply between tests that
             // pass with a margin: fired exactly when the weight sum is positive, and whose remaining
             // inputs are not negative (its bounds assume x >= 0; rows are ascending).  Any other start (a
             // neuron that fired on its bias alone, a row that begins below zero) is stepped through
             // from the first input on.
-            const bool plain = fired_cur[c] == (wsum[c] > 0.0f) && !fired_cur[c] && first_x >= 0.0f;
-            armed[c] = live[c] && n_full > 0 && plain;
-            kflag[c] = (live[c] && n_full > 0 && !plain) ? 0 : -1;
+            const bool plain = fired0 == (wsum[c] > 0.0f) && !fired0 && first_x >= 0.0f;
+            fired[c] = ballot(fired0);
+            fin[c] = ballot(!live);
+            armed[c] = ballot(live && n_full > 0 && plain);
+            step[c] = ballot(live && n_full > 0 && !plain);
+            any_armed |= armed[c];
         }
 
-        // Passes: the fast loop for the armed scans that are furthest behind, then the recorded
-        // chunks step by step.  A scan that does not close in its recorded chunk is armed again.
+        // Passes: the fast loop for the armed scans that are furthest behind, then the scans it left behind
+        // step by step.  A scan that does not close there is armed again.
         // Practically every item takes one pass and a second look without work.
-        bool first_pass = true;
+        int kmin = any_armed != 0 ? 0 : NONE;               // every armed scan starts at input 0
         for (;;) {
-            int kmin = NONE;
+            uint64_t ran[CH];                               // the scans that take part in this pass's fast loop
 #pragma unroll
-            for (int c = 0; c < CH; ++c) kmin = armed[c] ? min(kmin, kcur[c]) : kmin;
-            if (first_pass) {                               // every armed scan starts at input 0
-                kmin = __builtin_amdgcn_ballot_w64(kmin != NONE) != 0 ? 0 : NONE;
-            } else {
-#pragma unroll
-                for (int d = kWave / 2; d > 0; d >>= 1) kmin = min(kmin, __shfl_xor(kmin, d, kWave));
-                kmin = __builtin_amdgcn_readfirstlane(kmin);
-            }
-            first_pass = false;
+            for (int c = 0; c < CH; ++c) ran[c] = armed[c] & ballot(kcur[c] == kmin);
             if (kmin != NONE) {
-                uint64_t open[CH];                          // lanes whose scan runs in this loop
-                bool ran[CH];
+                uint64_t open[CH];                          // lanes whose scan still runs in it
 #pragma unroll
                 for (int c = 0; c < CH; ++c) {
-                    ran[c] = armed[c] && kcur[c] == kmin;
-                    open[c] = __builtin_amdgcn_ballot_w64(ran[c]);
-                    armed[c] = armed[c] && !ran[c];
-                    kcur[c] = ran[c] ? n_full : kcur[c];    // unless the scan records a chunk below
+                    open[c] = ran[c];
+                    armed[c] &= ~ran[c];
+                    kcur[c] = in_mask(ran[c]) ? n_full : kcur[c];          // unless the scan stops earlier
                 }
-                // The (x, row) stream of a segment is the same for all its lanes.  If every lane fetched
-                // the eight entries of a chunk itself, a wavefront would move four kilobytes per chunk
-                // through the vector memory path, which then bounds the kernel.  Instead the four lanes
-                // of a quad fetch entries q and q + 4 of both arrays (q = lane % 4: four dwords per lane
-                // and chunk, through buffer loads that need no address arithmetic), and a value reaches
-                // the other lanes of the quad as a quad broadcast: free for the row offsets, which enter
-                // the LDS address through an add that takes the broadcast as an operand modifier, one
-                // move per input time (shared by the lane's CH scans).
-                // Per phase, with c the chunk being consumed: request the entries of chunk c+RING-1, read
-                // the weights of chunk c+1 from LDS, run chunk c.
-                float wv[2][CH][CHUNK];                     // [buffer][scan][step]
-                auto weights = [&](int slot, float (&wo)[CH][CHUNK]) {
-                    unsigned al[4], ah[4];
-                    quad_row_addresses<ROW_SHIFT>(rpl[slot], wbase, al);
-                    quad_row_addresses<ROW_SHIFT>(rph[slot], wbase, ah);
-#pragma unroll
-                    for (int u = 0; u < CHUNK; ++u) {
-                        float wr[CH];
-                        read_columns<CH>(reinterpret_cast<lds_cfloat*>((uintptr_t)(u < 4 ? al[u] : ah[u - 4])), wr);
-#pragma unroll
-                        for (int c = 0; c < CH; ++c) wo[c][u] = wr[c];
-                    }
-                };
-                // Input times: with DPP alone every lane needs a move per time and chunk.  Where a
-                // segment spans several quads, its first quad instead leaves the eight times of the
-                // next chunk in a small LDS buffer of the wavefront (two chunks deep) and every lane
-                // reads them back as two 16-byte broadcasts, a phase ahead like the weights.  LDS
-                // serves the requests of a wavefront in order, so the reads find what was written.
-                float xq[2][CHUNK];
-                auto stage_times = [&](int slot, int buf) {
-                    if constexpr (XLDS) {
-                        float* __restrict__ xb = xbuf + buf * SEGS * CHUNK;
-                        if (x_writer) {
-                            xb[quad_lane] = rxl[slot];
-                            xb[quad_lane + 4] = rxh[slot];
-                        }
-                        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                        __builtin_amdgcn_wave_barrier();
-                        const float4 lo = *reinterpret_cast<const float4*>(xb), hi = *reinterpret_cast<const float4*>(xb + 4);
-                        xq[buf][0] = lo.x; xq[buf][1] = lo.y; xq[buf][2] = lo.z; xq[buf][3] = lo.w;
-                        xq[buf][4] = hi.x; xq[buf][5] = hi.y; xq[buf][6] = hi.z; xq[buf][7] = hi.w;
-                    }
-                };
-                if (!(ring_at_zero && kmin == 0)) {
-#pragma unroll
-                    for (int b = 0; b < RING - 1; ++b) request(b, kmin + b * CHUNK);
-                }
-                ring_at_zero = false;
-                weights(0, wv[0]);
-                // (every lane "uses" the first chunk's times here: otherwise the compiler moves their loads
-                // under the writers' branch of stage_times and waits for all 28 requests there)
-                if constexpr (XLDS) asm volatile("" : "+v"(rxl[0]), "+v"(rxh[0]));
-                stage_times(0, 0);
-
-                // One phase; its number is a compile-time value.  (The phases of a round are chained by a fold
-                // expression, not by a loop with a break: behind such a loop the compiler waits in every
-                // phase for all but the last four row loads, which makes the ring one chunk deep in effect.)
-                auto phase = [&](auto ph_c, int k) {
-                    constexpr int ph = decltype(ph_c)::value;
-                    request((ph + RING - 1) % RING, k + (RING - 1) * CHUNK);
-                    weights((ph + 1) % RING, wv[(ph + 1) % 2]);
-                    stage_times((ph + 1) % RING, (ph + 1) % 2);
-                    // The requests above stay ahead of the arithmetic below: what this phase consumes
-                    // was requested a phase or more ago, and what it requests has the whole phase to
-                    // arrive.
-                    __builtin_amdgcn_sched_barrier(0);
-                    float x[CHUNK];
-                    if constexpr (XLDS) {
-#pragma unroll
-                        for (int u = 0; u < CHUNK; ++u) x[u] = xq[ph % 2][u];
+                // The weights of a chunk are read in two halves of four inputs.  Per half, with h the half
+                // being consumed: read the weights of half h + NH - 1, then run half h; NH = 2 keeps
+                // four-neuron lanes within the registers of a 16-wavefront workgroup, the others read
+                // a whole chunk ahead.  H counts halves from the start of the round.
+                constexpr int NH = CH == 4 ? 2 : 4;
+                float wv[NH][CH][4];                        // [half buffer][scan][step]
+                auto weights = [&](auto h_c) {
+                    constexpr int H = decltype(h_c)::value, P = H / 2, HH = H % 2;
+                    unsigned at[4];
+                    if constexpr (BY_ROW) {
+                        constexpr int b = P / ROUND;
+                        row_row_addresses<(P % ROUND) * 4 + HH * 2>((int)rp[b].x << ROW_SHIFT, (int)rp[b].y << ROW_SHIFT, wbase, at);
                     } else {
-                        const int xl = __float_as_int(rxl[ph % RING]), xh = __float_as_int(rxh[ph % RING]);
-                        x[0] = __int_as_float(quad_broadcast<0>(xl)); x[1] = __int_as_float(quad_broadcast<1>(xl));
-                        x[2] = __int_as_float(quad_broadcast<2>(xl)); x[3] = __int_as_float(quad_broadcast<3>(xl));
-                        x[4] = __int_as_float(quad_broadcast<0>(xh)); x[5] = __int_as_float(quad_broadcast<1>(xh));
-                        x[6] = __int_as_float(quad_broadcast<2>(xh)); x[7] = __int_as_float(quad_broadcast<3>(xh));
+                        constexpr int b = P % ROUND;
+                        quad_row_addresses<HH>((int)rp[b].x << ROW_SHIFT, (int)rp[b].y << ROW_SHIFT, wbase, at);
                     }
-                    const float thrx = x[CHUNK - 1] * end_w, x7s = x[CHUNK - 1] * FILTER_END_XW;
-                    const float dx = x[CHUNK - 1] - x[0];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        float wr[CH];
+                        read_columns<CH>(reinterpret_cast<lds_cfloat*>((uintptr_t)at[u]), wr);
+#pragma unroll
+                        for (int c = 0; c < CH; ++c) wv[H % NH][c][u] = wr[c];
+                    }
+                };
+                auto times = [&](auto h_c, float (&x)[4]) {
+                    constexpr int H = decltype(h_c)::value, P = H / 2, HH = H % 2;
+                    if constexpr (BY_ROW) {
+                        constexpr int N = P * 4 + HH * 2;
+                        const float xe = __uint_as_float(rx[0].x), xo = __uint_as_float(rx[0].y);
+                        x[0] = row_broadcast<N>(xe); x[1] = row_broadcast<N>(xo);
+                        x[2] = row_broadcast<N + 1>(xe); x[3] = row_broadcast<N + 1>(xo);
+                    } else {
+                        const float xe = __uint_as_float(rx[P].x), xo = __uint_as_float(rx[P].y);
+                        x[0] = quad_broadcast<2 * HH>(xe); x[1] = quad_broadcast<2 * HH>(xo);
+                        x[2] = quad_broadcast<2 * HH + 1>(xe); x[3] = quad_broadcast<2 * HH + 1>(xo);
+                    }
+                };
+                weights(std::integral_constant<int, 0>{});
+                if constexpr (NH == 4) {
+                    weights(std::integral_constant<int, 1>{});
+                    weights(std::integral_constant<int, 2>{});
+                }
+                // One chunk: wb / yb are the scans' sums behind its inputs.  The requests stay ahead of the
+                // arithmetic: what a half consumes was requested a half or more ago, and what it requests has the
+                // whole half to arrive.
+                float yb[CH], x0, x7;
+                auto chunk = [&](auto ph_c, int k) {
+                    constexpr int ph = decltype(ph_c)::value;
+                    if constexpr (!BY_ROW) request((ph + ROUND - 1) % ROUND, k + (ROUND - 1) * CHUNK);
+                    auto half = [&](auto half_c) {
+                        constexpr int hh = decltype(half_c)::value, H = 2 * ph + hh;
+                        weights(std::integral_constant<int, H + NH - 1>{});
+                        __builtin_amdgcn_sched_barrier(0);
+                        float x[4];
+                        times(std::integral_constant<int, H>{}, x);
+                        if (hh == 0) x0 = x[0];
+                        else x7 = x[3];
+#pragma unroll
+                        for (int u = 0; u < 4; ++u)
+#pragma unroll
+                            for (int c = 0; c < CH; ++c) {
+                                const float wc = wv[H % NH][c][u];
+                                const bool start = hh == 0 && u == 0;
+                                wb[c] = (start ? wsum[c] : wb[c]) + wc;
+                                yb[c] = __fmaf_rn(x[u], wc, start ? ysum[c] : yb[c]);
+                            }
+                    };
+                    half(std::integral_constant<int, 0>{});
+                    half(std::integral_constant<int, 1>{});
+                };
+                // rows: the next round's block moves up, the one after it is requested
+                auto next_round = [&] {
+                    if constexpr (BY_ROW) {
+#pragma unroll
+                        for (int b = 0; b + 1 < BLOCKS; ++b) { rx[b] = rx[b + 1]; rp[b] = rp[b + 1]; }
+                    }
+                };
+                auto start_round = [&](int k0) {
+                    if constexpr (BY_ROW) request(BLOCKS - 1, k0 + (BLOCKS - 1) * BLOCK_INPUTS);
+                };
+                auto test = [&](int k) {
+                    const float dx = x7 - x0, x7s = x7 * FILTER_END_XW;
+                    const float thrx = __fmaf_rn(dx, w4, x7 * end_w);
 #pragma unroll
                     for (int c = 0; c < CH; ++c)
-                        filter_chunk(wsum[c], ysum[c], kflag[c], open[c], k, thrx, dx, x7s, x, wv[ph % 2][c]);
+                        filter_test(wsum[c], ysum[c], kcur[c], open[c], k, wb[c], yb[c], x7, thrx, dx, x7s, w4);
                 };
-                for (int k0 = kmin;; k0 += RING * CHUNK) {
-                    rotate_wave_priority(k0 / (RING * CHUNK) + (wave >> 2));
-                    const bool stop = !for_each_phase<RING>([&](auto ph_c) {
-                        const int k = k0 + decltype(ph_c)::value * CHUNK;
-                        const uint64_t inside = __builtin_amdgcn_ballot_w64(k < n_full);
-                        uint64_t any = 0;
-#pragma unroll
-                        for (int c = 0; c < CH; ++c) {
-                            open[c] &= inside;
-                            any |= open[c];
-                        }
-                        if (any == 0) return false;
-                        phase(ph_c, k);
-                        return true;
-                    });
-                    if (stop) break;
-                }
-#pragma unroll
-                for (int c = 0; c < CH; ++c) fired_cur[c] = ran[c] ? wsum[c] > 0.0f : fired_cur[c];
-            }
-
-            // Recorded chunks, stepped through with the reference's tests: every lane fetches its own
-            // eight inputs (positions are multiples of eight inside the full chunks of the row).  A scan
-            // that closes is finished.  One that does not goes back to the fast loop if its fired state is
-            // the plain one; otherwise (fired on a negative weight sum, say) it keeps stepping here, chunk
-            // by chunk.
-            bool need[CH], any_need = false, any_armed = false;
-            Chunk pc[CH];
-#pragma unroll
-            for (int c = 0; c < CH; ++c) {
-                need[c] = kflag[c] >= 0;
-                kcur[c] = need[c] ? kflag[c] : kcur[c];
-                kflag[c] = -1;
-                any_need |= need[c];
-                any_armed |= armed[c];
-            }
-            if (__builtin_amdgcn_ballot_w64(any_need) != 0) {
-                int round = 0;
-                do {
-                    // (fetched on demand: a second round is rare, requesting its entries ahead of time
-                    // would cost every item eight more loads per scan)
-#pragma unroll
-                    for (int c = 0; c < CH; ++c) load_chunk_flat(pc[c], xs, pr, need[c] ? kcur[c] : 0);
-                    any_need = false;
+                // Whole rounds as long as the longest row has one left, without an exit inside the round: behind an
+                // exit test between a request and its use, several chunks later, the compiler would move the
+                // request right in front of the use, and the wavefront would wait for the whole round trip.
+                // Scans whose row has ended are masked.  The last chunks of the longest row follow one by one.
+                auto inside = [&](int k) {
+                    const uint64_t in = __builtin_amdgcn_ballot_w64(k < n_full);
+                    uint64_t any = 0;
 #pragma unroll
                     for (int c = 0; c < CH; ++c) {
-                        float pw[CHUNK], px[CHUNK];
-#pragma unroll
-                        for (int u = 0; u < CHUNK; ++u) {
-                            pw[u] = wcol[pc[c].p[u] * COLS + c];
-                            px[u] = pc[c].x[u];
-                        }
-                        // Later rounds are for the rare scan that missed its close by a rounding: weight
-                        // sum positive, not fired (D < 0).  It cannot fire, let alone close, before the
-                        // weight sum has been negative long enough for D to come back up to zero, and it
-                        // walks on here, a chunk per round, usually in a wavefront that is alone by then.
-                        // While every scan of the round is in that state, a chunk is only accumulated and
-                        // bounded: with all t = ysum - x*wsum below -thr (the fast loop's margin) and all
-                        // weight sums positive, the reference's `fired` test is false after each of the
-                        // eight inputs, and that is all it evaluates for a scan that has not fired.
-                        bool walked = false;
-                        if (round > 0) {
-                            const bool stuck = need[c] && !fired_cur[c] && wsum[c] > 0.0f && px[0] >= 0.0f;
-                            if (__builtin_amdgcn_ballot_w64(need[c] && !stuck) == 0) {
-                                float wb = wsum[c], yb = ysum[c], tmax = -INFINITY, wmin = INFINITY;
-#pragma unroll
-                                for (int u = 0; u < CHUNK; ++u) {
-                                    wb += pw[u];
-                                    yb = __fmaf_rn(px[u], pw[u], yb);
-                                    tmax = fmaxf(tmax, __fmaf_rn(-px[u], wb, yb));
-                                    wmin = fminf(wmin, wb);
-                                }
-                                const float thr = __fmaf_rn(FILTER_REL, fabsf(yb), px[CHUNK - 1] * thr_w);
-                                walked = stuck && tmax < -thr && wmin > 0.0f;
-                                wsum[c] = walked ? wb : wsum[c];
-                                ysum[c] = walked ? yb : ysum[c];
-                            }
-                        }
-                        float ya = wsum[c] < 0.0f ? -ysum[c] : ysum[c];
-                        float yg = fired_cur[c] ? ya : INFINITY;
-                        uint64_t exited = 0;
-                        int kc = kcur[c] + (walked ? CHUNK : 0);
-                        const uint64_t run = __builtin_amdgcn_ballot_w64(need[c] && !walked);
-                        if (run != 0) scan_chunk_vector<true>(wsum[c], ysum[c], ya, yg, kc, exited, run, px, pw);
-                        const bool closed_here = (exited >> lane) & 1;
-                        kcur[c] = kc;                       // inputs consumed
-                        fin[c] = fin[c] || closed_here;
-                        fired_cur[c] = closed_here || yg < INFINITY;
-                        const bool more = need[c] && !closed_here && kc + CHUNK <= n_full;
-                        const bool plain = fired_cur[c] == (wsum[c] > 0.0f) && px[CHUNK - 1] >= 0.0f;
-                        armed[c] = armed[c] || (more && plain);
-                        any_armed |= more && plain;
-                        need[c] = more && !plain;
-                        any_need |= need[c];
+                        open[c] &= in;
+                        any |= open[c];
                     }
-                    ++round;
-                } while (__builtin_amdgcn_ballot_w64(any_need) != 0);
-            }
-            if (__builtin_amdgcn_ballot_w64(any_armed) == 0) break;
-        }
-
-        // Whatever is left of a row -- fewer than eight inputs behind the full chunks -- step by step,
-        // then the output.  The leftover entries and their weights are fetched in one go for the
-        // lane's CH scans (a load per step would put a memory round trip into every one of them); rows
-        // are padded beyond their length, so the eight entries from n_full on can always be read.
-        LaneState st[CH];
-        int kc[CH];
-        bool still[CH], any_left = false;
-#pragma unroll
-        for (int c = 0; c < CH; ++c) {
-            st[c].wsum = wsum[c]; st[c].ysum = ysum[c]; st[c].wa = fabsf(wsum[c]);
-            st[c].ya = wsum[c] < 0.0f ? -ysum[c] : ysum[c];
-            st[c].fired = fired_cur[c];
-            kc[c] = kcur[c];
-            still[c] = live[c] && !fin[c];
-            any_left |= still[c] && kc[c] < n_seg;
-        }
-        if (__builtin_amdgcn_ballot_w64(any_left) != 0) {
-            Chunk tc;
-            load_chunk_flat(tc, xs, pr, n_full < n_seg ? n_full : 0);
-            float tw[CH][CHUNK];
-#pragma unroll
-            for (int c = 0; c < CH; ++c)
-#pragma unroll
-                for (int u = 0; u < CHUNK; ++u) tw[c][u] = wcol[tc.p[u] * COLS + c];
-#pragma unroll
-            for (int u = 0; u < CHUNK - 1; ++u) {
-                bool any_step = false;
+                    return any != 0;
+                };
+                int k0 = kmin;
+                bool more = true;
+                for (; k0 + ROUND * CHUNK <= n_full_max && more; k0 += ROUND * CHUNK) {
+                    rotate_wave_priority(k0 / (ROUND * CHUNK) + (wave >> 2));
+                    start_round(k0);
+                    for_each_phase<ROUND>([&](auto ph_c) {
+                        const int k = k0 + decltype(ph_c)::value * CHUNK;
+                        inside(k);
+                        chunk(ph_c, k);
+                        test(k);
+                        return true;
+                    });
+                    next_round();
+                    more = inside(k0 + ROUND * CHUNK);
+                }
+                if (more)
+                    for_each_phase<ROUND>([&](auto ph_c) {
+                        const int k = k0 + decltype(ph_c)::value * CHUNK;
+                        if (!inside(k)) return false;
+                        chunk(ph_c, k);
+                        test(k);
+                        return true;
+                    });
 #pragma unroll
                 for (int c = 0; c < CH; ++c) {
-                    const bool step = still[c] && kc[c] == n_full + u && n_full + u < n_seg;
-                    if (step) {
-                        still[c] = scan_step(st[c], tc.x[u], tw[c][u]);
-                        if (still[c]) ++kc[c];
-                    }
-                    any_step |= step;
+                    fired[c] = (fired[c] & ~ran[c]) | (ballot(wsum[c] > 0.0f) & ran[c]);
+                    step[c] |= ran[c] & ballot(kcur[c] < n_full);
                 }
-                if (__builtin_amdgcn_ballot_w64(any_step) == 0) break;
             }
+
+            // Stopped scans, evaluated with the reference's tests: every lane fetches its own eight inputs
+            // (positions are multiples of eight inside the full chunks of the row).  A scan that closes is
+            // finished.  One that does not is stepped on for two more chunks -- the fast test fails early where
+            // the weight sum is small, and starting the fast loop for a chunk or two costs more -- and goes back
+            // to the fast loop then, if its fired state is the plain one; otherwise (fired on a negative weight
+            // sum, say) it keeps stepping here.
+            //   sure: the scan is in the plain state with ysum - x*wsum well above zero (close_chunk_vector)
+            uint64_t sure[CH], any_step = 0;
+#pragma unroll
+            for (int c = 0; c < CH; ++c) {
+                sure[c] = ran[c];
+                any_step |= step[c];
+            }
+            for (int round = 0; any_step != 0;) {
+                uint64_t stuck[CH];
+                // (the entries of all the lane's scans are requested before the first is worked on: one memory
+                // round trip per round, not CH)
+                Chunk pc[CH];
+#pragma unroll
+                for (int c = 0; c < CH; ++c) {
+                    stuck[c] = 0;
+                    load_chunk_flat(pc[c], xs, pr, in_mask(step[c]) ? kcur[c] : 0);
+                }
+                for_each_phase<CH>([&](auto c_c) {
+                    constexpr int c = decltype(c_c)::value;
+                    const uint64_t need = step[c];
+                    if (need == 0) return true;
+                    float pw[CHUNK];
+#pragma unroll
+                    for (int u = 0; u < CHUNK; ++u) pw[u] = wcol[pc[c].p[u] * COLS + c];
+                    const float w0 = wsum[c], y0 = ysum[c], x7 = pc[c].x[CHUNK - 1];
+                    const int k_start = kcur[c];
+                    float x_exit;
+                    const float slack = __fmaf_rn(FILTER_END_Y, fabsf(y0), __fmaf_rn(x7 * FILTER_END_XW, fabsf(w0), x7 * end_w));
+                    const uint64_t exited = close_chunk_vector<WANT_K>(wsum[c], ysum[c], kcur[c], x_exit, need & sure[c], pc[c].x, pw, slack);
+                    uint64_t positive = ballot(wsum[c] > 0.0f), now_fired = positive;
+                    uint64_t closed = exited & positive & ballot(ysum[c] <= x_exit * wsum[c]);
+                    const uint64_t redo = need & (~sure[c] | (exited & ~closed));
+                    if (!WANT_K) kcur[c] = in_mask(need & ~closed) ? k_start + CHUNK : k_start;
+                    if (redo != 0) {
+                        const bool mine = in_mask(redo);
+                        wsum[c] = mine ? w0 : wsum[c];
+                        ysum[c] = mine ? y0 : ysum[c];
+                        const bool fired0 = in_mask((sure[c] & ballot(w0 > 0.0f)) | (~sure[c] & fired[c]));
+                        float ya = wsum[c] < 0.0f ? -ysum[c] : ysum[c];
+                        float yg = fired0 ? ya : INFINITY;
+                        uint64_t unused = 0;
+                        int kc = k_start;
+                        scan_chunk_vector<true>(wsum[c], ysum[c], ya, yg, kc, unused, redo, pc[c].x, pw);
+                        kcur[c] = mine ? kc : kcur[c];
+                        const uint64_t gone = redo & ballot(kc != k_start + CHUNK);            // closed before its last input
+                        closed |= gone;
+                        positive = ballot(wsum[c] > 0.0f);
+                        now_fired = (now_fired & ~redo) | (redo & (gone | ballot(yg < INFINITY)));
+                        sure[c] &= ~redo;
+                    }
+                    const uint64_t ahead = ballot(x7 >= 0.0f);                  // the inputs behind this chunk are not negative
+                    const uint64_t more = need & ~closed & ballot(kcur[c] + CHUNK <= n_full);
+                    const uint64_t back = round >= 2 ? more & ahead & ~(now_fired ^ positive) : 0;
+                    fired[c] = (fired[c] & ~need) | (now_fired & need);
+                    fin[c] |= need & closed;
+                    armed[c] |= back;
+                    step[c] = more & ~back;
+                    stuck[c] = step[c] & ~now_fired & positive & ahead;
+                    return true;
+                });
+                ++round;
+                // A scan that missed its close by a rounding is left with a positive weight sum and not fired
+                // (ysum - x*wsum < 0) -- one in about 1e5.  It cannot fire, let alone close, while the weight
+                // sum stays positive, and would walk on here to the end of its row, a chunk per round, in
+                // a wavefront that is alone by then.  In rounds 1, 2, 4, 8, ... the wavefront looks
+                // ahead for it (never_fires): if the weight sum stays positive to the end, the scan is done.
+                // (256 -> 256 channels on 14x14, 32 images, 2304 inputs: 536 -> 500 us.)
+                if ((round & (round - 1)) == 0) {
+                    for (;;) {
+                        uint64_t lanes = 0;
+                        int c_now = 0, k = 0;
+                        float ws = 0.0f, ys = 0.0f;
+                        for_each_phase<CH>([&](auto c_c) {
+                            constexpr int c = decltype(c_c)::value;
+                            if (stuck[c] == 0) return true;
+                            lanes = stuck[c];
+                            c_now = c; k = kcur[c]; ws = wsum[c]; ys = ysum[c];
+                            stuck[c] &= stuck[c] - 1;
+                            return false;
+                        });
+                        if (lanes == 0) break;
+                        const int src = __builtin_ctzll(lanes);
+                        const size_t row0 = (size_t)__builtin_amdgcn_readlane(seg, src) * stride;
+                        const bool never = never_fires<COLS>(
+                            sorted + row0, perm + row0, wl + CH * (src % LANES) + c_now, __builtin_amdgcn_readlane(k, src),
+                            __builtin_amdgcn_readlane(n_seg, src), __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ws), src)),
+                            __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ys), src)), lane);
+                        const uint64_t bit = ballot(never) != 0 ? lanes & -lanes : 0;             // (a uniform value)
+                        for_each_phase<CH>([&](auto c_c) {
+                            constexpr int c = decltype(c_c)::value;
+                            fin[c] |= c == c_now ? bit : 0;
+                            step[c] &= ~(c == c_now ? bit : 0);
+                            return true;
+                        });
+                    }
+                }
+                any_step = 0;
+#pragma unroll
+                for (int c = 0; c < CH; ++c) any_step |= step[c];
+            }
+            any_armed = 0;
+#pragma unroll
+            for (int c = 0; c < CH; ++c) any_armed |= armed[c];
+            if (any_armed == 0) break;
+            kmin = NONE;
+#pragma unroll
+            for (int c = 0; c < CH; ++c) kmin = in_mask(armed[c]) ? min(kmin, kcur[c]) : kmin;
+#pragma unroll
+            for (int d = kWave / 2; d > 0; d >>= 1) kmin = min(kmin, __shfl_xor(kmin, d, kWave));
+            kmin = __builtin_amdgcn_readfirstlane(kmin);
+            request_first(kmin);
         }
+
+        // Whatever is left of a row -- fewer than eight inputs behind the full chunks -- step by step, then
+        // the output.  (Rows are padded beyond their length, so the eight entries from n_full on can always be
+        // read.)
+        const uint64_t leftover = ballot(n_full < n_seg);
+        uint64_t any_left = 0;
+#pragma unroll
+        for (int c = 0; c < CH; ++c) any_left |= ~fin[c] & leftover;
+        if (any_left != 0) {
+            Chunk tail;
+            load_chunk_flat(tail, xs, pr, n_full < n_seg ? n_full : 0);
+            for_each_phase<CH>([&](auto c_c) {
+                constexpr int c = decltype(c_c)::value;
+                const uint64_t start = ~fin[c] & leftover;
+                uint64_t run = start;
+                if (run == 0) return true;
+                float tw[CHUNK - 1];
+#pragma unroll
+                for (int u = 0; u < CHUNK - 1; ++u) tw[u] = wcol[tail.p[u] * COLS + c];
+                float ya = wsum[c] < 0.0f ? -ysum[c] : ysum[c];
+                float yg = in_mask(fired[c]) ? ya : INFINITY;
+                uint64_t closed = 0;
+                for_each_phase<CHUNK - 1>([&](auto u_c) {
+                    constexpr int u = decltype(u_c)::value;
+                    if (u > 0) run &= ballot(n_full + u < n_seg);
+                    if (run == 0) return false;
+                    scan_step_vector(wsum[c], ysum[c], ya, yg, kcur[c], run, tail.x[u], tw[u]);
+                    const uint64_t gone = run & ballot(kcur[c] == n_full + u);                 // did not consume the input
+                    closed |= gone;
+                    run &= ~gone;
+                    return true;
+                });
+                fired[c] = (fired[c] & ~start) | (start & (closed | ballot(yg < INFINITY)));
+                return true;
+            });
+        }
+        float y[CH], r[CH];
 #pragma unroll
         for (int c = 0; c < CH; ++c) {
-            if (!live[c]) continue;
-            // (a scan that stands before the full chunks' end here does not occur; it would be walked like this)
-            for (int k = kc[c]; k < n_seg && still[c]; ++k) {
-                still[c] = scan_step(st[c], xs[k], wcol[pr[k] * COLS + c]);
-                if (still[c]) ++kc[c];
+            y[c] = np.max_time; r[c] = 0.0f;
+            if (in_mask(fired[c])) {
+                r[c] = 1.0f / wsum[c];
+                y[c] = ysum[c] * r[c];
+                if (y[c] >= np.max_time) { y[c] = np.max_time; r[c] = 0.0f; }
             }
-            float y = np.max_time, r = 0.0f;
-            if (st[c].fired) {
-                r = 1.0f / st[c].wsum;
-                y = st[c].ysum * r;
-                if (y >= np.max_time) { y = np.max_time; r = 0.0f; }
+        }
+        if (seg_raw < S) {
+            const size_t o = (size_t)seg * J + j;
+            store_columns<CH>(y_out + o, y, J - j, J);
+            store_columns<CH>(rcp_out + o, r, J - j, J);
+            if (copy.dst) store_columns<CH>(copy.dst + time_copy_pixel(copy, seg) * J + j, y, J - j, J);
+            if (WANT_K) {
+#pragma unroll
+                for (int c = 0; c < CH; ++c)
+                    if (j + c < J) k_out[o + c] = (in_mask(fired[c]) && r[c] != 0.0f) ? kcur[c] : -1;
             }
-            const size_t o = (size_t)seg * J + j + c;
-            y_out[o] = y;
-            rcp_out[o] = r;
-            if (copy.dst) copy.dst[time_copy_pixel(copy, seg) * J + j + c] = y;
-            if (WANT_K) k_out[o] = (st[c].fired && r != 0.0f) ? kc[c] : -1;
         }
     }
 }
@@ -1361,21 +1432,44 @@ unpad_rows_kernel(const float* __restrict__ sorted, const int32_t* __restrict__ 
 }  // namespace
 
 namespace {
-// Neurons per lane of the instantiation for large launches: two (four need 151 registers: too few
-// wavefronts per SIMD, measured slower), except with 8-column slices, whose 32-byte weight rows make
-// the 8-byte reads of two-neuron lanes collide in the LDS banks (sixteen rows per read on four bank
-// groups): one neuron per lane reads eight rows at 4 bytes a lane.
-constexpr int filter_ch(int cols) { return cols == 8 ? 1 : 2; }
+// Neurons per lane of the instantiations: one, two or four; two at most with 8-column slices (a quad of lanes has
+// to stay within one segment).
+template <int COLS>
+constexpr int FILTER_MAX_CH = COLS == 8 ? 2 : 4;
+
+// How many of them a launch of S segments of I inputs uses: the form with the smallest estimated time.  A SIMD
+// works on its wavefronts four at a time; the time of a chunk with w of them at work and the fixed share of an
+// item (first requests, evaluation of the closing chunks, leftover inputs, output) in chunks are measured
+// (in 10 ns and chunks; 784 -> 800 at 32 ... 4096 rows, 27- to 4608-input patches).  More neurons per lane cost
+// less per neuron where wavefronts abound, fewer where a SIMD gets one or two wavefronts of long rows or the
+// rows are short.  With a single slice of at most 32 columns the rows come from HBM once: quads hold three
+// chunks ahead of the one at work, too few bytes in flight for that.
+template <int COLS>
+int filter_neurons(int64_t S, int64_t I, int n_slices, int cus) {
+    static const int chunk_time[3][4] = {{17, 20, 25, 30}, {23, 29, 36, 43}, {39, 48, 58, 69}};
+    static const int fixed_chunks[3] = {8, 10, 17};
+    int best = 1;
+    int64_t best_time = INT64_MAX;
+    for (int k = 0, ch = 1; ch <= FILTER_MAX_CH<COLS>; ++k, ch *= 2) {
+        if (ch > 1 && n_slices == 1 && COLS <= 32 && COLS / ch < 16) break;
+        const int64_t segs = kWave / COLS * ch;
+        const int64_t waves = ((S + segs - 1) / segs * n_slices + cus * 4 - 1) / (cus * 4);       // per SIMD
+        const int64_t t = (waves / 4 * chunk_time[k][3] + (waves % 4 ? chunk_time[k][waves % 4 - 1] : 0)) * (I / CHUNK + fixed_chunks[k]);
+        if (t < best_time) { best_time = t; best = ch; }
+    }
+    return best;
+}
+constexpr size_t FILTER_WIDE_COPY_BYTES = 48 * 1024;        // slices from here on are copied by 16 wavefronts
 
 template <int COLS>
 int raise_scan_lds_limits() {
     const void* whole[] = {
-        reinterpret_cast<const void*>(scan_lds_kernel<COLS, true>),
-        reinterpret_cast<const void*>(scan_lds_kernel<COLS, false>),
         reinterpret_cast<const void*>(scan_filter_kernel<COLS, 1, true>),
         reinterpret_cast<const void*>(scan_filter_kernel<COLS, 1, false>),
-        reinterpret_cast<const void*>(scan_filter_kernel<COLS, filter_ch(COLS), true>),
-        reinterpret_cast<const void*>(scan_filter_kernel<COLS, filter_ch(COLS), false>)};
+        reinterpret_cast<const void*>(scan_filter_kernel<COLS, 2, true>),
+        reinterpret_cast<const void*>(scan_filter_kernel<COLS, 2, false>),
+        reinterpret_cast<const void*>(scan_filter_kernel<COLS, FILTER_MAX_CH<COLS>, true>),
+        reinterpret_cast<const void*>(scan_filter_kernel<COLS, FILTER_MAX_CH<COLS>, false>)};
     for (const void* k : whole)
         SNNTC_HIP_CHECK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_SCAN_BYTES));
     const void* split[] = {reinterpret_cast<const void*>(scan_lds_split_kernel<COLS, true>),
@@ -1433,74 +1527,52 @@ int launch_scan_lds(const float* sorted, const int32_t* perm, const int32_t* n_r
     SNNTC_HIP_CHECK(hipGetDevice(&dev));
     const int prep = scan_prepare_device(dev, &cus);
     if (prep) return prep;
-    constexpr int SEGS = kWave / COLS;
     const int n_slices = (int)((J + COLS - 1) / COLS);
-    const int64_t items = (S + SEGS - 1) / SEGS;
-    // workgroups the chip holds at once (two per CU when two weight slices fit in its LDS)
-    const int wgs_per_cu = (lds_bytes + filter_extra_lds(COLS, 1, 16)) * 2 <= (size_t)LDS_SCAN_BYTES ? 2 : 1;
-    const int64_t capacity = (int64_t)cus * wgs_per_cu;
-    // A launch whose work items all find a wavefront of their own in workgroups of four (one
-    // wavefront per SIMD of a CU, and four times the threads of a single wavefront for copying the
-    // weight slice) runs the low-latency instantiation: the same work packed into a few full
-    // workgroups would leave most of the chip idle.  Larger launches get the workgroup size, 4 to
-    // 16 wavefronts, that spreads them over all CUs in one go.
-    const bool low_latency = (items + 3) / 4 * n_slices <= capacity;
-    int WAVES = LOW_LATENCY_THREADS / kWave;
-    if (!low_latency) {
-        const int64_t per_wg = (items * n_slices + capacity - 1) / capacity;
-        WAVES = (int)(per_wg >= 16 ? 16 : (per_wg + 3) / 4 * 4);
-    }
-    // With at least four wavefronts of multi-neuron lanes for every SIMD, CH neurons per lane (CH times
-    // the segments per wavefront) is the cheaper instruction stream; in between, one neuron per
-    // lane in 16-wave workgroups balances better -- as long as those workgroups fit the chip in one
-    // go: once one-neuron lanes would need a second round of workgroups, the multi-neuron form, which
-    // still fits, is the faster one (800 x 800 at B = 384: 55 against 79 us).
-    constexpr int CH = filter_ch(COLS);
-    const int64_t multi_items = (S + CH * SEGS - 1) / (CH * SEGS);
-    const bool multi = !low_latency && (multi_items * n_slices >= (int64_t)cus * 4 * 4 ||
-                                        (CH > 1 && items * n_slices > capacity * 16));
-    if (multi) {
-        const int64_t per_wg = (multi_items * n_slices + capacity - 1) / capacity;
-        WAVES = (int)(per_wg >= 16 ? 16 : (per_wg + 3) / 4 * 4);
-    }
     // Fewer items than CUs: a whole workgroup per item, its wavefronts sharing the item's tests.
     constexpr int SPLIT_SEGS = split_lanes(COLS) / COLS;
     const int64_t split_items = (S + SPLIT_SEGS - 1) / SPLIT_SEGS;
     const size_t split_lds = split_lds_bytes(split_lanes(COLS), SPLIT_SEGS, (int)stride);
-    const bool split = low_latency && split_items * n_slices <= (int64_t)cus && I >= 2 * CHUNK * SPLIT_WAVES &&
+    const bool split = split_items * n_slices <= (int64_t)cus && I >= 2 * CHUNK * SPLIT_WAVES &&
                        split_lds + SPLIT_STATIC_LDS <= (size_t)LDS_SCAN_BYTES &&
                        // the gather addresses W by 24-bit multiplies and a 32-bit byte offset
                        I + np.bias < (1 << 24) && J < (1 << 22) && (I + np.bias) * J * 4 < 0x7fffffffLL;
-    if (split) WAVES = 1;                                   // items per workgroup pass
-    const int64_t work_items = split ? split_items : multi ? multi_items : items;
-    const bool filt = !(split || low_latency);
-    if (filt) {
-        // the chunk buffers of the wavefronts share the LDS with the slice: fewer wavefronts where it is tight
-        // (LDS_SCAN_TARGET leaves room for four)
-        while (WAVES > 4 && lds_bytes + filter_extra_lds(COLS, multi ? CH : 1, WAVES) > (size_t)LDS_SCAN_BYTES) WAVES -= 4;
+    if (split) {
+        const int64_t n_groups = split_items < cus / n_slices ? split_items : cus / n_slices;
+        auto kern = causal_k ? scan_lds_split_kernel<COLS, true> : scan_lds_split_kernel<COLS, false>;
+        {
+            KernelTimerScope timer_("scan", stream);
+            hipLaunchKernelGGL(kern, dim3((unsigned)(n_slices * n_groups)), dim3(SPLIT_THREADS), split_lds, stream, sorted, perm,
+                               n_real, w, y, rcp, causal_k, (int)S, (int)I, (int)stride, (int)J, n_slices, (int)n_groups, np,
+                               copy);
+        }
+        SNNTC_HIP_CHECK(hipGetLastError());
+        return SNNTC_OK;
     }
-    // split the segments so that slices x groups covers the chip without a second round of workgroups
+
+    const int ch = filter_neurons<COLS>(S, I, n_slices, cus);
+    const int segs = kWave / COLS * ch;                     // segments per wavefront
+    const int64_t items = (S + segs - 1) / segs;
+    // One workgroup per CU (its 16 wavefronts take all registers; small slices let two of up to eight share a CU),
+    // and as many of them as there are items for: a CU that holds few wavefronts of its own copies the slice
+    // with a full workgroup all the same.
+    const int64_t per_cu = (items * n_slices + cus - 1) / cus;
+    const bool shared = per_cu <= 8 && (lds_bytes + FILTER_RED_BYTES) * 2 <= (size_t)LDS_SCAN_BYTES;
+    const int64_t capacity = (int64_t)cus * (shared ? 2 : 1);
+    const int64_t per_wg = (items * n_slices + capacity - 1) / capacity;
+    const int waves = (int)(per_wg >= 16 ? 16 : (per_wg + 3) / 4 * 4);
     int64_t n_groups = capacity / n_slices;
-    const int64_t max_groups = (work_items + WAVES - 1) / WAVES;
+    const int64_t max_groups = (items + waves - 1) / waves;
     if (n_groups > max_groups) n_groups = max_groups;
     if (n_groups < 1) n_groups = 1;
-    auto kern_k = filt ? (multi ? scan_filter_kernel<COLS, CH, true> : scan_filter_kernel<COLS, 1, true>)
-                  : split ? scan_lds_split_kernel<COLS, true> : scan_lds_kernel<COLS, true>;
-    auto kern = filt ? (multi ? scan_filter_kernel<COLS, CH, false> : scan_filter_kernel<COLS, 1, false>)
-                : split ? scan_lds_split_kernel<COLS, false> : scan_lds_kernel<COLS, false>;
-    dim3 grid((unsigned)(n_slices * n_groups)), block((unsigned)((split && !filt) ? SPLIT_THREADS : WAVES * kWave));
+    const int threads = lds_bytes > FILTER_WIDE_COPY_BYTES && !shared ? LDS_SCAN_THREADS : waves * kWave;
+    auto kern = ch == 1   ? (causal_k ? scan_filter_kernel<COLS, 1, true> : scan_filter_kernel<COLS, 1, false>)
+                : ch == 2 ? (causal_k ? scan_filter_kernel<COLS, 2, true> : scan_filter_kernel<COLS, 2, false>)
+                          : (causal_k ? scan_filter_kernel<COLS, FILTER_MAX_CH<COLS>, true> : scan_filter_kernel<COLS, FILTER_MAX_CH<COLS>, false>);
     {
         KernelTimerScope timer_("scan", stream);
-        const size_t dyn_lds = filt ? lds_bytes + filter_extra_lds(COLS, multi ? CH : 1, WAVES) : split ? split_lds : lds_bytes;
-        if (dyn_lds > (size_t)LDS_SCAN_BYTES)
-            return fail(SNNTC_ERR_UNSUPPORTED, "scan: %zu bytes of LDS for %d rows x %d columns exceed the %d available",
-                        dyn_lds, (int)(I + np.bias), COLS, LDS_SCAN_BYTES);
-        if (causal_k)
-            hipLaunchKernelGGL(kern_k, grid, block, dyn_lds, stream, sorted, perm, n_real, w, y, rcp, causal_k,
-                               (int)S, (int)I, (int)stride, (int)J, n_slices, (int)n_groups, np, copy);
-        else
-            hipLaunchKernelGGL(kern, grid, block, dyn_lds, stream, sorted, perm, n_real, w, y, rcp, causal_k,
-                               (int)S, (int)I, (int)stride, (int)J, n_slices, (int)n_groups, np, copy);
+        hipLaunchKernelGGL(kern, dim3((unsigned)(n_slices * n_groups)), dim3((unsigned)threads), lds_bytes + FILTER_RED_BYTES, stream,
+                           sorted, perm, n_real, w, y, rcp, causal_k, (int)S, (int)I, (int)stride, (int)J, n_slices, (int)n_groups,
+                           waves, np, copy);
     }
     SNNTC_HIP_CHECK(hipGetLastError());
     return SNNTC_OK;
@@ -1515,8 +1587,6 @@ int launch_scan(const float* sorted, const int32_t* perm, const int32_t* n_real,
     int cols = 64;
     while (cols > 8 && (rows * cols * sizeof(float) > (size_t)LDS_SCAN_TARGET || cols / 2 >= J)) cols >>= 1;
     const size_t lds_bytes = rows * cols * sizeof(float);
-    // (LDS_SCAN_TARGET, not the full 160 KB: whichever LDS kernel the launch shape selects must find room for
-    // its chunk buffers behind the slice -- 8-column slices of 5055..5120 rows would fit on their own only)
     if (lds_bytes <= (size_t)LDS_SCAN_TARGET) {
         switch (cols) {
             case 64: return launch_scan_lds<64>(sorted, perm, n_real, w, y, rcp, causal_k, S, I, stride, J, np, copy, lds_bytes, stream);

@@ -1,0 +1,59 @@
+"""The margin-filtered scan in each of its forms -- one, two or four neurons per lane, rows spread over sixteen
+lanes or over quads -- at the edges of its rounds, chunks, slices and wavefronts, bit for bit against the oracle."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import dense_case
+from oracle import capi
+from test_gpu_parity import _adversarial_dense
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def t(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).to(DEV)
+
+
+def _check(x, w, p):
+    import snntc_amd as snn
+    ref_out, ref_k, _, _ = capi.fc_forward_dev(x, w, p, want_aux=True)
+    out, _, _, ck = snn.snnfc(t(x), t(w), p, return_aux=True)
+    out2 = snn.snnfc(t(x), t(w), p)
+    torch.cuda.synchronize()
+    assert np.array_equal(ck.cpu().numpy(), ref_k), "causal-set sizes differ"
+    assert np.array_equal(out.cpu().numpy().view(np.uint32), ref_out.view(np.uint32)), "y / 1/S not bit-exact"
+    assert torch.equal(out, out2)
+
+
+@pytest.mark.parametrize("B,I,J", [
+    (20011, 31, 64), (20011, 33, 63), (12007, 72, 128),     # 64-column slices, four neurons: below, above, between rounds
+    (9001, 7, 50), (9001, 8, 50), (9001, 9, 50), (9001, 1, 40),          # rows of less than a chunk, one, one and a bit
+    (6007, 650, 96), (3001, 785, 101),                      # 32-column slices: quads, and a ragged last slice
+    (6007, 1301, 37), (700, 2305, 66),                      # 16-column slices
+    (1500, 4600, 9), (40, 4601, 23),                        # 8-column slices, many wavefronts and few
+    (1100, 400, 200), (300, 500, 70),                       # two neurons and one
+])
+def test_scan_forms(B, I, J):
+    """A tenth of the inputs (and all of every fiftieth row) never spiked, so rows of one wavefront differ in length."""
+    x, w, p, _ = dense_case(B + I, B, I, J, True, "baseline")
+    rng = np.random.default_rng(I)
+    x[rng.random(x.shape) < 0.1] = 1e5
+    x[::50] = 2e5
+    _check(x, w, p)
+
+
+@pytest.mark.parametrize("kind,B,I,J", [("randn", 20000, 90, 64), ("ties", 12000, 100, 61), ("negative", 9000, 75, 64),
+                                        ("bias_fires", 9000, 131, 64), ("late", 9000, 330, 32), ("sparse", 4000, 700, 40)])
+def test_four_neuron_lanes_off_the_common_path(kind, B, I, J):
+    x, w = _adversarial_dense(kind, 3, B, I, J)
+    _check(x, w, capi.fc_params(1.0))
+
+
+def test_scans_that_miss_their_close_by_a_rounding():
+    """Among 1.5 million scans about a dozen pass their closing time unnoticed (the sums round the wrong way): they are
+    left with a positive weight sum, not fired, and must be carried to the end of their rows, where practically all
+    of them stay silent."""
+    x, w, p, _ = dense_case(5, 24000, 600, 64, True, "baseline")
+    _check(x, w, p)
