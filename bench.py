@@ -251,8 +251,7 @@ def account(torch, snn, layers, extras=None):
     """Per kernel name: algorithmic fp32 flops and HBM bytes of one step, from the causal-set sizes the
     forward actually produces.  Formulas (S segments of length I, J outputs, b = bias flag):
       steps = sum over (s,j) of consumed inputs + b ;   pairs = sum over fired (s,j) of (k + b)
-      sort_segments : bytes 4*(in + 2*S*I), or 4*3*in when only the pixels' channels are sorted (merge path)
-      merge_patches : bytes 4*(2*in + 2*S*I)                       flops 0 (comparisons are not flops)
+      sort_segments (dense rows, 1x1 patches), order_patches : bytes 4*(in + 2*S*I)   flops 0 (comparisons are not flops)
       scan          : bytes 4*(2*S*I + (I+b)*J + 2*S*J)            flops 4*steps
       dX kernels    : bytes 4*(2*S*J + in + I*J + in)              flops 2*pairs
       grad_weight   : bytes 4*(2*S*J + in + (I+b)*J)               flops 3*pairs
@@ -282,7 +281,7 @@ def account(torch, snn, layers, extras=None):
                 x_op = inp
                 _, sz, _, ck = snn.snnfc(x_op, W, layer.Params, return_aux=True)
                 max_t, bias = float(layer.Params[0]), int(layer.Params[5] > 1e-8)
-                merged = False
+                order = "sort_segments"
             else:
                 x_op = inp
                 if padded is not True:               # a network layer: the layer pads (SAME) or crops (VALID) first;
@@ -291,7 +290,7 @@ def account(torch, snn, layers, extras=None):
                         add("pad_time", 0.0, 4.0 * (inp.numel() + x_op.numel()))
                 _, sz, _, ck = snn.snncv(x_op, W, layer.Params, return_aux=True)
                 max_t, bias = float(layer.Params[0]), int(layer.Params[11] > 1e-8)
-                merged = layer.C >= 32 and layer.C % 4 == 0 and layer.Kw >= 2
+                order = "order_patches" if layer.Kh * layer.Kw > 1 and sz.shape[1] <= 8192 else "sort_segments"
         S, I = sz.shape
         J = ck.shape[1]
         n_real = (sz <= np.float32(max_t) - np.float32(0.1)).sum(dim=1, keepdim=True)
@@ -300,11 +299,7 @@ def account(torch, snn, layers, extras=None):
         steps = float((consumed + bias).sum().item())
         pairs = float((torch.where(fired, ck, torch.zeros_like(ck)) + bias * fired).sum().item())
         n_in = float(x_op.numel())
-        if merged:
-            add("sort_segments", 0.0, 4.0 * 3.0 * n_in)
-            add("merge_patches", 0.0, 4.0 * (2.0 * n_in + 2.0 * S * I))
-        else:
-            add("sort_segments", 0.0, 4.0 * (n_in + 2.0 * S * I))
+        add(order, 0.0, 4.0 * (n_in + 2.0 * S * I))
         add("scan", 4.0 * steps, 4.0 * (2.0 * S * I + (I + bias) * J + 2.0 * S * J))
         if dense and J <= 16:
             add("fc_backward_narrow", 5.0 * pairs + S * J, 4.0 * (3.0 * S * J + 2.0 * n_in + 2.0 * (I + bias) * J))

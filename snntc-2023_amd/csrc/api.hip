@@ -131,22 +131,19 @@ int fc_check(int64_t B, int64_t I, int64_t J, int64_t w_rows, const float* param
     return SNNTC_OK;
 }
 
-// Forward scratch.  n_pix / pix_c > 0 adds the per-pixel sorted channels the conv merge path needs.
+// Forward scratch.
 struct FcFwdWs {
-    float* sorted; int32_t* perm; int32_t* n_real; float* pix_z; int32_t* pix_c;
+    float* sorted; int32_t* perm; int32_t* n_real;
     void* long_keys;                                      // merge passes of segments longer than one network
-    int64_t stride, pix_stride; size_t bytes;
+    int64_t stride; size_t bytes;
 };
-FcFwdWs fc_fwd_ws(void* ws, int64_t S, int64_t I, int64_t n_pix = 0, int64_t pix_c = 0) {
+FcFwdWs fc_fwd_ws(void* ws, int64_t S, int64_t I) {
     Carver c(ws);
     FcFwdWs r;
     r.stride = padded_stride(I);
-    r.pix_stride = padded_stride(pix_c);
     r.sorted = c.take<float>(S * r.stride);
     r.perm = c.take<int32_t>(S * r.stride);
     r.n_real = c.take<int32_t>(S);
-    r.pix_z = c.take<float>(n_pix * r.pix_stride);
-    r.pix_c = c.take<int32_t>(n_pix * r.pix_stride);
     const size_t long_bytes = sort_long_workspace_bytes(S, I);
     r.long_keys = long_bytes ? c.take<unsigned char>((int64_t)long_bytes) : nullptr;
     r.bytes = c.used;
@@ -274,21 +271,14 @@ int cv_forward_impl(const float* xpad, const float* w, const float* params, floa
     }
     if (g.S == 0 || Kc == 0) return SNNTC_OK;
     if (!xpad || !w || !out) return fail(SNNTC_ERR_BAD_ARGUMENT, "snntc_cv_forward: NULL tensor pointer");
-    const bool merge = merge_sort_supported(g);
-    FcFwdWs ws = fc_fwd_ws(workspace, g.S, g.P, merge ? B * H * W : 0, merge ? C : 0);
+    FcFwdWs ws = fc_fwd_ws(workspace, g.S, g.P);
     rc = check_workspace(workspace, workspace_bytes, ws.bytes);
     if (rc) return rc;
     hipStream_t st = static_cast<hipStream_t>(stream);
     const NeuronParams np = neuron_params(params[0], params[4], params[11]);
-    if (!merge)
+    if (!order_patches_supported(g))
         return forward_chain(conv_source(xpad, g), ws, w, out, sorted_z, perm, causal_k, g.S, g.P, Kc, np, copy, st);
-    // sort every pixel's channels once, then assemble the patches by rank merging
-    SegmentSource pixels{};
-    pixels.base = xpad; pixels.conv = 0; pixels.I = (int)C;
-    rc = launch_sort(pixels, B * H * W, ws.pix_z, ws.pix_c, nullptr, (int)ws.pix_stride, np.max_cmp, nullptr, st);
-    if (rc) return rc;
-    rc = launch_merge_patches(ws.pix_z, ws.pix_c, ws.pix_stride, ws.sorted, ws.perm, ws.n_real, g, ws.stride,
-                              np.max_cmp, st);
+    rc = launch_order_patches(xpad, ws.sorted, ws.perm, ws.n_real, g, ws.stride, np.max_cmp, st);
     if (rc) return rc;
     rc = launch_unpad_rows(ws.sorted, ws.perm, sorted_z, perm, g.S, g.P, ws.stride, st);
     if (rc) return rc;
@@ -313,7 +303,7 @@ int prepare_device(int dev, void** scratch_out) {
     std::lock_guard<std::mutex> lock(g_init_mutex);
     if (!g_scratch_ptr[dev]) {
         int rc = scan_prepare_device(dev, nullptr);
-        if (!rc) rc = merge_prepare_device(dev);
+        if (!rc) rc = order_prepare_device();
         if (rc) return rc;
         void* ptr = nullptr;
         SNNTC_HIP_CHECK(hipGetSymbolAddress(&ptr, HIP_SYMBOL(::scratch)));
@@ -705,8 +695,7 @@ int snntc_cv_forward_workspace_bytes(int64_t B, int64_t H, int64_t W, int64_t C,
     int rc = cv_geom(B, H, W, C, Kc, 0, params_host, false, "snntc_cv_forward_workspace_bytes", &g);
     if (rc) return rc;
     if (!bytes) return fail(SNNTC_ERR_BAD_ARGUMENT, "snntc_cv_forward_workspace_bytes: bytes is NULL");
-    const bool merge = merge_sort_supported(g);
-    *bytes = fc_fwd_ws(nullptr, g.S, g.P, merge ? B * H * W : 0, merge ? C : 0).bytes;
+    *bytes = fc_fwd_ws(nullptr, g.S, g.P).bytes;
     return SNNTC_OK;
 }
 

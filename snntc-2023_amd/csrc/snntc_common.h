@@ -147,11 +147,10 @@ size_t sort_long_workspace_bytes(int64_t S, int64_t I);
 int launch_sort(const SegmentSource& src, int64_t S, float* sorted, int32_t* perm, int32_t* n_real,
                 int out_stride, float max_cmp, void* long_ws, hipStream_t stream);
 
-// Conv patch sort by merging pre-sorted pixels (merge.hip): pix_z / pix_c are the [B*H*W, Cs] outputs
-// of launch_sort on the image's pixels.
-bool merge_sort_supported(const ConvGeom& g);
-int launch_merge_patches(const float* pix_z, const int32_t* pix_c, int64_t Cs, float* sorted, int32_t* perm,
-                         int32_t* n_real, const ConvGeom& g, int64_t stride, float max_cmp, hipStream_t stream);
+// Conv patches in ascending order (order.hip), every image region ranked once for all patches over it.
+bool order_patches_supported(const ConvGeom& g);
+int launch_order_patches(const float* xpad, float* sorted, int32_t* perm, int32_t* n_real, const ConvGeom& g, int64_t stride,
+                         float max_cmp, hipStream_t stream);
 
 // Copies the first I entries of every padded row into dense [S,I] arrays (either may be NULL).
 int launch_unpad_rows(const float* sorted, const int32_t* perm, float* sorted_out, int32_t* perm_out,
@@ -170,10 +169,10 @@ void set_scan_wait_polls(int polls);
 int read_scan_giveups(int64_t* count, hipStream_t stream);
 
 // One-time set-up on device `dev`, which must be the current device: the dynamic-LDS limits of every
-// scan / merge instantiation (and the CU count the scan sizes its launches with).  The launchers call
+// scan / ordering instantiation (and the CU count the scan sizes its launches with).  The launchers call
 // them on their first use of a device; snntc_init() calls them ahead of time.
 int scan_prepare_device(int dev, int* cu_count_out);
-int merge_prepare_device(int dev);
+int order_prepare_device();
 
 // upm = valid ? grad*rcp : 0   (valid: y <= MAX-0.1; n elements), and, in the same launch, the weight copy dX reads from: mode 0 none, mode 1
 // wt[cols, rows] = w[rows, cols]^T, mode 2 the regrouped copy of a conv layer's weights
