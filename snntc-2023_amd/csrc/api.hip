@@ -165,16 +165,15 @@ int forward_chain(const SegmentSource& src, const FcFwdWs& ws, const float* w, f
 // area is sized for the worst case of 256 slices only when slicing can happen at all.
 struct BwdWs { float* upm; float* wt; float* dxp; float* partial; int max_split; size_t bytes; };
 // patch_scratch: elements of the per-patch gradient of conv layers whose dX goes through patch space
-// narrow_split: slices the one-launch backward of a narrow dense layer needs (0: not that path)
+// dense_split: slices of a dense layer's dW (0: a conv layer)
 BwdWs bwd_ws(void* ws, int64_t S, int64_t rows, int64_t J, int64_t min_base_blocks, int64_t patch_scratch = 0,
-             int narrow_split = 0) {
+             int dense_split = 0) {
     Carver c(ws);
     BwdWs r;
     r.upm = c.take<float>(S * J);
-    r.wt = c.take<float>(rows * J);
+    r.wt = c.take<float>(rows * J);                        // (only conv layers use it; the size callers may rely on has room for it)
     r.dxp = c.take<float>(patch_scratch);
-    r.max_split = weight_grad_splits(S, min_base_blocks);
-    if (narrow_split > r.max_split) r.max_split = narrow_split;
+    r.max_split = dense_split > 0 ? dense_split : weight_grad_splits(S, min_base_blocks);
     r.partial = c.take<float>(r.max_split > 1 ? (int64_t)r.max_split * rows * J : 0);
     r.bytes = c.used;
     return r;
@@ -304,6 +303,7 @@ int prepare_device(int dev, void** scratch_out) {
     if (!g_scratch_ptr[dev]) {
         int rc = scan_prepare_device(dev, nullptr);
         if (!rc) rc = order_prepare_device();
+        if (!rc) rc = grad_prepare_device();
         if (rc) return rc;
         void* ptr = nullptr;
         SNNTC_HIP_CHECK(hipGetSymbolAddress(&ptr, HIP_SYMBOL(::scratch)));
@@ -582,10 +582,15 @@ static int fc_narrow_split(int64_t B, int64_t I, int64_t J) {
     return (I >= 1 && B >= 1 && fc_backward_narrow_supported(J)) ? fc_backward_narrow_splits(B) : 0;
 }
 
+static int fc_splits(int64_t B, int64_t I, int64_t J) {
+    const int narrow = fc_narrow_split(B, I, J);
+    return narrow ? narrow : grad_weight_dense_splits(B, I, J);
+}
+
 int snntc_fc_backward_workspace_bytes(int64_t B, int64_t I, int64_t J, size_t* bytes) {
     if (!bytes || B < 0 || I < 0 || J < 0)
         return fail(SNNTC_ERR_BAD_ARGUMENT, "snntc_fc_backward_workspace_bytes: bad argument");
-    *bytes = bwd_ws(nullptr, B, I + 1, J, grad_weight_blocks(I, J), 0, fc_narrow_split(B, I, J)).bytes;
+    *bytes = bwd_ws(nullptr, B, I + 1, J, 0, 0, fc_splits(B, I, J)).bytes;
     return SNNTC_OK;
 }
 
@@ -655,27 +660,24 @@ int snntc_fc_backward(const float* grad, const float* x, const float* w, const f
     }
     if (!grad || !x || !w || !oldout) return fail(SNNTC_ERR_BAD_ARGUMENT, "snntc_fc_backward: NULL tensor pointer");
     const int narrow = fc_narrow_split(B, I, J);
-    BwdWs ws = bwd_ws(workspace, B, I + 1, J, grad_weight_blocks(I, J), 0, narrow);
+    BwdWs ws = bwd_ws(workspace, B, I + 1, J, 0, 0, fc_splits(B, I, J));
     rc = check_workspace(workspace, workspace_bytes, ws.bytes);
     if (rc) return rc;
     const NeuronParams np = neuron_params(params_host[0], params_host[2], params_host[5]);
     if (narrow)                                          // a classifier head: everything in one launch
         return launch_fc_backward_narrow(x, w, grad, oldout, oldout + B * J, dx, dw, ws.partial, dparams, 6, B, I, J,
                                          np, st);
-    // wt[J, I] for dX (the bias row is not needed) is written by the same launch
-    rc = launch_backward_prologue(grad, oldout, oldout + B * J, ws.upm, B * J, np, dx ? 1 : 0, w, ws.wt, I, J,
-                                  0, dparams, 6, st);
+    rc = launch_backward_prologue(grad, oldout, oldout + B * J, ws.upm, B * J, np, w, nullptr, I, J, 0, dparams, 6, st);
     if (rc) return rc;
     if (dx) {
-        rc = launch_fc_grad_input(x, ws.wt, ws.upm, oldout, dx, B, I, J, I, st);
+        rc = launch_fc_grad_input(x, w, ws.upm, oldout, dx, B, I, J, st);
         if (rc) return rc;
     }
     if (!dw) return SNNTC_OK;
     SegmentSource src{};
     src.base = x; src.conv = 0; src.I = (int)I;
-    int nsplit = weight_grad_splits(B, grad_weight_blocks(w_rows, J));
-    if (nsplit > ws.max_split) nsplit = ws.max_split;
-    rc = launch_grad_weight_rows(src, ws.upm, oldout, nsplit > 1 ? ws.partial : dw, nsplit, B, J, 0, np, st);
+    const int nsplit = ws.max_split;
+    rc = launch_grad_weight_rows(src, ws.upm, oldout, nsplit > 1 ? ws.partial : dw, nsplit, B, J, np, st);
     if (rc) return rc;
     return launch_reduce_partials(ws.partial, dw, w_rows * J, nsplit, st);
 }
@@ -758,17 +760,16 @@ static int cv_backward_impl(const float* grad, const float* xpad, const float* w
     rc = check_workspace(workspace, workspace_bytes, ws.bytes);
     if (rc) return rc;
     const NeuronParams np = neuron_params(params_host[0], params_host[4], params_host[11]);
-    // the weight copy dX reads from is written by the same launch: regrouped for the channel kernel,
-    // wt[Kc, P] for the generic one
+    // the regrouped weight copy the channel kernel reads from is written by the same launch
     const bool chan_dx = cv_grad_input_chan_supported(g);
     rc = launch_backward_prologue(grad, oldout, oldout + g.S * Kc, ws.upm, g.S * Kc, np,
-                                  !dxpad ? 0 : chan_dx ? 2 : 1, w, ws.wt, g.P, Kc, g.C, dparams, 12, st);
+                                  w, dxpad && chan_dx ? ws.wt : nullptr, g.P, Kc, g.C, dparams, 12, st);
     if (rc) return rc;
     if (dxpad) {
         if (chan_dx) {
             rc = launch_cv_grad_input_chan(xpad, ws.wt, ws.upm, oldout, dxpad, crop, g, np, st);
         } else {
-            rc = launch_cv_grad_input(conv_source(xpad, g), ws.wt, ws.upm, oldout, ws.dxp, dxpad, crop, g, g.P, st);
+            rc = launch_cv_grad_input(conv_source(xpad, g), w, ws.upm, oldout, ws.dxp, dxpad, crop, g, st);
         }
         if (rc) return rc;
     }
@@ -781,7 +782,7 @@ static int cv_backward_impl(const float* grad, const float* xpad, const float* w
     if (wide) {
         rc = launch_cv_grad_weight_wide(xpad, ws.upm, oldout, dst, nsplit, g, w_rows, np, st);
     } else {
-        rc = launch_grad_weight_rows(src, ws.upm, oldout, dst, nsplit, g.S, Kc, 0, np, st);
+        rc = launch_grad_weight_rows(src, ws.upm, oldout, dst, nsplit, g.S, Kc, np, st);
     }
     if (rc) return rc;
     return launch_reduce_partials(ws.partial, dw, w_rows * Kc, nsplit, st);

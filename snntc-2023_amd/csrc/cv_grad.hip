@@ -642,7 +642,7 @@ static float dx_mask_scale(float max_time) {
     return ldexpf(1.0f, 126 - e);
 }
 
-// wq: the weights regrouped by launch_backward_prologue (mode 2)
+// wq: the weights regrouped by launch_backward_prologue
 int launch_cv_grad_input_chan(const float* xpad, const float* wq, const float* upm, const float* ym,
                               float* dx, const CropGeom& crop, const ConvGeom& g, const NeuronParams& np,
                               hipStream_t stream) {

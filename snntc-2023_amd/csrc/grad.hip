@@ -14,6 +14,8 @@
 // so that a term of an output that takes no part vanishes whatever its mask says (the kernels read y
 // itself, under the parameter name ym); the weight-gradient mask is folded into arithmetic: for x <= y the term (x-y) is <= 0 and
 // for x > y it is > 0, hence [x <= y](x - y) == min(x - y, 0).
+#include <atomic>
+
 #include "snntc_common.h"
 
 namespace snntc {
@@ -21,18 +23,15 @@ namespace {
 
 // First launch of a backward pass.  The elementwise pass over the layer's outputs,
 //   upm = valid ? grad * rcp : 0   (valid: y <= MAX - 0.1),
-// and the weight copy dX reads from do not depend on each other: one launch does both, the first
-// prep_blocks workgroups the former, the rest the latter.
-//   mode 1: wt[cols, rows] = w[rows, cols]^T, a 32 x 32 tile per workgroup
-//   mode 2: w[(tap, c), kc] -> wt[tap][kc / 4][c][kc % 4], one 16-byte piece per thread (cols = Kc, a
-//           multiple of 4; chan = C)
+// and the regrouped weights the channel-lane dX of conv layers reads do not depend on each other: one launch does both, the
+// first prep_blocks workgroups the former, the rest the latter.
+//   w[(tap, c), kc] -> wt[tap][kc / 4][c][kc % 4], one 16-byte piece per thread (cols = Kc, a multiple of 4; chan = C)
 __global__ void __launch_bounds__(256)
 backward_prologue_kernel(const float* __restrict__ grad, const float* __restrict__ y,
                          const float* __restrict__ rcp, float* __restrict__ upm, int64_t n, float max_cmp,
-                         int prep_blocks, int vec4, int mode, const float* __restrict__ w,
+                         int prep_blocks, int vec4, const float* __restrict__ w,
                          float* __restrict__ wt, int rows, int cols, int chan, float* __restrict__ zeros,
                          int n_zeros) {
-    __shared__ float tile[32][33];
     if (blockIdx.x == 0 && (int)threadIdx.x < n_zeros) zeros[threadIdx.x] = 0.0f;    // the dParams output
     if ((int)blockIdx.x < prep_blocks) {
         const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -55,29 +54,14 @@ backward_prologue_kernel(const float* __restrict__ grad, const float* __restrict
         return;
     }
     const int blk = (int)blockIdx.x - prep_blocks;
-    if (mode == 1) {
-        const int tiles_x = (cols + 31) / 32;
-        const int tx = threadIdx.x % 32, ty = threadIdx.x / 32;       // 32 x 8
-        const int c0 = (blk % tiles_x) * 32, r0 = (blk / tiles_x) * 32;
-        for (int dy = ty; dy < 32; dy += 8) {
-            const int r = r0 + dy, c = c0 + tx;
-            tile[dy][tx] = (r < rows && c < cols) ? w[(size_t)r * cols + c] : 0.0f;
-        }
-        __syncthreads();
-        for (int dy = ty; dy < 32; dy += 8) {
-            const int c = c0 + dy, r = r0 + tx;
-            if (r < rows && c < cols) wt[(size_t)c * rows + r] = tile[tx][dy];
-        }
-    } else {
-        const int k4 = cols / 4;
-        const int64_t t = (int64_t)blk * blockDim.x + threadIdx.x;    // over (tap, c, kc / 4), kc / 4 fastest
-        if (t >= (int64_t)rows * k4) return;
-        const int64_t row = t / k4;                                   // tap * C + c
-        const int q = (int)(t - row * k4);
-        const int64_t tap = row / chan;
-        const int c = (int)(row - tap * chan);
-        reinterpret_cast<float4*>(wt)[(tap * k4 + q) * chan + c] = reinterpret_cast<const float4*>(w)[t];
-    }
+    const int k4 = cols / 4;
+    const int64_t t = (int64_t)blk * blockDim.x + threadIdx.x;    // over (tap, c, kc / 4), kc / 4 fastest
+    if (t >= (int64_t)rows * k4) return;
+    const int64_t row = t / k4;                                   // tap * C + c
+    const int q = (int)(t - row * k4);
+    const int64_t tap = row / chan;
+    const int c = (int)(row - tap * chan);
+    reinterpret_cast<float4*>(wt)[(tap * k4 + q) * chan + c] = reinterpret_cast<const float4*>(w)[t];
 }
 
 __global__ void __launch_bounds__(256) fill_zero_kernel(float* __restrict__ p, int64_t n) {
@@ -102,136 +86,185 @@ __device__ __forceinline__ const float* segment_base(const SegmentSource& src, i
     return src.base + ((size_t)(a * src.H + nh * src.Sh) * src.W + (size_t)nw * src.Sw) * src.C;
 }
 
-// ---------------------------------------------------------------------------------------------
-// Dense dX.  Lanes run across inputs i (wt[j, i] is read coalesced), each thread carries RB
-// samples whose y/up values are wave-uniform; the four wavefronts of a block split the j range
-// and are summed through LDS in a fixed order.
-// ---------------------------------------------------------------------------------------------
-constexpr int DX_RB = 4;
-constexpr int DX_STEP = 4;
+// The wavefront's own LDS traffic in program order: what it has written so far is what it reads from here on.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
 
-// PATCHES: the "samples" are the implicit patches of a conv layer (src.conv) and the result is the
-// gradient per patch element, dx[S, P], which cv_col2im_kernel then folds back onto the image.
-template <bool PATCHES>
-__global__ void __launch_bounds__(256)
-fc_grad_input_kernel(const SegmentSource src, const float* __restrict__ wt,
-                     const float* __restrict__ upm, const float* __restrict__ ym, float* __restrict__ dx,
-                     int B, int I, int J, int wt_stride) {
-    const float* __restrict__ x = src.base;
-    __shared__ float red[3][DX_RB][kWave];
+// ---------------------------------------------------------------------------------------------
+// Dense dX.  A wavefront owns a tile of 16 samples x 32 inputs, a lane 2 x 4 of it, and walks over outputs j, 16 at a time:
+// y, up and W of its rows come in 16-byte pieces, a chunk ahead, go to a piece of LDS of the wavefront's own, transposed, and
+// come back as three reads per output, one output ahead, for 24 vector instructions.  SPLIT wavefronts share a tile's outputs
+// and are added in order through LDS; with SPLIT 1 the four wavefronts of a workgroup have tiles of their own.
+// What bounds it: the compare, multiply-add and select of a term (3.3 clocks each at 4096 samples).  Before, one input and
+// four samples per lane, a transposed copy of W streamed past scalar y / up: four samples per weight read, and lines of the
+// scalar cache fetched four times over.  us: 333 x 1521 -> 777 60 -> 46, 4096 x 784 -> 800 519 -> 239, 256 x 784 -> 800 31 ->
+// 25, 128 x 784 -> 800 20 -> 16, 16 200 patches x 500 -> 50 46 -> 27, and the copy, some 2.  (4 x 4 per lane: 228 at 4096 samples, 61
+// at 333.)
+// ---------------------------------------------------------------------------------------------
+constexpr int DX_A = 2, DX_S = 8 * DX_A, DX_I = 32, DX_JC = 16, DX_PITCH = 36;         // (pitch: the transposing writes of the pieces spread over the banks)
+constexpr int dx_threads(int split) { return (split == 1 ? 4 : split) * kWave; }
+constexpr int dx_lds_bytes(int split) { return dx_threads(split) / kWave * 3 * DX_JC * DX_PITCH * 4; }
+
+// PATCHES: the "samples" are the implicit patches of a conv layer (src.conv) and the
+// result is the gradient per patch element, dx[S, P], which cv_col2im_kernel then folds back onto the image.
+template <int SPLIT, bool PATCHES>
+__global__ void __launch_bounds__(dx_threads(SPLIT), 4)
+fc_grad_input_kernel(const SegmentSource src, const float* __restrict__ w, const float* __restrict__ upm,
+                     const float* __restrict__ ym, float* __restrict__ dx, int B, int I, int J, int tiles_i, int n_tiles) {
+    constexpr int A = DX_A, TS = DX_S, LANES = DX_JC / 4, ROWS = kWave / LANES, S_PASSES = TS / ROWS, I_PASSES = DX_I / ROWS;
+    static_assert(S_PASSES * ROWS == TS && I_PASSES * ROWS == DX_I, "whole passes");
+    extern __shared__ __align__(16) float dx_lds[];
     const int lane = threadIdx.x % kWave;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int i = blockIdx.y * kWave + lane;
-    const unsigned ic = (unsigned)min(i, I - 1);
-    const int b0 = blockIdx.x * DX_RB;
+    const int block = xcd_contiguous(blockIdx.x, gridDim.x);
+    const int tile_raw = SPLIT == 1 ? block * 4 + wave : block;
+    const int tile = min(tile_raw, n_tiles - 1);
+    const int ts = tile / tiles_i, s0 = ts * TS, i0 = (tile - ts * tiles_i) * DX_I;
+    const int sg = lane / 8, ig = lane % 8;
 
-    float xr[DX_RB], acc[DX_RB];
-    // the y / up rows of the block's samples: one base pointer each and a byte offset per sample (eight
-    // scalar registers instead of sixteen for eight pointers; samples past the batch repeat the last row)
-    const float* __restrict__ ybase = ym + (size_t)b0 * J;
-    const float* __restrict__ ubase = upm + (size_t)b0 * J;
-    int row_bytes[DX_RB];
+    float xr[A][4], acc[A][4];
 #pragma unroll
-    for (int r = 0; r < DX_RB; ++r) {
-        const int brow = min(b0 + r, B - 1);
-        xr[r] = PATCHES ? segment_base(src, brow)[row_offset(src, (int)ic)] : x[(size_t)brow * I + ic];
-        row_bytes[r] = (brow - b0) * J * (int)sizeof(float);
-        acc[r] = 0.0f;
-    }
-    const int jq = (J + 3) / 4;
-    const int j_lo = wave * jq, j_hi = min(J, j_lo + jq);
-    const float* __restrict__ wcol = wt + ic;
-    int j = j_lo;
-    // DX_STEP columns at a time.  The y / up values of the block's samples are wave-uniform and arrive
-    // through the scalar path; scalar loads return in no fixed order, so a wavefront can only wait for
-    // all of them, and a load issued right before its use costs a round trip every time.  The loop
-    // therefore runs one step ahead: wait for the values of this step (requested a step ago), request
-    // those of the next into the other set of registers, then do this step's arithmetic.  The
-    // weights (vector loads, which return in order) run one step ahead as well.
-    {
-        typedef float f4 __attribute__((ext_vector_type(4)));
-        auto request = [&](f4 (&yv)[DX_RB], f4 (&uv)[DX_RB], int jj) {
-            const int off = jj * (int)sizeof(float);
+    for (int a = 0; a < A; ++a) {
+        const int s = min(s0 + sg * A + a, B - 1);
+        const float* xs = PATCHES ? segment_base(src, s) : src.base + (size_t)s * I;
 #pragma unroll
-            for (int r = 0; r < DX_RB; ++r) {
-                const int o = row_bytes[r] + off;
-                asm volatile("s_load_dwordx4 %0, %1, %2" : "=s"(yv[r]) : "s"(ybase), "s"(o));
-                asm volatile("s_load_dwordx4 %0, %1, %2" : "=s"(uv[r]) : "s"(ubase), "s"(o));
-            }
-        };
-        auto arrived = [&](f4 (&yv)[DX_RB], f4 (&uv)[DX_RB]) {
-            asm volatile("s_waitcnt lgkmcnt(0)"
-                         : "+s"(yv[0]), "+s"(yv[1]), "+s"(yv[2]), "+s"(yv[3]), "+s"(uv[0]), "+s"(uv[1]), "+s"(uv[2]),
-                           "+s"(uv[3]));
-        };
-        auto weights = [&](float (&wv)[DX_STEP], int jj) {
-#pragma unroll
-            for (int u = 0; u < DX_STEP; ++u) wv[u] = (wt + (size_t)(jj + u) * wt_stride)[ic];
-        };
-        // acc[r] += up * w where x <= y; the others are skipped, as in the reference
-        // (snnfcgrad_kernels.cu.cc:60), not added as zeros.  (Writing the compare into EXEC and running
-        // the multiply-add under it saves the select but no time: the EXEC round trip stalls the issue.)
-        auto macs = [&](const f4 (&yv)[DX_RB], const f4 (&uv)[DX_RB], const float (&wv)[DX_STEP]) {
-#pragma unroll
-            for (int r = 0; r < DX_RB; ++r) {
-#pragma unroll
-                for (int u = 0; u < DX_STEP; ++u)
-                    acc[r] = xr[r] <= yv[r][u] ? __fmaf_rn(uv[r][u], wv[u], acc[r]) : acc[r];
-            }
-        };
-        static_assert(DX_RB == 4 && DX_STEP == 4, "register sets of the pipelined loop");
-        const int steps = (j_hi - j_lo) / DX_STEP;
-        if (steps > 0) {
-            f4 ya[DX_RB], ua[DX_RB], yb[DX_RB], ub[DX_RB];
-            float wa[DX_STEP], wb[DX_STEP];
-            const int j_last = j_lo + (steps - 1) * DX_STEP;      // requests past the last step re-read it
-            request(ya, ua, j);
-            weights(wa, j);
-            for (int sidx = 0; sidx + 2 <= steps; sidx += 2) {
-                const int jn = j + DX_STEP, jnn = min(j + 2 * DX_STEP, j_last);
-                arrived(ya, ua);
-                request(yb, ub, jn);
-                weights(wb, jn);
-                __builtin_amdgcn_sched_barrier(0);                 // requests first, then the arithmetic
-                macs(ya, ua, wa);
-                __builtin_amdgcn_sched_barrier(0);
-                arrived(yb, ub);
-                request(ya, ua, jnn);
-                weights(wa, jnn);
-                __builtin_amdgcn_sched_barrier(0);
-                macs(yb, ub, wb);
-                __builtin_amdgcn_sched_barrier(0);
-                j += 2 * DX_STEP;
-            }
-            arrived(ya, ua);                                       // nothing stays in flight
-            if (steps & 1) macs(ya, ua, wa);
-            j = j_lo + steps * DX_STEP;
+        for (int b = 0; b < 4; ++b) {
+            const int i = min(i0 + ig * 4 + b, I - 1);
+            xr[a][b] = xs[PATCHES ? row_offset(src, i) : i];
+            acc[a][b] = 0.0f;
         }
     }
-    for (; j < j_hi; ++j) {
-        const float wv = wcol[(size_t)j * wt_stride];
+    // A sample's sums must not depend on the batch it is in, so the order of its additions depends on J alone: chunk c of the
+    // outputs belongs to part c % 16, a part's chunks are added in turn, parts p and p + 8, the pairs p and p + 4, ... in a
+    // tree -- which a wavefront with parts v, v + 8 (, v + 4, v + 12) begins.  Fewer than 64 outputs are one part.
+    constexpr int PARTS = SPLIT == 1 ? 1 : 16 / SPLIT, STEP = SPLIT == 1 ? 1 : 16;
+    const int chunks = (J + DX_JC - 1) / DX_JC;
+    auto part = [&](int k) { return SPLIT == 1 ? 0 : wave + (k & 1) * 8 + (k >> 1) * 4; };
+    auto next_chunk = [&](int k, int c) {                   // behind chunk c of the k-th part; chunks if there is none
+        if (c + STEP < chunks) return c + STEP;
+        int next = chunks;
 #pragma unroll
-        for (int r = 0; r < DX_RB; ++r) {
-            const int e = row_bytes[r] / (int)sizeof(float) + j;
-            acc[r] = xr[r] <= ybase[e] ? __fmaf_rn(ubase[e], wv, acc[r]) : acc[r];
+        for (int m = PARTS - 1; m > 0; --m)
+            if (m > k && part(m) < chunks) next = part(m);
+        return next;
+    };
+    const int pr = lane / LANES, pj = lane % LANES * 4;     // the lane's piece: row pr (+ ROWS per pass), outputs pj ... + 3
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    typedef float fa __attribute__((ext_vector_type(A)));
+    f4 yv[S_PASSES], uv[S_PASSES], wv[I_PASSES];
+    typedef float f4_any __attribute__((ext_vector_type(4), aligned(4)));             // (four floats need no more alignment than one)
+    auto piece = [&](const float* row, int j, bool whole) {
+        f4 v;
+        if (whole) {
+            v = *reinterpret_cast<const f4_any*>(row + j);
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[q] = row[min(j + q, J - 1)];
         }
-    }
-    if (wave > 0) {
+        return v;
+    };
+    auto request = [&](int j0) {
+        const bool whole = j0 + DX_JC <= J;
 #pragma unroll
-        for (int r = 0; r < DX_RB; ++r) red[wave - 1][r][lane] = acc[r];
-    }
-    __syncthreads();
-    if (wave == 0 && i < I) {
+        for (int t = 0; t < S_PASSES; ++t) {
+            const size_t row = (size_t)min(s0 + t * ROWS + pr, B - 1) * J;
+            yv[t] = piece(ym + row, j0 + pj, whole);
+            uv[t] = piece(upm + row, j0 + pj, whole);
+        }
 #pragma unroll
-        for (int r = 0; r < DX_RB; ++r) {
-            if (b0 + r < B)
-                dx[(size_t)(b0 + r) * I + i] = ((acc[r] + red[0][r][lane]) + red[1][r][lane]) + red[2][r][lane];
+        for (int t = 0; t < I_PASSES; ++t) wv[t] = piece(w + (size_t)min(i0 + t * ROWS + pr, I - 1) * J, j0 + pj, whole);
+    };
+    float* ys = dx_lds + wave * 3 * DX_JC * DX_PITCH;       // [output][sample | sample | input]
+    float* us = ys + DX_JC * DX_PITCH;
+    float* ws = us + DX_JC * DX_PITCH;
+    float total[A][4], pair[A][4];
+    if (part(0) < chunks) request(part(0) * DX_JC);
+#pragma unroll
+    for (int k = 0; k < PARTS; ++k) {
+        for (int c = part(k); c < chunks; c += STEP) {
+            const int j0 = c * DX_JC;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const bool in = j0 + pj + q < J;                // outputs past the end take no part
+#pragma unroll
+                for (int t = 0; t < S_PASSES; ++t) {
+                    ys[(pj + q) * DX_PITCH + t * ROWS + pr] = in ? yv[t][q] : -INFINITY;
+                    us[(pj + q) * DX_PITCH + t * ROWS + pr] = in ? uv[t][q] : 0.0f;
+                }
+#pragma unroll
+                for (int t = 0; t < I_PASSES; ++t) ws[(pj + q) * DX_PITCH + t * ROWS + pr] = wv[t][q];
+            }
+            const int next = next_chunk(k, c);
+            if (next < chunks) request(next * DX_JC);
+            wave_lds_order();
+            fa y[2], u[2];
+            f4 wj[2];
+            auto fetch = [&](int b, int j) {
+                y[b] = *reinterpret_cast<const fa*>(ys + j * DX_PITCH + sg * A);
+                u[b] = *reinterpret_cast<const fa*>(us + j * DX_PITCH + sg * A);
+                wj[b] = *reinterpret_cast<const f4*>(ws + j * DX_PITCH + ig * 4);
+            };
+            fetch(0, 0);
+#pragma unroll
+            for (int j = 0; j < DX_JC; ++j) {
+                const int b2 = j & 1;
+                if (j + 1 < DX_JC) fetch(b2 ^ 1, j + 1);
+                __builtin_amdgcn_sched_barrier(0);
+                // acc += up * w where x <= y; the others are skipped, as in the reference (snnfcgrad_kernels.cu.cc:60), not
+                // added as zeros
+#pragma unroll
+                for (int a = 0; a < A; ++a)
+#pragma unroll
+                    for (int b = 0; b < 4; ++b)
+                        acc[a][b] = xr[a][b] <= y[b2][a] ? __fmaf_rn(u[b2][a], wj[b2][b], acc[a][b]) : acc[a][b];
+            }
+            wave_lds_order();
+        }
+#pragma unroll
+        for (int a = 0; a < A; ++a)
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                if (k == 0) total[a][b] = acc[a][b];
+                else if (k == 1) total[a][b] += acc[a][b];
+                else if (k == 2) pair[a][b] = acc[a][b];
+                else total[a][b] += pair[a][b] + acc[a][b];
+                acc[a][b] = 0.0f;
+            }
+    }
+    if constexpr (SPLIT == 1) {
+        if (tile_raw >= n_tiles) return;
+#pragma unroll
+        for (int a = 0; a < A; ++a)
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                const int s = s0 + sg * A + a, i = i0 + ig * 4 + b;
+                if (s < B && i < I) dx[(size_t)s * I + i] = total[a][b];
+            }
+    } else {
+        __syncthreads();
+        float* red = dx_lds + wave * TS * DX_I;             // [wave][sample][input]
+#pragma unroll
+        for (int a = 0; a < A; ++a)
+            *reinterpret_cast<f4*>(red + (sg * A + a) * DX_I + ig * 4) = f4{total[a][0], total[a][1], total[a][2], total[a][3]};
+        __syncthreads();
+        for (int e = threadIdx.x; e < TS * DX_I; e += dx_threads(SPLIT)) {
+            const int s = s0 + e / DX_I, i = i0 + e % DX_I;
+            float sum[SPLIT];
+#pragma unroll
+            for (int v = 0; v < SPLIT; ++v) sum[v] = dx_lds[v * TS * DX_I + e];
+#pragma unroll
+            for (int h = SPLIT / 2; h > 0; h /= 2)
+#pragma unroll
+                for (int v = 0; v < h; ++v) sum[v] += sum[v + h];
+            if (s < B && i < I) dx[(size_t)s * I + i] = sum[0];
         }
     }
 }
 
 // ---------------------------------------------------------------------------------------------
-// dW for dense rows or implicit conv patches.  Lanes run across outputs j (y/up rows are read
+// dW for implicit conv patches.  Lanes run across outputs j (y/up rows are read
 // coalesced); each thread carries RI consecutive weight rows whose x values are wave-uniform.
 // The segment range is cut into gridDim.z slices; a slice is further split over the four
 // wavefronts of the block.  With more than one slice the per-slice sums go to `partial` and are
@@ -242,14 +275,14 @@ constexpr int DW_UNROLL = 4;
 
 __global__ void __launch_bounds__(256)
 grad_weight_kernel(SegmentSource src, const float* __restrict__ upm, const float* __restrict__ ym,
-                   float* __restrict__ dst, int S, int J, int rows, int row_start, int seg_per_slice,
+                   float* __restrict__ dst, int S, int J, int rows, int seg_per_slice,
                    float biasvolt, float neg_s, float post) {
     __shared__ float red[3][DW_RI][kWave];
     const int lane = threadIdx.x % kWave;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int j = blockIdx.x * kWave + lane;
     const unsigned jc = (unsigned)min(j, J - 1);
-    const int i0 = row_start + blockIdx.y * DW_RI;
+    const int i0 = blockIdx.y * DW_RI;
     const int I = src.I;
 
     const int s_begin = blockIdx.z * seg_per_slice;
@@ -328,123 +361,104 @@ grad_weight_kernel(SegmentSource src, const float* __restrict__ upm, const float
 }
 
 // ---------------------------------------------------------------------------------------------
-// dW of a dense layer.  Same mapping as grad_weight_kernel (lane = output j, DW_RI weight rows per
-// block, the block's samples shared out over its four wavefronts), arranged so that a wavefront
-// waits for memory a few times instead of once per four samples -- at a batch of a few hundred
-// samples the wavefronts are short-lived and there are too few of them to hide those waits:
-//  * the x values of the block's rows, 256 samples at a time, are staged in LDS by all threads (the
-//    tile after the current one is already on its way) and read back as broadcasts; rows past the
-//    inputs read biasvolt, so the bias row needs no code of its own;
-//  * the ym / upm values of DWD_BATCH samples are requested together before the first one is used.
+// dW of a dense layer.  A workgroup owns 64 weight rows x 64 outputs, its wavefronts take the slice's samples eight at a
+// time in turn, a lane 8 x 8 of the tile: a sample's 64 inputs, output times and upstream values are three coalesced loads, a
+// batch ahead, go to a piece of LDS of the wavefront's own and come back as six 16-byte reads for 128 vector instructions.
+// Rows past the inputs read biasvolt, so the bias row needs no code of its own.  The wavefronts' sums are added in order
+// through LDS.
+// What bounds it: the addition and the multiply-add of a term (3.3 clocks each at 4096 samples).  Before, eight rows and one
+// output per lane: two LDS reads of 8 clocks and 512 bytes of y / up per 16 instructions.  us: 4096 x 784 -> 800 254 -> 158,
+// 1024 rows 69 -> 47 (both + 6 for adding up slices), 333 x 1521 -> 777 48 -> 40, 128 x 784 -> 800 15 -> 13.  (The times are scaled as they
+// are staged: a sum of two registers issues faster than a multiply-add of three, 225 us.)
 // ---------------------------------------------------------------------------------------------
-#ifndef SNNTC_DWD_BATCH
-#define SNNTC_DWD_BATCH 16
-#endif
-constexpr int DWD_BATCH = SNNTC_DWD_BATCH;
-constexpr int DWD_TILE = 256;                              // samples per staged tile: 64 per wavefront
-static_assert(DW_RI == 8, "the staging below moves eight rows per sample");
+constexpr int DWD_T = 64, DWD_BATCH = 4;
 
-__global__ void __launch_bounds__(256)
+template <int WAVES>
+__global__ void __launch_bounds__(WAVES * kWave, 4)
 grad_weight_dense_kernel(const float* __restrict__ x, const float* __restrict__ upm, const float* __restrict__ ym,
                          float* __restrict__ dst, int S, int I, int J, int rows, int seg_per_slice, float biasvolt,
                          float neg_s, float post) {
-    __shared__ __align__(16) float xt[2][DWD_TILE][DW_RI];
-    __shared__ float red[3][DW_RI][kWave];
+    // staging: [wave][sample][x 64 | y 64 | up 64]; sums: [wave][row 32][output 64], half a tile at a time
+    constexpr int STAGE = DWD_BATCH * 3 * DWD_T, SUMS = DWD_T / 2 * DWD_T;
+    __shared__ __align__(16) float lds[WAVES * (STAGE > SUMS ? STAGE : SUMS)];
+    typedef float f4 __attribute__((ext_vector_type(4)));
     const int lane = threadIdx.x % kWave;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int j = blockIdx.x * kWave + lane;
-    const unsigned jc = (unsigned)min(j, J - 1);
-    const int i0 = blockIdx.y * DW_RI;
-    const int s_begin = blockIdx.z * seg_per_slice;
-    const int s_end = __builtin_amdgcn_readfirstlane(min(S, s_begin + seg_per_slice));
-    // ym / upm of the slice through buffer descriptors: the sample's row is a scalar offset, the lane's
-    // column a constant one, and no address is computed per lane (the launcher keeps a slice below 2 GB)
-    const int slice_bytes = max(s_end - s_begin, 0) * J * (int)sizeof(float);
-    const __amdgpu_buffer_rsrc_t ybuf =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(ym + (size_t)s_begin * J), 0, slice_bytes, 0x00020000);
-    const __amdgpu_buffer_rsrc_t ubuf =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(upm + (size_t)s_begin * J), 0, slice_bytes, 0x00020000);
-    const int col_bytes = (int)(jc * sizeof(float)), row_bytes = J * (int)sizeof(float);
+    const int j0 = blockIdx.x * DWD_T, i0 = blockIdx.y * DWD_T;
+    const int s_begin = blockIdx.z * seg_per_slice, s_end = min(S, s_begin + seg_per_slice);
+    const int rg = lane / 8, cg = lane % 8;
 
-    float acc[DW_RI];
-#pragma unroll
-    for (int r = 0; r < DW_RI; ++r) acc[r] = 0.0f;
+    const bool is_input = i0 + lane < I;
+    const float* __restrict__ xcol = x + min(i0 + lane, I - 1);
+    const int jc = min(j0 + lane, J - 1);
+    const float* __restrict__ ycol = ym + jc;
+    const float* __restrict__ ucol = upm + jc;
+    float* stage = lds + wave * STAGE;
 
-    // element e = threadIdx.x + 256 * k of a tile: sample e / 8, row e % 8
-    const int st_row = threadIdx.x % DW_RI;
-    const int st_smp = threadIdx.x / DW_RI;                 // + 32 * k
-    const bool st_input = i0 + st_row < I;
-    const float* __restrict__ st_src = x + (st_input ? i0 + st_row : 0);
-    float pending[DW_RI];
-    auto fetch_tile = [&](int c0) {
+    float acc[8][8];
 #pragma unroll
-        for (int k = 0; k < DW_RI; ++k) {
-            const int s = min(c0 + st_smp + 32 * k, s_end - 1);
-            pending[k] = st_input ? st_src[(size_t)s * I] : biasvolt;
-        }
-    };
-    auto store_tile = [&](int buf) {
+    for (int r = 0; r < 8; ++r)
 #pragma unroll
-        for (int k = 0; k < DW_RI; ++k) xt[buf][st_smp + 32 * k][st_row] = pending[k];
-    };
-
-    // ym / upm of DWD_BATCH samples are requested together, then the batch is worked on.  (Requesting a
-    // batch ahead of the arithmetic changes nothing: alone, the requests of a launch keep L2 busy for
-    // about as long as the arithmetic keeps the vector units busy, and the two overlap only in part.)
-    auto load_batch = [&](float (&yv)[DWD_BATCH], float (&uv)[DWD_BATCH], int sb) {
+        for (int c = 0; c < 8; ++c) acc[r][c] = 0.0f;
+    float xv[DWD_BATCH], yv[DWD_BATCH], uv[DWD_BATCH];
+    auto request = [&](int sb) {
 #pragma unroll
         for (int q = 0; q < DWD_BATCH; ++q) {
-            const int sc = __builtin_amdgcn_readfirstlane(min(sb + q, s_end - 1));   // past the end: the last sample again
-            const int off = (sc - s_begin) * row_bytes;
-            yv[q] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ybuf, col_bytes, off, 0));
-            uv[q] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ubuf, col_bytes, off, 0));
+            const int s = min(sb + q, s_end - 1);
+            xv[q] = xcol[(size_t)s * I];
+            yv[q] = ycol[(size_t)s * J];
+            uv[q] = ucol[(size_t)s * J];
         }
     };
-    auto run_batch = [&](const float (&yv)[DWD_BATCH], const float (&uv)[DWD_BATCH], int sb, int buf, int h) {
+    int sb = s_begin + wave * DWD_BATCH;
+    if (sb < s_end) request(sb);
+    for (; sb < s_end; sb += WAVES * DWD_BATCH) {
 #pragma unroll
         for (int q = 0; q < DWD_BATCH; ++q) {
-            const float4* xq = reinterpret_cast<const float4*>(&xt[buf][wave * (DWD_TILE / 4) + h + q][0]);
-            const float4 xa = xq[0], xb = xq[1];
-            const float xr[DW_RI] = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
-            const float ys = yv[q] * -neg_s;
-            const float u = sb + q < s_end ? uv[q] : 0.0f;  // the surplus of the last batch weighs nothing
-#pragma unroll
-            for (int r = 0; r < DW_RI; ++r) acc[r] = __fmaf_rn(scaled_lead(xr[r], neg_s, ys), u, acc[r]);
+            stage[q * 3 * DWD_T + lane] = (is_input ? xv[q] : biasvolt) * neg_s;
+            stage[q * 3 * DWD_T + DWD_T + lane] = yv[q] * -neg_s;
+            stage[q * 3 * DWD_T + 2 * DWD_T + lane] = sb + q < s_end ? uv[q] : 0.0f;       // samples past the end weigh nothing
         }
-    };
-
-    if (s_begin < s_end) {
-        fetch_tile(s_begin);
-        store_tile(0);
-        int buf = 0;
-        for (int c0 = s_begin; c0 < s_end; c0 += DWD_TILE, buf ^= 1) {
-            __syncthreads();                                // tile `buf` is complete; the other one is free
-            const bool more = c0 + DWD_TILE < s_end;
-            if (more) fetch_tile(c0 + DWD_TILE);
-            const int w0 = c0 + wave * (DWD_TILE / 4);
-#pragma unroll 1
-            for (int h = 0; h < DWD_TILE / 4; h += DWD_BATCH) {
-                const int sb = w0 + h;
-                if (sb >= s_end) break;                     // wavefront-uniform
-                float yv[DWD_BATCH], uv[DWD_BATCH];
-                load_batch(yv, uv, sb);
-                run_batch(yv, uv, sb, buf, h);
+        if (sb + WAVES * DWD_BATCH < s_end) request(sb + WAVES * DWD_BATCH);
+        wave_lds_order();
+#pragma unroll 2
+        for (int q = 0; q < DWD_BATCH; ++q) {
+            const float* at = stage + q * 3 * DWD_T;
+            float xr[8], yr[8], ur[8];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const f4 a = *reinterpret_cast<const f4*>(at + rg * 8 + 4 * h);
+                const f4 b = *reinterpret_cast<const f4*>(at + DWD_T + cg * 8 + 4 * h);
+                const f4 c = *reinterpret_cast<const f4*>(at + 2 * DWD_T + cg * 8 + 4 * h);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) { xr[4 * h + e] = a[e]; yr[4 * h + e] = b[e]; ur[4 * h + e] = c[e]; }
             }
-            if (more) store_tile(buf ^ 1);
+#pragma unroll
+            for (int r = 0; r < 8; ++r)
+#pragma unroll
+                for (int c = 0; c < 8; ++c)
+                    acc[r][c] = __fmaf_rn(__builtin_amdgcn_fmed3f(xr[r] + yr[c], 0.0f, 1.0f), ur[c], acc[r][c]);
         }
+        wave_lds_order();
     }
-    if (wave > 0) {
+    float* out = dst + (size_t)blockIdx.z * rows * J;
 #pragma unroll
-        for (int r = 0; r < DW_RI; ++r) red[wave - 1][r][lane] = acc[r];
-    }
-    __syncthreads();
-    if (wave == 0 && j < J) {
-        float* out = dst + (size_t)blockIdx.z * rows * J;
+    for (int half = 0; half < 2; ++half) {
+        __syncthreads();                                    // (the staging, or the first half, has been read)
+        float* mine = lds + wave * SUMS;
 #pragma unroll
-        for (int r = 0; r < DW_RI; ++r) {
-            if (i0 + r < rows)
-                out[(size_t)(i0 + r) * J + j] =
-                    (((acc[r] + red[0][r][lane]) + red[1][r][lane]) + red[2][r][lane]) * post;
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                *reinterpret_cast<f4*>(mine + (rg * 4 + r) * DWD_T + cg * 8 + 4 * h) =
+                    f4{acc[4 * half + r][4 * h], acc[4 * half + r][4 * h + 1], acc[4 * half + r][4 * h + 2], acc[4 * half + r][4 * h + 3]};
+        __syncthreads();
+        for (int e = threadIdx.x; e < SUMS; e += WAVES * kWave) {
+            const int tr = e / DWD_T, i = i0 + tr / 4 * 8 + 4 * half + tr % 4, j = j0 + e % DWD_T;
+            float sum = lds[e];
+#pragma unroll
+            for (int v = 1; v < WAVES; ++v) sum += lds[v * SUMS + e];
+            if (i < rows && j < J) out[(size_t)i * J + j] = sum * post;
         }
     }
 }
@@ -647,21 +661,18 @@ int blocks_for(int64_t n, int block) { return (int)((n + block - 1) / block); }
 }  // namespace
 
 int launch_backward_prologue(const float* grad, const float* y, const float* rcp, float* upm, int64_t n,
-                             const NeuronParams& np, int mode, const float* w, float* wt, int64_t rows,
+                             const NeuronParams& np, const float* w, float* wt, int64_t rows,
                              int64_t cols, int64_t chan, float* zeros, int n_zeros, hipStream_t stream) {
     if (!zeros) n_zeros = 0;
     const bool vec4 = n % 4 == 0 && (((uintptr_t)grad | (uintptr_t)y | (uintptr_t)rcp | (uintptr_t)upm) & 15) == 0;
     const int64_t prep_blocks = vec4 ? (n / 4 + 255) / 256 : (n + 255) / 256;
-    int64_t copy_blocks = 0;
-    if (mode == 1) copy_blocks = ((cols + 31) / 32) * ((rows + 31) / 32);
-    else if (mode == 2) copy_blocks = (rows * (cols / 4) + 255) / 256;
-    if (mode != 0 && (rows <= 0 || cols <= 0)) { mode = 0; copy_blocks = 0; }
+    const int64_t copy_blocks = wt ? (rows * (cols / 4) + 255) / 256 : 0;
     if (prep_blocks + copy_blocks <= 0) return n_zeros > 0 ? launch_fill_zero(zeros, n_zeros, stream) : SNNTC_OK;
     if (prep_blocks + copy_blocks > 0x7fffffffLL) return fail(SNNTC_ERR_TOO_LARGE, "backward: grid too large");
     {
         KernelTimerScope timer_("prep_upstream", stream);
         hipLaunchKernelGGL(backward_prologue_kernel, dim3((unsigned)(prep_blocks + copy_blocks)), dim3(256), 0, stream,
-                           grad, y, rcp, upm, n, np.max_cmp, (int)prep_blocks, vec4 ? 1 : 0, mode, w, wt, (int)rows, (int)cols,
+                           grad, y, rcp, upm, n, np.max_cmp, (int)prep_blocks, vec4 ? 1 : 0, w, wt, (int)rows, (int)cols,
                            (int)chan, zeros, n_zeros);
     }
     SNNTC_HIP_CHECK(hipGetLastError());
@@ -677,20 +688,58 @@ int launch_fill_zero(float* p, int64_t n, hipStream_t stream) {
     return SNNTC_OK;
 }
 
-int launch_fc_grad_input(const float* x, const float* wt, const float* upm, const float* ym, float* dx,
-                         int64_t B, int64_t I, int64_t J, int64_t wt_stride, hipStream_t stream) {
-    if (B <= 0 || I <= 0) return SNNTC_OK;
-    if (J <= 0) return launch_fill_zero(dx, B * I, stream);
-    dim3 grid((unsigned)((B + DX_RB - 1) / DX_RB), (unsigned)((I + kWave - 1) / kWave));
-    if (grid.y > 65535u) return fail(SNNTC_ERR_TOO_LARGE, "dense backward: input size %lld too large", (long long)I);
-    { KernelTimerScope timer_("fc_grad_input", stream);
-    SegmentSource src{};
-    src.base = x; src.conv = 0; src.I = (int)I;
-    hipLaunchKernelGGL(fc_grad_input_kernel<false>, grid, dim3(256), 0, stream, src, wt, upm, ym, dx, (int)B, (int)I,
-                       (int)J, (int)wt_stride);
+namespace {
+// Wavefronts per tile.  Many tiles: four, which leave a CU's several workgroups to fill its SIMDs; fewer: more, so that every
+// SIMD has two or so (us with 4 / 8 / 16 at 800 outputs: 200 tiles 27 / 21 / 19, 400: 30 / 28.5 / 34, 800: 47 / 49 / 63); not
+// below 16 outputs each, and a single one for fewer than 64 outputs (16 200 x 500 -> 50: 26 against 32).
+int dx_split(int64_t tiles, int64_t J) {
+    if (J < 64) return 1;
+    int split = tiles >= 640 ? 4 : tiles >= 256 ? 8 : 16;
+    while (split > 4 && J < DX_JC * split) split /= 2;
+    return split;
+}
+
+template <bool PATCHES>
+int launch_dx(const char* name, const SegmentSource& src, const float* w, const float* upm, const float* ym, float* dx, int64_t B,
+              int64_t I, int64_t J, hipStream_t stream) {
+    const int rc = grad_prepare_device();
+    if (rc) return rc;
+    const int64_t tiles_i = (I + DX_I - 1) / DX_I, tiles = (B + DX_S - 1) / DX_S * tiles_i;
+    const int split = dx_split(tiles, J);
+    const int64_t blocks = split == 1 ? (tiles + 3) / 4 : tiles;
+    if (blocks > 0x1fffffffLL) return fail(SNNTC_ERR_TOO_LARGE, "backward: %lld x %lld input gradients are too many", (long long)B, (long long)I);
+    {
+        KernelTimerScope timer_(name, stream);
+        auto kern = split == 1 ? fc_grad_input_kernel<1, PATCHES> : split == 4 ? fc_grad_input_kernel<4, PATCHES>
+                  : split == 8 ? fc_grad_input_kernel<8, PATCHES> : fc_grad_input_kernel<16, PATCHES>;
+        hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(dx_threads(split)), dx_lds_bytes(split), stream, src, w, upm, ym, dx, (int)B, (int)I, (int)J,
+                           (int)tiles_i, (int)tiles);
     }
     SNNTC_HIP_CHECK(hipGetLastError());
     return SNNTC_OK;
+}
+}  // namespace
+
+// The dynamic-LDS limits of the current device, once.
+int grad_prepare_device() {
+    static std::atomic<bool> ready[kMaxDevices];
+    int dev = 0;
+    SNNTC_HIP_CHECK(hipGetDevice(&dev));
+    if (dev < 0 || dev >= kMaxDevices) return fail(SNNTC_ERR_UNSUPPORTED, "backward: device index %d not supported", dev);
+    if (ready[dev].load(std::memory_order_acquire)) return SNNTC_OK;
+    for (const void* k : {reinterpret_cast<const void*>(fc_grad_input_kernel<16, false>), reinterpret_cast<const void*>(fc_grad_input_kernel<16, true>)})
+        SNNTC_HIP_CHECK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, dx_lds_bytes(16)));
+    ready[dev].store(true, std::memory_order_release);
+    return SNNTC_OK;
+}
+
+int launch_fc_grad_input(const float* x, const float* w, const float* upm, const float* ym, float* dx,
+                         int64_t B, int64_t I, int64_t J, hipStream_t stream) {
+    if (B <= 0 || I <= 0) return SNNTC_OK;
+    if (J <= 0) return launch_fill_zero(dx, B * I, stream);
+    SegmentSource src{};
+    src.base = x; src.conv = 0; src.I = (int)I;
+    return launch_dx<false>("fc_grad_input", src, w, upm, ym, dx, B, I, J, stream);
 }
 
 // Number of slices the segment range is cut into for dW: none when the (row-block x column-block)
@@ -719,27 +768,44 @@ int grad_weight_blocks(int64_t rows, int64_t J) {
     return (int)(((J + kWave - 1) / kWave) * ((rows + DW_RI - 1) / DW_RI));
 }
 
-// Rows [row_start, rows) of dW, or of every partial-sum slice when nsplit > 1 (dst = slices).
+// Slices of a dense layer's samples.  A CU needs about 100 clocks per sample for a tile of 64 x 64; the launch lasts as long as
+// the CU with the most of them, and adding up slices costs another launch (about 5 us and the slices' traffic).
+int grad_weight_dense_splits(int64_t S, int64_t I, int64_t J) {
+    const int64_t tiles = ((J + DWD_T - 1) / DWD_T) * ((I + 1 + DWD_T - 1) / DWD_T);
+    int best = 1;
+    double best_time = 1e30;
+    for (int n = 1; n <= 16 && (n == 1 || S / n >= 64); ++n) {
+        const double time = (double)((tiles * n + 255) / 256) * 100.0 * (double)((S + n - 1) / n) +
+                            (n > 1 ? 12000.0 + 8.0 * n * (double)(I + 1) * (double)J / 1500.0 : 0.0);
+        if (time < best_time * 0.97) { best_time = time; best = n; }
+    }
+    return best;
+}
+
+// dW, or every partial-sum slice of it, when nsplit > 1 (dst = slices).
 int launch_grad_weight_rows(const SegmentSource& src, const float* upm, const float* ym, float* dst,
-                            int nsplit, int64_t S, int64_t J, int64_t row_start, const NeuronParams& np,
+                            int nsplit, int64_t S, int64_t J, const NeuronParams& np,
                             hipStream_t stream) {
     const int64_t rows = (int64_t)src.I + np.bias;
-    if (rows <= row_start || J <= 0 || S <= 0) return SNNTC_OK;
+    if (rows <= 0 || J <= 0 || S <= 0) return SNNTC_OK;
     if (nsplit < 1) nsplit = 1;
     const int seg_per_slice = (int)((S + nsplit - 1) / nsplit);
-    dim3 grid((unsigned)((J + kWave - 1) / kWave), (unsigned)((rows - row_start + DW_RI - 1) / DW_RI),
-              (unsigned)nsplit);
+    const int rows_per_block = src.conv ? DW_RI : DWD_T;
+    dim3 grid((unsigned)((J + kWave - 1) / kWave), (unsigned)((rows + rows_per_block - 1) / rows_per_block), (unsigned)nsplit);
     if (grid.y > 65535u) return fail(SNNTC_ERR_TOO_LARGE, "weight gradient: too many weight rows");
     {
-        KernelTimerScope timer_(row_start ? "grad_weight_tail" : "grad_weight", stream);
+        KernelTimerScope timer_("grad_weight", stream);
         const LeadScale ls = lead_scale(np.max_time);
-        // (the dense kernel addresses a slice of ym / upm with 32-bit byte offsets)
-        if (!src.conv && row_start == 0 && ((int64_t)seg_per_slice + DWD_TILE) * J * (int64_t)sizeof(float) < 0x7fffffffLL)
-            hipLaunchKernelGGL(grad_weight_dense_kernel, grid, dim3(256), 0, stream, src.base, upm, ym, dst, (int)S,
-                               (int)src.I, (int)J, (int)rows, seg_per_slice, np.biasvolt, ls.neg_s, ls.post);
-        else
+        if (src.conv) {
             hipLaunchKernelGGL(grad_weight_kernel, grid, dim3(256), 0, stream, src, upm, ym, dst, (int)S, (int)J,
-                               (int)rows, (int)row_start, seg_per_slice, np.biasvolt, ls.neg_s, ls.post);
+                               (int)rows, seg_per_slice, np.biasvolt, ls.neg_s, ls.post);
+        } else {
+            // eight wavefronts per tile where there are too few tiles to give every SIMD two otherwise
+            const bool wide = (int64_t)grid.x * grid.y * grid.z < 512;
+            auto kern = wide ? grad_weight_dense_kernel<8> : grad_weight_dense_kernel<4>;
+            hipLaunchKernelGGL(kern, grid, dim3((wide ? 8 : 4) * kWave), 0, stream, src.base, upm, ym, dst, (int)S,
+                               (int)src.I, (int)J, (int)rows, seg_per_slice, np.biasvolt, ls.neg_s, ls.post);
+        }
     }
     SNNTC_HIP_CHECK(hipGetLastError());
     return SNNTC_OK;
@@ -787,18 +853,13 @@ int launch_fc_backward_narrow(const float* x, const float* w, const float* grad,
 }
 
 // dxp: scratch of S * P floats (gradient per patch element)
-int launch_cv_grad_input(const SegmentSource& src, const float* wt, const float* upm, const float* ym, float* dxp,
-                         float* dx, const CropGeom& crop, const ConvGeom& g, int64_t wt_stride, hipStream_t stream) {
+int launch_cv_grad_input(const SegmentSource& src, const float* w, const float* upm, const float* ym, float* dxp,
+                         float* dx, const CropGeom& crop, const ConvGeom& g, hipStream_t stream) {
     const int64_t n = g.B * g.H * g.W * g.C;
     if (n <= 0) return SNNTC_OK;
     if (g.Kc <= 0 || g.S <= 0) return launch_fill_zero(dx, g.B * crop.h * crop.w * g.C, stream);
-    dim3 grid((unsigned)((g.S + DX_RB - 1) / DX_RB), (unsigned)((g.P + kWave - 1) / kWave));
-    if (grid.y > 65535u) return fail(SNNTC_ERR_TOO_LARGE, "conv backward: patch length %lld too large", (long long)g.P);
-    { KernelTimerScope timer_("cv_grad_input", stream);
-    hipLaunchKernelGGL(fc_grad_input_kernel<true>, grid, dim3(256), 0, stream, src, wt, upm, ym, dxp, (int)g.S,
-                       (int)g.P, (int)g.Kc, (int)wt_stride);
-    }
-    SNNTC_HIP_CHECK(hipGetLastError());
+    const int rc = launch_dx<true>("cv_grad_input", src, w, upm, ym, dxp, g.S, g.P, g.Kc, stream);
+    if (rc) return rc;
     { KernelTimerScope timer_("cv_col2im", stream);
     hipLaunchKernelGGL(cv_col2im_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, stream, dxp, dx, crop, n, (int)g.H,
                        (int)g.W, (int)g.C, (int)g.Kh, (int)g.Kw, (int)g.Sh, (int)g.Sw, (int)g.Nh, (int)g.Nw);

@@ -174,22 +174,23 @@ int read_scan_giveups(int64_t* count, hipStream_t stream);
 int scan_prepare_device(int dev, int* cu_count_out);
 int order_prepare_device();
 
-// upm = valid ? grad*rcp : 0   (valid: y <= MAX-0.1; n elements), and, in the same launch, the weight copy dX reads from: mode 0 none, mode 1
-// wt[cols, rows] = w[rows, cols]^T, mode 2 the regrouped copy of a conv layer's weights
-// (wt[tap][cols / 4][chan][cols % 4] from w[(tap, chan), cols], rows = taps * chan).  `zeros`, if not
-// NULL, are n_zeros (<= 256) floats the launch clears: the op's all-zero dParams output.
-int launch_backward_prologue(const float* grad, const float* y, const float* rcp, float* upm, int64_t n, const NeuronParams& np, int mode, const float* w, float* wt, int64_t rows,
+// upm = valid ? grad*rcp : 0   (valid: y <= MAX-0.1; n elements), and, in the same launch, if wt is not NULL, the regrouped copy of
+// a conv layer's weights that launch_cv_grad_input_chan reads (wt[tap][cols / 4][chan][cols % 4] from w[(tap, chan), cols], rows =
+// taps * chan).  `zeros`, if not NULL, are n_zeros (<= 256) floats the launch clears: the op's all-zero dParams output.
+int launch_backward_prologue(const float* grad, const float* y, const float* rcp, float* upm, int64_t n, const NeuronParams& np, const float* w, float* wt, int64_t rows,
                              int64_t cols, int64_t chan, float* zeros, int n_zeros, hipStream_t stream);
 
-int launch_fc_grad_input(const float* x, const float* wt, const float* upm, const float* ym, float* dx,
-                         int64_t B, int64_t I, int64_t J, int64_t wt_stride, hipStream_t stream);
+int launch_fc_grad_input(const float* x, const float* w, const float* upm, const float* ym, float* dx,
+                         int64_t B, int64_t I, int64_t J, hipStream_t stream);
+int grad_prepare_device();
 
 // dW for dense rows or implicit patches.  The segment range may be cut into `nsplit` slices whose
 // partial sums (scratch `dst`, nsplit x rows x J) are added in slice order by launch_reduce_partials.
 int weight_grad_splits(int64_t S, int64_t base_blocks);
 int grad_weight_blocks(int64_t rows, int64_t J);
+int grad_weight_dense_splits(int64_t S, int64_t I, int64_t J);
 int launch_grad_weight_rows(const SegmentSource& src, const float* upm, const float* ym, float* dst,
-                            int nsplit, int64_t S, int64_t J, int64_t row_start, const NeuronParams& np,
+                            int nsplit, int64_t S, int64_t J, const NeuronParams& np,
                             hipStream_t stream);
 int launch_reduce_partials(const float* partial, float* dw, int64_t n, int nsplit, hipStream_t stream);
 
@@ -204,7 +205,7 @@ int launch_fc_backward_narrow(const float* x, const float* w, const float* grad,
 
 // Conv layers with many channels: lane = channel (dX) / wide row blocks (dW), see cv_grad.hip.
 bool cv_grad_input_chan_supported(const ConvGeom& g);
-// launch_cv_grad_input_chan reads the weights from the copy regrouped by launch_backward_prologue (mode 2).
+// launch_cv_grad_input_chan reads the weights from the copy regrouped by launch_backward_prologue.
 int launch_cv_grad_input_chan(const float* xpad, const float* wq, const float* upm, const float* ym,
                               float* dx, const CropGeom& crop, const ConvGeom& g, const NeuronParams& np,
                               hipStream_t stream);
@@ -214,8 +215,8 @@ int launch_cv_grad_weight_wide(const float* xpad, const float* upm, const float*
                                const ConvGeom& g, int64_t rows, const NeuronParams& np, hipStream_t stream);
 
 // Conv dX for layers launch_cv_grad_input_chan does not take; dxp is scratch of S * P floats.
-int launch_cv_grad_input(const SegmentSource& src, const float* wt, const float* upm, const float* ym, float* dxp,
-                         float* dx, const CropGeom& crop, const ConvGeom& g, int64_t wt_stride, hipStream_t stream);
+int launch_cv_grad_input(const SegmentSource& src, const float* w, const float* upm, const float* ym, float* dxp,
+                         float* dx, const CropGeom& crop, const ConvGeom& g, hipStream_t stream);
 
 int launch_fill_zero(float* p, int64_t n, hipStream_t stream);
 

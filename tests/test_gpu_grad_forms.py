@@ -1,0 +1,43 @@
+"""The dense and patch gradients in each of their forms -- one, four, eight or sixteen wavefronts per tile of dX, four or eight
+per tile of dW, with and without slices -- at ragged edges of tiles, chunks and pieces, against the fp64 oracle sums."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import capi
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def t(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).to(DEV)
+
+
+@pytest.mark.parametrize("B,I,J", [
+    (1, 1, 17), (17, 33, 18), (15, 31, 63), (16, 32, 64), (17, 65, 65),   # one wavefront per tile, four; less and more than a tile
+    (33, 40, 255), (20, 63, 257),                                         # eight and sixteen wavefronts
+    (260, 520, 130), (700, 500, 40), (1100, 1000, 101),                   # many tiles: eight, one, four
+    (129, 64, 300), (515, 127, 64), (1030, 300, 257),                     # slices of the samples
+    (300, 1500, 1299),                                                    # four wavefronts per tile of dW
+])
+def test_dense_gradients(B, I, J):
+    import snntc_amd as snn
+    rng = np.random.default_rng(B + I + J)
+    x = np.exp(rng.random((B, I))).astype(np.float32)
+    x[rng.random((B, I)) < 0.1] = 1e5
+    y = np.exp(1.2 * rng.random((B, J))).astype(np.float32)
+    y[rng.random((B, J)) < 0.1] = 1e5
+    x[0, : min(I, J)] = y[0, : min(I, J)]                                 # equal times count
+    w = rng.standard_normal((I + 1, J)).astype(np.float32)
+    out = np.concatenate([y, rng.random((B, J)).astype(np.float32)])
+    g = np.zeros((2 * B, J), np.float32)
+    g[:B] = rng.standard_normal((B, J))
+    p = capi.fc_params(1.0)
+    dx, dw, _ = (v.cpu().numpy() for v in snn.snnfc_grad(t(g), t(x), t(w), p, t(out)))
+    again = snn.snnfc_grad(t(g), t(x), t(w), p, t(out))
+    assert np.array_equal(dx, again[0].cpu().numpy()) and np.array_equal(dw, again[1].cpu().numpy())
+    rdx, rdw, _ = capi.fc_backward_dev(g, x, w, p, out, wide=True)
+    adx, adw, _ = capi.fc_backward_dev(np.abs(g), x, np.abs(w), p, out, wide=True)      # sums of absolute terms
+    assert np.all(np.abs(dx - rdx) <= 1e-6 * np.abs(adx) + 1e-30)
+    assert np.all(np.abs(dw - rdw) <= 1e-6 * np.abs(adw) + 1e-30)
