@@ -311,9 +311,15 @@ SNNTC_API int snntc_recipe_total(const int64_t* rows, const int64_t* cols, int64
  *       the next launch on (process-wide; polls < 0 restores the default of 2^20).  With 0 every wait that
  *       is not already satisfied at its first poll gives up, which drives the give-up path while every
  *       kernel still runs to its end.
+ *   snntc_debug_order_tile(B,H,W,C,params,aligned,tile)  test hook, host code only: how a conv layer's patches
+ *       are put in order on 256 CUs when Xpad is 16-byte aligned (aligned != 0) or not.  tile[4] = patches of a
+ *       tile down and across, pixels of its region that get a bitmap of their own (0: none), bytes of LDS; all
+ *       zero for a layer whose patches are sorted one by one.
  * ------------------------------------------------------------------------------------------- */
 SNNTC_API int snntc_scan_status(int64_t* giveups, void* stream);
 SNNTC_API int snntc_debug_set_scan_wait_polls(int polls);
+SNNTC_API int snntc_debug_order_tile(int64_t B, int64_t H, int64_t W, int64_t C, const float* params_host, int aligned,
+                                     int64_t* tile);
 
 /* ---------------------------------------------------------------------------------------------
  * Per-kernel timing (no counterpart in the reference, which only times whole scripts with

@@ -543,6 +543,14 @@ int snntc_debug_set_scan_wait_polls(int polls) {
     return SNNTC_OK;
 }
 
+int snntc_debug_order_tile(int64_t B, int64_t H, int64_t W, int64_t C, const float* params_host, int aligned, int64_t* tile) {
+    ConvGeom g;
+    const int rc = cv_geom(B, H, W, C, 1, 0, params_host, false, "snntc_debug_order_tile", &g);
+    if (rc) return rc;
+    if (!tile) return fail(SNNTC_ERR_BAD_ARGUMENT, "snntc_debug_order_tile: tile is NULL");
+    return order_tile(g, aligned != 0, tile);
+}
+
 int snntc_profile_enable(int on) {
     std::lock_guard<std::mutex> lock(g_prof_mutex);
     prof_drain();

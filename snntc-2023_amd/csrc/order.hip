@@ -738,15 +738,21 @@ struct OrderPlan {
 constexpr int ORDER_MAX_REGION = 8192;
 constexpr int ORDER_PIXEL_CHANNELS = 32;
 
+// LDS of a tile whose region has n inputs, 0 if the kernel does not take it.
+size_t order_tile_lds(int64_t n, const OrderForm& form, int stride, int patches, int region_pixels) {
+    if (n > ORDER_MAX_REGION || n > (int64_t)form.threads * ORDER_EPT) return 0;
+    const size_t lds = order_lds_bytes((int)n, form.threads, stride, form.wave ? form.threads / kWave : 0, patches, region_pixels);
+    return lds <= (size_t)ORDER_LDS_BYTES - 1024 ? lds : 0;
+}
+
 // Tile of a layer: the one with the smallest estimated time among the tiles that cut rows and columns evenly.  A
 // workgroup issues some 450 vector instructions per wavefront, 230 per 256 inputs it ranks and 13 per 64 inputs it
 // orders; alone on a CU it takes about 14000 clocks for the ranks and, per patch in turn, 1000 and 220 per 64 inputs.
 // The workgroups that share a CU take about the sum of one's latency and everyone's instructions, and overlap the better
 // the more they are.
-OrderPlan order_plan(const ConvGeom& g, const OrderForm& form, bool quads, int cus) {
+OrderPlan order_best_tile(const ConvGeom& g, const OrderForm& form, bool pixels, int cus) {
     OrderPlan best{};
     float best_time = 1e30f;
-    const bool pixels = quads && g.C >= ORDER_PIXEL_CHANNELS;
     const int T = form.threads, W = T / kWave, stride = (int)padded_stride(g.P), members = form.wave ? kWave : T;
     const int iters = (int)((g.P + members - 1) / members);
     const float patch_work = form.wave ? 60.f + 13.f * iters : W * (20.f + 13.f * iters);
@@ -756,9 +762,8 @@ OrderPlan order_plan(const ConvGeom& g, const OrderForm& form, bool quads, int c
         for (int64_t nx = (g.Nw + 15) / 16, tw = 0; nx <= g.Nw; nx = tw > 1 ? (g.Nw + tw - 2) / (tw - 1) : g.Nw + 1) {
             tw = (g.Nw + nx - 1) / nx;
             const int64_t px = ((th - 1) * g.Sh + g.Kh) * ((tw - 1) * g.Sw + g.Kw), n = px * g.C;
-            if (n > ORDER_MAX_REGION || n > (int64_t)T * ORDER_EPT) continue;
-            const size_t lds = order_lds_bytes((int)n, T, stride, form.wave ? W : 0, (int)(th * tw), pixels ? (int)px : 0);
-            if (lds > (size_t)ORDER_LDS_BYTES - 1024) continue;
+            const size_t lds = order_tile_lds(n, form, stride, (int)(th * tw), pixels ? (int)px : 0);
+            if (lds == 0) continue;
             const int64_t tiles = g.B * ny * nx, fit = std::min((int64_t)(ORDER_LDS_BYTES / (lds + 512)), (int64_t)(form.waves_per_cu / W));
             const int64_t resident = std::max((int64_t)1, std::min(fit, (tiles + cus - 1) / cus));
             const float patches = (float)(th * tw), turns = form.wave ? (float)((th * tw + W - 1) / W) : patches;
@@ -775,6 +780,14 @@ OrderPlan order_plan(const ConvGeom& g, const OrderForm& form, bool quads, int c
     return best;
 }
 
+// A bitmap per pixel of the region takes region^2 / C / 8 bytes: with large kernels not even a single patch's pixels fit next
+// to the rest (7x7 with 164 channels, 16x16 with 32), and the patches set their bits themselves, as for fewer channels.
+OrderPlan order_plan(const ConvGeom& g, const OrderForm& form, bool quads, int cus) {
+    OrderPlan plan{};
+    if (quads && g.C >= ORDER_PIXEL_CHANNELS) plan = order_best_tile(g, form, true, cus);
+    return plan.n_cap ? plan : order_best_tile(g, form, false, cus);
+}
+
 }  // namespace
 
 int order_prepare_device() {
@@ -788,8 +801,19 @@ int order_prepare_device() {
 // Patches of one pixel share nothing, patches of up to 64 inputs are sorted in registers by one wavefront faster than they
 // are ranked (50 176 of 27 inputs: 16.5 against 25.7 us; of 50: 25.8 / 27.5; of 72: 42.6 / 27.9), and the same holds up to
 // 128 inputs while there are only a few patches per CU and the latency of one workgroup counts (784 of 72: 6.3 / 8.3 us).
+// The tile that asks for least is a single patch that sets its own bits; it is among the ones order_plan looks at.
 bool order_patches_supported(const ConvGeom& g) {
-    return g.Kh * g.Kw > 1 && g.P > (g.S <= 4096 ? 128 : 64) && g.P <= ORDER_MAX_REGION;
+    return g.Kh * g.Kw > 1 && g.P > (g.S <= 4096 ? 128 : 64) && g.P <= ORDER_MAX_REGION &&
+           order_tile_lds(g.P, order_form_of(g.P), (int)padded_stride(g.P), 1, 0) > 0;
+}
+
+int order_tile(const ConvGeom& g, bool aligned, int64_t tile[4]) {
+    for (int i = 0; i < 4; ++i) tile[i] = 0;
+    if (!order_patches_supported(g)) return SNNTC_OK;
+    const OrderPlan plan = order_plan(g, order_form_of(g.P), g.C % 4 == 0 && aligned, 256);
+    if (plan.n_cap == 0) return fail(SNNTC_ERR_UNSUPPORTED, "order: no tile for patches of %lld inputs", (long long)g.P);
+    tile[0] = plan.th; tile[1] = plan.tw; tile[2] = plan.region_pixels; tile[3] = (int64_t)plan.lds;
+    return SNNTC_OK;
 }
 
 int launch_order_patches(const float* xpad, float* sorted, int32_t* perm, int32_t* n_real, const ConvGeom& g, int64_t stride,

@@ -38,7 +38,7 @@ EXPORTS = (
     "snntc_pad_time_forward", "snntc_pad_time_backward",
     "snntc_encode_time", "snntc_label_loss", "snntc_weight_cost_workspace_bytes", "snntc_weight_cost_sums",
     "snntc_weight_cost_grad", "snntc_recipe_total",
-    "snntc_scan_status", "snntc_debug_set_scan_wait_polls",
+    "snntc_scan_status", "snntc_debug_set_scan_wait_polls", "snntc_debug_order_tile",
     "snntc_profile_enable", "snntc_profile_collect", "snntc_profile_entry",
 )
 
@@ -131,6 +131,7 @@ def load():
     lib.snntc_recipe_total.argtypes = [pi64, pi64, i64, c.c_float, c.c_float, vp, vp, i64, vp, vp, vp, sz, vp]
     lib.snntc_scan_status.argtypes = [c.POINTER(i64), vp]
     lib.snntc_debug_set_scan_wait_polls.argtypes = [c.c_int]
+    lib.snntc_debug_order_tile.argtypes = [i64, i64, i64, i64, fparams, c.c_int, c.POINTER(i64)]
     lib.snntc_profile_enable.argtypes = [c.c_int]
     lib.snntc_profile_collect.argtypes = []
     lib.snntc_profile_entry.argtypes = [c.c_int, c.POINTER(c.c_char_p), c.POINTER(i64), c.POINTER(c.c_double)]

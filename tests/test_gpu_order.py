@@ -27,6 +27,9 @@ FORMS = [
     (1, 4, 5, 321, 4, 2, 1, 1),         # P = 2568
     (1, 6, 5, 512, 3, 3, 1, 1),
     (1, 3, 4, 2048, 2, 2, 1, 2),        # P = 8192, the longest
+    (1, 8, 8, 164, 7, 7, 1, 1),         # P = 8036 and, below, 4896 (the shortest), 8192: no room for a bitmap per pixel
+    (1, 10, 21, 32, 9, 17, 1, 2),
+    (2, 16, 17, 32, 16, 16, 1, 1),
 ]
 
 
