@@ -10,6 +10,10 @@
 // Scratch comes from PyTorch's caching allocator per call: it is stream-ordered, belongs to the graph's
 // pool while a stream is captured, and is safe with several threads and streams without a pool of ours.
 // The GIL is released while an op runs.
+//
+// The nodes below know reverse mode over ordinary tensors.  Everything else PyTorch can hand an op -- forward-mode
+// tangents, functorch's wrappers, tensors of Python modes, a tracer that has to see the call -- goes to the
+// torch.autograd.Function of the same op in ops.py, which refuses or records it as any such function does (`plain`).
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 #include <dlfcn.h>
@@ -17,6 +21,8 @@
 #include <ATen/ATen.h>
 #include <ATen/core/grad_mode.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/autograd.h>
@@ -24,6 +30,7 @@
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include <array>
 #include <optional>
@@ -59,6 +66,7 @@ struct Library {
 PyObject* g_library_error = nullptr;   // snntc_amd._lib.SnntcLibraryError
 PyObject* g_error = nullptr;           // snntc_amd._lib.SnntcError
 PyObject* g_params = nullptr;          // snntc_amd._lib.params_array: any sequence -> contiguous float32 vector
+PyObject* g_general = nullptr;         // snntc_amd.ops.GENERAL: name of a differentiable op -> its torch.autograd.Function
 
 // Raises a Python exception of class `cls` from code that may run without the GIL (an autograd thread).
 [[noreturn]] void raise_class(PyObject* cls, PyObject* (*args)(int, const std::string&), int status, const std::string& msg) {
@@ -122,6 +130,20 @@ Tensor first_half(const Tensor& y, int64_t B) {
 
 bool wants_grad(const Tensor& a) { return at::GradMode::is_enabled() && a.requires_grad(); }
 bool wants_grad(const Tensor& a, const Tensor& b) { return at::GradMode::is_enabled() && (a.requires_grad() || b.requires_grad()); }
+
+// Whether the native nodes may stand for PyTorch's own machinery: no tangent to carry on, no wrapper without memory of
+// its own, no mode, transform or tracer that has to see the operation.
+bool plain(std::initializer_list<std::reference_wrapper<const Tensor>> tensors) {
+    static const c10::DispatchKeySet special{
+        c10::DispatchKey::Python, c10::DispatchKey::Functionalize, c10::DispatchKey::Conjugate, c10::DispatchKey::Negative,
+        c10::DispatchKey::ZeroTensor, c10::DispatchKey::Batched, c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper};
+    if (torch::jit::tracer::isTracing() || c10::impl::TorchDispatchModeTLS::any_modes_set() ||
+        c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode))
+        return false;
+    for (const Tensor& t : tensors)
+        if (t.defined() && (t.key_set().has_any(special) || t._fw_grad(0).defined())) return false;
+    return true;
+}
 
 // ---- the ops -------------------------------------------------------------------------------------------------------
 
@@ -732,6 +754,12 @@ Feed feed_arg(PyObject* dst, PyObject* top, PyObject* left) {
     return Feed{optional_tensor(dst, "next_xpad"), int_arg(top), int_arg(left)};
 }
 
+PyObject* general(const char* name, PyObject* const* a, Py_ssize_t n) {
+    PyObject* f = PyDict_GetItemString(g_general, name);
+    TORCH_CHECK(f, "no general path for ", name);
+    return PyObject_Vectorcall(f, a, n, nullptr);
+}
+
 #define SNNTC_METHOD(name) PyObject* name(PyObject*, PyObject* const* a, Py_ssize_t n)
 
 // fc_forward(X, W, params) -> Y[2B,J]
@@ -755,6 +783,7 @@ SNNTC_METHOD(py_fc_layer) {
     HANDLE_TH_ERRORS
     arity(n, 4, "fc_layer");
     const Tensor x = tensor_arg(a[0], "X"), w = tensor_arg(a[1], "W");
+    if (!plain({x, w})) return general("fc_layer", a, n);
     const auto p = params_arg<6>(a[2]);
     const bool times = bool_arg(a[3]);
     Tensor out;
@@ -806,6 +835,7 @@ SNNTC_METHOD(py_cv_layer) {
     HANDLE_TH_ERRORS
     arity(n, 4, "cv_layer");
     const Tensor x = tensor_arg(a[0], "X"), w = tensor_arg(a[1], "W");
+    if (!plain({x, w})) return general("cv_layer", a, n);
     const auto p = params_arg<12>(a[2]);
     const bool times = bool_arg(a[3]);
     Tensor out;
@@ -827,6 +857,7 @@ SNNTC_METHOD(py_cv_same) {
     const Pads pad{int_arg(a[3]), int_arg(a[4]), int_arg(a[5]), int_arg(a[6])};
     const Tensor xpad = optional_tensor(a[7], "xpad");
     const Feed feed = feed_arg(a[8], a[9], a[10]);
+    if (!plain({x, w, xpad, feed.dst})) return general("cv_same", a, n);
     Tensor out;
     {
         NoGil nogil;
@@ -891,6 +922,7 @@ SNNTC_METHOD(py_min_pool_layer) {
     const Tensor x = tensor_arg(a[0], "x");
     const PoolShape s = pool_arg(a + 1);
     const Feed feed = feed_arg(a[10], a[11], a[12]);
+    if (!plain({x, feed.dst})) return general("min_pool_layer", a, n);
     Tensor out;
     {
         NoGil nogil;
@@ -905,6 +937,7 @@ SNNTC_METHOD(py_pad_layer) {
     HANDLE_TH_ERRORS
     arity(n, 6, "pad_layer");
     const Tensor x = tensor_arg(a[0], "x");
+    if (!plain({x})) return general("pad_layer", a, n);
     const Pads pad{int_arg(a[1]), int_arg(a[2]), int_arg(a[3]), int_arg(a[4])};
     const float value = float_arg(a[5]);
     Tensor out;
@@ -937,6 +970,7 @@ SNNTC_METHOD(py_loss_layer) {
     HANDLE_TH_ERRORS
     arity(n, 2, "loss_layer");
     const Tensor t = tensor_arg(a[0], "times"), l = tensor_arg(a[1], "label");
+    if (!plain({t, l})) return general("loss_layer", a, n);
     Tensor out;
     {
         NoGil nogil;
@@ -974,6 +1008,15 @@ std::vector<Tensor> tensor_list(PyObject* o, const char* name) {
     std::vector<Tensor> v;
     for (Py_ssize_t i = 0; i < PyList_GET_SIZE(o); ++i) v.push_back(tensor_arg(PyList_GET_ITEM(o, i), name));
     return v;
+}
+
+// plain(tensors...): whether the native entry points that have no general path may take them
+SNNTC_METHOD(py_plain) {
+    HANDLE_TH_ERRORS
+    bool ok = plain({});
+    for (Py_ssize_t i = 0; ok && i < n; ++i) ok = plain({tensor_arg(a[i], "argument")});
+    return PyBool_FromLong(ok);
+    END_HANDLE_TH_ERRORS
 }
 
 // encode_time(image) -> exp(1 - image) for a float32 device tensor
@@ -1023,15 +1066,16 @@ SNNTC_METHOD(py_recipe_step) {
     END_HANDLE_TH_ERRORS
 }
 
-// bind(path, SnntcLibraryError, SnntcError, params_array): looks the C ABI up in the library loaded from `path`
+// bind(path, SnntcLibraryError, SnntcError, params_array, general paths): looks the C ABI up in the library loaded from `path`
 SNNTC_METHOD(py_bind) {
     HANDLE_TH_ERRORS
-    arity(n, 4, "bind");
+    arity(n, 5, "bind");
     const char* path = PyUnicode_AsUTF8(a[0]);
     if (!path) throw python_error();
-    Py_INCREF(a[1]); Py_INCREF(a[2]); Py_INCREF(a[3]);
-    Py_XDECREF(g_library_error); Py_XDECREF(g_error); Py_XDECREF(g_params);
-    g_library_error = a[1]; g_error = a[2]; g_params = a[3];
+    TORCH_CHECK_TYPE(PyDict_Check(a[4]), "bind takes a dict of general paths");
+    for (int i = 1; i < 5; ++i) Py_INCREF(a[i]);
+    Py_XDECREF(g_library_error); Py_XDECREF(g_error); Py_XDECREF(g_params); Py_XDECREF(g_general);
+    g_library_error = a[1]; g_error = a[2]; g_params = a[3]; g_general = a[4];
     void* handle = dlopen(path, RTLD_NOW | RTLD_LOCAL);
     if (!handle) raise_class(g_library_error, message_args, 0, std::string("cannot load ") + path + ": " + dlerror());
     Library l;
@@ -1049,8 +1093,8 @@ SNNTC_METHOD(py_bind) {
 PyMethodDef g_methods[] = {SNNTC_ENTRY(bind), SNNTC_ENTRY(fc_forward), SNNTC_ENTRY(fc_layer), SNNTC_ENTRY(fc_backward),
                            SNNTC_ENTRY(cv_forward), SNNTC_ENTRY(cv_layer), SNNTC_ENTRY(cv_same), SNNTC_ENTRY(cv_backward),
                            SNNTC_ENTRY(min_pool), SNNTC_ENTRY(min_pool_layer), SNNTC_ENTRY(pad_layer), SNNTC_ENTRY(time_loss),
-                           SNNTC_ENTRY(loss_layer), SNNTC_ENTRY(sgd_update), SNNTC_ENTRY(encode_time), SNNTC_ENTRY(constraint_cost),
-                           SNNTC_ENTRY(recipe_step), {nullptr, nullptr, 0, nullptr}};
+                           SNNTC_ENTRY(loss_layer), SNNTC_ENTRY(sgd_update), SNNTC_ENTRY(plain), SNNTC_ENTRY(encode_time),
+                           SNNTC_ENTRY(constraint_cost), SNNTC_ENTRY(recipe_step), {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_binding", "Native host path of the SNN-TC ops.", -1, g_methods,
                         nullptr, nullptr, nullptr, nullptr};

@@ -153,7 +153,8 @@ def native():
         except ImportError as e:
             raise SnntcLibraryError(f"snntc_amd/_binding.so is missing or cannot be loaded ({e}): build it with "
                                     f"`make -C {CSRC_DIR}`. There is no CPU fallback for the SNN-TC ops.") from e
-        _binding.bind(lib_path(), SnntcLibraryError, SnntcError, params_array)
+        from . import ops
+        _binding.bind(lib_path(), SnntcLibraryError, SnntcError, params_array, ops.GENERAL)
         _native = _binding
     return _native
 

@@ -10,10 +10,13 @@ Counterparts of the reference's op handles (SNN_TC_Modules.py:29-33, 89-93):
 ``SnnFc`` / ``SnnCv`` are the differentiable ops that replace ``@ops.RegisterGradient``.
 Tensors must be float32 on a ROCm device; ``Params`` is the host-side float32 vector the layers
 build.  PyTorch supplies device memory, the current HIP stream and the autograd engine; the host side
-of a call (checks, allocation, launches, graph nodes) is csrc/binding.cpp.
+of a call (checks, allocation, launches, graph nodes) is csrc/binding.cpp.  The differentiable ops are
+``torch.autograd.Function`` classes whose ``apply`` is that native path; it hands a call with forward-mode
+tangents, functorch transforms, tracers or tensor wrappers in it to the function itself (``GENERAL``).
 """
 import ctypes
 
+import numpy as np
 import torch
 
 from . import _lib
@@ -178,42 +181,93 @@ def snncv_grad(grad, X, W, Params, Y, want_dparams=True, want_dx=True, want_dw=T
                                      None if crop is None else tuple(crop))
 
 
-class SnnFc:
+def _keep(ctx, X, W, Y, Params):
+    ctx.save_for_backward(X, W, Y)
+    ctx.params = np.array(Params, dtype=np.float32, copy=True)
+
+
+def _layer_grads(op, ctx, grad, **how):
+    X, W, Y = ctx.saved_tensors
+    return op(grad, X, W, ctx.params, Y, want_dparams=False, want_dx=ctx.needs_input_grad[0],
+              want_dw=ctx.needs_input_grad[1], **how)[:2]
+
+
+class SnnFc(torch.autograd.Function):
     """Y = snnfc(X, W, Params) with the gradient the reference registers for "SnnFc"
     (SNN_TC_Modules.py:31-33): the backward op receives the full [2B,J] forward output."""
 
-    @staticmethod
-    def apply(X, W, Params):
+    @classmethod
+    def apply(cls, X, W, Params):
         return _lib.native().fc_layer(X, W, Params, False)
 
-
-class SnnCv:
-    """Y = snncv(Xpad, W, Params) with the gradient registered for "SnnCv" (SNN_TC_Modules.py:91-93)."""
+    @staticmethod
+    def forward(ctx, X, W, Params):
+        Y = snnfc(X, W, Params)
+        _keep(ctx, X, W, Y, Params)
+        return Y
 
     @staticmethod
-    def apply(X, W, Params):
+    def backward(ctx, grad):
+        return *_layer_grads(snnfc_grad, ctx, grad), None
+
+
+class SnnCv(torch.autograd.Function):
+    """Y = snncv(Xpad, W, Params) with the gradient registered for "SnnCv" (SNN_TC_Modules.py:91-93)."""
+
+    @classmethod
+    def apply(cls, X, W, Params):
         return _lib.native().cv_layer(X, W, Params, False)
 
+    @staticmethod
+    def forward(ctx, X, W, Params):
+        Y = snncv(X, W, Params)
+        _keep(ctx, X, W, Y, Params)
+        return Y
 
-class SnnFcTimes:
+    @staticmethod
+    def backward(ctx, grad):
+        return *_layer_grads(snncv_grad, ctx, grad), None
+
+
+class SnnFcTimes(torch.autograd.Function):
     """What SNN_dense.call returns (SNN_TC_Modules.py:73-75): the spike times Y[:B] of snnfc.  The full
     [2B,J] output is kept for the backward op, which then takes the [B,J] upstream gradient directly --
     slicing the output of SnnFc instead costs a zero fill and a copy of [2B,J] per backward pass."""
 
-    @staticmethod
-    def apply(X, W, Params):
+    @classmethod
+    def apply(cls, X, W, Params):
         return _lib.native().fc_layer(X, W, Params, True)
 
-
-class SnnCvTimes:
-    """Spike times Y[:B] of snncv, as SNN_conv.call returns them (SNN_TC_Modules.py:168-170)."""
+    @staticmethod
+    def forward(ctx, X, W, Params):
+        Y = snnfc(X, W, Params)
+        _keep(ctx, X, W, Y, Params)
+        return Y[:X.shape[0]]
 
     @staticmethod
-    def apply(X, W, Params):
+    def backward(ctx, grad):
+        return *_layer_grads(snnfc_grad, ctx, grad, first_half_grad=True), None
+
+
+class SnnCvTimes(torch.autograd.Function):
+    """Spike times Y[:B] of snncv, as SNN_conv.call returns them (SNN_TC_Modules.py:168-170)."""
+
+    @classmethod
+    def apply(cls, X, W, Params):
         return _lib.native().cv_layer(X, W, Params, True)
 
+    @staticmethod
+    def forward(ctx, X, W, Params):
+        Y = snncv(X, W, Params)
+        _keep(ctx, X, W, Y, Params)
+        return Y[:X.shape[0]]
 
-class SnnCvSame:
+    @staticmethod
+    def backward(ctx, grad):
+        return *_layer_grads(snncv_grad, ctx, grad, first_half_grad=True), None
+
+
+class SnnCvSame(torch.autograd.Function):
     """SNN_conv with SAME padding as one differentiable step on the un-padded image x[B,H,W,C]: pad with
     MAX_SPIKE_TIME, snncv, and in the backward pass the gradient with respect to x itself (the op stores
     only that window of the padded gradient, so no separate crop runs).
@@ -223,10 +277,27 @@ class SnnCvSame:
       next_xpad None, or the padded input buffer of the conv layer that follows: the spike times are
                 written there as well, at pixel offset next_offset."""
 
-    @staticmethod
-    def apply(x, W, Params, pads, xpad, next_xpad, next_offset):
+    @classmethod
+    def apply(cls, x, W, Params, pads, xpad, next_xpad, next_offset):
         return _lib.native().cv_same(x, W, Params, pads[0], pads[1], pads[2], pads[3], xpad, next_xpad, next_offset[0],
                                      next_offset[1])
+
+    @staticmethod
+    def forward(ctx, x, W, Params, pads, xpad, next_xpad, next_offset):
+        top, bottom, left, right = pads
+        B, H, Wd, C = x.shape
+        if xpad is None:
+            xpad = pad_time(x, top, bottom, left, right, float(Params[0])) if any(pads) else x
+        elif tuple(xpad.shape) != (B, top + H + bottom, left + Wd + right, C):
+            raise ValueError(f"padded buffer {tuple(xpad.shape)} does not match input {tuple(x.shape)} and pads {pads}")
+        Y = snncv(xpad, W, Params, next_xpad=next_xpad, next_offset=next_offset)
+        _keep(ctx, xpad, W, Y, Params)
+        ctx.crop = (H, Wd, top, left)
+        return Y[:B]
+
+    @staticmethod
+    def backward(ctx, grad):
+        return *_layer_grads(snncv_grad, ctx, grad, first_half_grad=True, crop=ctx.crop), None, None, None, None, None
 
 
 def softmax_time_loss(times, label, want_loss=True, want_grad=True):
@@ -246,12 +317,22 @@ def sgd_update(params, grads, lr):
         _lib.native().sgd_update(params, grads, lr)
 
 
-class SoftmaxTimeLoss:
+class SoftmaxTimeLoss(torch.autograd.Function):
     """mean_b CE(label_b, softmax(-times_b)); the gradient is produced by the forward kernel."""
 
-    @staticmethod
-    def apply(times, label):
+    @classmethod
+    def apply(cls, times, label):
         return _lib.native().loss_layer(times, label)
+
+    @staticmethod
+    def forward(ctx, times, label):
+        loss, grad = softmax_time_loss(times, label, want_grad=times.requires_grad)
+        ctx.save_for_backward(*[] if grad is None else [grad])
+        return loss.mean()
+
+    @staticmethod
+    def backward(ctx, upstream):
+        return (ctx.saved_tensors[0] * upstream if ctx.saved_tensors else None), None
 
 
 def min_pool(x, kernel, stride, pad, out_hw, pad_value=1e5, want_arg=True, next_xpad=None, next_offset=(0, 0)):
@@ -280,14 +361,27 @@ def min_pool_grad(grad_y, arg, in_shape, kernel, stride, pad):
     return dx
 
 
-class SnnMinPool:
+class SnnMinPool(torch.autograd.Function):
     """SNN_maxpool2d on device tensors: min over the (implicitly padded) window, gradient to the
     position that attained it."""
 
-    @staticmethod
-    def apply(x, kernel, stride, pad, out_hw, pad_value, next_xpad=None, next_offset=(0, 0)):
+    @classmethod
+    def apply(cls, x, kernel, stride, pad, out_hw, pad_value, next_xpad=None, next_offset=(0, 0)):
         return _lib.native().min_pool_layer(x, kernel[0], kernel[1], stride[0], stride[1], pad[0], pad[1], out_hw[0], out_hw[1],
                                             pad_value, next_xpad, next_offset[0], next_offset[1])
+
+    @staticmethod
+    def forward(ctx, x, kernel, stride, pad, out_hw, pad_value, next_xpad, next_offset):
+        y, arg = min_pool(x, kernel, stride, pad, out_hw, pad_value, want_arg=x.requires_grad, next_xpad=next_xpad,
+                          next_offset=next_offset)
+        ctx.geom = (tuple(x.shape), kernel, stride, pad)
+        ctx.save_for_backward(*[] if arg is None else [arg])
+        return y
+
+    @staticmethod
+    def backward(ctx, grad_y):
+        dx = min_pool_grad(grad_y, ctx.saved_tensors[0], *ctx.geom) if ctx.saved_tensors else None
+        return dx, None, None, None, None, None, None, None
 
 
 def pad_time(x, top, bottom, left, right, value):
@@ -315,9 +409,35 @@ def pad_time_grad(dxpad, in_shape, top, left):
     return dx
 
 
-class SnnPadTime:
+class SnnPadTime(torch.autograd.Function):
     """SAME padding of a conv layer's input with MAX_SPIKE_TIME, one kernel each way."""
 
-    @staticmethod
-    def apply(x, top, bottom, left, right, value):
+    @classmethod
+    def apply(cls, x, top, bottom, left, right, value):
         return _lib.native().pad_layer(x, top, bottom, left, right, value)
+
+    @staticmethod
+    def forward(ctx, x, top, bottom, left, right, value):
+        ctx.geom = (tuple(x.shape), top, left)
+        return pad_time(x, top, bottom, left, right, value)
+
+    @staticmethod
+    def backward(ctx, dxpad):
+        return pad_time_grad(dxpad, *ctx.geom), None, None, None, None, None
+
+
+def _function(cls, *args):
+    return super(cls, cls).apply(*args)                     # torch.autograd.Function's own
+
+
+#: the differentiable ops with the arguments of their native entry points, as torch.autograd.Function runs them
+GENERAL = {
+    "fc_layer": lambda X, W, Params, times: _function(SnnFcTimes if times else SnnFc, X, W, Params),
+    "cv_layer": lambda X, W, Params, times: _function(SnnCvTimes if times else SnnCv, X, W, Params),
+    "cv_same": lambda x, W, Params, top, bottom, left, right, xpad, next_xpad, ntop, nleft: _function(
+        SnnCvSame, x, W, Params, (top, bottom, left, right), xpad, next_xpad, (ntop, nleft)),
+    "min_pool_layer": lambda x, kh, kw, sh, sw, top, left, nh, nw, value, next_xpad, ntop, nleft: _function(
+        SnnMinPool, x, (kh, kw), (sh, sw), (top, left), (nh, nw), value, next_xpad, (ntop, nleft)),
+    "pad_layer": lambda x, top, bottom, left, right, value: _function(SnnPadTime, x, top, bottom, left, right, value),
+    "loss_layer": lambda times, label: _function(SoftmaxTimeLoss, times, label),
+}
