@@ -93,3 +93,81 @@ def test_a_trace_records_the_op(name):
         traced = torch.jit.trace(module, (x,))
         for y in (x, 2.0 - 0.5 * x):
             assert torch.equal(traced(y), module(y))
+
+
+# ---- the recipe's encoding and weight-constraint cost: stock ops wherever the kernels would lose something ------------
+
+def _stock_cost(weights, k, k2):
+    return (k * sum(torch.clamp(1.0 - w.sum(0), min=0.0).mean() for w in weights)
+            + k2 * sum(torch.square(w).mean() for w in weights))
+
+
+class _Held(torch.nn.Module):
+    """Something with layers whose weights are whatever tensors it is given."""
+
+    class Layer(torch.nn.Module):
+        w_sum_cost = None
+
+        def __init__(self, weight):
+            super().__init__()
+            self.weight = weight
+
+    def __init__(self, *weights):
+        super().__init__()
+        self.layers = torch.nn.ModuleList(self.Layer(w) for w in weights)
+
+
+def _weights():
+    return [_rand(13, 20) / 13, _rand(21, 5) / 40]
+
+
+def test_encoding_keeps_tangents_transforms_and_strides():
+    from snntc_amd import train
+    x, t = torch.rand(4, 6, device=DEV), torch.rand(4, 6, device=DEV)
+    want = torch.exp(1.0 - x)
+    with fwAD.dual_level():
+        out = fwAD.unpack_dual(train.encode_input(fwAD.make_dual(x, t)))
+        assert torch.allclose(out.tangent, -want * t) and torch.allclose(out.primal, want)
+    assert torch.allclose(torch.func.vmap(train.encode_input)(x), want)
+    assert torch.allclose(torch.func.grad(lambda v: train.encode_input(v).sum())(x), -want)
+    assert torch.allclose(torch.jit.trace(train.encode_input, (x,))(t), torch.exp(1.0 - t))
+    assert torch.allclose(torch.compile(train.encode_input, backend="eager", fullgraph=True)(x), want)
+    assert train.encode_input(x.t()).stride() == x.t().stride() and torch.equal(train.encode_input(x.t()), train.encode_input(x).t())
+
+
+def test_cost_keeps_tangents_transforms_and_factors():
+    from snntc_amd import train
+    ws = _weights()
+
+    def cost(*w, k=100.0, k2=1e-2):
+        return train.constraint_cost(_Held(*w), k, k2)
+
+    tangents = [torch.rand_like(w) for w in ws]
+    grads = torch.func.grad(_stock_cost)(ws, 100.0, 1e-2)
+    directional = sum((g * t).sum() for g, t in zip(grads, tangents))
+    with fwAD.dual_level():
+        out = fwAD.unpack_dual(cost(*[fwAD.make_dual(w, t) for w, t in zip(ws, tangents)]))
+        assert torch.allclose(out.tangent, directional, rtol=1e-5)
+    for g, want in zip(torch.func.grad(cost, argnums=(0, 1))(*ws), grads):
+        assert torch.allclose(g, want, rtol=1e-5)
+    many = [torch.stack([w, 2 * w]) for w in ws]
+    each = torch.stack([_stock_cost(ws, 100.0, 1e-2), _stock_cost([2 * w for w in ws], 100.0, 1e-2)])
+    assert torch.allclose(torch.func.vmap(cost)(*many), each, rtol=1e-5)
+    k, k2 = (torch.tensor(v, device=DEV, requires_grad=True) for v in (100.0, 1e-2))
+    got = torch.autograd.grad(cost(*ws, k=k, k2=k2), [k, k2])
+    for g, want in zip(got, torch.autograd.grad(_stock_cost(ws, k, k2), [k, k2])):
+        assert torch.allclose(g, want, rtol=1e-5)
+
+
+def test_recipe_step_with_a_factor_that_is_a_tensor():
+    import snntc_amd as snn
+    from snntc_amd import train
+    w = torch.rand(13, 4).numpy() / 4
+    images, labels = torch.rand(5, 12, device=DEV), torch.randint(0, 4, (5,), device=DEV)
+    results = []
+    for k in (100.0, torch.tensor(100.0, device=DEV)):
+        model = snn.SNN_dense(12, 4, weight=w).to(DEV)
+        loss, correct = train.train_step(model, torch.optim.SGD(model.parameters(), lr=0.1), images, labels, 4, weight_k=k)
+        results.append((loss, correct, model.weight.detach()))
+    for a, b in zip(*results):
+        assert torch.allclose(a.float(), b.float(), rtol=1e-5, atol=1e-6)
