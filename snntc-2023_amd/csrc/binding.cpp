@@ -379,9 +379,7 @@ struct LossNode : public Node {
     variable_list apply(variable_list&& grads) override {
         std::lock_guard<std::mutex> lock(mutex_);
         if (!grads[0].defined()) return variable_list(1);
-        const Tensor g = grad.unpack();
-        at::AutoGradMode no_grad(false);
-        return {g * grads[0]};
+        return {grad.unpack() * grads[0]};                  // (differentiable in the upstream factor)
     }
 };
 
@@ -585,7 +583,14 @@ struct CostNode : public Node {
         if (!grads[0].defined()) return out;
         std::vector<Tensor> w;
         for (SavedVariable& s : weights) w.push_back(s.unpack());
-        at::AutoGradMode no_grad(false);
+        if (at::GradMode::is_enabled() || !plain({grads[0]})) {        // a graph of the gradient is wanted: differentiable ops
+            for (size_t i = 0; i < w.size(); ++i) {
+                if (!task_should_compute_output(i)) continue;
+                const Tensor low = (1.0 - w[i].detach().sum(0)).ge(0).to(at::kFloat);
+                out[i] = grads[0] * (low * (-k / (float)w[i].size(1)) + w[i] * (2.0f * k2 / (float)w[i].numel()));
+            }
+            return out;
+        }
         const Tensor up = grads[0].contiguous();
         const c10::DeviceGuard guard(up.device());
         CostArgs args(w);

@@ -171,3 +171,38 @@ def test_recipe_step_with_a_factor_that_is_a_tensor():
         results.append((loss, correct, model.weight.detach()))
     for a, b in zip(*results):
         assert torch.allclose(a.float(), b.float(), rtol=1e-5, atol=1e-6)
+
+
+def test_gradients_of_the_gradient():
+    """A penalty on the cost's gradient, and the loss's gradient in its upstream factor: the same second derivatives as the
+    stock composition in float64."""
+    import snntc_amd as snn
+    from snntc_amd import train
+    ws = [w.requires_grad_(True) for w in _weights()]
+    ref = [w.detach().double().cpu().requires_grad_(True) for w in ws]
+    scale, ref_scale = torch.tensor(3.0, device=DEV, requires_grad=True), torch.tensor(3.0, dtype=torch.float64, requires_grad=True)
+
+    def penalty(cost, weights, s):
+        first = torch.autograd.grad(cost * s, weights, create_graph=True)
+        return [*first, *torch.autograd.grad(sum((g * g).sum() for g in first), [*weights, s])]
+
+    for g, want in zip(penalty(train.constraint_cost(_Held(*ws), 100.0, 1e-2), ws, scale), penalty(_stock_cost(ref, 100.0, 1e-2), ref, ref_scale)):
+        assert torch.allclose(g.double().cpu(), want, rtol=1e-5, atol=1e-9)
+
+    times = _rand(4, 5).requires_grad_(True)
+    label = torch.eye(5, device=DEV)[:4]
+    first, = torch.autograd.grad(snn.loss_func(logit=times, label=label) * scale, [times], create_graph=True)
+    by_scale, = torch.autograd.grad((first * first).sum(), [scale])
+    assert torch.allclose(by_scale, 2.0 * (first.detach() ** 2).sum() / 3.0, rtol=1e-5)
+
+
+def test_batched_upstream_gradients_of_cost_and_loss():
+    import snntc_amd as snn
+    from snntc_amd import train
+    ws = [w.requires_grad_(True) for w in _weights()]
+    times, label = _rand(4, 5).requires_grad_(True), torch.eye(5, device=DEV)[:4]
+    up = torch.tensor([1.0, 0.5, -2.0], device=DEV)
+    for out, inputs in ((train.constraint_cost(_Held(*ws)), ws), (snn.loss_func(logit=times, label=label), [times])):
+        one = torch.autograd.grad(out, inputs, retain_graph=True)
+        for g, want in zip(torch.autograd.grad(out, inputs, up, is_grads_batched=True), one):
+            assert torch.allclose(g, up.view(-1, 1, 1) * want, rtol=1e-5)
