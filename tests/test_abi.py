@@ -124,6 +124,18 @@ def test_workspace_queries(lib):
     assert n.value >= 64 * 32 * 32 * 576 * 8
 
 
+def test_tall_narrow_dense_gradients_are_sliced_for_the_whole_chip(lib):
+    """The backward workspace holds the partial weight gradients, one per slice of the samples: tiles of 64 x 64 times slices
+    give half of the 256 CUs a workgroup wherever slices of 64 samples allow it."""
+    n = ctypes.c_size_t()
+    for B, I, J in [(65536, 64, 17), (65536, 64, 64), (65536, 63, 33), (20000, 100, 100), (4096, 200, 64), (9000, 300, 40), (2048, 50, 20)]:
+        assert lib.snntc_fc_backward_workspace_bytes(B, I, J, ctypes.byref(n)) == 0
+        slices = (n.value - (B * J + (I + 1) * J) * 4) // ((I + 1) * J * 4)
+        tiles = -(-J // 64) * -(-(I + 1) // 64)
+        assert tiles * slices >= min(128, tiles * (B // 64) // 2), (B, I, J, slices)
+        assert B // slices >= 60, (B, I, J, slices)
+
+
 def test_python_ops_map_status_to_exceptions():
     from snntc_amd import _lib
     lib = _lib.load()

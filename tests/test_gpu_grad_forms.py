@@ -20,6 +20,7 @@ def t(a):
     (260, 520, 130), (700, 500, 40), (1100, 1000, 101),                   # many tiles: eight, one, four
     (129, 64, 300), (515, 127, 64), (1030, 300, 257),                     # slices of the samples
     (300, 1500, 1299),                                                    # four wavefronts per tile of dW
+    (2200, 63, 33), (4200, 64, 65),                                       # one and four tiles: more slices than sixteen
 ])
 def test_dense_gradients(B, I, J):
     import snntc_amd as snn
