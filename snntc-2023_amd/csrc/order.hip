@@ -13,7 +13,8 @@
 // decades).  An input's rank is the number of inputs before its 32-bit word plus the bits below its own.  About one input
 // in eight lies in a word where two share a bit; these go to a list, are gathered by word and compared with the two or three
 // others there.  Inputs that never spiked all carry the same largest time: they keep their index order behind the others,
-// by a prefix count.  Should any other value repeat more than ORDER_BUCKET_LIMIT times, a bitonic network sorts the region.
+// by a prefix count.  Where another value repeats (or values crowd) so that more than ORDER_BUCKET_LIMIT inputs share a word,
+// the region's inputs are ranked by a stable radix sort instead, eight bits a pass.
 //
 // A patch's bitmap is the union of its pixels' (patches of 32 channels and more; built once per region) or is set bit by bit.
 // Patches of up to 1152 inputs belong to a wavefront, which needs no barrier for them; longer ones to the workgroup.
@@ -24,6 +25,13 @@
 // them by merge path (chains of dependent LDS reads), in us: those 65 536 patches 188 -> 93, 100 352 of 576 297 -> 129, 25 088
 // of 1152 227 -> 84, 6272 of 2304 144 -> 56, 1568 of 4608 79 -> 43, 3136 of 576 34 -> 16; 401 408 of 147 (7x7x3, stride 2),
 // sorted patch by patch before, 438 -> 155.
+//
+// Ties, on 8-bit images (as they are / a third of the rows saturated / smooth / one value), us, next to continuous values and to
+// the order by networks and merges that this replaced (any values): 65 536 patches of 576 inputs 158 / 174 / 182 / 194 (88; 205),
+// 401 408 of 147 177 / 228 / 240 / 319 (138; 430), 131 072 of 75 43 / 52 / 51 / 58 (41; 89), 6272 of 2304 109 / 119 / 133 / 134 (50; 140);
+// above it only at few long and at short strided patches: 1568 of 4608 88 / 115 / 108 / 96 (39; 77), 16 384 of 180 33 / 52 / 38 / 45
+// (18; 33).  A bitonic network over the region in the radix sort's place took 173 / 420 / 469 / 724 for the first.  With up to
+// 64 inputs compared per word instead of 16 they take up to 37 % longer (smooth 248), with 8 the continuous ones do (96).
 #include <algorithm>
 #include <atomic>
 
@@ -34,8 +42,9 @@ namespace {
 
 constexpr int ORDER_COARSE = 1024;
 constexpr int ORDER_COARSE_BITS = 10;
-constexpr int ORDER_BUCKET_LIMIT = 64;
+constexpr int ORDER_BUCKET_LIMIT = 16;                       // inputs of a word that are still compared with each other
 constexpr int ORDER_EPT = 16;                              // region inputs per thread at most
+constexpr int ORDER_RADIX_PITCH = 260;                     // 256 digit counts and a shift of the banks
 constexpr int ORDER_LDS_BYTES = 160 * 1024;
 
 struct OrderGeom {
@@ -102,13 +111,12 @@ __device__ __forceinline__ uint32_t pack_ranks(uint32_t r) { return ((r >> 2) & 
 // LDS: values [n_cap] u32, ranks [n_cap] u16, then -- one after the other -- the ranking's tables or the patches' bitmaps
 // and staging buffers.
 inline size_t order_lds_bytes(int n_cap, int threads, int stride, int waves, int patches, int region_pixels) {
-    size_t pow2 = 64;
-    while (pow2 < (size_t)n_cap) pow2 *= 2;
     const size_t bit_len = ((size_t)(n_cap + 31) / 32 + 3) / 4 * 4;
     const size_t head = ((size_t)n_cap * 6 + 15) / 16 * 16;
     const size_t list_cap = ((size_t)n_cap + 4 * threads - 1) / (4 * threads) * (4 * threads);
     size_t tables = (ORDER_COARSE + kWave) * 4 + (((size_t)n_cap + 7) / 8 * 4 + kWave) * 8 + ((size_t)n_cap + 1) / 2 * 4 + list_cap * 2 + 64;
-    if (tables < pow2 * 2) tables = pow2 * 2;
+    const size_t radix = ((size_t)n_cap + 3) / 4 * 16 + (size_t)threads / kWave * ORDER_RADIX_PITCH * 4;
+    if (tables < radix) tables = radix;
     const size_t per_patch = waves ? (size_t)waves * (bit_len * 8 + (size_t)stride * 4)             // a patch per wavefront
                                    : (size_t)patches * bit_len * 8 + (size_t)stride * 8;
     const size_t after = (size_t)region_pixels * bit_len * 4 + per_patch;
@@ -379,7 +387,7 @@ order_patches_kernel(const float* __restrict__ xpad, float* __restrict__ sorted,
     if (lane == 0) bases[1][wave] = carry;
     if (__builtin_amdgcn_ballot_w64(fullest > ORDER_BUCKET_LIMIT) != 0 && lane == 0) overflow = 1;
     __syncthreads();
-    const bool give_up = overflow != 0;
+    const bool give_up = __builtin_amdgcn_readfirstlane((int)overflow) != 0;
     if (!give_up) {
         uint32_t base = 0;
 #pragma unroll
@@ -494,23 +502,71 @@ order_patches_kernel(const float* __restrict__ xpad, float* __restrict__ sorted,
             count(e, k, word);
         }
     } else {
-        // a value repeats too often: bitonic network over the inputs' indexes, compared by (value, index)
-        uint16_t* item = reinterpret_cast<uint16_t*>(area);
-        int pow2 = 64;
-        while (pow2 < n) pow2 *= 2;
-        for (int i = tid; i < pow2; i += T) item[i] = (uint16_t)i;
-        __syncthreads();
-        auto full_key = [&](uint32_t i) { return (unsigned long long)(i < (uint32_t)n ? order_key(value[i]) : ~0u) << 32 | i; };
-        for (int k = 1; k < pow2; k *= 2)
-            for (int j = k; j > 0; j /= 2) {
-                for (int i = tid; i < pow2 / 2; i += T) {
-                    const int lo = 2 * i - (i & (j - 1)), hi = lo + j;
-                    const uint16_t a = item[lo], b = item[hi];
-                    if ((full_key(a) > full_key(b)) == ((lo & (2 * k)) == 0)) { item[lo] = b; item[hi] = a; }
-                }
-                __syncthreads();
+        // a value repeats too often: stable radix sort of the inputs' indexes, eight bits of the distance from the
+        // smallest key a pass; the last pass leaves ranks.  A wavefront takes a run of inputs, 64 at a time.
+        constexpr int DIGITS = 256, PITCH = ORDER_RADIX_PITCH, GROUP = WAVES / 4;
+        const int rounds = (n + T - 1) / T, half = (g.n_cap + 3) / 4 * 4;
+        uint16_t* item = reinterpret_cast<uint16_t*>(area);                              // [2][half], from pass to pass
+        uint32_t* count = area + half;                      // [wavefront][digit]
+        uint32_t* own = count + wave * PITCH;
+        const uint32_t spread = k_max - k_min;
+        int shift = 0;
+        do {
+            const bool last_pass = spread >> shift < DIGITS;
+            const uint16_t* from = item + ((shift / 8) & 1) * half;
+            uint16_t* to = item + ((shift / 8 + 1) & 1) * half;
+            auto index_at = [&](int at) { return shift == 0 ? (uint32_t)at : (uint32_t)from[at]; };
+            auto digit_of = [&](uint32_t e) { return ((order_key(value[e]) - k_min) >> shift) & (DIGITS - 1); };
+            reinterpret_cast<uint4*>(own)[lane] = make_uint4(0, 0, 0, 0);
+            lds_order();
+#pragma unroll 1
+            for (int r = 0; r < rounds; ++r) {
+                const int at = (wave * rounds + r) * kWave + lane;
+                if (at < n) atomicAdd(&own[digit_of(index_at(at))], 1u);
             }
-        for (int i = tid; i < n; i += T) rank[item[i]] = (uint16_t)pack_ranks((uint32_t)i);
+            __syncthreads();
+            // inputs before the ones of a wavefront and digit: in order of (digit, wavefront), four wavefronts per thread
+            const int digit = tid / GROUP, first = tid % GROUP * 4;
+            uint32_t c[4], sum = 0;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) sum += c[q] = count[(first + q) * PITCH + digit];
+            uint32_t at_or_below = wave_prefix(sum);
+            if (lane == kWave - 1) bases[0][wave] = at_or_below;
+            __syncthreads();
+            uint32_t start = at_or_below - sum;
+#pragma unroll 1
+            for (int v = 0; v < wave; ++v) start += bases[0][v];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                count[(first + q) * PITCH + digit] = start;
+                start += c[q];
+            }
+            __syncthreads();
+#pragma unroll 1
+            for (int r = 0; r < rounds; ++r) {
+                const int at = (wave * rounds + r) * kWave + lane;
+                const uint32_t e = at < n ? index_at(at) : 0, dg = digit_of(e);
+                const uint64_t some = __builtin_amdgcn_ballot_w64(at < n);
+                uint32_t lo = (uint32_t)some, hi = (uint32_t)(some >> 32);               // lanes with the same digit
+#pragma unroll 4
+                for (int b = 0; b < 8; ++b) {               // (in two goes: all eight at once cost every launch 12 registers)
+                    const uint32_t unset = ((dg >> b) & 1) - 1;
+                    const uint64_t set = __builtin_amdgcn_ballot_w64(unset == 0);
+                    lo &= (uint32_t)set ^ unset;
+                    hi &= (uint32_t)(set >> 32) ^ unset;
+                }
+                const uint64_t same = (uint64_t)hi << 32 | lo;
+                if (at < n) {
+                    const uint32_t before = own[dg], place = before + lanes_below(same);
+                    if ((same >> lane) == 1) own[dg] = place + 1;                        // the last of them
+                    if (last_pass) rank[e] = (uint16_t)pack_ranks(place);
+                    else to[place] = (uint16_t)e;
+                }
+                lds_order();
+            }
+            __syncthreads();
+            shift += 8;
+        } while (shift < 32 && spread >> shift);
     }
     __syncthreads();                                        // ranks are in place, the tables are free
 

@@ -47,12 +47,16 @@ def _values(kind, rng, shape):
         x = rng.standard_normal(shape).astype(np.float32)
         x[rng.random(shape) < 0.01] = 0.0
         x[rng.random(shape) < 0.01] = -0.0
+    elif kind == "bytes":                                   # an 8-bit image with a saturated part and one of a single value
+        x = np.exp(1.0 - rng.integers(0, 256, shape) / 255.0).astype(np.float32)
+        x[:, : shape[1] // 3] = 1.0
+        x[-1] = 1.5
     elif kind == "repeats":                                 # half the inputs share one value
         x[rng.random(shape) < 0.5] = 1.25
     return x
 
 
-@pytest.mark.parametrize("kind", ["plain", "silent", "crowded", "signs", "repeats"])
+@pytest.mark.parametrize("kind", ["plain", "silent", "crowded", "signs", "repeats", "bytes"])
 @pytest.mark.parametrize("B,H,W,C,Kh,Kw,Sh,Sw", FORMS)
 def test_patch_order(B, H, W, C, Kh, Kw, Sh, Sw, kind):
     import snntc_amd as snn
