@@ -804,6 +804,21 @@ __device__ __forceinline__ void read_columns(__attribute__((address_space(3))) c
 // exceeds thr, which is the condition above.  With weight sums that stay above 4W the bound is t_7 itself;
 // below, a chunk may fail although none of its inputs closes the set, by (x_7 - x_0)*4W at most.
 // Two additions per input and ten instructions per chunk and neuron.
+//
+// That slack is small next to ysum - x*wsum, which starts at theta*x, where weights are small and the sum soon leaves zero;
+// under zero-mean weights of a larger spread (the layers' own initialiser, sqrt(15 / inputs)) it stops most scans several
+// times each, and every stop costs steps and another pass over the row.  There (TIGHT) the smallest weight sum of the chunk is
+// tracked, one three-way minimum per two inputs, and the lane accepts if
+//     fma(x_7 - x_0, min(0, wsum_0 .. wsum_7), t_7)  >  thr + the last term above.
+// A workgroup decides by the size of its slice's weights: W * sqrt(inputs) against theta is about 4.5 times the spread of a
+// whole row's weight sum in units of the threshold.  us, bounded / tracked, at W*sqrt(I)/theta of about 5, 7, 9, 13 and 18:
+//   784 -> 800, 4096 rows            334 / 346   336 / 348   351 / 340   381 / 352   507 / 356
+//   784 -> 800, 256 rows              40 / 41     46 / 42     53 / 45     60 / 48     86 / 50
+//   65 536 patches of 576, 64        230 / 252   238 / 252   260 / 254   305 / 261   448 / 288
+//   401 408 patches of 147, 64       605 / 611   643 / 571   762 / 549  1278 / 555  1674 / 585
+//   131 072 patches of 288, 32       160 / 170   175 / 167   200 / 164   281 / 171   345 / 173
+//   1568 patches of 4608, 512        652 / 656   656 / 662   656 / 660   680 / 677   692 / 679
+constexpr float TIGHT_FROM = 7.0f;
 constexpr float FILTER_END_Y = 0x1p-19f;                  // 32u >= 4u + 17.2u, times |ysum_7|
 constexpr float FILTER_END_XW = 0x1p-19f;                 // 32u >= 17.2u, times x_7 * |wsum_7|
 constexpr float FILTER_END_W = 0x1p-15f;                  // 512u >= 36u + 310u, times x_7 * max|w| of the slice
@@ -813,11 +828,12 @@ constexpr float FILTER_END_W = 0x1p-15f;                  // 512u >= 36u + 310u,
 // first index as kcur and leave `open`.  The arithmetic does not depend on EXEC or branches (lanes that
 // are not open compute along and discard), so the compiler is free to interleave it with the LDS traffic
 // of the next chunk; the decision works on lane masks in scalar registers.
-// dx = x[7] - x[0], x7s = FILTER_END_XW * x[7], thrx = FILTER_END_W * W * x[7] + dx * w4, w4 = 4W.
+// dx = x[7] - x[0], x7s = FILTER_END_XW * x[7], thrx = FILTER_END_W * W * x[7] (+ dx * 4W where the smallest weight sum is
+// bounded), low: the smallest weight sum or zero, or its bound + 4W.
 __device__ __forceinline__ void filter_test(float& wsum, float& ysum, int& kcur, uint64_t& open, int k, float wb, float yb,
-                                            float x7, float thrx, float dx, float x7s, float w4) {
+                                            float x7, float thrx, float dx, float x7s, float low) {
     const float t7 = __fmaf_rn(-x7, wb, yb);
-    const float bound = __fmaf_rn(dx, fminf(fminf(wsum, wb), w4), t7);
+    const float bound = __fmaf_rn(dx, low, t7);
     const float thr = __fmaf_rn(FILTER_END_Y, fabsf(yb), __fmaf_rn(x7s, fabsf(wb), thrx));
     uint64_t stop;
     // (two statements: the first has scalar results only, so the masks stay uniform values for the compiler
@@ -1002,17 +1018,20 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
     const float w_max = block_max(fill_weight_slice<COLS>(wl, w, rows, J, j0), wl + rows * COLS);
     const float end_w = FILTER_END_W * w_max;               // margin of the fast loop
     const float w4 = 4.0f * 1.00001f * w_max;               // 4W of its bound on the weight sums
+    const bool tight = __builtin_amdgcn_readfirstlane(w_max * sqrtf((float)I) > TIGHT_FROM * np.theta);
 
+    constexpr int NONE = 0x7fffffff;
+    constexpr int ROW_SHIFT = COLS == 64 ? 8 : COLS == 32 ? 7 : COLS == 16 ? 6 : 5;      // a weight row is COLS * 4 bytes
+    static_assert(COLS == 64 || COLS == 32 || COLS == 16 || COLS == 8, "slice width");
+
+    auto scan_items = [&](auto tight_c) {                   // the rest of the kernel, in both forms
+    constexpr bool TIGHT = decltype(tight_c)::value;
     const int lane = threadIdx.x % kWave;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int sub = lane / LANES, cg = lane - sub * LANES;
     const int j = j0 + CH * cg;                            // first of the lane's columns
     const float* __restrict__ wcol = wl + CH * cg;
     const unsigned wbase = (unsigned)(uintptr_t)(lds_cfloat*)wcol;          // LDS byte address of the lane's columns
-    constexpr int NONE = 0x7fffffff;
-    constexpr int ROW_SHIFT = COLS == 64 ? 8 : COLS == 32 ? 7 : COLS == 16 ? 6 : 5;      // a weight row is COLS * 4 bytes
-    static_assert(COLS == 64 || COLS == 32 || COLS == 16 || COLS == 8, "slice width");
-
     // `waves` wavefronts of the workgroup work on items; the others have only helped to copy the slice
     for (int item = group * waves + wave; wave < waves && item * SEGS < S; item += n_groups * waves) {
         const int seg_raw = item * SEGS + sub;
@@ -1153,7 +1172,7 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
                 // One chunk: wb / yb are the scans' sums behind its inputs.  The requests stay ahead of the
                 // arithmetic: what a half consumes was requested a half or more ago, and what it requests has the
                 // whole half to arrive.
-                float yb[CH], x0, x7;
+                float yb[CH], low[CH], x0, x7;
                 auto chunk = [&](auto ph_c, int k) {
                     constexpr int ph = decltype(ph_c)::value;
                     if constexpr (!BY_ROW) request((ph + ROUND - 1) % ROUND, k + (ROUND - 1) * CHUNK);
@@ -1171,8 +1190,10 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
                             for (int c = 0; c < CH; ++c) {
                                 const float wc = wv[H % NH][c][u];
                                 const bool start = hh == 0 && u == 0;
+                                const float before = wb[c];
                                 wb[c] = (start ? wsum[c] : wb[c]) + wc;
                                 yb[c] = __fmaf_rn(x[u], wc, start ? ysum[c] : yb[c]);
+                                if (TIGHT && u % 2 == 1) low[c] = fminf(fminf(hh == 0 && u == 1 ? 0.0f : low[c], before), wb[c]);
                             }
                     };
                     half(std::integral_constant<int, 0>{});
@@ -1190,10 +1211,11 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
                 };
                 auto test = [&](int k) {
                     const float dx = x7 - x0, x7s = x7 * FILTER_END_XW;
-                    const float thrx = __fmaf_rn(dx, w4, x7 * end_w);
+                    const float thrx = TIGHT ? x7 * end_w : __fmaf_rn(dx, w4, x7 * end_w);
 #pragma unroll
                     for (int c = 0; c < CH; ++c)
-                        filter_test(wsum[c], ysum[c], kcur[c], open[c], k, wb[c], yb[c], x7, thrx, dx, x7s, w4);
+                        filter_test(wsum[c], ysum[c], kcur[c], open[c], k, wb[c], yb[c], x7, thrx, dx, x7s,
+                                    TIGHT ? low[c] : fminf(fminf(wsum[c], wb[c]), w4));
                 };
                 // Whole rounds as long as the longest row has one left, without an exit inside the round: behind an
                 // exit test between a request and its use, several chunks later, the compiler would move the
@@ -1415,6 +1437,11 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
             }
         }
     }
+    };
+    // (Values computed before the branch would be kept for both forms and cost the loops scalar registers: 1 % of the time.)
+    asm volatile("" : "+s"(n_groups), "+s"(waves), "+s"(S), "+s"(stride), "+s"(J));
+    if (tight) scan_items(std::true_type{});
+    else scan_items(std::false_type{});
 }
 
 __global__ void __launch_bounds__(256)

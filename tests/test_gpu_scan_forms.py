@@ -27,17 +27,25 @@ def _check(x, w, p):
     assert torch.equal(out, out2)
 
 
-@pytest.mark.parametrize("B,I,J", [
+SIZES = [
     (20011, 31, 64), (20011, 33, 63), (12007, 72, 128),     # 64-column slices, four neurons: below, above, between rounds
     (9001, 7, 50), (9001, 8, 50), (9001, 9, 50), (9001, 1, 40),          # rows of less than a chunk, one, one and a bit
     (6007, 650, 96), (3001, 785, 101),                      # 32-column slices: quads, and a ragged last slice
     (6007, 1301, 37), (700, 2305, 66),                      # 16-column slices
     (1500, 4600, 9), (40, 4601, 23),                        # 8-column slices, many wavefronts and few
     (1100, 400, 200), (300, 500, 70),                       # two neurons and one
-])
-def test_scan_forms(B, I, J):
+]
+
+
+@pytest.mark.parametrize("law", ["baseline", "initial"])    # the smallest weight sum of a chunk bounded, or tracked
+@pytest.mark.parametrize("B,I,J", SIZES)
+def test_scan_forms(B, I, J, law):
     """A tenth of the inputs (and all of every fiftieth row) never spiked, so rows of one wavefront differ in length."""
+    from snntc_amd.layers import init_weight
     x, w, p, _ = dense_case(B + I, B, I, J, True, "baseline")
+    if law == "initial":
+        np.random.seed(B + I)
+        w = init_weight(I, J, 1.0)
     rng = np.random.default_rng(I)
     x[rng.random(x.shape) < 0.1] = 1e5
     x[::50] = 2e5
@@ -46,8 +54,11 @@ def test_scan_forms(B, I, J):
 
 @pytest.mark.parametrize("kind,B,I,J", [("randn", 20000, 90, 64), ("ties", 12000, 100, 61), ("negative", 9000, 75, 64),
                                         ("bias_fires", 9000, 131, 64), ("late", 9000, 330, 32), ("sparse", 4000, 700, 40)])
-def test_four_neuron_lanes_off_the_common_path(kind, B, I, J):
+@pytest.mark.parametrize("small", [False, True])             # weights as they are, or scaled so that the weight sums are bounded
+def test_four_neuron_lanes_off_the_common_path(kind, B, I, J, small):
     x, w = _adversarial_dense(kind, 3, B, I, J)
+    if small:
+        w = (w * (6.0 / (np.abs(w).max() * I ** 0.5))).astype(np.float32)
     _check(x, w, capi.fc_params(1.0))
 
 
