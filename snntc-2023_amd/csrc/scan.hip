@@ -806,19 +806,22 @@ __device__ __forceinline__ void read_columns(__attribute__((address_space(3))) c
 // Two additions per input and ten instructions per chunk and neuron.
 //
 // That slack is small next to ysum - x*wsum, which starts at theta*x, where weights are small and the sum soon leaves zero;
-// under zero-mean weights of a larger spread (the layers' own initialiser, sqrt(15 / inputs)) it stops most scans several
+// under weights of a larger spread (the layers' own initialiser: mean 0, deviation sqrt(15 / inputs)) it stops most scans several
 // times each, and every stop costs steps and another pass over the row.  There (TIGHT) the smallest weight sum of the chunk is
 // tracked, one three-way minimum per two inputs, and the lane accepts if
 //     fma(x_7 - x_0, min(0, wsum_0 .. wsum_7), t_7)  >  thr + the last term above.
-// A workgroup decides by the size of its slice's weights: W * sqrt(inputs) against theta is about 4.5 times the spread of a
-// whole row's weight sum in units of the threshold.  us, bounded / tracked, at W*sqrt(I)/theta of about 5, 7, 9, 13 and 18:
-//   784 -> 800, 4096 rows            334 / 346   336 / 348   351 / 340   381 / 352   507 / 356
-//   784 -> 800, 256 rows              40 / 41     46 / 42     53 / 45     60 / 48     86 / 50
-//   65 536 patches of 576, 64        230 / 252   238 / 252   260 / 254   305 / 261   448 / 288
-//   401 408 patches of 147, 64       605 / 611   643 / 571   762 / 549  1278 / 555  1674 / 585
-//   131 072 patches of 288, 32       160 / 170   175 / 167   200 / 164   281 / 171   345 / 173
-//   1568 patches of 4608, 512        652 / 656   656 / 662   656 / 660   680 / 677   692 / 679
-constexpr float TIGHT_FROM = 7.0f;
+// A workgroup decides by the largest weight of its slice, next to the threshold that ysum - x*wsum starts from; where
+// a wavefront has a single item nothing hides the extra passes, and the line lies lower.  us, bounded / tracked (W / theta),
+// weights of mean 4 / I and standard deviation s / sqrt(I):
+//                                          s = 1             s = 1.5           s = 2             s = 3             s = 3.87
+//   784 -> 800, 4096 rows            334 / 346 (0.19)  336 / 348 (0.28)  351 / 340 (0.36)  430 / 352 (0.55)  507 / 356 (0.70)
+//   65 536 patches of 576, 64        230 / 252 (0.19)  238 / 252 (0.28)  260 / 254 (0.38)  342 / 262 (0.56)  448 / 288 (0.72)
+//   401 408 patches of 147, 64       605 / 611 (0.35)  643 / 571 (0.51)  762 / 549 (0.68) 1278 / 555 (1.00) 1674 / 585 (1.28)
+//   25 088 patches of 1152, 128      424 / 454 (0.13)  423 / 455 (0.20)  447 / 457 (0.26)  487 / 459 (0.39)  563 / 466 (0.51)
+//   1568 patches of 4608, 512        652 / 656 (0.08)  656 / 662 (0.12)  656 / 660 (0.16)  672 / 667 (0.24)  692 / 679 (0.30)
+//   784 -> 800, 256 rows              40 / 41  (0.19)   46 / 42  (0.28)   53 / 45  (0.36)   65 / 48  (0.55)   86 / 50  (0.70)
+//   784 patches of 1152, 128          37 / 38  (0.13)   42 / 38  (0.20)   51 / 41  (0.26)   56 / 47  (0.39)   61 / 52  (0.51)
+constexpr float TIGHT_FROM = 0.36f, TIGHT_FROM_SINGLE = 0.2f;
 constexpr float FILTER_END_Y = 0x1p-19f;                  // 32u >= 4u + 17.2u, times |ysum_7|
 constexpr float FILTER_END_XW = 0x1p-19f;                 // 32u >= 17.2u, times x_7 * |wsum_7|
 constexpr float FILTER_END_W = 0x1p-15f;                  // 512u >= 36u + 310u, times x_7 * max|w| of the slice
@@ -1018,7 +1021,8 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
     const float w_max = block_max(fill_weight_slice<COLS>(wl, w, rows, J, j0), wl + rows * COLS);
     const float end_w = FILTER_END_W * w_max;               // margin of the fast loop
     const float w4 = 4.0f * 1.00001f * w_max;               // 4W of its bound on the weight sums
-    const bool tight = __builtin_amdgcn_readfirstlane(w_max * sqrtf((float)I) > TIGHT_FROM * np.theta);
+    const bool single = (S + SEGS - 1) / SEGS <= n_groups * waves;      // a wavefront has one item
+    const bool tight = __builtin_amdgcn_readfirstlane(w_max > (single ? TIGHT_FROM_SINGLE : TIGHT_FROM) * np.theta);
 
     constexpr int NONE = 0x7fffffff;
     constexpr int ROW_SHIFT = COLS == 64 ? 8 : COLS == 32 ? 7 : COLS == 16 ? 6 : 5;      // a weight row is COLS * 4 bytes
