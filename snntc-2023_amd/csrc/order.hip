@@ -20,13 +20,13 @@
 // Patches of up to 1152 inputs belong to a wavefront, which needs no barrier for them; longer ones to the workgroup.
 //
 // What bounds it: vector instructions, LDS cycles and stores in about equal parts (65 536 patches of 576 inputs: 53, 46 and
-// 50 us of 93).  An input costs some 110 / (patches over it) + 19 vector and 1 + 5 LDS instructions per 64; the 8 bytes per
-// input it writes are 302 MB there.  Measured against pixels sorted by a network of their own and patches put together from
-// them by merge path (chains of dependent LDS reads), in us: those 65 536 patches 188 -> 93, 100 352 of 576 297 -> 129, 25 088
-// of 1152 227 -> 84, 6272 of 2304 144 -> 56, 1568 of 4608 79 -> 43, 3136 of 576 34 -> 16; 401 408 of 147 (7x7x3, stride 2),
-// sorted patch by patch before, 438 -> 155.
+// 50 us of 83 to 93, by card).  An input costs some 110 / (patches over it) + 19 vector and 1 + 5 LDS instructions per 64; the 8
+// bytes per input it writes are 302 MB there.  Measured against pixels sorted by a network of their own and patches put together
+// from them by merge path (chains of dependent LDS reads), in us: those 65 536 patches 188 -> 83, 100 352 of 576 297 -> 124,
+// 25 088 of 1152 227 -> 86, 6272 of 2304 144 -> 54, 1568 of 4608 79 -> 42; 401 408 of 147 (7x7x3, stride 2), sorted patch by patch
+// before, 438 -> 137.
 //
-// Ties, on 8-bit images (as they are / a third of the rows saturated / smooth / one value), us, next to continuous values and to
+// Ties, on 8-bit images (as they are / a third of the rows saturated / smooth / one value), us between events, next to continuous values and to
 // the order by networks and merges that this replaced (any values): 65 536 patches of 576 inputs 158 / 174 / 182 / 194 (88; 205),
 // 401 408 of 147 177 / 228 / 240 / 319 (138; 430), 131 072 of 75 43 / 52 / 51 / 58 (41; 89), 6272 of 2304 109 / 119 / 133 / 134 (50; 140);
 // above it only at few long and at short strided patches: 1568 of 4608 88 / 115 / 108 / 96 (39; 77), 16 384 of 180 33 / 52 / 38 / 45
