@@ -780,7 +780,7 @@ __device__ __forceinline__ void read_columns(__attribute__((address_space(3))) c
 // reference test and never close; a NaN bound or threshold fails the fast test.
 //
 // CH (1, 2 or 4) adjacent neurons per lane: one row address, one input time and one 4-, 8- or 16-byte LDS read
-// serve CH scans, and a wavefront covers 64*CH/COLS segments.  What bounds the loop is vector issue (127
+// serve CH scans, and a wavefront covers 64*CH/COLS segments.  What bounds the loop is vector issue (120
 // instructions per chunk of 4 x 64 neurons) and, under it, the power limit: the same instruction stream runs
 // 16 % slower on random weights than on zeros.  Per 64 neuron-steps, 16 wavefronts per CU: 21.2 / 15.7 / 12.7
 // clocks with one, two and four neurons per lane (17.8 for the two-neuron form that tracked the smallest
@@ -803,7 +803,7 @@ __device__ __forceinline__ void read_columns(__attribute__((address_space(3))) c
 // bound itself; sums inside the chunk differ from the final ones by at most seven inputs).  Every t_u then
 // exceeds thr, which is the condition above.  With weight sums that stay above 4W the bound is t_7 itself;
 // below, a chunk may fail although none of its inputs closes the set, by (x_7 - x_0)*4W at most.
-// Two additions per input and ten instructions per chunk and neuron.
+// Two additions per input and seven instructions per chunk and neuron.
 //
 // That slack is small next to ysum - x*wsum, which starts at theta*x, where weights are small and the sum soon leaves zero;
 // under weights of a larger spread (the layers' own initialiser: mean 0, deviation sqrt(15 / inputs)) it stops most scans several
@@ -825,19 +825,30 @@ constexpr float TIGHT_FROM = 0.36f, TIGHT_FROM_SINGLE = 0.2f;
 constexpr float FILTER_END_Y = 0x1p-19f;                  // 32u >= 4u + 17.2u, times |ysum_7|
 constexpr float FILTER_END_XW = 0x1p-19f;                 // 32u >= 17.2u, times x_7 * |wsum_7|
 constexpr float FILTER_END_W = 0x1p-15f;                  // 512u >= 36u + 310u, times x_7 * max|w| of the slice
+// The fast test takes the first two terms into its operands: t_7 is evaluated at x_7 * (1 + 64u), and x_7 - x_0 is
+// enlarged by 256u * x_7.  With A = 4W - min(..) >= 0 (tracked form: -min(0, ..)), passing means
+// t' - dx' * A > 512u * x_7 * W, and with T = ysum_7 - x_7 * wsum_7 and dx = x_7 - x_0 <= x_7
+//   wsum_7 >= 0:  T >= (1 - u) t' + 62.9u * x_7 * wsum_7 and dx' * A >= (1 + 128u) dx * A, so
+//                 T - dx * A >= 126u * t' + 62.9u * x_7 * wsum_7 + 510u * x_7 * W;
+//   wsum_7 < 0:   T >= (1 - u) t' - 65.2u * x_7 * |wsum_7|, and A >= |wsum_7|, so dx' * A >= (1 + 64u) dx * A +
+//                 192u * x_7 * |wsum_7| and T - dx * A >= 62u * t' + 125u * x_7 * |wsum_7| + 510u * x_7 * W;
+// both are above 21.2u * |ysum_7| + 17.2u * x_7 * |wsum_7| + 346u * x_7 * W, since |ysum_7| <= T + x_7 * |wsum_7|.  (What is
+// left covers the roundings of t', dx', the bound and the threshold.)  Two vector instructions per neuron and chunk
+// less than with a threshold of the neuron's own: 65 536 segments of 576 to 64 neurons 276 -> 265 us, 784 -> 800 at
+// 4096 rows 368 -> 341, 6272 segments of 2304 to 256 neurons 423 -> 405 (kernel traces on one card).
+constexpr float FILTER_AT = 1.0f + 0x1p-18f;
+constexpr float FILTER_DX = 0x1p-16f;
 
 // The test of a chunk for one scan of every lane: wb, yb are the sums behind it.  Lanes in the mask `open`
 // that pass take them over; open lanes that fail keep the sums from before the chunk, take the chunk's
 // first index as kcur and leave `open`.  The arithmetic does not depend on EXEC or branches (lanes that
 // are not open compute along and discard), so the compiler is free to interleave it with the LDS traffic
 // of the next chunk; the decision works on lane masks in scalar registers.
-// dx = x[7] - x[0], x7s = FILTER_END_XW * x[7], thrx = FILTER_END_W * W * x[7] (+ dx * 4W where the smallest weight sum is
-// bounded), low: the smallest weight sum or zero, or its bound + 4W.
+// x7e = FILTER_AT * x[7], dx = x[7] - x[0] + FILTER_DX * x[7], thr = FILTER_END_W * W * x[7] (+ dx * 4W where the smallest weight
+// sum is bounded), low: the smallest weight sum or zero, or its bound + 4W.
 __device__ __forceinline__ void filter_test(float& wsum, float& ysum, int& kcur, uint64_t& open, int k, float wb, float yb,
-                                            float x7, float thrx, float dx, float x7s, float low) {
-    const float t7 = __fmaf_rn(-x7, wb, yb);
-    const float bound = __fmaf_rn(dx, low, t7);
-    const float thr = __fmaf_rn(FILTER_END_Y, fabsf(yb), __fmaf_rn(x7s, fabsf(wb), thrx));
+                                            float x7e, float thr, float dx, float low) {
+    const float bound = __fmaf_rn(dx, low, __fmaf_rn(-x7e, wb, yb));
     uint64_t stop;
     // (two statements: the first has scalar results only, so the masks stay uniform values for the compiler
     // also where no branch depends on them)
@@ -1214,11 +1225,11 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
                     if constexpr (BY_ROW) request(BLOCKS - 1, k0 + (BLOCKS - 1) * BLOCK_INPUTS);
                 };
                 auto test = [&](int k) {
-                    const float dx = x7 - x0, x7s = x7 * FILTER_END_XW;
-                    const float thrx = TIGHT ? x7 * end_w : __fmaf_rn(dx, w4, x7 * end_w);
+                    const float dx = __fmaf_rn(x7, FILTER_DX, x7 - x0), x7e = x7 * FILTER_AT;
+                    const float thr = TIGHT ? x7 * end_w : __fmaf_rn(dx, w4, x7 * end_w);
 #pragma unroll
                     for (int c = 0; c < CH; ++c)
-                        filter_test(wsum[c], ysum[c], kcur[c], open[c], k, wb[c], yb[c], x7, thrx, dx, x7s,
+                        filter_test(wsum[c], ysum[c], kcur[c], open[c], k, wb[c], yb[c], x7e, thr, dx,
                                     TIGHT ? low[c] : fminf(fminf(wsum[c], wb[c]), w4));
                 };
                 // Whole rounds as long as the longest row has one left, without an exit inside the round: behind an
