@@ -780,13 +780,19 @@ __device__ __forceinline__ void read_columns(__attribute__((address_space(3))) c
 // reference test and never close; a NaN bound or threshold fails the fast test.
 //
 // CH (1, 2 or 4) adjacent neurons per lane: one row address, one input time and one 4-, 8- or 16-byte LDS read
-// serve CH scans, and a wavefront covers 64*CH/COLS segments.  What bounds the loop is vector issue (120
-// instructions per chunk of 4 x 64 neurons) and, under it, the power limit: the same instruction stream runs
-// 16 % slower on random weights than on zeros.  Per 64 neuron-steps, 16 wavefronts per CU: 21.2 / 15.7 / 12.7
-// clocks with one, two and four neurons per lane (17.8 for the two-neuron form that tracked the smallest
-// weight sum of a chunk and passed the input times through LDS).  3x3 patches of 64 channels to 64 neurons,
-// 65 536 segments: 310 -> 238 us; 128 -> 128 channels on 28x28, 32 images: 472 -> 416; 256 -> 256 on 14x14: 555 -> 440;
-// dense 784 -> 800 at 4096 rows: 379 -> 302.
+// serve CH scans, and a wavefront covers 64*CH/COLS segments.  Two loops:
+//   * the full chip (four neurons per lane; two with eight-column slices): what bounds it is vector issue (120
+//     instructions per chunk of 4 x 64 neurons) and, under it, the power limit: the same instruction stream runs
+//     16 % slower on random weights than on zeros.  3x3 patches of 64 channels to 64 neurons, 65 536 segments: 310 -> 238 us;
+//     128 -> 128 channels on 28x28, 32 images: 472 -> 416; 256 -> 256 on 14x14: 555 -> 440; dense 784 -> 800 at 4096 rows: 379 -> 302,
+//     and with the shorter test and evenly dealt items 270;
+//   * few wavefronts (LONE: one neuron per lane, two with slices of sixteen columns and more): a SIMD has a wavefront or
+//     three, and each pays about 4.3 clocks for an instruction whatever it is.  52 instructions per chunk of 64 neurons
+//     instead of 75: broadcasts as operands, the test's operands computed once per block of four chunks in the lanes that hold
+//     it, end-of-row masks folded into them, decisions taken half a chunk later, entries kept in a ring without moves.
+//     98 chunks of a lone wavefront 15.2 -> 10.9 us; whole launches: 784 -> 800 at 16 / 128 / 256 rows 24.2 / 28.0 / 38.2 -> 19.2 / 23.5 /
+//     34.0; 2048 -> 512 at 16 rows 48.4 -> 36.6; 49 patches of 4608 -> 512 122 -> 88; 196 of 2304 -> 256 63 -> 49.  (Sixteen-byte
+//     weight reads transposed between lane groups by permlane swaps: 29 us for the first; a swap costs 8.4 clocks.)
 // ---------------------------------------------------------------------------------------------
 // The fast loop does not evaluate the eight t of a chunk: it bounds them from the last one.  With the
 // sums as computed, D_u = ysum_u - x_u*wsum_u obeys  D_{u-1} = D_u + (x_u - x_{u-1})*wsum_{u-1} - e_u,
@@ -961,6 +967,66 @@ __device__ __forceinline__ void quad_row_addresses(int even, int odd, unsigned b
             : [e] "v"(even), [o] "v"(odd), [base] "v"(base));
 }
 
+// The pieces of the fast loop for few wavefronts.  Every instruction costs such a wavefront about 4.3 clocks, whatever it is and
+// whatever it depends on, except that a lane mask that goes from the vector to the scalar side and back in consecutive
+// instructions costs 16 more.  So broadcasts are operands (DPP) and not moves, and the decision on a chunk is taken in the
+// middle of the next one.  (What lanes read from others -- xe, xo, even, odd and the test's nx, dx, thr -- passes through a
+// volatile statement with two wait states behind the last write, which a DPP read needs.)
+//
+// DPP control "lane N of the row of sixteen" or "lane N of the quad".
+#define SNNTC_BCAST_ROW "row_newbcast:%[n] row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+#define SNNTC_BCAST_ROW1 "row_newbcast:%[n1] row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+#define SNNTC_BCAST_AT "row_newbcast:%[m] row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+#define SNNTC_BCAST_AT1 "row_newbcast:%[m1] row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+#define SNNTC_BCAST_QUAD "quad_perm:[%[n],%[n],%[n],%[n]] row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+#define SNNTC_BCAST_QUAD1 "quad_perm:[%[n1],%[n1],%[n1],%[n1]] row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+#define SNNTC_BCAST_QAT "quad_perm:[%[m],%[m],%[m],%[m]] row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+#define SNNTC_BCAST_QAT1 "quad_perm:[%[m1],%[m1],%[m1],%[m1]] row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+
+// Four inputs of a scan: s[0..3] the weight sums behind them, ys the other sum; the times are those that lanes N and N + 1 hold.
+#define SNNTC_HALF(B, B1)                                                                                              \
+    "v_add_f32_e32 %[s0], %[ws], %[w0]\n" "v_fmac_f32_dpp %[ys], %[xe], %[w0] " B                                      \
+    "v_add_f32_e32 %[s1], %[s0], %[w1]\n" "v_fmac_f32_dpp %[ys], %[xo], %[w1] " B                                      \
+    "v_add_f32_e32 %[s2], %[s1], %[w2]\n" "v_fmac_f32_dpp %[ys], %[xe], %[w2] " B1                                     \
+    "v_add_f32_e32 %[s3], %[s2], %[w3]\n" "v_fmac_f32_dpp %[ys], %[xo], %[w3] " B1
+template <bool BY_ROW, int N>
+__device__ __forceinline__ void accumulate_half(float ws, float (&s)[4], float& ys, float xe, float xo, const float (&w)[4]) {
+#define SNNTC_HALF_OPERANDS                                                                                            \
+    : [s0] "=&v"(s[0]), [s1] "=&v"(s[1]), [s2] "=&v"(s[2]), [s3] "=&v"(s[3]), [ys] "+v"(ys)                            \
+    : [ws] "v"(ws), [xe] "v"(xe), [xo] "v"(xo), [w0] "v"(w[0]), [w1] "v"(w[1]), [w2] "v"(w[2]), [w3] "v"(w[3]),        \
+      [n] "n"(N), [n1] "n"(N + 1)
+    if constexpr (BY_ROW) asm(SNNTC_HALF(SNNTC_BCAST_ROW, SNNTC_BCAST_ROW1) SNNTC_HALF_OPERANDS);
+    else asm(SNNTC_HALF(SNNTC_BCAST_QUAD, SNNTC_BCAST_QUAD1) SNNTC_HALF_OPERANDS);
+}
+// LDS addresses of the four weight rows whose shifted indices lanes M and M + 1 hold.
+#define SNNTC_ADDRESSES(B, B1)                                                                                         \
+    "v_add_u32_dpp %[a0], %[e], %[base] " B "v_add_u32_dpp %[a1], %[o], %[base] " B                                    \
+    "v_add_u32_dpp %[a2], %[e], %[base] " B1 "v_add_u32_dpp %[a3], %[o], %[base] " B1
+template <bool BY_ROW, int M>
+__device__ __forceinline__ void weight_addresses(unsigned (&a)[4], unsigned even, unsigned odd, unsigned base) {
+#define SNNTC_ADDRESS_OPERANDS                                                                                         \
+    : [a0] "=&v"(a[0]), [a1] "=&v"(a[1]), [a2] "=&v"(a[2]), [a3] "=&v"(a[3])                                           \
+    : [e] "v"(even), [o] "v"(odd), [base] "v"(base), [m] "n"(M), [m1] "n"(M + 1)
+    if constexpr (BY_ROW) asm(SNNTC_ADDRESSES(SNNTC_BCAST_AT, SNNTC_BCAST_AT1) SNNTC_ADDRESS_OPERANDS);
+    else asm(SNNTC_ADDRESSES(SNNTC_BCAST_QAT, SNNTC_BCAST_QAT1) SNNTC_ADDRESS_OPERANDS);
+}
+// Whether a chunk passes (see filter_test): ysum - thr - x7e * wsum + dx * low > 0.  (Taking thr off first adds
+// u * (|ysum| + thr) to the roundings, which the margins above leave room for.)  The operands of chunk P are those of lane 4 * P
+// of the row (BY_ROW) or the lane's own.
+template <bool BY_ROW, int P>
+__device__ __forceinline__ uint64_t chunk_passes(float wb, float yb, float nx, float dx, float thr, float low) {
+    float t;
+    uint64_t pass;
+    if constexpr (BY_ROW)
+        asm("v_subrev_f32_dpp %[t], %[thr], %[yb] " SNNTC_BCAST_ROW "v_fmac_f32_dpp %[t], %[nx], %[wb] " SNNTC_BCAST_ROW
+            "v_fmac_f32_dpp %[t], %[dx], %[low] " SNNTC_BCAST_ROW
+            : [t] "=&v"(t) : [thr] "v"(thr), [yb] "v"(yb), [nx] "v"(nx), [wb] "v"(wb), [dx] "v"(dx), [low] "v"(low), [n] "n"(4 * P));
+    else
+        t = __fmaf_rn(dx, low, __fmaf_rn(nx, wb, yb - thr));
+    asm("v_cmp_lt_f32_e64 %[pass], 0, %[t]" : [pass] "=s"(pass) : [t] "v"(t));        // false for NaN
+    return pass;
+}
+
 typedef __attribute__((address_space(3))) const float lds_cfloat;
 
 // f(integral_constant<int, 0>), f(<1>), ... f(<N-1>) until one returns false; true if none did.  The
@@ -1009,7 +1075,7 @@ __device__ __forceinline__ void row_row_addresses(int even, int odd, unsigned ba
         : [e] "v"(even), [o] "v"(odd), [base] "v"(base), [n0] "n"(N), [n1] "n"(N + 1));
 }
 
-template <int COLS, int CH, bool WANT_K>
+template <int COLS, int CH, bool LONE, bool WANT_K>
 __global__ void __launch_bounds__(LDS_SCAN_THREADS)
 scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__ perm,
                    const int32_t* __restrict__ n_real, const float* __restrict__ w, float* __restrict__ y_out,
@@ -1047,8 +1113,13 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
     const int j = j0 + CH * cg;                            // first of the lane's columns
     const float* __restrict__ wcol = wl + CH * cg;
     const unsigned wbase = (unsigned)(uintptr_t)(lds_cfloat*)wcol;          // LDS byte address of the lane's columns
-    // `waves` wavefronts of the workgroup work on items; the others have only helped to copy the slice
-    for (int item = group * waves + wave; wave < waves && item * SEGS < S; item += n_groups * waves) {
+    // `waves` wavefronts of the workgroup work on items; the others have only helped to copy the slice.  A group takes
+    // neighbouring items where they fill its SIMDs evenly.  Otherwise (several turns, or one that fills 13 of 16 wavefronts or
+    // fewer) they are dealt out one by one, so that no group has a wavefront more per SIMD than it must (1536 rows of 784 -> 800
+    // 154 -> 122 us, 200 704 patches of 147 to 64 neurons 243 -> 232, 392 of 4608 to 512 200 -> 166).
+    const int n_items = (S + SEGS - 1) / SEGS;
+    const bool deal = n_items > n_groups * waves || (waves == 16 && n_items <= n_groups * 13);
+    for (int item = deal ? wave * n_groups + group : group * waves + wave; wave < waves && item * SEGS < S; item += n_groups * waves) {
         const int seg_raw = item * SEGS + sub;
         const int seg = seg_raw < S ? seg_raw : S - 1;      // idle lanes shadow a valid segment
         const float* __restrict__ xs = sorted + (size_t)seg * stride;
@@ -1073,16 +1144,19 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
         // held: rows: block b holds the round b rounds ahead of the current one; quads: a ring of chunks.
         // The first entries are requested here, next to the two loads above and before anything waits for
         // them: practically every item starts its first pass at input 0.
-        constexpr int BLOCKS = BY_ROW ? (CH == 4 ? 2 : 3) : ROUND;
+        constexpr int BLOCKS = BY_ROW ? (LONE ? 3 : 2) : LONE ? 2 * ROUND : ROUND;
+        constexpr int PHASES = BY_ROW ? ROUND * BLOCKS : BLOCKS;     // chunks held (the loop for one and two neurons per lane)
         constexpr int BLOCK_INPUTS = BY_ROW ? ROUND * CHUNK : CHUNK;
         u32x2 rx[BLOCKS], rp[BLOCKS];
         auto request = [&](int b, int k) {
             rx[b] = __builtin_amdgcn_raw_buffer_load_b64(rows_of_item.xs, lane_bytes, k * (int)sizeof(float), 0);
             rp[b] = __builtin_amdgcn_raw_buffer_load_b64(rows_of_item.pr, lane_bytes, k * (int)sizeof(float), 0);
         };
+        // (no further than that: short rows would fetch the rows behind them)
+        const int last_block = stride - CHUNK;
         auto request_first = [&](int k) {
 #pragma unroll
-            for (int b = 0; b < BLOCKS - 1; ++b) request(b, k + b * BLOCK_INPUTS);
+            for (int b = 0; b < BLOCKS - (LONE ? 0 : 1); ++b) request(b, LONE ? min(k + b * BLOCK_INPUTS, last_block) : k + b * BLOCK_INPUTS);
         };
         request_first(0);
         const int n_full = n_seg & ~(CHUNK - 1);
@@ -1140,8 +1214,133 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
                 for (int c = 0; c < CH; ++c) {
                     open[c] = ran[c];
                     armed[c] &= ~ran[c];
-                    kcur[c] = in_mask(ran[c]) ? n_full : kcur[c];          // unless the scan stops earlier
+                    if (!LONE) kcur[c] = in_mask(ran[c]) ? n_full : kcur[c];       // unless the scan stops earlier
                 }
+                if constexpr (LONE) {
+                    // Half h (four inputs) is worked on while the weights of the next three are on their way.
+                    constexpr int NH = 4, HALVES = 2 * PHASES;
+                    float wv[NH][CH][4];                    // [half buffer][scan][input]
+                    float run_w[CH], run_y[CH], end_w_of[CH], end_y_of[CH];
+                    uint64_t pass[CH];
+                    unsigned passed[CH];                    // chunks
+                    u32x2 at[BLOCKS];                       // LDS offsets of the rows of the entries held
+                    float nx, dx, thr;                      // the test's operands
+                    auto shifted = [&](const u32x2& r) { return u32x2{r.x << ROW_SHIFT, r.y << ROW_SHIFT}; };
+                    // They are those of the lane's quad in block b (rows) or in ring slot b (quads), from input k on.  Behind the end of a
+                    // row nothing passes.
+                    const int last_at = n_full - (BY_ROW ? (lane & 12) * (CHUNK / 4) : 0);
+                    auto test_operands = [&](int b, int k) {
+                        const float x0 = quad_broadcast<0>(__uint_as_float(rx[b].x)), x7 = quad_broadcast<3>(__uint_as_float(rx[b].y));
+                        dx = __fmaf_rn(x7, FILTER_DX, x7 - x0);
+                        nx = -x7 * FILTER_AT;
+                        thr = TIGHT ? x7 * end_w : __fmaf_rn(dx, w4, x7 * end_w);
+                        if (SEGS > 1) thr = k < last_at ? thr : INFINITY;
+                    };
+#pragma unroll
+                    for (int c = 0; c < CH; ++c) { run_w[c] = wsum[c]; run_y[c] = ysum[c]; }
+                    // (the first chunk decides on one that moves nothing)
+#pragma unroll
+                    for (int c = 0; c < CH; ++c) { end_w_of[c] = wsum[c]; end_y_of[c] = ysum[c]; pass[c] = ~0ull; passed[c] = ~0u; }
+                    auto weights = [&](auto h_c) {
+                        constexpr int H = decltype(h_c)::value, P = H / 2, HH = H % 2;
+                        constexpr int B = (BY_ROW ? P / ROUND : P) % BLOCKS, M = BY_ROW ? (P % ROUND) * 4 + HH * 2 : HH * 2;
+                        unsigned a[4];
+                        weight_addresses<BY_ROW, M>(a, at[B].x, at[B].y, wbase);
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) {
+                            float wr[CH];
+                            read_columns<CH>(reinterpret_cast<lds_cfloat*>((uintptr_t)a[u]), wr);
+#pragma unroll
+                            for (int c = 0; c < CH; ++c) wv[H % NH][c][u] = wr[c];
+                        }
+                    };
+                    // The chunk tested last: scans that passed take its sums over.
+                    auto decide = [&] {
+#pragma unroll
+                        for (int c = 0; c < CH; ++c) {
+                            open[c] &= pass[c];
+                            asm("v_cndmask_b32_e64 %[ws], %[ws], %[wb], %[open]\n"
+                                "v_cndmask_b32_e64 %[ys], %[ys], %[yb], %[open]\n"
+                                "v_addc_co_u32_e64 %[k], vcc, 0, %[k], %[open]\n"
+                                : [ws] "+v"(wsum[c]), [ys] "+v"(ysum[c]), [k] "+v"(passed[c])
+                                : [open] "s"(open[c]), [wb] "v"(end_w_of[c]), [yb] "v"(end_y_of[c]) : "vcc");
+                        }
+                    };
+                    auto chunk = [&](auto ph_c, int k) {
+                        constexpr int ph = decltype(ph_c)::value, R = BY_ROW ? ph / ROUND : ph;
+                        // The next entry (block of four chunks, chunk) whose weights will be read, and the test's operands
+                        if constexpr (!BY_ROW || ph % ROUND == 0) {
+                            constexpr int B = BY_ROW ? (R + 1) % BLOCKS : (ph + 2) % BLOCKS;
+                            at[B] = shifted(rp[B]);
+                            test_operands(R, k);
+                            asm volatile("s_nop 1" : "+v"(rx[R].x), "+v"(rx[R].y), "+v"(at[B].x), "+v"(at[B].y), "+v"(nx), "+v"(dx), "+v"(thr));
+                        }
+                        float start[CH], low[CH];
+                        auto half = [&](auto half_c) {
+                            constexpr int hh = decltype(half_c)::value, H = 2 * ph + hh, N = BY_ROW ? (ph % ROUND) * 4 + hh * 2 : 2 * hh;
+                            weights(std::integral_constant<int, H + NH - 1>{});
+                            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                            for (int c = 0; c < CH; ++c) {
+                                float sums[4];
+                                if (hh == 0) start[c] = run_w[c];
+                                accumulate_half<BY_ROW, N>(run_w[c], sums, run_y[c], __uint_as_float(rx[R].x), __uint_as_float(rx[R].y), wv[H % NH][c]);
+                                run_w[c] = sums[3];
+                                if (TIGHT)
+                                    low[c] = fminf(fminf(fminf(fminf(hh == 0 ? 0.0f : low[c], sums[0]), sums[1]), sums[2]), sums[3]);
+                            }
+                            __builtin_amdgcn_sched_barrier(0);
+                        };
+                        half(std::integral_constant<int, 0>{});
+                        decide();
+                        half(std::integral_constant<int, 1>{});
+#pragma unroll
+                        for (int c = 0; c < CH; ++c) {
+                            if (!TIGHT) low[c] = fminf(fminf(start[c], run_w[c]), w4);
+                            pass[c] = chunk_passes<BY_ROW, BY_ROW ? ph % ROUND : 0>(run_w[c], run_y[c], nx, dx, thr, low[c]);
+                            end_w_of[c] = run_w[c];
+                            end_y_of[c] = run_y[c];
+                        }
+                        if constexpr (!BY_ROW) request(ph, min(k + BLOCKS * CHUNK, last_block));
+                        else if constexpr (ph % ROUND == ROUND - 1) request(R, min(k - (ROUND - 1) * CHUNK + BLOCKS * BLOCK_INPUTS, last_block));
+                    };
+                    // the first weights
+                    at[0] = shifted(rp[0]);
+                    asm volatile("s_nop 1" : "+v"(at[0].x), "+v"(at[0].y));
+                    if constexpr (!BY_ROW) {
+                        at[1] = shifted(rp[1]);
+                        asm volatile("s_nop 1" : "+v"(at[1].x), "+v"(at[1].y));
+                    }
+                    weights(std::integral_constant<int, 0>{});
+                    weights(std::integral_constant<int, 1>{});
+                    weights(std::integral_constant<int, 2>{});
+                    int k0 = kmin;
+                    bool more = true;
+                    // Whole rounds as long as the longest row has one left, without an exit inside (behind an exit between a request
+                    // and its use the compiler would move the request to the use), then its last chunks one by one.
+                    const bool rotate = waves > 4;          // (more than a wavefront per SIMD)
+                    for (; k0 + PHASES * CHUNK <= n_full_max && more; k0 += PHASES * CHUNK) {
+                        if (rotate) rotate_wave_priority(k0 / (PHASES * CHUNK) + (wave >> 2));
+                        for_each_phase<PHASES>([&](auto ph_c) {
+                            chunk(ph_c, k0 + decltype(ph_c)::value * CHUNK);
+                            return true;
+                        });
+                        uint64_t any = 0;
+#pragma unroll
+                        for (int c = 0; c < CH; ++c) any |= open[c];
+                        more = any != 0;
+                    }
+                    if (more)
+                        for_each_phase<PHASES>([&](auto ph_c) {
+                            const int k = k0 + decltype(ph_c)::value * CHUNK;
+                            if (k >= n_full_max) return false;
+                            chunk(ph_c, k);
+                            return true;
+                        });
+                    decide();
+#pragma unroll
+                    for (int c = 0; c < CH; ++c) kcur[c] = in_mask(ran[c]) ? kmin + (int)passed[c] * CHUNK : kcur[c];
+                } else {
                 // The weights of a chunk are read in two halves of four inputs.  Per half, with h the half
                 // being consumed: read the weights of half h + NH - 1, then run half h; NH = 2 keeps
                 // four-neuron lanes within the registers of a 16-wavefront workgroup, the others read
@@ -1269,6 +1468,7 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
                         test(k);
                         return true;
                     });
+                }
 #pragma unroll
                 for (int c = 0; c < CH; ++c) {
                     fired[c] = (fired[c] & ~ran[c]) | (ballot(wsum[c] > 0.0f) & ran[c]);
@@ -1482,36 +1682,59 @@ constexpr int FILTER_MAX_CH = COLS == 8 ? 2 : 4;
 // How many of them a launch of S segments of I inputs uses: the form with the smallest estimated time.  A SIMD
 // works on its wavefronts four at a time; the time of a chunk with w of them at work and the fixed share of an
 // item (first requests, evaluation of the closing chunks, leftover inputs, output) in chunks are measured
-// (in 10 ns and chunks; 784 -> 800 at 32 ... 4096 rows, 27- to 4608-input patches).  More neurons per lane cost
-// less per neuron where wavefronts abound, fewer where a SIMD gets one or two wavefronts of long rows or the
-// rows are short.  With a single slice of at most 32 columns the rows come from HBM once: quads hold three
-// chunks ahead of the one at work, too few bytes in flight for that.
+// (in 10 ns and chunks; 784 -> 800 at 64 ... 2048 rows, 27- to 4608-input patches of 1 ... 32 images).  More neurons per lane
+// cost less per neuron where wavefronts abound, fewer where a SIMD gets one or two wavefronts of long rows.  us with one / two /
+// four neurons per lane: 784 -> 800 at 128 rows 23.6 / 26.7 / 47.4, 384 rows 64.8 / 43.6 / 54.8, 768 rows 95 / 103 / 70; 49 patches of
+// 4608 to 512 neurons 86 / 116; 200 704 patches of 147 to 64 neurons 350 / 302 / 243.
 template <int COLS>
 int filter_neurons(int64_t S, int64_t I, int n_slices, int cus) {
-    static const int chunk_time[3][4] = {{17, 20, 25, 30}, {23, 29, 36, 43}, {39, 48, 58, 69}};
-    static const int fixed_chunks[3] = {8, 10, 17};
+    static const int wide[3][4] = {{14, 19, 22, 32}, {20, 29, 40, 53}, {38, 50, 62, 77}};
+    static const int narrow[2][4] = {{14, 19, 22, 32}, {25, 33, 46, 58}};                         // eight-column slices
+    static const int fixed_chunks[3] = {4, 5, 8};
+    // A single slice of 8 or 16 columns: rows come from HBM once, and quads hold too few bytes in flight for that (262 144
+    // patches of 144 to 16 neurons 134 / 147 / 174 us).
+    if (n_slices == 1 && COLS <= 16) return 1;
     int best = 1;
     int64_t best_time = INT64_MAX;
     for (int k = 0, ch = 1; ch <= FILTER_MAX_CH<COLS>; ++k, ch *= 2) {
-        if (ch > 1 && n_slices == 1 && COLS <= 32 && COLS / ch < 16) break;
         const int64_t segs = kWave / COLS * ch;
-        const int64_t waves = ((S + segs - 1) / segs * n_slices + cus * 4 - 1) / (cus * 4);       // per SIMD
-        const int64_t t = (waves / 4 * chunk_time[k][3] + (waves % 4 ? chunk_time[k][waves % 4 - 1] : 0)) * (I / CHUNK + fixed_chunks[k]);
+        const int64_t groups = n_slices < cus ? cus / n_slices : 1;                               // workgroups per slice
+        const int64_t per_group = ((S + segs - 1) / segs + groups - 1) / groups;                  // items of the fullest
+        const int* chunk_time = COLS == 8 ? narrow[k % 2] : wide[k];
+        const int64_t t = (per_group < 16 ? 16 * chunk_time[(per_group + 3) / 4 - 1] : per_group * chunk_time[3]) * (I / CHUNK + fixed_chunks[k]);
         if (t < best_time) { best_time = t; best = ch; }
     }
     return best;
 }
+// Eight-column slices of rows shorter than this keep the loop of the full chip with one neuron per lane too: the other one
+// requests eight chunks ahead there, which such rows do not have (401 408 rows of 75 to 8 neurons 90 against 100 us).
+constexpr int FILTER_LONE_FROM = 128;
 constexpr size_t FILTER_WIDE_COPY_BYTES = 48 * 1024;        // slices from here on are copied by 16 wavefronts
+
+// The instantiation for ch neurons per lane.
+template <int COLS, bool WANT_K>
+decltype(&scan_filter_kernel<COLS, 1, true, WANT_K>) filter_kernel(int ch, bool lone) {
+    if (ch == 1) {
+        if constexpr (COLS == 8) {
+            if (!lone) return scan_filter_kernel<COLS, 1, false, WANT_K>;
+        }
+        return scan_filter_kernel<COLS, 1, true, WANT_K>;
+    }
+    if constexpr (COLS == 8) return scan_filter_kernel<COLS, 2, false, WANT_K>;
+    else return ch == 2 ? scan_filter_kernel<COLS, 2, true, WANT_K> : scan_filter_kernel<COLS, 4, false, WANT_K>;
+}
 
 template <int COLS>
 int raise_scan_lds_limits() {
     const void* whole[] = {
-        reinterpret_cast<const void*>(scan_filter_kernel<COLS, 1, true>),
-        reinterpret_cast<const void*>(scan_filter_kernel<COLS, 1, false>),
-        reinterpret_cast<const void*>(scan_filter_kernel<COLS, 2, true>),
-        reinterpret_cast<const void*>(scan_filter_kernel<COLS, 2, false>),
-        reinterpret_cast<const void*>(scan_filter_kernel<COLS, FILTER_MAX_CH<COLS>, true>),
-        reinterpret_cast<const void*>(scan_filter_kernel<COLS, FILTER_MAX_CH<COLS>, false>)};
+        reinterpret_cast<const void*>(filter_kernel<COLS, true>(1, true)),
+        reinterpret_cast<const void*>(filter_kernel<COLS, false>(1, true)),
+        reinterpret_cast<const void*>(filter_kernel<COLS, true>(1, false)),
+        reinterpret_cast<const void*>(filter_kernel<COLS, false>(1, false)),
+        reinterpret_cast<const void*>(filter_kernel<COLS, true>(2, true)),
+        reinterpret_cast<const void*>(filter_kernel<COLS, false>(2, true)),
+        reinterpret_cast<const void*>(filter_kernel<COLS, true>(FILTER_MAX_CH<COLS>, false)),
+        reinterpret_cast<const void*>(filter_kernel<COLS, false>(FILTER_MAX_CH<COLS>, false))};
     for (const void* k : whole)
         SNNTC_HIP_CHECK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_SCAN_BYTES));
     const void* split[] = {reinterpret_cast<const void*>(scan_lds_split_kernel<COLS, true>),
@@ -1607,9 +1830,8 @@ int launch_scan_lds(const float* sorted, const int32_t* perm, const int32_t* n_r
     if (n_groups > max_groups) n_groups = max_groups;
     if (n_groups < 1) n_groups = 1;
     const int threads = lds_bytes > FILTER_WIDE_COPY_BYTES && !shared ? LDS_SCAN_THREADS : waves * kWave;
-    auto kern = ch == 1   ? (causal_k ? scan_filter_kernel<COLS, 1, true> : scan_filter_kernel<COLS, 1, false>)
-                : ch == 2 ? (causal_k ? scan_filter_kernel<COLS, 2, true> : scan_filter_kernel<COLS, 2, false>)
-                          : (causal_k ? scan_filter_kernel<COLS, FILTER_MAX_CH<COLS>, true> : scan_filter_kernel<COLS, FILTER_MAX_CH<COLS>, false>);
+    const bool lone = ch < FILTER_MAX_CH<COLS> && !(COLS == 8 && I < FILTER_LONE_FROM);
+    auto kern = causal_k ? filter_kernel<COLS, true>(ch, lone) : filter_kernel<COLS, false>(ch, lone);
     {
         KernelTimerScope timer_("scan", stream);
         hipLaunchKernelGGL(kern, dim3((unsigned)(n_slices * n_groups)), dim3((unsigned)threads), lds_bytes + FILTER_RED_BYTES, stream,

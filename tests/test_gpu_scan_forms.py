@@ -54,6 +54,38 @@ def test_scan_forms(B, I, J, law):
     _check(x, w, p)
 
 
+# Launches that leave a SIMD a wavefront or two: rounds of twelve chunks (rows of sixteen lanes) and of eight (quads)
+LONE_SIZES = [
+    (700, 7, 64), (700, 95, 64), (700, 96, 64), (700, 97, 64), (700, 201, 63),          # 64-column slices, one neuron per lane
+    (900, 96, 20), (900, 193, 20), (1200, 95, 10), (1200, 192, 16), (1200, 104, 11),    # 32 and 16 columns, rows of a wavefront in pairs and fours
+    (1300, 127, 8), (1300, 128, 8), (1300, 192, 7), (1300, 259, 8), (40, 2689, 16),     # 8 columns: below and from the line on, several slices
+    (6000, 288, 64), (6000, 299, 50), (2100, 700, 96), (512, 1345, 250),                # two neurons: 64, 32 and 16 columns
+    (1536, 200, 130), (3300, 300, 96),                                                  # several turns, the last one partial
+]
+
+
+@pytest.mark.parametrize("law", ["baseline", "initial"])
+@pytest.mark.parametrize("B,I,J", LONE_SIZES)
+def test_scan_forms_of_small_launches(B, I, J, law):
+    from snntc_amd.layers import init_weight
+    x, w, p, _ = dense_case(B + I + J, B, I, J, True, "baseline")
+    if law == "initial":
+        np.random.seed(B + I)
+        w = init_weight(I, J, 1.0)
+    rng = np.random.default_rng(I)
+    x[rng.random(x.shape) < 0.1] = 1e5
+    x[::50] = 2e5
+    x[7::50, I // 2:] = 1e5                                  # and rows that end early
+    _check(x, w, p)
+
+
+@pytest.mark.parametrize("kind,B,I,J", [("randn", 700, 190, 64), ("ties", 900, 200, 25), ("negative", 1200, 175, 16),
+                                        ("bias_fires", 1300, 200, 8), ("late", 700, 330, 64), ("sparse", 6000, 290, 64)])
+def test_small_launches_off_the_common_path(kind, B, I, J):
+    x, w = _adversarial_dense(kind, 3, B, I, J)
+    _check(x, w, capi.fc_params(1.0))
+
+
 @pytest.mark.parametrize("kind,B,I,J", [("randn", 20000, 90, 64), ("ties", 12000, 100, 61), ("negative", 9000, 75, 64),
                                         ("bias_fires", 9000, 131, 64), ("late", 9000, 330, 32), ("sparse", 4000, 700, 40)])
 @pytest.mark.parametrize("small", [False, True])             # weights as they are, or scaled so that the smallest weight sum is bounded
