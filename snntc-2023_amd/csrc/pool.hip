@@ -33,7 +33,7 @@ FastDiv make_fast_div(int64_t d, int64_t max_n) {
 // blockIdx.x = output row (b, nh); a thread takes VEC consecutive channels of one (nw, c) position of
 // the row (VEC = 4 when C is a multiple of 4 and the tensors are 16-byte aligned): 32-bit index
 // arithmetic only, consecutive lanes on consecutive channels.
-template <int VEC>
+template <int VEC, int BATCH>
 __global__ void __launch_bounds__(256)
 min_pool_forward_kernel(const float* __restrict__ x, float* __restrict__ y, int32_t* __restrict__ arg, int H, int W,
                         int C, int Kh, int Kw, int Sh, int Sw, int pad_top, int pad_left, int Nh, int Nw,
@@ -48,27 +48,35 @@ min_pool_forward_kernel(const float* __restrict__ x, float* __restrict__ y, int3
     float best[VEC];
     int where[VEC];
 #pragma unroll
-    for (int v = 0; v < VEC; ++v) { best[v] = INFINITY; where[v] = 0; }
-    for (int kh = 0; kh < Kh; ++kh) {
-        const int h = h0 + kh;
-        for (int kw = 0; kw < Kw; ++kw) {
-            const int w = w0 + kw;
-            float val[VEC];
+    for (int v = 0; v < VEC; ++v) { best[v] = (H <= 0 || W <= 0) && pad_value < INFINITY ? pad_value : INFINITY; where[v] = 0; }
+    // The window's positions in (kh, kw) order, BATCH requests at a time: a global pool would otherwise wait for memory once per
+    // position (7x7 of one image, 512 channels: 19.3 -> 9.2 us).  Requests outside the image go to its nearest pixel; the last position is
+    // repeated to fill the last batch, which changes nothing since only a smaller value replaces the minimum.
+    const int total = H > 0 && W > 0 ? Kh * Kw : 0;
+    int kh = 0, kw = 0;
+    for (int p0 = 0; p0 < total; p0 += BATCH) {
+        float val[BATCH][VEC];
+        bool in[BATCH];
 #pragma unroll
-            for (int v = 0; v < VEC; ++v) val[v] = pad_value;
-            if (h >= 0 && h < H && w >= 0 && w < W) {
-                const float* p = img + ((size_t)h * W + w) * C;
-                if (VEC == 4) {
-                    const float4 q = *reinterpret_cast<const float4*>(p);
-                    val[0] = q.x; val[1] = q.y; val[2] = q.z; val[3] = q.w;
-                } else {
-                    val[0] = *p;
-                }
+        for (int i = 0; i < BATCH; ++i) {
+            const int h = h0 + kh, w = w0 + kw;
+            in[i] = h >= 0 && h < H && w >= 0 && w < W;
+            const float* p = img + ((size_t)min(max(h, 0), H - 1) * W + min(max(w, 0), W - 1)) * C;
+            if (VEC == 4) {
+                const float4 q = *reinterpret_cast<const float4*>(p);
+                val[i][0] = q.x; val[i][1] = q.y; val[i][2] = q.z; val[i][3] = q.w;
+            } else {
+                val[i][0] = *p;
             }
-#pragma unroll
-            for (int v = 0; v < VEC; ++v)
-                if (val[v] < best[v]) { best[v] = val[v]; where[v] = kh * Kw + kw; }
+            if (p0 + i + 1 < total && ++kw == Kw) { kw = 0; ++kh; }
         }
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i)
+#pragma unroll
+            for (int v = 0; v < VEC; ++v) {
+                const float now = in[i] ? val[i][v] : pad_value;
+                if (now < best[v]) { best[v] = now; where[v] = min(p0 + i, total - 1); }
+            }
     }
     const size_t t = (size_t)row * Nw * C + e;
     if (VEC == 4) {
@@ -229,7 +237,8 @@ int launch_min_pool_forward(const float* x, float* y, int32_t* arg, const PoolGe
     if (grid.y > 65535u) return fail(SNNTC_ERR_TOO_LARGE, "pooling: output row of %lld elements too long", (long long)per_row);
     {
         KernelTimerScope timer_("min_pool", stream);
-        auto kern = vec ? min_pool_forward_kernel<4> : min_pool_forward_kernel<1>;
+        auto kern = g.Kh * g.Kw <= 4 ? (vec ? min_pool_forward_kernel<4, 4> : min_pool_forward_kernel<1, 4>)
+                                     : (vec ? min_pool_forward_kernel<4, 9> : min_pool_forward_kernel<1, 9>);
         hipLaunchKernelGGL(kern, grid, dim3(256), 0, stream, x, y, arg, (int)g.H, (int)g.W, (int)g.C, (int)g.Kh,
                            (int)g.Kw, (int)g.Sh, (int)g.Sw, (int)g.pad_top, (int)g.pad_left, (int)g.Nh, (int)g.Nw,
                            pad_value, make_fast_div(g.C, per_row), copy);

@@ -77,6 +77,26 @@ def test_hip_pooling_matches_the_oracle(B, H, W, C, Kh, Kw, Sh, Sw, same):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("k", [(1, 1), (2, 2), (2, 3), (3, 3), (2, 5), (4, 5), (6, 6)])     # 1 to 36 positions: around batches of four and nine
+@pytest.mark.parametrize("C", [1, 4, 6])
+def test_hip_pooling_windows_around_a_batch(k, C):
+    import snntc_amd as snn
+    rng = np.random.default_rng(k[0] * 10 + k[1])
+    x = np.round(np.exp(rng.random((2, 9, 11, C))) * 4).astype(np.float32) / 4                # ties
+    s = (min(2, k[0]), min(3, k[1]))
+    y, arg, pad = cf.min_pool(x, k[0], k[1], s[0], s[1], True)
+    y2, arg2 = snn.min_pool(torch.from_numpy(x).to("cuda:0"), k, s, pad, y.shape[1:3])
+    assert np.array_equal(arg2.cpu().numpy(), arg) and np.array_equal(y2.cpu().numpy(), y)
+
+
+@pytest.mark.gpu
+def test_hip_pooling_of_an_empty_image_is_padding():
+    import snntc_amd as snn
+    y, arg = snn.min_pool(torch.empty(2, 0, 4, 8, device="cuda:0"), (2, 2), (1, 1), (1, 0), (1, 3))
+    assert torch.all(y == 1e5) and torch.all(arg == 0)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("B,H,W,C", [(32, 7, 7, 512), (3, 5, 9, 7), (2, 1, 1, 4), (1, 14, 14, 256)])
 def test_hip_global_min_pool_matches_the_oracle(B, H, W, C):
     """SNN_globalminpool2d = one VALID window the size of the image (the ImageNet-shaped net's head):
