@@ -154,6 +154,8 @@ FcFwdWs fc_fwd_ws(void* ws, int64_t S, int64_t I) {
 int forward_chain(const SegmentSource& src, const FcFwdWs& ws, const float* w, float* out, float* sorted_z,
                   int32_t* perm, int32_t* causal_k, int64_t S, int64_t I, int64_t J, const NeuronParams& np,
                   const TimeCopy& copy, hipStream_t st) {
+    if (!src.conv && !sorted_z && !perm && !causal_k && scan_sorts_rows(S, I, ws.stride, J, np))
+        return launch_scan(src.base, nullptr, nullptr, w, out, out + S * J, nullptr, S, I, ws.stride, J, np, copy, st);
     int rc = launch_sort(src, S, ws.sorted, ws.perm, ws.n_real, (int)ws.stride, np.max_cmp, ws.long_keys, st);
     if (rc) return rc;
     rc = launch_unpad_rows(ws.sorted, ws.perm, sorted_z, perm, S, I, ws.stride, st);

@@ -25,6 +25,7 @@
 #include <utility>
 
 #include "snntc_common.h"
+#include "sort_network.h"
 
 namespace snntc {
 namespace {
@@ -312,6 +313,19 @@ __device__ __forceinline__ void accumulate_chunk(float& wsum, float& ysum, int& 
                  : SNNTC_SCAN_INPUTS("v", x));
 }
 
+// Eight inputs added to one sum, their factors the values that lanes FIRST ... of the row of sixteen hold.
+template <int FIRST>
+__device__ __forceinline__ void accumulate_row(float& acc, float x, const float (&w)[CHUNK]) {
+#define SNNTC_ROW_STEP(U) "v_fmac_f32_dpp %[acc], %[x], %[w" #U "] row_newbcast:%[n" #U "] row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+    if (FIRST == 0) asm volatile("s_nop 1" : "+v"(x));      // (wait states, should the compiler have moved it)
+    asm(SNNTC_ROW_STEP(0) SNNTC_ROW_STEP(1) SNNTC_ROW_STEP(2) SNNTC_ROW_STEP(3) SNNTC_ROW_STEP(4) SNNTC_ROW_STEP(5)
+            SNNTC_ROW_STEP(6) SNNTC_ROW_STEP(7)
+        : [acc] "+v"(acc)
+        : [x] "v"(x), [w0] "v"(w[0]), [w1] "v"(w[1]), [w2] "v"(w[2]), [w3] "v"(w[3]), [w4] "v"(w[4]), [w5] "v"(w[5]), [w6] "v"(w[6]),
+          [w7] "v"(w[7]), [n0] "n"(FIRST), [n1] "n"(FIRST + 1), [n2] "n"(FIRST + 2), [n3] "n"(FIRST + 3), [n4] "n"(FIRST + 4),
+          [n5] "n"(FIRST + 5), [n6] "n"(FIRST + 6), [n7] "n"(FIRST + 7));
+}
+
 // Copies columns [j0, j0 + COLS) of all `rows` rows of W[rows, J] into LDS as wl[row][COLS] (zeros
 // past column J).  Loads are issued in batches so that a small workgroup does not pay one memory
 // latency per element.
@@ -421,7 +435,7 @@ __device__ __forceinline__ float fill_weight_slice(float* __restrict__ wl, const
 // measured no faster.)
 constexpr int SPLIT_WAVES = 8, SPLIT_TESTERS = SPLIT_WAVES - 1;
 constexpr int SPLIT_THREADS = SPLIT_WAVES * kWave;
-constexpr int SPLIT_STATIC_LDS = 3 * SPLIT_WAVES * kWave * 4 + 16;
+constexpr int SPLIT_STATIC_LDS = 3 * SPLIT_WAVES * kWave * 4 + 16 + 2 * 4 * CHUNK * 4;
 constexpr int SPLIT_SPIN_LIMIT = 1 << 20;                  // default number of polls of the progress counter before a
                                                            // tester gives up (NeuronParams::wait_polls carries the one in force)
 // Tester wavefronts that gave up since the process started: one word per device, written (a vector
@@ -431,6 +445,9 @@ constexpr int SPLIT_PAD = 4;                               // floats between the
                                                            // reads of eight neighbouring lanes fall on distinct banks
 constexpr int SPLIT_ROUND = 4;                             // chunks per round of the producer
 constexpr int split_lanes(int cols) { return cols == 64 ? 64 : 32; }
+// Slices whose items have one or two rows can order them in the workgroup (more rows per item leave a network too few threads).
+constexpr bool split_sorts(int cols) { return cols == 32 || cols == 16; }
+constexpr int SPLIT_SORT_MAX = 1024;                       // inputs
 
 // dynamic LDS of the split kernel: gathered weights [lanes][stride + pad], sorted rows [segs][stride],
 // sums after every chunk [chunks + round][2][lanes].  Reads run up to a round past the end of a row
@@ -439,8 +456,15 @@ __host__ __device__ inline size_t split_lds_bytes(int lanes, int segs, int strid
     return ((size_t)lanes * (stride + SPLIT_PAD) + (size_t)segs * stride +
             (size_t)(stride / CHUNK + SPLIT_ROUND) * 2 * lanes) * sizeof(float);
 }
+// Items of 32 lanes: the upper half of the producer forms the weight sums as multiply-adds with ones, a round of which stands here
+// (and a round ahead, which it requests as it does of the times).
+constexpr int SPLIT_ONES = 2 * SPLIT_ROUND * CHUNK;
 
-template <int COLS, bool WANT_K>
+// NPAD > 0: the workgroup orders the rows of its item itself, with a network of NPAD keys per row, from `sorted` = the input
+// values as they are [S][I]; perm and n_real are not read.  Every slice orders the same rows again, on CUs that would be idle, and a
+// launch (with its ramp, a store and a trip to memory) is gone: one row of 784 to 800 neurons 5.6 + 12.2 -> 15.4 us, 128 items of
+// two rows of 800 6.8 + 12.4 -> 17.6.
+template <int COLS, int NPAD, bool WANT_K>
 __global__ void __launch_bounds__(SPLIT_THREADS)
 scan_lds_split_kernel(const float* __restrict__ sorted, const int32_t* __restrict__ perm,
                       const int32_t* __restrict__ n_real, const float* __restrict__ w, float* __restrict__ y_out,
@@ -450,6 +474,7 @@ scan_lds_split_kernel(const float* __restrict__ sorted, const int32_t* __restric
     __shared__ int k_found[SPLIT_WAVES][kWave];
     __shared__ float w_found[SPLIT_WAVES][kWave], y_found[SPLIT_WAVES][kWave];
     __shared__ int progress;                               // chunks whose sums are in LDS
+    __shared__ __align__(16) float ones[SPLIT_ONES];
     constexpr int LANES = split_lanes(COLS), SEGS = LANES / COLS;
     constexpr int NONE = 0x7fffffff;
     const int block = xcd_contiguous(blockIdx.x, gridDim.x);
@@ -479,7 +504,44 @@ scan_lds_split_kernel(const float* __restrict__ sorted, const int32_t* __restric
         const int seg = seg_raw < S ? seg_raw : S - 1;
         const int row = seg - seg0;                         // idle lanes shadow the item's last segment
         const float* __restrict__ xs = xrows + row * stride;
-        const int n = scans ? n_real[seg] : 0;              // (requested before the rows: one round trip less)
+        int n = 0;
+        if (NPAD == 0 && scans) n = n_real[seg];            // (requested before the rows: one round trip less)
+        // row indices in LDS, where the sums will stand
+        int32_t* __restrict__ own_perm = reinterpret_cast<int32_t*>(sums);
+        if constexpr (NPAD > 0) {
+            constexpr int G = SPLIT_THREADS / SEGS, EPT = NPAD / G;
+            static_assert(EPT >= 1 && EPT * G == NPAD && G >= kWave, "a row is sorted by whole wavefronts");
+            int tseg = threadIdx.x % G;
+            const int own = threadIdx.x / G;
+            asm volatile("" : "+v"(tseg));                  // (or the network's lane masks would be kept across items, in spilled registers)
+            const float* __restrict__ p = sorted + (size_t)min(seg0 + own, S - 1) * I;
+            u64 v[EPT];
+#pragma unroll
+            for (int r = 0; r < EPT; ++r) {
+                const int e = tseg * EPT + r;
+                v[r] = ((u64)(e < I ? float_to_key(p[e]) : 0xffffffffu) << 32) | (uint32_t)e;
+            }
+            bitonic_sort<EPT, G>(v, tseg, reinterpret_cast<u64*>(wg) + own * NPAD);       // (the weights come later)
+            int below = 0;
+#pragma unroll
+            for (int r = 0; r < EPT; ++r) {
+                const int e = tseg * EPT + r;
+                const bool real = e < I;
+                const float f = key_to_float((uint32_t)(v[r] >> 32));
+                below += real && f <= np.max_cmp;
+                if (e < stride) {
+                    xrows[own * stride + e] = real ? f : INFINITY;
+                    own_perm[own * stride + e] = real ? (int32_t)(uint32_t)v[r] : 0;
+                }
+            }
+#pragma unroll
+            for (int d = 1; d < kWave; d <<= 1) below += __shfl_xor(below, d, kWave);
+            if (lane == 0) k_found[wave][0] = below;
+            __syncthreads();
+            constexpr int ROW_WAVES = G / kWave;
+            for (int q = 0; q < ROW_WAVES; ++q) n += k_found[row * ROW_WAVES + q][0];
+            if (!scans) n = 0;
+        }
         {
             // Weights in scan order: a thread keeps its column and takes four consecutive entries of a
             // row at a time (one 16-byte read of row indices, four weights, one 16-byte LDS write);
@@ -491,7 +553,7 @@ scan_lds_split_kernel(const float* __restrict__ sorted, const int32_t* __restric
             const int gc = threadIdx.x % COLS, gk = threadIdx.x / COLS;
             const bool col_live = j0 + gc < J;
             const int groups = n_segs * stride / 4;        // stride is a multiple of 16 entries
-            const int4* __restrict__ gp = reinterpret_cast<const int4*>(perm + (size_t)seg0 * stride);
+            const int4* __restrict__ gp = reinterpret_cast<const int4*>(NPAD > 0 ? own_perm : perm + (size_t)seg0 * stride);
             const __amdgpu_buffer_rsrc_t wbuf = __builtin_amdgcn_make_buffer_rsrc(
                 const_cast<float*>(w), 0, (int)((size_t)(I + np.bias) * J * sizeof(float)), 0x00020000);
             const unsigned pitch = (unsigned)J * 4u, col_bytes = (unsigned)(j0 + gc) * 4u;
@@ -508,8 +570,10 @@ scan_lds_split_kernel(const float* __restrict__ sorted, const int32_t* __restric
             };
             request_rows(gk);
             __builtin_amdgcn_sched_barrier(0);
-            const float4* __restrict__ gx = reinterpret_cast<const float4*>(sorted + (size_t)seg0 * stride);
-            for (int e = threadIdx.x; e < groups; e += SPLIT_THREADS) reinterpret_cast<float4*>(xrows)[e] = gx[e];
+            if constexpr (NPAD == 0) {
+                const float4* __restrict__ gx = reinterpret_cast<const float4*>(sorted + (size_t)seg0 * stride);
+                for (int e = threadIdx.x; e < groups; e += SPLIT_THREADS) reinterpret_cast<float4*>(xrows)[e] = gx[e];
+            }
             for (int g0 = gk;;) {
                 float4 wv[GB];
 #pragma unroll
@@ -529,6 +593,7 @@ scan_lds_split_kernel(const float* __restrict__ sorted, const int32_t* __restric
                 request_rows(g0);
             }
             if (threadIdx.x == 0) progress = 0;
+            if (threadIdx.x < SPLIT_ONES) ones[threadIdx.x] = 1.0f;
         }
         __syncthreads();                                    // rows and weights are in place
 
@@ -547,17 +612,33 @@ scan_lds_split_kernel(const float* __restrict__ sorted, const int32_t* __restric
 
         if (wave == 0) {
             // ---- producer -----------------------------------------------------------------------
-            // chunk c is consumed from buf[c % NBUF]; after it, chunk c + NBUF is read into its place
+            // Chunk c is consumed from buf[c % NBUF]; after it, chunk c + NBUF is read into its place.  With 32 lanes an item
+            // has a lane per sum: the lower half of the wavefront forms ysum = fma(x, w, ysum), the upper wsum = fma(1, w, wsum),
+            // eight instructions a chunk instead of sixteen (98 chunks: 5.8 -> 4.6 us; the testers take 6.1, and are now what is waited
+            // for: dismissing chunks by the margin test, or fifteen testers, made the launch no shorter).
             constexpr int NBUF = SPLIT_ROUND;
+            constexpr bool HALVES = LANES * 2 == kWave;
+            const bool ones_half = HALVES && lane >= LANES;
+            float acc = ones_half ? wsum : ysum;                        // ysum alone where a lane has both sums
+            const float* xp = ones_half ? ones : xs;                    // the times of the round at work
+            const int xp_step = ones_half ? 0 : NBUF * CHUNK;
             float bx[NBUF][CHUNK], bw[NBUF][CHUNK];
-            auto fetch = [&](float (&x)[CHUNK], float (&wv)[CHUNK], int k) {
-                const float4 x0 = *reinterpret_cast<const float4*>(xs + k), x1 = *reinterpret_cast<const float4*>(xs + k + 4);
-                const float4 w0 = *reinterpret_cast<const float4*>(wrow + k), w1 = *reinterpret_cast<const float4*>(wrow + k + 4);
-                x[0] = x0.x; x[1] = x0.y; x[2] = x0.z; x[3] = x0.w; x[4] = x1.x; x[5] = x1.y; x[6] = x1.z; x[7] = x1.w;
-                wv[0] = w0.x; wv[1] = w0.y; wv[2] = w0.z; wv[3] = w0.w; wv[4] = w1.x; wv[5] = w1.y; wv[6] = w1.z; wv[7] = w1.w;
+            auto fetch = [&](float (&v)[CHUNK], const float* q) {
+                const float4 a = *reinterpret_cast<const float4*>(q), b = *reinterpret_cast<const float4*>(q + 4);
+                v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
             };
+            // Times by DPP, where the sixteen lanes of a row scan one segment: a register holds two chunks, a lane an input (an LDS
+            // request costs a lone wavefront some 14 clocks: 4.5 instead of 6 a chunk).
+            constexpr bool BY_ROW = HALVES && COLS >= 16;
+            float rows[NBUF / 2];
+            auto fetch_rows = [&](int h, const float* q) { rows[h] = q[h * 16 + lane % 16]; };
 #pragma unroll
-            for (int b = 0; b < NBUF; ++b) fetch(bx[b], bw[b], b * CHUNK);
+            for (int b = 0; b < NBUF; ++b) {
+                fetch(bw[b], wrow + b * CHUNK);
+                if (!BY_ROW) fetch(bx[b], xp + b * CHUNK);
+                else if (b % 2 == 1) fetch_rows(b / 2, xp);
+                asm volatile("" ::: "memory");              // (in the loop's order: it waits for what either way in has to wait for)
+            }
             // chunks of this item: the longest row decides the counter's final value, the shortest how
             // long no lane needs a mask
             int n_full_max = n_full, n_full_min = scans ? n_full : NONE;
@@ -573,11 +654,17 @@ scan_lds_split_kernel(const float* __restrict__ sorted, const int32_t* __restric
             // not waited for: LDS serves a wavefront's requests in order, so the sums it covers, stored
             // a phase earlier, are in place before it.  Nothing moves across a phase boundary (the
             // compiler would otherwise wait for every outstanding request before each accumulation).
-            auto publish = [&](int k) {
+            // (`also`: the sum behind the chunk before, published along)
+            auto publish = [&](int k, float also, bool pair) {
                 asm volatile("" ::: "memory");
                 float* out = sums + (k / CHUNK) * 2 * LANES;
-                out[la] = wsum;
-                out[LANES + la] = ysum;
+                if (HALVES) {
+                    out[lane ^ LANES] = pair ? also : acc;              // wsum first
+                    if (pair) out[2 * LANES + (lane ^ LANES)] = acc;
+                } else {
+                    out[la] = wsum;
+                    out[LANES + la] = acc;
+                }
                 asm volatile("" ::: "memory");
                 __hip_atomic_store(&progress, k / CHUNK, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                 asm volatile("" ::: "memory");
@@ -588,26 +675,52 @@ scan_lds_split_kernel(const float* __restrict__ sorted, const int32_t* __restric
                 for (int ph = 0; ph < NBUF; ++ph) {
                     const int k = k0 + ph * CHUNK;
                     __builtin_amdgcn_sched_barrier(0);
+                    if constexpr (BY_ROW) {
+                        if (ph % 2 == 0) {
+                            accumulate_row<0>(acc, rows[ph / 2], bw[ph]);
+                            const float behind_first = acc;
+                            accumulate_row<8>(acc, rows[ph / 2], bw[ph + 1]);
+                            publish(k, behind_first, true);
+                            fetch(bw[ph], wrow + k + NBUF * CHUNK);
+                            fetch(bw[ph + 1], wrow + k + (NBUF + 1) * CHUNK);
+                            fetch_rows(ph / 2, xp + NBUF * CHUNK);
+                        }
+                    } else {
 #pragma unroll
-                    for (int u = 0; u < CHUNK; ++u) {
-                        wsum += bw[ph][u];
-                        ysum = __fmaf_rn(bx[ph][u], bw[ph][u], ysum);
+                        for (int u = 0; u < CHUNK; ++u) {
+                            if (!HALVES) wsum += bw[ph][u];
+                            acc = __fmaf_rn(bx[ph][u], bw[ph][u], acc);
+                        }
+                        publish(k, 0.0f, false);
+                        fetch(bx[ph], xp + (NBUF + ph) * CHUNK);
+                        fetch(bw[ph], wrow + k + NBUF * CHUNK);
                     }
-                    publish(k);
-                    fetch(bx[ph], bw[ph], k + NBUF * CHUNK);
                 }
+                xp += xp_step;
             }
+            if (BY_ROW && k0 < n_full_max)
+#pragma unroll
+                for (int b = 0; b < NBUF; ++b) fetch(bx[b], xp + b * CHUNK);
             for (; k0 < n_full_max; k0 += NBUF * CHUNK) {
 #pragma unroll
                 for (int ph = 0; ph < NBUF; ++ph) {
                     const int k = k0 + ph * CHUNK;
                     const uint64_t run = __ballot(k < n_full);
                     int unused = 0;
+                    float unused_sum = 0.0f;
                     __builtin_amdgcn_sched_barrier(0);
-                    accumulate_chunk(wsum, ysum, unused, run, bx[ph], bw[ph]);
-                    publish(k);
-                    fetch(bx[ph], bw[ph], k + NBUF * CHUNK);
+                    accumulate_chunk(HALVES ? unused_sum : wsum, acc, unused, run, bx[ph], bw[ph]);
+                    publish(k, 0.0f, false);
+                    fetch(bx[ph], xp + (NBUF + ph) * CHUNK);
+                    fetch(bw[ph], wrow + k + NBUF * CHUNK);
                 }
+                xp += xp_step;
+            }
+            if (HALVES) {
+                wsum = __shfl(acc, lane | LANES, kWave);
+                ysum = __shfl(acc, la, kWave);
+            } else {
+                ysum = acc;
             }
             // the last chunk's sums: wait for them, then let the counter reach its final value
             __hip_atomic_store(&progress, (n_full_max + CHUNK - 1) / CHUNK, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -1685,12 +1798,13 @@ constexpr int FILTER_MAX_CH = COLS == 8 ? 2 : 4;
 // (in 10 ns and chunks; 784 -> 800 at 64 ... 2048 rows, 27- to 4608-input patches of 1 ... 32 images).  More neurons per lane
 // cost less per neuron where wavefronts abound, fewer where a SIMD gets one or two wavefronts of long rows.  us with one / two /
 // four neurons per lane: 784 -> 800 at 128 rows 23.6 / 26.7 / 47.4, 384 rows 64.8 / 43.6 / 54.8, 768 rows 95 / 103 / 70; 49 patches of
-// 4608 to 512 neurons 86 / 116; 200 704 patches of 147 to 64 neurons 350 / 302 / 243.
+// 4608 to 512 neurons 86 / 116; 200 704 patches of 147 to 64 neurons 350 / 302 / 243;
+// 25 000 rows of 5 to 379 neurons 67 / 55 / 53.
 template <int COLS>
 int filter_neurons(int64_t S, int64_t I, int n_slices, int cus) {
-    static const int wide[3][4] = {{14, 19, 22, 32}, {20, 29, 40, 53}, {38, 50, 62, 77}};
+    static const int wide[3][4] = {{14, 19, 22, 32}, {20, 29, 40, 53}, {38, 52, 62, 77}};
     static const int narrow[2][4] = {{14, 19, 22, 32}, {25, 33, 46, 58}};                         // eight-column slices
-    static const int fixed_chunks[3] = {4, 5, 8};
+    static const int fixed_chunks[3] = {6, 7, 9};
     // A single slice of 8 or 16 columns: rows come from HBM once, and quads hold too few bytes in flight for that (262 144
     // patches of 144 to 16 neurons 134 / 147 / 174 us).
     if (n_slices == 1 && COLS <= 16) return 1;
@@ -1737,8 +1851,11 @@ int raise_scan_lds_limits() {
         reinterpret_cast<const void*>(filter_kernel<COLS, false>(FILTER_MAX_CH<COLS>, false))};
     for (const void* k : whole)
         SNNTC_HIP_CHECK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_SCAN_BYTES));
-    const void* split[] = {reinterpret_cast<const void*>(scan_lds_split_kernel<COLS, true>),
-                           reinterpret_cast<const void*>(scan_lds_split_kernel<COLS, false>)};
+    constexpr bool SORTS = split_sorts(COLS);
+    const void* split[] = {reinterpret_cast<const void*>(scan_lds_split_kernel<COLS, 0, true>),
+                           reinterpret_cast<const void*>(scan_lds_split_kernel<COLS, 0, false>),
+                           reinterpret_cast<const void*>(scan_lds_split_kernel<COLS, SORTS ? 512 : 0, false>),
+                           reinterpret_cast<const void*>(scan_lds_split_kernel<COLS, SORTS ? 1024 : 0, false>)};
     for (const void* k : split)
         SNNTC_HIP_CHECK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
                                             LDS_SCAN_BYTES - SPLIT_STATIC_LDS));
@@ -1782,28 +1899,50 @@ int read_scan_giveups(int64_t* count, hipStream_t stream) {
     return SNNTC_OK;
 }
 
+constexpr int split_segs(int cols) { return split_lanes(cols) / cols; }
+// Whether a launch with slices of `cols` columns goes to scan_lds_split_kernel.
+static bool takes_split(int cols, int64_t S, int64_t I, int64_t stride, int64_t J, const NeuronParams& np, int cus) {
+    const int64_t items = (S + split_segs(cols) - 1) / split_segs(cols) * ((J + cols - 1) / cols);
+    return items <= (int64_t)cus && I >= 2 * CHUNK * SPLIT_WAVES &&
+           split_lds_bytes(split_lanes(cols), split_segs(cols), (int)stride) + SPLIT_STATIC_LDS <= (size_t)LDS_SCAN_BYTES &&
+           // the gather addresses W by 24-bit multiplies and a 32-bit byte offset
+           I + np.bias < (1 << 24) && J < (1 << 22) && (I + np.bias) * J * 4 < 0x7fffffffLL;
+}
+
+// Widest column slice (8..64) whose I + bias rows fit in LDS; 0: none does.  (The split kernel's items are 32 lanes: where such
+// slices are few enough for it they are taken: 512 -> 1000 of one row 4.2 + 13 -> 11.8 us with the order.)
+static int slice_columns(int64_t S, int64_t I, int64_t stride, int64_t J, const NeuronParams& np, int cus) {
+    const size_t rows = (size_t)I + np.bias;
+    int cols = 64;
+    while (cols > 8 && (rows * cols * sizeof(float) > (size_t)LDS_SCAN_TARGET || cols / 2 >= J)) cols >>= 1;
+    if (rows * cols * sizeof(float) > (size_t)LDS_SCAN_TARGET) return 0;
+    return cols == 64 && takes_split(32, S, I, stride, J, np, cus) ? 32 : cols;
+}
+
+bool scan_sorts_rows(int64_t S, int64_t I, int64_t stride, int64_t J, const NeuronParams& np) {
+    if (S <= 0 || J <= 0 || I > SPLIT_SORT_MAX) return false;
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess || scan_prepare_device(dev, &cus) != SNNTC_OK) return false;
+    const int cols = slice_columns(S, I, stride, J, np, cus);
+    return cols != 0 && split_sorts(cols) && takes_split(cols, S, I, stride, J, np, cus);
+}
+
 template <int COLS>
 int launch_scan_lds(const float* sorted, const int32_t* perm, const int32_t* n_real, const float* w, float* y,
                     float* rcp, int32_t* causal_k, int64_t S, int64_t I, int64_t stride, int64_t J,
-                    const NeuronParams& np_in, const TimeCopy& copy, size_t lds_bytes, hipStream_t stream) {
+                    const NeuronParams& np_in, const TimeCopy& copy, size_t lds_bytes, int cus, hipStream_t stream) {
     NeuronParams np = np_in;
     np.wait_polls = g_wait_polls.load(std::memory_order_relaxed);
-    int dev = 0, cus = 0;
-    SNNTC_HIP_CHECK(hipGetDevice(&dev));
-    const int prep = scan_prepare_device(dev, &cus);
-    if (prep) return prep;
     const int n_slices = (int)((J + COLS - 1) / COLS);
     // Fewer items than CUs: a whole workgroup per item, its wavefronts sharing the item's tests.
-    constexpr int SPLIT_SEGS = split_lanes(COLS) / COLS;
-    const int64_t split_items = (S + SPLIT_SEGS - 1) / SPLIT_SEGS;
-    const size_t split_lds = split_lds_bytes(split_lanes(COLS), SPLIT_SEGS, (int)stride);
-    const bool split = split_items * n_slices <= (int64_t)cus && I >= 2 * CHUNK * SPLIT_WAVES &&
-                       split_lds + SPLIT_STATIC_LDS <= (size_t)LDS_SCAN_BYTES &&
-                       // the gather addresses W by 24-bit multiplies and a 32-bit byte offset
-                       I + np.bias < (1 << 24) && J < (1 << 22) && (I + np.bias) * J * 4 < 0x7fffffffLL;
+    const int64_t split_items = (S + split_segs(COLS) - 1) / split_segs(COLS);
+    const size_t split_lds = split_lds_bytes(split_lanes(COLS), split_segs(COLS), (int)stride);
+    const bool split = takes_split(COLS, S, I, stride, J, np, cus);
     if (split) {
         const int64_t n_groups = split_items < cus / n_slices ? split_items : cus / n_slices;
-        auto kern = causal_k ? scan_lds_split_kernel<COLS, true> : scan_lds_split_kernel<COLS, false>;
+        constexpr bool SORTS = split_sorts(COLS);
+        auto kern = causal_k ? scan_lds_split_kernel<COLS, 0, true> : scan_lds_split_kernel<COLS, 0, false>;
+        if (!perm) kern = I <= 512 ? scan_lds_split_kernel<COLS, SORTS ? 512 : 0, false> : scan_lds_split_kernel<COLS, SORTS ? 1024 : 0, false>;
         {
             KernelTimerScope timer_("scan", stream);
             hipLaunchKernelGGL(kern, dim3((unsigned)(n_slices * n_groups)), dim3(SPLIT_THREADS), split_lds, stream, sorted, perm,
@@ -1846,17 +1985,18 @@ int launch_scan(const float* sorted, const int32_t* perm, const int32_t* n_real,
                 float* rcp, int32_t* causal_k, int64_t S, int64_t I, int64_t stride, int64_t J,
                 const NeuronParams& np, const TimeCopy& copy, hipStream_t stream) {
     if (S <= 0 || J <= 0) return SNNTC_OK;
-    // widest column slice (8..64) whose I+bias rows fit in LDS; none fits -> stream W from memory
-    const size_t rows = (size_t)I + np.bias;
-    int cols = 64;
-    while (cols > 8 && (rows * cols * sizeof(float) > (size_t)LDS_SCAN_TARGET || cols / 2 >= J)) cols >>= 1;
-    const size_t lds_bytes = rows * cols * sizeof(float);
-    if (lds_bytes <= (size_t)LDS_SCAN_TARGET) {
+    int dev = 0, cus = 0;
+    SNNTC_HIP_CHECK(hipGetDevice(&dev));
+    const int prep = scan_prepare_device(dev, &cus);
+    if (prep) return prep;
+    const int cols = slice_columns(S, I, stride, J, np, cus);            // none: W is streamed from memory
+    const size_t lds_bytes = ((size_t)I + np.bias) * cols * sizeof(float);
+    if (cols) {
         switch (cols) {
-            case 64: return launch_scan_lds<64>(sorted, perm, n_real, w, y, rcp, causal_k, S, I, stride, J, np, copy, lds_bytes, stream);
-            case 32: return launch_scan_lds<32>(sorted, perm, n_real, w, y, rcp, causal_k, S, I, stride, J, np, copy, lds_bytes, stream);
-            case 16: return launch_scan_lds<16>(sorted, perm, n_real, w, y, rcp, causal_k, S, I, stride, J, np, copy, lds_bytes, stream);
-            default: return launch_scan_lds<8>(sorted, perm, n_real, w, y, rcp, causal_k, S, I, stride, J, np, copy, lds_bytes, stream);
+            case 64: return launch_scan_lds<64>(sorted, perm, n_real, w, y, rcp, causal_k, S, I, stride, J, np, copy, lds_bytes, cus, stream);
+            case 32: return launch_scan_lds<32>(sorted, perm, n_real, w, y, rcp, causal_k, S, I, stride, J, np, copy, lds_bytes, cus, stream);
+            case 16: return launch_scan_lds<16>(sorted, perm, n_real, w, y, rcp, causal_k, S, I, stride, J, np, copy, lds_bytes, cus, stream);
+            default: return launch_scan_lds<8>(sorted, perm, n_real, w, y, rcp, causal_k, S, I, stride, J, np, copy, lds_bytes, cus, stream);
         }
     }
     const int j_blocks = (int)((J + kWave - 1) / kWave);

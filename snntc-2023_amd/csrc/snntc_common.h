@@ -159,6 +159,10 @@ int launch_unpad_rows(const float* sorted, const int32_t* perm, float* sorted_ou
 
 // Causal-set scan over sorted segments (rows of length `stride`, n_real inputs each):
 // y[S,J], rcp[S,J], optional causal_k[S,J].
+// Whether the scan of such a launch orders dense rows itself; launch_scan then takes the input values [S, I] as `sorted`, with
+// perm and n_real (and causal_k) NULL.
+bool scan_sorts_rows(int64_t S, int64_t I, int64_t stride, int64_t J, const NeuronParams& np);
+
 int launch_scan(const float* sorted, const int32_t* perm, const int32_t* n_real, const float* w, float* y,
                 float* rcp, int32_t* causal_k, int64_t S, int64_t I, int64_t stride, int64_t J,
                 const NeuronParams& np, const TimeCopy& copy, hipStream_t stream);

@@ -79,6 +79,26 @@ def test_scan_forms_of_small_launches(B, I, J, law):
     _check(x, w, p)
 
 
+# Launches whose workgroups order their own rows: one and two rows per item, networks of 512 and 1024, several slices
+SORTING_SIZES = [(1, 784, 800), (1, 128, 30), (1, 129, 33), (3, 300, 20), (5, 511, 16), (6, 512, 40), (7, 513, 10), (5, 1023, 16), (2, 1024, 100),
+                 (255, 800, 10), (1, 512, 1000), (100, 200, 64)]
+
+
+@pytest.mark.parametrize("ties", [False, True])
+@pytest.mark.parametrize("B,I,J", SORTING_SIZES)
+def test_scans_that_order_their_rows(B, I, J, ties):
+    x, w, p, _ = dense_case(B + I + J, B, I, J, True, "baseline")
+    rng = np.random.default_rng(I + J)
+    if ties:
+        x = (np.round(x * 16) / 16).astype(np.float32)
+        x[:, ::7] = -0.0
+        x[:, 3::7] = 0.0
+    x[rng.random(x.shape) < 0.1] = 1e5
+    x[-1, I // 3:] = 1e5
+    x[B // 2, :] = 2e5
+    _check(x, w, p)
+
+
 @pytest.mark.parametrize("kind,B,I,J", [("randn", 700, 190, 64), ("ties", 900, 200, 25), ("negative", 1200, 175, 16),
                                         ("bias_fires", 1300, 200, 8), ("late", 700, 330, 64), ("sparse", 6000, 290, 64)])
 def test_small_launches_off_the_common_path(kind, B, I, J):
