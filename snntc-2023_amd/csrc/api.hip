@@ -156,7 +156,9 @@ int forward_chain(const SegmentSource& src, const FcFwdWs& ws, const float* w, f
                   const TimeCopy& copy, hipStream_t st) {
     if (!src.conv && !sorted_z && !perm && !causal_k && scan_sorts_rows(S, I, ws.stride, J, np))
         return launch_scan(src.base, nullptr, nullptr, w, out, out + S * J, nullptr, S, I, ws.stride, J, np, copy, st);
-    int rc = launch_sort(src, S, ws.sorted, ws.perm, ws.n_real, (int)ws.stride, np.max_cmp, ws.long_keys, st);
+    int rc = !src.conv && order_rows_supported(S, I)
+                 ? launch_order_rows(src.base, ws.sorted, ws.perm, ws.n_real, S, I, ws.stride, np.max_cmp, st)
+                 : launch_sort(src, S, ws.sorted, ws.perm, ws.n_real, (int)ws.stride, np.max_cmp, ws.long_keys, st);
     if (rc) return rc;
     rc = launch_unpad_rows(ws.sorted, ws.perm, sorted_z, perm, S, I, ws.stride, st);
     if (rc) return rc;

@@ -36,6 +36,7 @@
 #include <atomic>
 
 #include "snntc_common.h"
+#include "sort_network.h"
 
 namespace snntc {
 namespace {
@@ -123,9 +124,11 @@ inline size_t order_lds_bytes(int n_cap, int threads, int stride, int waves, int
     return head + (tables > after ? tables : after);
 }
 
+// ROWS > 0: the region is one dense row of up to ROWS inputs and its only patch: an input's rank is its place.  Where values
+// repeat or crowd, the row is sorted by a network instead.
 // T threads; ITERS inputs per lane (WAVE: a patch belongs to a wavefront) or per thread (a patch belongs to
 // the workgroup) of a patch; VEC = 4: rows of the image are read in aligned groups of four (C a multiple of four).
-template <int T, bool WAVE, int ITERS, int FULL, int VEC, bool PIXELS>
+template <int T, bool WAVE, int ITERS, int FULL, int VEC, bool PIXELS, int ROWS = 0>
 __global__ void __launch_bounds__(T)
 order_patches_kernel(const float* __restrict__ xpad, float* __restrict__ sorted, int32_t* __restrict__ perm,
                      int32_t* __restrict__ n_real, OrderGeom g) {
@@ -157,7 +160,8 @@ order_patches_kernel(const float* __restrict__ xpad, float* __restrict__ sorted,
     uint16_t* dirty_list = slots + (g.n_cap + 1) / 2 * 2 + wave * ((n + 4 * T - 1) / (4 * T)) * 4 * kWave;       // (a list per wavefront)
 
     // input j of a thread's round
-    auto begun = [&](int round) { return VEC == 4 ? (round * T + wave * kWave) * 4 < n : round * 4 * T + wave * kWave < n; };      // wave-uniform
+    bool crowded = false;                                   // ROWS: nothing is left to rank
+    auto begun = [&](int round) { return !(ROWS > 0 && crowded) && (VEC == 4 ? (round * T + wave * kWave) * 4 < n : round * 4 * T + wave * kWave < n); };      // wave-uniform
     auto input = [&](int round, int j) { return VEC == 4 ? (round * T + tid) * 4 + j : (round * 4 + j) * T + tid; };
 
     // ---- the region's inputs ---------------------------------------------------------------------------------------
@@ -296,6 +300,12 @@ order_patches_kernel(const float* __restrict__ xpad, float* __restrict__ sorted,
     uint32_t before = wave_prefix(held_sum);
     if (lane == kWave - 1) bases[0][wave] = before;
     before -= held_sum;
+    if constexpr (ROWS > 0) {                               // a value of an eighth of the inputs would fill its word
+        uint32_t most = 0;
+#pragma unroll
+        for (int q = 0; q < HELD; ++q) most = max(most, held[q]);
+        if (most > (uint32_t)n / 8) overflow = 1;
+    }
     if (has_last && wave == 0) {
         const int m = (n + 4 * T - 1) / (4 * T) * WAVES * (VEC == 1 ? 4 : 1);
         uint32_t carry = 0;
@@ -306,6 +316,7 @@ order_patches_kernel(const float* __restrict__ xpad, float* __restrict__ sorted,
         }
     }
     __syncthreads();
+    if constexpr (ROWS > 0) crowded = __builtin_amdgcn_readfirstlane((int)overflow) != 0;
     uint32_t n_first = 0;                                   // inputs before the ones of the largest time
 #pragma unroll
     for (int v = 0; v < WAVES; ++v) {
@@ -501,6 +512,18 @@ order_patches_kernel(const float* __restrict__ xpad, float* __restrict__ sorted,
             gather(e, k, word);
             count(e, k, word);
         }
+    } else if constexpr (ROWS > 0) {
+        constexpr int EPT = ROWS / T;
+        u64 v[EPT];
+#pragma unroll
+        for (int q = 0; q < EPT; ++q) {
+            const int e = tid * EPT + q;
+            v[q] = (u64)(e < n ? order_key(value[e]) : ~0u) << 32 | (uint32_t)e;
+        }
+        bitonic_sort<EPT, T>(v, tid, reinterpret_cast<u64*>(area));
+#pragma unroll
+        for (int q = 0; q < EPT; ++q)
+            if (const uint32_t e = (uint32_t)v[q]; e < (uint32_t)n) rank[e] = (uint16_t)pack_ranks((uint32_t)(tid * EPT + q));
     } else {
         // a value repeats too often: stable radix sort of the inputs' indexes, eight bits of the distance from the
         // smallest key a pass; the last pass leaves ranks.  A wavefront takes a run of inputs, 64 at a time.
@@ -569,6 +592,42 @@ order_patches_kernel(const float* __restrict__ xpad, float* __restrict__ sorted,
         } while (shift < 32 && spread >> shift);
     }
     __syncthreads();                                        // ranks are in place, the tables are free
+
+    if constexpr (ROWS > 0) {
+        uint32_t* at = area;                                // the input at every place of the row, 0 behind its end
+        for (int e = tid; e < n; e += T) {
+            const uint32_t r = rank[e];
+            at[(r & 0x7ffu) * 4 + (r >> 11)] = (uint32_t)e;
+        }
+        for (int i = n + tid; i < g.stride; i += T) at[i] = 0;
+        // inputs that take part: keys below that of -inf are NaN, which do not (those above key_cmp are out already)
+        uint32_t nans = 0;
+        if (k_min < order_key(0xff800000u)) {
+            for (int e = tid; e < n; e += T) nans += order_key(value[e]) < order_key(0xff800000u);
+            nans = (uint32_t)__builtin_amdgcn_readlane((int)wave_prefix(nans), kWave - 1);
+            if (lane == 0) bases[1][wave] = nans;
+        }
+        __syncthreads();
+        if (tid == 0) {
+            uint32_t m = reals;
+            if (k_min < order_key(0xff800000u))
+                for (int v = 0; v < WAVES; ++v) m -= bases[1][v];
+            n_real[image] = (int)m;
+        }
+        float* __restrict__ zs = sorted + (size_t)image * g.stride;
+        int32_t* __restrict__ ps = perm + (size_t)image * g.stride;
+        for (int i = tid * 4; i < g.stride; i += T * 4) {
+            const uint4 q = *reinterpret_cast<const uint4*>(at + i);
+            uint4 z = make_uint4(value[q.x], value[q.y], value[q.z], value[q.w]);
+            if (i >= n) z.x = 0x7f800000u;
+            if (i + 1 >= n) z.y = 0x7f800000u;
+            if (i + 2 >= n) z.z = 0x7f800000u;
+            if (i + 3 >= n) z.w = 0x7f800000u;
+            *reinterpret_cast<uint4*>(zs + i) = z;
+            *reinterpret_cast<uint4*>(ps + i) = q;
+        }
+        return;
+    }
 
     // ---- patches ---------------------------------------------------------------------------------------------------
     // bits[w]: a patch's inputs as bits at their ranks and, behind it, the byte offset in LDS of the stage entry that the
@@ -846,7 +905,83 @@ OrderPlan order_plan(const ConvGeom& g, const OrderForm& form, bool quads, int c
 
 }  // namespace
 
+namespace {
+// The kernels' LDS limits on a device, once.
+int order_ready(int dev) {
+    static std::atomic<bool> ready[kMaxDevices];
+    if (dev < 0 || dev >= kMaxDevices) return fail(SNNTC_ERR_UNSUPPORTED, "order: device index %d not supported", dev);
+    if (!ready[dev].load(std::memory_order_acquire)) {
+        const int rc = order_prepare_device();
+        if (rc) return rc;
+        ready[dev].store(true, std::memory_order_release);
+    }
+    return SNNTC_OK;
+}
+
+// Dense rows by length.
+struct OrderRowsForm {
+    int inputs, threads;
+    OrderKernel single, quads;
+};
+template <int T, int N>
+constexpr OrderRowsForm order_rows_form() {
+    return OrderRowsForm{N, T, order_patches_kernel<T, true, 1, 0, 1, false, N>, order_patches_kernel<T, true, 1, 0, 4, false, N>};
+}
+const OrderRowsForm kOrderRowsForms[] = {order_rows_form<256, 512>(), order_rows_form<256, 1024>(), order_rows_form<256, 2048>(),
+                                         order_rows_form<512, 4096>(), order_rows_form<1024, 8192>()};
+
+size_t order_rows_lds(int64_t I, const OrderRowsForm& form) {
+    const size_t ranks = order_lds_bytes((int)I, form.threads, (int)padded_stride(I), 1, 0, 0);
+    const size_t network = ((size_t)I * 6 + 15) / 16 * 16 + (size_t)form.inputs * 8;
+    return std::max(ranks, network);
+}
+}  // namespace
+
+// Dense rows: against the sorting networks, us, 2 / 128 / 2048 / 8192 rows:
+//   of 300     4.5 / 4.8 / 12.4 / 35 -> - / - / 10.2 / 27       of 2048    9.5 / 12 / 45 / 129 -> 6.9 / 9.1 / 25 / 67
+//   of 784     5.8 / 6.7 / 29 / 71   -> - / 6.2 / 21 / 35       of 4096    18 / 22 / 91        -> 8.3 / 12 / 42
+//   of 1521    9.6 / 11 / 44 / 122   -> 7.0 / 9.0 / 22 / 61     of 8192    34 / 36 / 204       -> 12 / 13 / 93
+// A network's steps grow with the square of the length's logarithm, the ranking's do not; below some 300 inputs, and for few rows of
+// up to 1024, both wait for a workgroup's latency and the network is as fast.  Rows whose values repeat are found out after the
+// histogram (a value of an eighth of the inputs) or in the bitmap and go to the network all the same: 4096 rows of 784 with 256 levels 41 -> 38 us,
+// mostly background 41 -> 45; of 1521 69 -> 76 and 68 -> 87.  (By radix sort, as regions are: 784 mostly background 81, 4096 454.)
+bool order_rows_supported(int64_t S, int64_t I) {
+    return S > 0 && I <= ORDER_MAX_REGION && (I > 1024 || (I > 512 && S >= 100) || (I > 256 && S >= 1536));
+}
+
+int launch_order_rows(const float* x, float* sorted, int32_t* perm, int32_t* n_real, int64_t S, int64_t I, int64_t stride,
+                      float max_cmp, hipStream_t stream) {
+    int dev = 0;
+    SNNTC_HIP_CHECK(hipGetDevice(&dev));
+    const int rc = order_ready(dev);
+    if (rc) return rc;
+    const OrderRowsForm* form = kOrderRowsForms;
+    while (I > form->inputs) ++form;
+    OrderGeom og{};
+    og.H = 1; og.W = (int)I; og.C = 1; og.Kh = 1; og.Kw = (int)I; og.Sh = 1; og.Sw = 1; og.Nh = 1; og.Nw = 1; og.P = (int)I;
+    og.th = og.tw = og.tiles_y = og.tiles_x = 1;
+    og.n_cap = (int)I;
+    og.words = (int)((I + 31) / 32);
+    og.stride = (int)stride;
+    og.max_cmp = max_cmp;
+    og.per_image_magic = og.tiles_x_magic = order_magic(1);
+    og.kw_len_magic = og.c_magic = og.row_magic[0] = og.row_magic[1] = order_magic((int)I);
+    if (S > 0x7fffffffLL) return fail(SNNTC_ERR_TOO_LARGE, "order: grid too large");
+    const bool quads = I % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
+    {
+        KernelTimerScope timer_("order_rows", stream);
+        hipLaunchKernelGGL(quads ? form->quads : form->single, dim3((unsigned)S), dim3(form->threads), order_rows_lds(I, *form), stream, x,
+                           sorted, perm, n_real, og);
+    }
+    SNNTC_HIP_CHECK(hipGetLastError());
+    return SNNTC_OK;
+}
+
 int order_prepare_device() {
+    for (const OrderRowsForm& f : kOrderRowsForms)
+        for (OrderKernel k : {f.single, f.quads})
+            SNNTC_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                ORDER_LDS_BYTES - 1024));
     for (const OrderForm& f : kOrderForms)
         for (OrderKernel k : {f.quads_pixels, f.quads, f.single})
             SNNTC_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -878,12 +1013,8 @@ int launch_order_patches(const float* xpad, float* sorted, int32_t* perm, int32_
     SNNTC_HIP_CHECK(hipGetDevice(&dev));
     const int prep = scan_prepare_device(dev, &cus);
     if (prep) return prep;
-    static std::atomic<bool> ready[kMaxDevices];
-    if (!ready[dev].load(std::memory_order_acquire)) {
-        const int rc = order_prepare_device();
-        if (rc) return rc;
-        ready[dev].store(true, std::memory_order_release);
-    }
+    const int rc = order_ready(dev);
+    if (rc) return rc;
     const bool quads = g.C % 4 == 0 && reinterpret_cast<uintptr_t>(xpad) % 16 == 0;
     const OrderForm& form = order_form_of(g.P);
     const OrderPlan plan = order_plan(g, form, quads, cus);

@@ -149,6 +149,10 @@ int launch_sort(const SegmentSource& src, int64_t S, float* sorted, int32_t* per
 
 // Conv patches in ascending order (order.hip), every image region ranked once for all patches over it.
 bool order_patches_supported(const ConvGeom& g);
+// The same ranking for dense rows x[S, I], where it is faster than launch_sort.
+bool order_rows_supported(int64_t S, int64_t I);
+int launch_order_rows(const float* x, float* sorted, int32_t* perm, int32_t* n_real, int64_t S, int64_t I, int64_t stride,
+                      float max_cmp, hipStream_t stream);
 int order_tile(const ConvGeom& g, bool aligned, int64_t tile[4]);        // of a launch on 256 CUs; zeros where the layer is not supported
 int launch_order_patches(const float* xpad, float* sorted, int32_t* perm, int32_t* n_real, const ConvGeom& g, int64_t stride,
                          float max_cmp, hipStream_t stream);

@@ -71,3 +71,51 @@ def test_patch_order(B, H, W, C, Kh, Kw, Sh, Sw, kind):
     assert np.array_equal(sz, ref_sorted)
     assert np.array_equal(ck, ref_k)
     assert np.array_equal(out.view(np.uint32), ref_out.view(np.uint32))
+
+
+ROWS = [(1536, 257), (1536, 512), (100, 513), (128, 784), (100, 1023), (101, 1024), (3, 1025), (2, 2048), (5, 2049), (3, 4096), (2, 4097), (2, 8191),
+        (3, 8192)]
+
+
+@pytest.mark.parametrize("kind", ["plain", "silent", "crowded", "signs", "repeats", "bytes", "ink", "one", "odd"])
+@pytest.mark.parametrize("B,I", ROWS)
+def test_dense_row_order(B, I, kind):
+    """Dense rows that are ranked (or, where values repeat, sorted by a network after all), at the edges of their length classes."""
+    import snntc_amd as snn
+    rng = np.random.default_rng(B * 7 + I)
+    if kind in ("ink", "one", "odd"):
+        x = np.full((B, I), np.float32(np.e))
+        if kind == "ink":                                   # mostly background, the rest in 256 levels
+            ink = rng.random((B, I)) < 0.2
+            x[ink] = np.exp(1.0 - rng.integers(1, 256, ink.sum()) / 255.0).astype(np.float32)
+        elif kind == "odd":                                 # infinities, NaN of both signs, zeros of both, the smallest numbers
+            x = np.exp(rng.random((B, I))).astype(np.float32)
+            pick = np.array([np.inf, -np.inf, np.nan, -np.nan, 0.0, -0.0, 1e-45, -1e-45, 3.4e38, 1e5, 1e5 - 0.1], np.float32)
+            some = rng.random((B, I)) < 0.2
+            x[some] = pick[rng.integers(0, len(pick), some.sum())]
+    else:
+        x = _values(kind, rng, (B, 1, 1, I)).reshape(B, I)
+    xt = torch.from_numpy(x).to(DEV)
+    w = torch.from_numpy(rng.standard_normal((I + 1, 3)).astype(np.float32)).to(DEV)
+    _, z, perm, _ = snn.snnfc(xt, w, capi.fc_params(1.0), return_aux=True)
+    bits = np.where(x == 0, np.float32(0), x).view(np.uint32)
+    key = np.where(bits >> 31 == 1, ~bits, bits | np.uint32(0x80000000))
+    want = np.argsort(key, axis=1, kind="stable")
+    assert np.array_equal(perm.cpu().numpy(), want)
+    assert np.array_equal(z.cpu().numpy().view(np.uint32), np.take_along_axis(bits, want, 1))
+
+
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("B,I", [(128, 784), (128, 785), (4, 3000)])
+def test_dense_rows_at_any_alignment(B, I, offset):
+    import snntc_amd as snn
+    from oracle.capi import fc_forward_dev
+    rng = np.random.default_rng(I + offset)
+    x = np.exp(rng.random((B, I))).astype(np.float32)
+    w = (4.0 / I + rng.standard_normal((I + 1, 40)) / np.sqrt(I)).astype(np.float32)
+    room = torch.zeros(B * I + 1, device=DEV)
+    view = room[offset:offset + B * I].view(B, I)
+    view.copy_(torch.from_numpy(x))
+    out = snn.snnfc(view, torch.from_numpy(w).to(DEV), capi.fc_params(1.0))
+    ref = fc_forward_dev(x, w, capi.fc_params(1.0))
+    assert np.array_equal(out.cpu().numpy().view(np.uint32), (ref[0] if isinstance(ref, tuple) else ref).view(np.uint32))
