@@ -108,18 +108,35 @@ constexpr int DX_A = 2, DX_S = 8 * DX_A, DX_I = 32, DX_JC = 16, DX_PITCH = 36;  
 constexpr int dx_threads(int split) { return (split == 1 ? 4 : split) * kWave; }
 constexpr int dx_lds_bytes(int split) { return dx_threads(split) / kWave * 3 * DX_JC * DX_PITCH * 4; }
 
+// Upstream values of a backward pass: the prologue's, or (RAW) formed where they are staged, which saves small batches a launch.
+struct Upstream {
+    const float* up;                                       // upm, or grad
+    const float* rcp;
+    float max_cmp;
+};
+template <bool RAW, class V>
+__device__ __forceinline__ V upstream_value(V up, V rcp, V y, float max_cmp) {
+    if constexpr (!RAW) return up;
+    else if constexpr (sizeof(V) == sizeof(float)) return y <= max_cmp ? up * rcp : 0.0f;
+    else {
+        V u;
+#pragma unroll
+        for (int q = 0; q < (int)(sizeof(V) / sizeof(float)); ++q) u[q] = y[q] <= max_cmp ? up[q] * rcp[q] : 0.0f;
+        return u;
+    }
+}
+
 // PATCHES: the "samples" are the implicit patches of a conv layer (src.conv) and the
 // result is the gradient per patch element, dx[S, P], which cv_col2im_kernel then folds back onto the image.
-template <int SPLIT, bool PATCHES>
-__global__ void __launch_bounds__(dx_threads(SPLIT), 4)
-fc_grad_input_kernel(const SegmentSource src, const float* __restrict__ w, const float* __restrict__ upm,
-                     const float* __restrict__ ym, float* __restrict__ dx, int B, int I, int J, int tiles_i, int n_tiles) {
+template <int SPLIT, bool PATCHES, bool RAW>
+__device__ __forceinline__ void
+fc_grad_input_tile(const SegmentSource& src, const float* __restrict__ w, const Upstream& upstream, const float* __restrict__ ym,
+                   float* __restrict__ dx, int B, int I, int J, int tiles_i, int n_tiles, int block_index, int blocks, float* dx_lds) {
     constexpr int A = DX_A, TS = DX_S, LANES = DX_JC / 4, ROWS = kWave / LANES, S_PASSES = TS / ROWS, I_PASSES = DX_I / ROWS;
     static_assert(S_PASSES * ROWS == TS && I_PASSES * ROWS == DX_I, "whole passes");
-    extern __shared__ __align__(16) float dx_lds[];
     const int lane = threadIdx.x % kWave;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int block = xcd_contiguous(blockIdx.x, gridDim.x);
+    const int block = xcd_contiguous(block_index, blocks);
     const int tile_raw = SPLIT == 1 ? block * 4 + wave : block;
     const int tile = min(tile_raw, n_tiles - 1);
     const int ts = tile / tiles_i, s0 = ts * TS, i0 = (tile - ts * tiles_i) * DX_I;
@@ -154,7 +171,9 @@ fc_grad_input_kernel(const SegmentSource src, const float* __restrict__ w, const
     const int pr = lane / LANES, pj = lane % LANES * 4;     // the lane's piece: row pr (+ ROWS per pass), outputs pj ... + 3
     typedef float f4 __attribute__((ext_vector_type(4)));
     typedef float fa __attribute__((ext_vector_type(A)));
-    f4 yv[S_PASSES], uv[S_PASSES], wv[I_PASSES];
+    f4 yv[S_PASSES], uv[S_PASSES], rv[S_PASSES], wv[I_PASSES];
+    const float* __restrict__ upm = upstream.up;
+    const float* __restrict__ rcp = upstream.rcp;
     typedef float f4_any __attribute__((ext_vector_type(4), aligned(4)));             // (four floats need no more alignment than one)
     auto piece = [&](const float* row, int j, bool whole) {
         f4 v;
@@ -173,6 +192,7 @@ fc_grad_input_kernel(const SegmentSource src, const float* __restrict__ w, const
             const size_t row = (size_t)min(s0 + t * ROWS + pr, B - 1) * J;
             yv[t] = piece(ym + row, j0 + pj, whole);
             uv[t] = piece(upm + row, j0 + pj, whole);
+            if constexpr (RAW) rv[t] = piece(rcp + row, j0 + pj, whole);
         }
 #pragma unroll
         for (int t = 0; t < I_PASSES; ++t) wv[t] = piece(w + (size_t)min(i0 + t * ROWS + pr, I - 1) * J, j0 + pj, whole);
@@ -186,6 +206,8 @@ fc_grad_input_kernel(const SegmentSource src, const float* __restrict__ w, const
     for (int k = 0; k < PARTS; ++k) {
         for (int c = part(k); c < chunks; c += STEP) {
             const int j0 = c * DX_JC;
+#pragma unroll
+            for (int t = 0; t < S_PASSES; ++t) uv[t] = upstream_value<RAW>(uv[t], rv[t], yv[t], upstream.max_cmp);
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const bool in = j0 + pj + q < J;                // outputs past the end take no part
@@ -262,6 +284,15 @@ fc_grad_input_kernel(const SegmentSource src, const float* __restrict__ w, const
             if (s < B && i < I) dx[(size_t)s * I + i] = sum[0];
         }
     }
+}
+
+template <int SPLIT, bool PATCHES>
+__global__ void __launch_bounds__(dx_threads(SPLIT), 4)
+fc_grad_input_kernel(const SegmentSource src, const float* __restrict__ w, const float* __restrict__ upm,
+                     const float* __restrict__ ym, float* __restrict__ dx, int B, int I, int J, int tiles_i, int n_tiles) {
+    extern __shared__ __align__(16) float dx_lds[];
+    fc_grad_input_tile<SPLIT, PATCHES, false>(src, w, Upstream{upm, nullptr, 0.0f}, ym, dx, B, I, J, tiles_i, n_tiles, blockIdx.x,
+                                              gridDim.x, dx_lds);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -374,26 +405,29 @@ grad_weight_kernel(SegmentSource src, const float* __restrict__ upm, const float
 // ---------------------------------------------------------------------------------------------
 constexpr int DWD_T = 64, DWD_BATCH = 4;
 
-template <int WAVES>
-__global__ void __launch_bounds__(WAVES * kWave, 4)
-grad_weight_dense_kernel(const float* __restrict__ x, const float* __restrict__ upm, const float* __restrict__ ym,
-                         float* __restrict__ dst, int S, int I, int J, int rows, int seg_per_slice, float biasvolt,
-                         float neg_s, float post) {
-    // staging: [wave][sample][x 64 | y 64 | up 64]; sums: [wave][row 32][output 64], half a tile at a time
-    constexpr int STAGE = DWD_BATCH * 3 * DWD_T, SUMS = DWD_T / 2 * DWD_T;
-    __shared__ __align__(16) float lds[WAVES * (STAGE > SUMS ? STAGE : SUMS)];
+// staging: [wave][sample][x 64 | y 64 | up 64]; sums: [wave][row 32][output 64], half a tile at a time
+constexpr int DWD_STAGE = DWD_BATCH * 3 * DWD_T, DWD_SUMS = DWD_T / 2 * DWD_T;
+constexpr int dwd_lds_floats(int waves) { return waves * (DWD_STAGE > DWD_SUMS ? DWD_STAGE : DWD_SUMS); }
+
+template <int WAVES, bool RAW>
+__device__ __forceinline__ void
+grad_weight_dense_tile(const float* __restrict__ x, const Upstream& upstream, const float* __restrict__ ym, float* __restrict__ dst,
+                       int S, int I, int J, int rows, int seg_per_slice, float biasvolt, float neg_s, float post, int bx, int by,
+                       int bz, float* lds) {
+    constexpr int STAGE = DWD_STAGE, SUMS = DWD_SUMS;
     typedef float f4 __attribute__((ext_vector_type(4)));
     const int lane = threadIdx.x % kWave;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int j0 = blockIdx.x * DWD_T, i0 = blockIdx.y * DWD_T;
-    const int s_begin = blockIdx.z * seg_per_slice, s_end = min(S, s_begin + seg_per_slice);
+    const int j0 = bx * DWD_T, i0 = by * DWD_T;
+    const int s_begin = bz * seg_per_slice, s_end = min(S, s_begin + seg_per_slice);
     const int rg = lane / 8, cg = lane % 8;
 
     const bool is_input = i0 + lane < I;
     const float* __restrict__ xcol = x + min(i0 + lane, I - 1);
     const int jc = min(j0 + lane, J - 1);
     const float* __restrict__ ycol = ym + jc;
-    const float* __restrict__ ucol = upm + jc;
+    const float* __restrict__ ucol = upstream.up + jc;
+    const float* __restrict__ rcol = RAW ? upstream.rcp + jc : nullptr;
     float* stage = lds + wave * STAGE;
 
     float acc[8][8];
@@ -401,7 +435,7 @@ grad_weight_dense_kernel(const float* __restrict__ x, const float* __restrict__ 
     for (int r = 0; r < 8; ++r)
 #pragma unroll
         for (int c = 0; c < 8; ++c) acc[r][c] = 0.0f;
-    float xv[DWD_BATCH], yv[DWD_BATCH], uv[DWD_BATCH];
+    float xv[DWD_BATCH], yv[DWD_BATCH], uv[DWD_BATCH], rv[DWD_BATCH];
     auto request = [&](int sb) {
 #pragma unroll
         for (int q = 0; q < DWD_BATCH; ++q) {
@@ -409,6 +443,8 @@ grad_weight_dense_kernel(const float* __restrict__ x, const float* __restrict__ 
             xv[q] = xcol[(size_t)s * I];
             yv[q] = ycol[(size_t)s * J];
             uv[q] = ucol[(size_t)s * J];
+            rv[q] = 0.0f;
+            if constexpr (RAW) rv[q] = rcol[(size_t)s * J];
         }
     };
     int sb = s_begin + wave * DWD_BATCH;
@@ -418,7 +454,7 @@ grad_weight_dense_kernel(const float* __restrict__ x, const float* __restrict__ 
         for (int q = 0; q < DWD_BATCH; ++q) {
             stage[q * 3 * DWD_T + lane] = (is_input ? xv[q] : biasvolt) * neg_s;
             stage[q * 3 * DWD_T + DWD_T + lane] = yv[q] * -neg_s;
-            stage[q * 3 * DWD_T + 2 * DWD_T + lane] = sb + q < s_end ? uv[q] : 0.0f;       // samples past the end weigh nothing
+            stage[q * 3 * DWD_T + 2 * DWD_T + lane] = sb + q < s_end ? upstream_value<RAW>(uv[q], rv[q], yv[q], upstream.max_cmp) : 0.0f;       // samples past the end weigh nothing
         }
         if (sb + WAVES * DWD_BATCH < s_end) request(sb + WAVES * DWD_BATCH);
         wave_lds_order();
@@ -442,7 +478,7 @@ grad_weight_dense_kernel(const float* __restrict__ x, const float* __restrict__ 
         }
         wave_lds_order();
     }
-    float* out = dst + (size_t)blockIdx.z * rows * J;
+    float* out = dst + (size_t)bz * rows * J;
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
         __syncthreads();                                    // (the staging, or the first half, has been read)
@@ -461,6 +497,39 @@ grad_weight_dense_kernel(const float* __restrict__ x, const float* __restrict__ 
             for (int v = 1; v < WAVES; ++v) sum += lds[v * SUMS + e];
             if (i < rows && j < J) out[(size_t)i * J + j] = sum * post;
         }
+    }
+}
+
+template <int WAVES>
+__global__ void __launch_bounds__(WAVES * kWave, 4)
+grad_weight_dense_kernel(const float* __restrict__ x, const float* __restrict__ upm, const float* __restrict__ ym,
+                         float* __restrict__ dst, int S, int I, int J, int rows, int seg_per_slice, float biasvolt,
+                         float neg_s, float post) {
+    __shared__ __align__(16) float lds[dwd_lds_floats(WAVES)];
+    grad_weight_dense_tile<WAVES, false>(x, Upstream{upm, nullptr, 0.0f}, ym, dst, S, I, J, rows, seg_per_slice, biasvolt, neg_s, post,
+                                         blockIdx.x, blockIdx.y, blockIdx.z, lds);
+}
+
+// The whole backward pass of a dense layer on a small batch in one launch: the first dx_blocks workgroups take dX tiles, the others
+// dW tiles, and both form the upstream values as they stage them.  Each part alone leaves the chip half empty and waits for its first
+// loads.  us, prologue, dX and dW / together, 784 -> 800: 1 row 18.5 / 14.0, 64 rows 22 / 16, 128 27 / 19.5, 256 41.5 / 38, 400 57 / 58,
+// 512 70 / 56; 128 rows of 2048 -> 512 35 / 30, of 128 -> 128 16.5 / 10.6.
+__global__ void __launch_bounds__(8 * kWave, 4)
+fc_backward_kernel(const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ grad, const float* __restrict__ y,
+                   const float* __restrict__ rcp, float* __restrict__ dx, float* __restrict__ dw, float* __restrict__ zeros, int n_zeros,
+                   int B, int I, int J, int rows, int tiles_i, int dx_blocks, int dw_cols, float max_cmp, float biasvolt, float neg_s,
+                   float post) {
+    constexpr int FLOATS = dwd_lds_floats(8) > dx_lds_bytes(8) / 4 ? dwd_lds_floats(8) : dx_lds_bytes(8) / 4;
+    __shared__ __align__(16) float lds[FLOATS];
+    const Upstream upstream{grad, rcp, max_cmp};
+    if (blockIdx.x == 0 && (int)threadIdx.x < n_zeros) zeros[threadIdx.x] = 0.0f;          // the dParams output
+    if ((int)blockIdx.x < dx_blocks) {
+        SegmentSource src{};
+        src.base = x; src.conv = 0; src.I = I;
+        fc_grad_input_tile<8, false, true>(src, w, upstream, y, dx, B, I, J, tiles_i, dx_blocks, blockIdx.x, dx_blocks, lds);
+    } else {
+        const int tile = (int)blockIdx.x - dx_blocks, by = tile / dw_cols;
+        grad_weight_dense_tile<8, true>(x, upstream, y, dw, B, I, J, rows, B, biasvolt, neg_s, post, tile - by * dw_cols, by, 0, lds);
     }
 }
 
@@ -821,6 +890,29 @@ int launch_reduce_partials(const float* partial, float* dw, int64_t n, int nspli
         KernelTimerScope timer_("reduce_partials", stream);
         hipLaunchKernelGGL(reduce_partials_kernel, dim3(blocks_for(n, RED_ELEMS)), dim3(RED_ELEMS * RED_GROUPS), 0,
                            stream, partial, dw, n, nsplit);
+    }
+    SNNTC_HIP_CHECK(hipGetLastError());
+    return SNNTC_OK;
+}
+
+// dX and dW of a dense layer in one launch (dX == NULL: dW alone), where its workgroups, of which a CU holds two, come in at most
+// two turns: beyond, the parts alone fill the chip, with tiles of their own.  (Eight wavefronts share a dX tile's outputs, sixteen each.)
+bool fc_backward_joint_supported(int64_t B, int64_t I, int64_t J, bool dx) {
+    const int64_t dx_tiles = dx ? (B + DX_S - 1) / DX_S * ((I + DX_I - 1) / DX_I) : 0;
+    const int64_t dw_tiles = ((J + DWD_T - 1) / DWD_T) * ((I + 1 + DWD_T - 1) / DWD_T);
+    return J >= DX_JC * 8 && dx_tiles + dw_tiles <= 1024;
+}
+
+int launch_fc_backward_joint(const float* x, const float* w, const float* grad, const float* y, const float* rcp, float* dx, float* dw,
+                             float* zeros, int n_zeros, int64_t B, int64_t I, int64_t J, const NeuronParams& np, hipStream_t stream) {
+    const int64_t rows = I + np.bias, tiles_i = (I + DX_I - 1) / DX_I, dx_blocks = dx ? (B + DX_S - 1) / DX_S * tiles_i : 0;
+    const int64_t dw_cols = (J + DWD_T - 1) / DWD_T, dw_blocks = dw_cols * ((rows + DWD_T - 1) / DWD_T);
+    const LeadScale ls = lead_scale(np.max_time);
+    {
+        KernelTimerScope timer_("fc_backward", stream);
+        hipLaunchKernelGGL(fc_backward_kernel, dim3((unsigned)(dx_blocks + dw_blocks)), dim3(8 * kWave), 0, stream, x, w, grad, y, rcp, dx,
+                           dw, zeros, zeros ? n_zeros : 0, (int)B, (int)I, (int)J, (int)rows, (int)tiles_i, (int)dx_blocks, (int)dw_cols,
+                           np.max_cmp, np.biasvolt, ls.neg_s, ls.post);
     }
     SNNTC_HIP_CHECK(hipGetLastError());
     return SNNTC_OK;

@@ -42,3 +42,36 @@ def test_dense_gradients(B, I, J):
     adx, adw, _ = capi.fc_backward_dev(np.abs(g), x, np.abs(w), p, out, wide=True)      # sums of absolute terms
     assert np.all(np.abs(dx - rdx) <= 1e-6 * np.abs(adx) + 1e-30)
     assert np.all(np.abs(dw - rdw) <= 1e-6 * np.abs(adw) + 1e-30)
+
+
+@pytest.mark.parametrize("bias", [True, False])
+@pytest.mark.parametrize("B,I,J", [
+    (1, 1, 128), (16, 32, 128), (17, 33, 129), (15, 64, 191), (33, 63, 320),                  # less than a tile, one, a bit more
+    (63, 191, 1000), (208, 2000, 130), (240, 2000, 130),                                    # both sides of the line to separate launches
+])
+def test_dense_gradients_in_one_launch(B, I, J, bias):
+    """dX and dW together, dW alone and dX alone: the same bits, and within the band of the fp64 sums."""
+    import snntc_amd as snn
+    rng = np.random.default_rng(B + I + J)
+    x = np.exp(rng.random((B, I))).astype(np.float32)
+    x[rng.random((B, I)) < 0.1] = 1e5
+    y = np.exp(1.2 * rng.random((B, J))).astype(np.float32)
+    y[rng.random((B, J)) < 0.1] = 1e5
+    rcp = np.where(y < 1e5, rng.standard_normal((B, J)), np.inf).astype(np.float32)          # outputs that take no part weigh nothing
+    w = rng.standard_normal((I + int(bias), J)).astype(np.float32)
+    out = np.concatenate([y, rcp])
+    g = np.zeros((2 * B, J), np.float32)
+    g[:B] = rng.standard_normal((B, J))
+    p = capi.fc_params(1.0 if bias else 0.0)
+    args = (t(g), t(x), t(w), p, t(out))
+    dx, dw, dp = snn.snnfc_grad(*args)
+    assert not torch.any(torch.as_tensor(dp))
+    assert torch.equal(dw, snn.snnfc_grad(*args, want_dx=False)[1])
+    assert torch.equal(dx, snn.snnfc_grad(*args, want_dw=False)[0])
+    dx, dw = dx.cpu().numpy(), dw.cpu().numpy()
+    out[B:][y >= 1e5] = 0.0
+    rdx, rdw, _ = capi.fc_backward_dev(g, x, w, p, out, wide=True)
+    out[B:] = np.abs(out[B:])
+    adx, adw, _ = capi.fc_backward_dev(np.abs(g), x, np.abs(w), p, out, wide=True)
+    assert np.all(np.abs(dx - rdx) <= 1e-6 * np.abs(adx) + 1e-30)
+    assert np.all(np.abs(dw - rdw) <= 1e-6 * np.abs(adw) + 1e-30)
