@@ -251,12 +251,13 @@ def account(torch, snn, layers, extras=None):
     """Per kernel name: algorithmic fp32 flops and HBM bytes of one step, from the causal-set sizes the
     forward actually produces.  Formulas (S segments of length I, J outputs, b = bias flag):
       steps = sum over (s,j) of consumed inputs + b ;   pairs = sum over fired (s,j) of (k + b)
-      sort_segments (dense rows, 1x1 patches), order_patches : bytes 4*(in + 2*S*I)   flops 0 (comparisons are not flops)
+      sort_segments (short rows, 1x1 patches), order_rows (dense rows), order_patches : bytes 4*(in + 2*S*I)   flops 0 (comparisons are not flops)
       scan          : bytes 4*(2*S*I + (I+b)*J + 2*S*J)            flops 4*steps
       dX kernels    : bytes 4*(2*S*J + in + I*J + in)              flops 2*pairs
       grad_weight   : bytes 4*(2*S*J + in + (I+b)*J)               flops 3*pairs
       prep_upstream : bytes 4*(3*S*J + S*J [+ 2*I*J])              flops S*J   (carries the weight copy conv dX reads)
-      fc_backward_narrow (J <= 16, the three above in one launch): bytes 4*(3*S*J + 2*in + 2*(I+b)*J), flops 5*pairs + S*J
+      fc_backward (dense, small batches; the three above in one launch): their operations, bytes 4*(3*S*J + 2*in + 2*(I+b)*J)
+      fc_backward_narrow (J <= 16, likewise): bytes 4*(3*S*J + 2*in + 2*(I+b)*J), flops 5*pairs + S*J
       pad_time : bytes 4*(in + out) ;  min_pool / min_pool_grad : bytes 4*(in + 2*out)
     `in` is the op's input tensor (B*I dense, B*H*W*C padded image for conv)."""
     acc = {}
@@ -281,7 +282,9 @@ def account(torch, snn, layers, extras=None):
                 x_op = inp
                 _, sz, _, ck = snn.snnfc(x_op, W, layer.Params, return_aux=True)
                 max_t, bias = float(layer.Params[0]), int(layer.Params[5] > 1e-8)
-                order = "sort_segments"
+                rows, length = sz.shape
+                ranked = length > 1024 or (length > 512 and rows >= 100) or (length > 256 and rows >= 1536)
+                order = "order_rows" if ranked and length <= 8192 else "sort_segments"
             else:
                 x_op = inp
                 if padded is not True:               # a network layer: the layer pads (SAME) or crops (VALID) first;
@@ -303,6 +306,11 @@ def account(torch, snn, layers, extras=None):
         add("scan", 4.0 * steps, 4.0 * (2.0 * S * I + (I + bias) * J + 2.0 * S * J))
         if dense and J <= 16:
             add("fc_backward_narrow", 5.0 * pairs + S * J, 4.0 * (3.0 * S * J + 2.0 * n_in + 2.0 * (I + bias) * J))
+            continue
+        tiles = -(-S // 16) * -(-I // 32) * bool(want_dx) + -(-J // 64) * -(-(I + 1) // 64)
+        if dense and J >= 128 and tiles <= 1024:             # dX tiles of 16 x 32, dW tiles of 64 x 64
+            add("fc_backward", (5.0 if want_dx else 3.0) * pairs + S * J,
+                4.0 * (3.0 * S * J + 2.0 * n_in + 2.0 * (I + bias) * J))
             continue
         if want_dx:
             add("fc_grad_input" if dense else "cv_grad_input", 2.0 * pairs, 4.0 * (2.0 * S * J + 2.0 * n_in + I * J))
