@@ -283,7 +283,7 @@ def account(torch, snn, layers, extras=None):
                 _, sz, _, ck = snn.snnfc(x_op, W, layer.Params, return_aux=True)
                 max_t, bias = float(layer.Params[0]), int(layer.Params[5] > 1e-8)
                 rows, length = sz.shape
-                ranked = length > 1024 or (length > 512 and rows >= 100) or (length > 256 and rows >= 1536)
+                ranked = length > 1024 or (length > 512 and rows >= 100) or (length > 256 and (2560 if length % 4 else 1536) <= rows <= 8192)
                 order = "order_rows" if ranked and length <= 8192 else "sort_segments"
             else:
                 x_op = inp

@@ -942,11 +942,13 @@ size_t order_rows_lds(int64_t I, const OrderRowsForm& form) {
 //   of 784     5.8 / 6.7 / 29 / 71   -> - / 6.2 / 21 / 35       of 4096    18 / 22 / 91        -> 8.3 / 12 / 42
 //   of 1521    9.6 / 11 / 44 / 122   -> 7.0 / 9.0 / 22 / 61     of 8192    34 / 36 / 204       -> 12 / 13 / 93
 // A network's steps grow with the square of the length's logarithm, the ranking's do not; below some 300 inputs, and for few rows of
-// up to 1024, both wait for a workgroup's latency and the network is as fast.  Rows whose values repeat are found out after the
+// up to 1024, both wait for a workgroup's latency and the network is as fast.  Up to 512 inputs the network is one wavefront's and a
+// full chip of them catches up (16 384 / 65 536 rows of 300 47 / 161 -> 46 / 171), sooner where rows are read an input at a time (of
+// 499 at 2009 / 5000 / 16 384 rows 13.3 / 30 / 49 -> 13.1 / 22 / 58).  Rows whose values repeat are found out after the
 // histogram (a value of an eighth of the inputs) or in the bitmap and go to the network all the same: 4096 rows of 784 with 256 levels 41 -> 38 us,
 // mostly background 41 -> 45; of 1521 69 -> 76 and 68 -> 87.  (By radix sort, as regions are: 784 mostly background 81, 4096 454.)
 bool order_rows_supported(int64_t S, int64_t I) {
-    return S > 0 && I <= ORDER_MAX_REGION && (I > 1024 || (I > 512 && S >= 100) || (I > 256 && S >= 1536));
+    return S > 0 && I <= ORDER_MAX_REGION && (I > 1024 || (I > 512 && S >= 100) || (I > 256 && S >= (I % 4 ? 2560 : 1536) && S <= 8192));
 }
 
 int launch_order_rows(const float* x, float* sorted, int32_t* perm, int32_t* n_real, int64_t S, int64_t I, int64_t stride,

@@ -73,7 +73,7 @@ def test_patch_order(B, H, W, C, Kh, Kw, Sh, Sw, kind):
     assert np.array_equal(out.view(np.uint32), ref_out.view(np.uint32))
 
 
-ROWS = [(1536, 257), (1536, 512), (100, 513), (128, 784), (100, 1023), (101, 1024), (3, 1025), (2, 2048), (5, 2049), (3, 4096), (2, 4097), (2, 8191),
+ROWS = [(1536, 257), (2560, 257), (8192, 260), (8193, 260), (1536, 512), (100, 513), (128, 784), (100, 1023), (101, 1024), (3, 1025), (2, 2048), (5, 2049), (3, 4096), (2, 4097), (2, 8191),
         (3, 8192)]
 
 
