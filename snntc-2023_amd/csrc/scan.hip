@@ -1126,17 +1126,21 @@ __device__ __forceinline__ void weight_addresses(unsigned (&a)[4], unsigned even
 // Whether a chunk passes (see filter_test): ysum - thr - x7e * wsum + dx * low > 0.  (Taking thr off first adds
 // u * (|ysum| + thr) to the roundings, which the margins above leave room for.)  The operands of chunk P are those of lane 4 * P
 // of the row (BY_ROW) or the lane's own.
+// (BY_ROW: one statement, since between two the compiler puts a wait state; its vector is v127, the last that a wavefront of a
+// workgroup of 16 has, because with a vector among its results the mask would count as divergent.  3136 and 6272 patches of 576 to
+// 64 neurons 26.7 -> 26.7 and 41.4 -> 40.0 us, 128 rows of 512 to 1000 19.3 -> 18.6.)
 template <bool BY_ROW, int P>
 __device__ __forceinline__ uint64_t chunk_passes(float wb, float yb, float nx, float dx, float thr, float low) {
-    float t;
     uint64_t pass;
-    if constexpr (BY_ROW)
-        asm("v_subrev_f32_dpp %[t], %[thr], %[yb] " SNNTC_BCAST_ROW "v_fmac_f32_dpp %[t], %[nx], %[wb] " SNNTC_BCAST_ROW
-            "v_fmac_f32_dpp %[t], %[dx], %[low] " SNNTC_BCAST_ROW
-            : [t] "=&v"(t) : [thr] "v"(thr), [yb] "v"(yb), [nx] "v"(nx), [wb] "v"(wb), [dx] "v"(dx), [low] "v"(low), [n] "n"(4 * P));
-    else
-        t = __fmaf_rn(dx, low, __fmaf_rn(nx, wb, yb - thr));
-    asm("v_cmp_lt_f32_e64 %[pass], 0, %[t]" : [pass] "=s"(pass) : [t] "v"(t));        // false for NaN
+    if constexpr (BY_ROW) {
+        asm("v_subrev_f32_dpp v127, %[thr], %[yb] " SNNTC_BCAST_ROW "v_fmac_f32_dpp v127, %[nx], %[wb] " SNNTC_BCAST_ROW
+            "v_fmac_f32_dpp v127, %[dx], %[low] " SNNTC_BCAST_ROW "v_cmp_lt_f32_e64 %[pass], 0, v127\n"              // false for NaN
+            : [pass] "=s"(pass) : [thr] "v"(thr), [yb] "v"(yb), [nx] "v"(nx), [wb] "v"(wb), [dx] "v"(dx), [low] "v"(low), [n] "n"(4 * P)
+            : "v127");
+    } else {
+        const float t = __fmaf_rn(dx, low, __fmaf_rn(nx, wb, yb - thr));
+        asm("v_cmp_lt_f32_e64 %[pass], 0, %[t]" : [pass] "=s"(pass) : [t] "v"(t));
+    }
     return pass;
 }
 
@@ -1797,12 +1801,12 @@ constexpr int FILTER_MAX_CH = COLS == 8 ? 2 : 4;
 // item (first requests, evaluation of the closing chunks, leftover inputs, output) in chunks are measured
 // (in 10 ns and chunks; 784 -> 800 at 64 ... 2048 rows, 27- to 4608-input patches of 1 ... 32 images).  More neurons per lane
 // cost less per neuron where wavefronts abound, fewer where a SIMD gets one or two wavefronts of long rows.  us with one / two /
-// four neurons per lane: 784 -> 800 at 128 rows 23.6 / 26.7 / 47.4, 384 rows 64.8 / 43.6 / 54.8, 768 rows 95 / 103 / 70; 49 patches of
-// 4608 to 512 neurons 86 / 116; 200 704 patches of 147 to 64 neurons 350 / 302 / 243;
+// four neurons per lane: 784 -> 800 at 128 rows 24.3 / 28.5 / 47.8, 384 rows 44.3 / 44.0 / 55.4, 768 rows 77 / 69 / 71, 2048 rows
+// 198 / 170 / 147; 49 patches of 4608 to 512 neurons 90 / 152; 200 704 patches of 147 to 64 neurons 349 / 307 / 221;
 // 25 000 rows of 5 to 379 neurons 67 / 55 / 53.
 template <int COLS>
 int filter_neurons(int64_t S, int64_t I, int n_slices, int cus) {
-    static const int wide[3][4] = {{14, 19, 22, 32}, {20, 29, 40, 53}, {38, 52, 62, 77}};
+    static const int wide[3][4] = {{14, 19, 22, 32}, {20, 29, 35, 53}, {38, 52, 62, 77}};
     static const int narrow[2][4] = {{14, 19, 22, 32}, {25, 33, 46, 58}};                         // eight-column slices
     static const int fixed_chunks[3] = {6, 7, 9};
     // A single slice of 8 or 16 columns: rows come from HBM once, and quads hold too few bytes in flight for that (262 144
