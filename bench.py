@@ -247,12 +247,24 @@ def capture_step(torch, wl):
 # ------------------------------------------------------------------------------------------------
 # roofline accounting: algorithmic flops / bytes per kernel, summed over the layers of one step
 # ------------------------------------------------------------------------------------------------
+def launched(torch, call):
+    """Names of the library's kernels that a call launches."""
+    from snntc_amd import _lib
+    _lib.profile_enable(True)
+    call()
+    torch.cuda.synchronize()
+    names = set(_lib.profile_collect())
+    _lib.profile_enable(False)
+    return names
+
+
 def account(torch, snn, layers, extras=None):
     """Per kernel name: algorithmic fp32 flops and HBM bytes of one step, from the causal-set sizes the
-    forward actually produces.  Formulas (S segments of length I, J outputs, b = bias flag):
+    forward actually produces, for the kernels that each layer's forward and backward launch.  Formulas (S segments of
+    length I, J outputs, b = bias flag):
       steps = sum over (s,j) of consumed inputs + b ;   pairs = sum over fired (s,j) of (k + b)
       sort_segments (short rows, 1x1 patches), order_rows (dense rows), order_patches : bytes 4*(in + 2*S*I)   flops 0 (comparisons are not flops)
-      scan          : bytes 4*(2*S*I + (I+b)*J + 2*S*J)            flops 4*steps
+      scan          : bytes 4*(2*S*I + (I+b)*J + 2*S*J)            flops 4*steps   (S*I where it orders the rows itself)
       dX kernels    : bytes 4*(2*S*J + in + I*J + in)              flops 2*pairs
       grad_weight   : bytes 4*(2*S*J + in + (I+b)*J)               flops 3*pairs
       prep_upstream : bytes 4*(3*S*J + S*J [+ 2*I*J])              flops S*J   (carries the weight copy conv dX reads)
@@ -282,9 +294,6 @@ def account(torch, snn, layers, extras=None):
                 x_op = inp
                 _, sz, _, ck = snn.snnfc(x_op, W, layer.Params, return_aux=True)
                 max_t, bias = float(layer.Params[0]), int(layer.Params[5] > 1e-8)
-                rows, length = sz.shape
-                ranked = length > 1024 or (length > 512 and rows >= 100) or (length > 256 and (2560 if length % 4 else 1536) <= rows <= 8192)
-                order = "order_rows" if ranked and length <= 8192 else "sort_segments"
             else:
                 x_op = inp
                 if padded is not True:               # a network layer: the layer pads (SAME) or crops (VALID) first;
@@ -293,7 +302,10 @@ def account(torch, snn, layers, extras=None):
                         add("pad_time", 0.0, 4.0 * (inp.numel() + x_op.numel()))
                 _, sz, _, ck = snn.snncv(x_op, W, layer.Params, return_aux=True)
                 max_t, bias = float(layer.Params[0]), int(layer.Params[11] > 1e-8)
-                order = "order_patches" if layer.Kh * layer.Kw > 1 and sz.shape[1] <= 8192 else "sort_segments"
+            forward, backward = (snn.snnfc, snn.snnfc_grad) if dense else (snn.snncv, snn.snncv_grad)
+            ran = launched(torch, lambda: forward(x_op, W, layer.Params))
+            y = forward(x_op, W, layer.Params)
+            ran |= launched(torch, lambda: backward(torch.zeros_like(y), x_op, W, layer.Params, y, want_dx=bool(want_dx)))
         S, I = sz.shape
         J = ck.shape[1]
         n_real = (sz <= np.float32(max_t) - np.float32(0.1)).sum(dim=1, keepdim=True)
@@ -302,13 +314,15 @@ def account(torch, snn, layers, extras=None):
         steps = float((consumed + bias).sum().item())
         pairs = float((torch.where(fired, ck, torch.zeros_like(ck)) + bias * fired).sum().item())
         n_in = float(x_op.numel())
-        add(order, 0.0, 4.0 * (n_in + 2.0 * S * I))
-        add("scan", 4.0 * steps, 4.0 * (2.0 * S * I + (I + bias) * J + 2.0 * S * J))
-        if dense and J <= 16:
+        order = ran & {"order_rows", "order_patches", "sort_segments"}
+        for name in order:
+            add(name, 0.0, 4.0 * (n_in + 2.0 * S * I))
+        add("scan_stream" if "scan_stream" in ran else "scan", 4.0 * steps,
+            4.0 * ((2.0 if order else 1.0) * S * I + (I + bias) * J + 2.0 * S * J))
+        if "fc_backward_narrow" in ran:
             add("fc_backward_narrow", 5.0 * pairs + S * J, 4.0 * (3.0 * S * J + 2.0 * n_in + 2.0 * (I + bias) * J))
             continue
-        tiles = -(-S // 16) * -(-I // 32) * bool(want_dx) + -(-J // 64) * -(-(I + 1) // 64)
-        if dense and J >= 128 and tiles <= 1024:             # dX tiles of 16 x 32, dW tiles of 64 x 64
+        if "fc_backward" in ran:
             add("fc_backward", (5.0 if want_dx else 3.0) * pairs + S * J,
                 4.0 * (3.0 * S * J + 2.0 * n_in + 2.0 * (I + bias) * J))
             continue

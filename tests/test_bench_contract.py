@@ -106,3 +106,27 @@ def test_record_line_is_short_and_parses_on_its_own():
     # a single workload: no per_config table
     one = bench.headline(per_config["cfg3"], None, 20, 5, "AMD Instinct MI355X")
     assert "per_config" not in one and len(json.dumps(one, separators=(",", ":"))) < bench.LINE_BUDGET
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,I,J", [(256, 800, 10), (4, 300, 20), (128, 784, 800), (16384, 64, 128), (4096, 784, 800), (9000, 300, 40)])
+@pytest.mark.parametrize("want_dx", [True, False])
+def test_accounting_names_the_kernels_that_run(B, I, J, want_dx):
+    """Rows ordered inside the scan, ranked rows, the joint backward, dW in slices: only what is launched is booked, and all of it."""
+    sys.path.insert(0, ROOT)
+    import bench
+    import torch
+    import snntc_amd as snn
+    rng = np.random.default_rng(B + I + J)
+    layer = snn.SNN_dense(I, J, biasvolt=1.0, weight=bench._w_init(rng, I, J)).to("cuda:0")
+    x = torch.from_numpy(np.exp(1.0 - rng.random((B, I))).astype(np.float32)).to("cuda:0")
+    booked = bench.account(torch, snn, [(layer, x, want_dx, False)])
+    y = snn.snnfc(x, layer.weight.data, layer.Params)
+
+    def step():
+        snn.snnfc(x, layer.weight.data, layer.Params)
+        snn.snnfc_grad(torch.zeros_like(y), x, layer.weight.data, layer.Params, y, want_dx=want_dx)
+
+    assert set(booked) == bench.launched(torch, step) - {"reduce_partials"}
+    orders = len({"order_rows", "sort_segments"} & set(booked))
+    assert booked["scan"][1] == 4.0 * ((1 + orders) * B * I + (I + 1) * J + 2 * B * J)
