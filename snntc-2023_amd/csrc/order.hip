@@ -34,6 +34,7 @@
 // 64 inputs compared per word instead of 16 they take up to 37 % longer (smooth 248), with 8 the continuous ones do (96).
 #include <algorithm>
 #include <atomic>
+#include <iterator>
 
 #include "snntc_common.h"
 #include "sort_network.h"
@@ -45,6 +46,8 @@ constexpr int ORDER_COARSE = 1024;
 constexpr int ORDER_COARSE_BITS = 10;
 constexpr int ORDER_BUCKET_LIMIT = 16;                       // inputs of a word that are still compared with each other
 constexpr int ORDER_EPT = 16;                              // region inputs per thread at most
+constexpr int ORDER_ROW_BUCKET_LIMIT = 32;                   // ... of a dense row
+constexpr int ORDER_GROUP_PITCH = ORDER_COARSE + 1;          // counts of a pair of wavefronts: buckets, and the largest time
 constexpr int ORDER_RADIX_PITCH = 260;                     // 256 digit counts and a shift of the banks
 constexpr int ORDER_LDS_BYTES = 160 * 1024;
 
@@ -125,7 +128,7 @@ inline size_t order_lds_bytes(int n_cap, int threads, int stride, int waves, int
 }
 
 // ROWS > 0: the region is one dense row of up to ROWS inputs and its only patch: an input's rank is its place.  Where values
-// repeat or crowd, the row is sorted by a network instead.
+// repeat, see there; where more than ORDER_ROW_BUCKET_LIMIT inputs share a word all the same, the row is sorted by a network.
 // T threads; ITERS inputs per lane (WAVE: a patch belongs to a wavefront) or per thread (a patch belongs to
 // the workgroup) of a patch; VEC = 4: rows of the image are read in aligned groups of four (C a multiple of four).
 template <int T, bool WAVE, int ITERS, int FULL, int VEC, bool PIXELS, int ROWS = 0>
@@ -133,11 +136,12 @@ __global__ void __launch_bounds__(T)
 order_patches_kernel(const float* __restrict__ xpad, float* __restrict__ sorted, int32_t* __restrict__ perm,
                      int32_t* __restrict__ n_real, OrderGeom g) {
     extern __shared__ __align__(16) uint32_t lds[];
-    constexpr int WAVES = T / kWave, ROUNDS = ORDER_EPT / 4;
-    constexpr uint32_t kNone = ~0u, kNegZero = 0x80000000u;
+    constexpr int EPT = ROWS > 0 ? (ROWS + 4 * T - 1) / (4 * T) * 4 : ORDER_EPT;         // region inputs per thread at most
+    constexpr int WAVES = T / kWave, ROUNDS = EPT / 4;
+    constexpr uint32_t kNone = ~0u, kFrequent = ~0u - 1, kNegZero = 0x80000000u;
     __shared__ uint4 red[WAVES];
     __shared__ uint32_t bases[2][WAVES];
-    __shared__ uint32_t overflow;
+    __shared__ uint32_t overflow, several;
     const int tid = threadIdx.x, lane = tid % kWave;
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int block = xcd_contiguous(blockIdx.x, gridDim.x);
@@ -160,8 +164,8 @@ order_patches_kernel(const float* __restrict__ xpad, float* __restrict__ sorted,
     uint16_t* dirty_list = slots + (g.n_cap + 1) / 2 * 2 + wave * ((n + 4 * T - 1) / (4 * T)) * 4 * kWave;       // (a list per wavefront)
 
     // input j of a thread's round
-    bool crowded = false;                                   // ROWS: nothing is left to rank
-    auto begun = [&](int round) { return !(ROWS > 0 && crowded) && (VEC == 4 ? (round * T + wave * kWave) * 4 < n : round * 4 * T + wave * kWave < n); };      // wave-uniform
+    bool tied = false, counted = false;                     // ROWS: values repeat; and nothing else is left to rank
+    auto begun = [&](int round) { return VEC == 4 ? (round * T + wave * kWave) * 4 < n : round * 4 * T + wave * kWave < n; };      // wave-uniform
     auto input = [&](int round, int j) { return VEC == 4 ? (round * T + tid) * 4 + j : (round * 4 + j) * T + tid; };
 
     // ---- the region's inputs ---------------------------------------------------------------------------------------
@@ -170,7 +174,7 @@ order_patches_kernel(const float* __restrict__ xpad, float* __restrict__ sorted,
     const uint32_t key_cmp = order_key(__float_as_uint(g.max_cmp));
     for (int i = tid; i < ORDER_COARSE / 4; i += T) reinterpret_cast<uint4*>(coarse)[i] = make_uint4(0, 0, 0, 0);
     for (int i = tid; i < (n_words + kWave) / 2; i += T) reinterpret_cast<uint4*>(words)[i] = make_uint4(0, 0, 0, 0);
-    uint32_t d[ORDER_EPT];                                               // key, then distance from the smallest key, then position
+    uint32_t d[EPT];                                                     // key, then distance from the smallest key, then position
 #pragma unroll
     for (int round = 0; round < ROUNDS; ++round) {
         if (!begun(round)) break;
@@ -243,14 +247,14 @@ order_patches_kernel(const float* __restrict__ xpad, float* __restrict__ sorted,
     const uint32_t reals = (uint32_t)n - (uint32_t)__builtin_amdgcn_readfirstlane((int)idle);        // inputs that take part in a scan
     const bool has_last = k_max > key_cmp;                  // inputs of the largest time: behind all others, in index order
     const int sh = range >> (ORDER_COARSE_BITS + 1) ? 32 - __builtin_clz(range) - ORDER_COARSE_BITS : 1;
-    const uint32_t d_limit = sh + ORDER_COARSE_BITS >= 32 ? kNone - 1 : ((uint32_t)ORDER_COARSE << sh) - 1;
+    const uint32_t d_limit = sh + ORDER_COARSE_BITS >= 32 ? kFrequent - 1 : ((uint32_t)ORDER_COARSE << sh) - 1;
 
     // ---- positions: 16 bits of a bitmap per input, shared out evenly over the coarse buckets ---------------------------
     // PLAIN: no input of the largest time and whole groups of four; threads past the end stay out.  Otherwise inputs of
     // the largest time, and threads past the end, go through the motions on entries of no consequence.
     uint32_t* last = reinterpret_cast<uint32_t*>(slots);    // inputs of the largest time before a wavefront's round
     const bool plain = VEC == 4 && !has_last;
-    auto coarse_of = [&](uint32_t dist) { return dist == kNone ? (uint32_t)(ORDER_COARSE + lane) : dist >> sh; };
+    auto coarse_of = [&](uint32_t dist) { return dist >= kFrequent ? (uint32_t)(ORDER_COARSE + lane) : dist >> sh; };
     const uint32_t spare = (uint32_t)(n_words + lane);      // a word of no consequence
     auto last_of = [&](int round, int j) { return __builtin_amdgcn_ballot_w64(d[round * 4 + j] == kNone && input(round, j) < n); };
     if (plain) {
@@ -297,14 +301,17 @@ order_patches_kernel(const float* __restrict__ xpad, float* __restrict__ sorted,
     uint32_t held[HELD], held_sum = 0;
 #pragma unroll
     for (int q = 0; q < HELD; ++q) held_sum += held[q] = coarse[tid * HELD + q];
+    if constexpr (ROWS > 0)                                 // in the upper half: buckets in use
+#pragma unroll
+        for (int q = 0; q < HELD; ++q) held_sum += held[q] ? 1u << 16 : 0u;
     uint32_t before = wave_prefix(held_sum);
     if (lane == kWave - 1) bases[0][wave] = before;
     before -= held_sum;
-    if constexpr (ROWS > 0) {                               // a value of an eighth of the inputs would fill its word
-        uint32_t most = 0;
+    uint32_t most = 0;                                      // ROWS: inputs of the thread's fullest bucket << 10 | the bucket
+    if constexpr (ROWS > 0) {
 #pragma unroll
-        for (int q = 0; q < HELD; ++q) most = max(most, held[q]);
-        if (most > (uint32_t)n / 8) overflow = 1;
+        for (int q = 0; q < HELD; ++q) most = max(most, held[q] << ORDER_COARSE_BITS | (uint32_t)(tid * HELD + q));
+        if (most >> ORDER_COARSE_BITS > max((uint32_t)ORDER_BUCKET_LIMIT, (uint32_t)n / 192)) overflow = 1;
     }
     if (has_last && wave == 0) {
         const int m = (n + 4 * T - 1) / (4 * T) * WAVES * (VEC == 1 ? 4 : 1);
@@ -316,7 +323,6 @@ order_patches_kernel(const float* __restrict__ xpad, float* __restrict__ sorted,
         }
     }
     __syncthreads();
-    if constexpr (ROWS > 0) crowded = __builtin_amdgcn_readfirstlane((int)overflow) != 0;
     uint32_t n_first = 0;                                   // inputs before the ones of the largest time
 #pragma unroll
     for (int v = 0; v < WAVES; ++v) {
@@ -324,15 +330,22 @@ order_patches_kernel(const float* __restrict__ xpad, float* __restrict__ sorted,
         if (v < wave) before += b;
         n_first += b;
     }
+    // Values repeat (or crowd): a bucket holds more inputs, or fewer buckets are in use, than evenly spread values make of it.
+    if constexpr (ROWS > 0) {
+        const uint32_t used = n_first >> 16;
+        n_first &= 0xffffu;
+        before &= 0xffffu;
+        tied = __builtin_amdgcn_readfirstlane((int)(overflow | (used * 5 < min(n_first, (range >> sh) + 1) * 3))) != 0;
+    }
 #pragma unroll
     for (int q = 0; q < HELD; ++q) {
         coarse[tid * HELD + q] = before << 19 | held[q];
         before += held[q];
     }
-    uint32_t last_before[VEC == 1 ? ORDER_EPT : ROUNDS];
+    uint32_t last_before[VEC == 1 ? EPT : ROUNDS];
     if (has_last) {
 #pragma unroll
-        for (int q = 0; q < (VEC == 1 ? ORDER_EPT : ROUNDS); ++q)
+        for (int q = 0; q < (VEC == 1 ? EPT : ROUNDS); ++q)
             last_before[q] = q * (VEC == 1 ? 1 : 4) * T < n ? last[q * WAVES + wave] : 0;
     }
     __syncthreads();
@@ -346,7 +359,128 @@ order_patches_kernel(const float* __restrict__ xpad, float* __restrict__ sorted,
         atomicOr(&w->x, 1u << ((at >> 15) & 31));
         atomicAdd(&w->y, 1u);
     };
-    if (plain) {
+    // Rows whose values repeat.  Where every bucket holds a single value, an input's place among its equals is all that is missing:
+    // a wavefront takes a run of inputs, 64 at a time, and counts them per bucket (a pair of wavefronts shares a word), which makes the ranks.
+    // Where one value repeats among others, its inputs stay out of the bitmap and keep their index order between the
+    // smaller and the larger ones, by a prefix count.
+    uint32_t k_frequent = 0, n_frequent = 0, n_lower = 0;   // the value that stays out, inputs of it and of smaller values
+    uint32_t frequent_before[VEC == 1 ? EPT : ROUNDS];
+    if constexpr (ROWS > 0) {
+        if (tied) {
+            uint16_t* one = slots + (g.n_cap + 1) / 2 * 2;  // an input of every bucket, where the lists will stand (1024 or more entries)
+            auto each = [&](auto&& f) {
+#pragma unroll
+                for (int round = 0; round < ROUNDS; ++round) {
+                    if (!begun(round)) break;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        if (input(round, j) < n && d[round * 4 + j] != kNone) f((uint32_t)input(round, j), d[round * 4 + j] >> sh);
+                }
+            };
+            most = wave_max(most);
+            if (lane == 0) bases[1][wave] = most;
+            if (tid == 0) overflow = several = 0;
+            each([&](uint32_t e, uint32_t b) { one[b] = (uint16_t)e; });
+            __syncthreads();
+#pragma unroll
+            for (int v = 0; v < WAVES; ++v) most = max(most, bases[1][v]);
+            const uint32_t frequent = value[one[most & (ORDER_COARSE - 1)]];             // (any, where the bucket holds several)
+            k_frequent = order_key(frequent);
+            uint32_t counts = 0;                            // inputs of it, and of smaller values << 16
+            bool differs = false;
+            each([&](uint32_t e, uint32_t b) {
+                const uint32_t v = value[e];
+                counts += v == frequent ? 1u : order_key(v) < k_frequent ? 1u << 16 : 0u;
+                differs |= v != value[one[b]];
+            });
+            counts = wave_prefix(counts);
+            if (lane == kWave - 1) bases[0][wave] = counts;
+            if (__builtin_amdgcn_ballot_w64(differs) != 0 && lane == 0) several = 1;
+            __syncthreads();
+            counts = 0;
+#pragma unroll
+            for (int v = 0; v < WAVES; ++v) counts += bases[0][v];
+            n_lower = counts >> 16;
+            n_frequent = counts & 0xffffu;
+            counted = __builtin_amdgcn_readfirstlane((int)several) == 0;
+            tied = __builtin_amdgcn_readfirstlane((int)n_frequent) > ORDER_ROW_BUCKET_LIMIT;
+        }
+        if (counted) {
+            uint32_t* counter = reinterpret_cast<uint32_t*>(words);                      // [pair of wavefronts][bucket]
+            for (int i = tid; i < WAVES / 2 * ORDER_GROUP_PITCH; i += T) counter[i] = 0;
+            __syncthreads();
+            constexpr int RUNS = ROWS / T;
+            const int runs = (n + T - 1) / T, half = wave % 2 * 16;
+            uint32_t place[RUNS];                           // bucket << 16 | inputs of it before, in the wavefront
+#pragma unroll
+            for (int r = 0; r < RUNS; ++r) {
+                const int e = (wave * runs + r) * kWave + lane;
+                if (r >= runs || e - lane >= n) break;
+                const uint32_t k = order_key(value[min(e, n - 1)]);
+                const uint32_t b = has_last && k == k_max ? (uint32_t)ORDER_COARSE : min(k - k_min, d_limit) >> sh;
+                const uint64_t some = __builtin_amdgcn_ballot_w64(e < n);
+                uint32_t lo = (uint32_t)some, hi = (uint32_t)(some >> 32);               // lanes of the same bucket
+#pragma unroll
+                for (int bit = 0; bit <= ORDER_COARSE_BITS; ++bit) {
+                    const uint32_t unset = ((b >> bit) & 1) - 1;
+                    const uint64_t set = __builtin_amdgcn_ballot_w64(unset == 0);
+                    lo &= (uint32_t)set ^ unset;
+                    hi &= (uint32_t)(set >> 32) ^ unset;
+                }
+                const uint64_t same = (uint64_t)hi << 32 | lo;
+                const uint32_t ahead = lanes_below(same);
+                uint32_t before_run = 0;
+                if (e < n && ahead == 0)
+                    before_run = atomicAdd(&counter[wave / 2 * ORDER_GROUP_PITCH + b], (uint32_t)__builtin_popcountll(same) << half);
+                before_run = (uint32_t)__shfl((int)before_run, e < n ? __builtin_ctzll(same) : lane, kWave);
+                place[r] = b << 16 | (((before_run >> half) & 0xffffu) + ahead);
+            }
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < RUNS; ++r) {
+                const int e = (wave * runs + r) * kWave + lane;
+                if (r >= runs || e - lane >= n) break;
+                if (e >= n) continue;
+                const uint32_t b = place[r] >> 16;
+                uint32_t at = (place[r] & 0xffffu) + (b == (uint32_t)ORDER_COARSE ? n_first : coarse[b] >> 19);
+                for (int p = 0; p < wave / 2; ++p) {
+                    const uint32_t c = counter[p * ORDER_GROUP_PITCH + b];
+                    at += (c & 0xffffu) + (c >> 16);
+                }
+                if (half) at += counter[wave / 2 * ORDER_GROUP_PITCH + b] & 0xffffu;
+                rank[e] = (uint16_t)pack_ranks(at);
+            }
+        } else if (tied) {
+#pragma unroll
+            for (int round = 0; round < ROUNDS; ++round) {
+                uint32_t c = 0;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int q = round * 4 + j, e = input(round, j);
+                    d[q] = e >= n ? kNone : d[q] != kNone && order_key(value[min(e, n - 1)]) == k_frequent ? kFrequent : d[q];
+                    if constexpr (VEC == 1) c = 0;
+                    c += (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(d[q] == kFrequent));
+                    if constexpr (VEC == 1) if (lane == 0) last[q * WAVES + wave] = c;
+                }
+                if constexpr (VEC == 4) if (lane == 0) last[round * WAVES + wave] = c;
+            }
+            __syncthreads();
+            constexpr int COUNTS = (VEC == 1 ? EPT : ROUNDS) * WAVES, TURNS = (COUNTS + kWave - 1) / kWave;
+            uint32_t prefix[TURNS], sum = n_lower;
+#pragma unroll
+            for (int t = 0; t < TURNS; ++t) {
+                const uint32_t v = t * kWave + lane < COUNTS ? last[t * kWave + lane] : 0, s = wave_prefix(v);
+                prefix[t] = sum + s - v;
+                sum += (uint32_t)__builtin_amdgcn_readlane((int)s, kWave - 1);
+            }
+#pragma unroll
+            for (int q = 0; q < (VEC == 1 ? EPT : ROUNDS); ++q)                          // (WAVES divides 64)
+                frequent_before[q] = (uint32_t)__builtin_amdgcn_readlane((int)prefix[q * WAVES / kWave], q * WAVES % kWave + wave);
+        }
+    }
+    const bool whole = plain && !(ROWS > 0 && tied);        // every group of four as it is
+    if (counted) {
+    } else if (whole) {
 #pragma unroll
         for (int round = 0; round < ROUNDS; ++round) {
             if (!begun(round)) break;
@@ -364,232 +498,252 @@ order_patches_kernel(const float* __restrict__ xpad, float* __restrict__ sorted,
             if (!begun(round)) break;
             uint32_t c[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) c[j] = coarse[coarse_of(d[round * 4 + j])];
+            for (int j = 0; j < 4; ++j) c[j] = coarse[coarse_of(d[round * 4 + j])];      // (those that stay out as well)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int q = round * 4 + j;
-                if (d[q] != kNone) enter(d[q] = min(position(d[q], c[j]), kNone - 1));
+                if (d[q] < kFrequent) enter(d[q] = min(position(d[q], c[j]), kFrequent - 1));
             }
         }
     }
-    __syncthreads();
-    // words: the bitmap and, behind it, the number of inputs before the word | inputs share a bit in it << 31
-    constexpr int STEPS = ORDER_EPT / 8;
-    const int steps = (n_words + 4 * T - 1) / (4 * T);
-    uint32_t count_of[STEPS][4];
-    uint32_t carry = 0, fullest = 0;
-#pragma unroll
-    for (int st = 0; st < STEPS; ++st) {
-        if (st >= steps) break;
-        const int w = ((wave * steps + st) * kWave + lane) * 4;
-        uint4 q[2] = {make_uint4(0, 0, 0, 0), make_uint4(0, 0, 0, 0)};
-        if (w < n_words) {
-            q[0] = *reinterpret_cast<const uint4*>(words + w);
-            q[1] = *reinterpret_cast<const uint4*>(words + w + 2);
-        }
-        const uint32_t sum = q[0].y + q[0].w + q[1].y + q[1].w, s = carry + wave_prefix(sum);
-        fullest = max(max(fullest, max(q[0].y, q[0].w)), max(q[1].y, q[1].w));
-        count_of[st][0] = (s - sum) | ((uint32_t)__builtin_popcount(q[0].x) != q[0].y ? 1u << 31 : 0u);
-        count_of[st][1] = (s - sum + q[0].y) | ((uint32_t)__builtin_popcount(q[0].z) != q[0].w ? 1u << 31 : 0u);
-        count_of[st][2] = (s - q[1].y - q[1].w) | ((uint32_t)__builtin_popcount(q[1].x) != q[1].y ? 1u << 31 : 0u);
-        count_of[st][3] = (s - q[1].w) | ((uint32_t)__builtin_popcount(q[1].z) != q[1].w ? 1u << 31 : 0u);
-        carry = (uint32_t)__builtin_amdgcn_readlane((int)s, kWave - 1);
-    }
-    if (lane == 0) bases[1][wave] = carry;
-    if (__builtin_amdgcn_ballot_w64(fullest > ORDER_BUCKET_LIMIT) != 0 && lane == 0) overflow = 1;
-    __syncthreads();
-    const bool give_up = __builtin_amdgcn_readfirstlane((int)overflow) != 0;
-    if (!give_up) {
-        uint32_t base = 0;
-#pragma unroll
-        for (int v = 0; v < WAVES; ++v)
-            if (v < wave) base += bases[1][v];
+    if (!counted) {
+        __syncthreads();
+        // words: the bitmap and, behind it, the number of inputs before the word | inputs share a bit in it << 31
+        constexpr int STEPS = (EPT + 7) / 8;
+        const int steps = (n_words + 4 * T - 1) / (4 * T);
+        uint32_t count_of[STEPS][4];
+        uint32_t carry = 0, fullest = 0;
 #pragma unroll
         for (int st = 0; st < STEPS; ++st) {
             if (st >= steps) break;
             const int w = ((wave * steps + st) * kWave + lane) * 4;
-            if (w < n_words)
-#pragma unroll
-                for (int t = 0; t < 4; ++t) words[w + t].y = count_of[st][t] + base;
+            uint4 q[2] = {make_uint4(0, 0, 0, 0), make_uint4(0, 0, 0, 0)};
+            if (w < n_words) {
+                q[0] = *reinterpret_cast<const uint4*>(words + w);
+                q[1] = *reinterpret_cast<const uint4*>(words + w + 2);
+            }
+            const uint32_t sum = q[0].y + q[0].w + q[1].y + q[1].w, s = carry + wave_prefix(sum);
+            fullest = max(max(fullest, max(q[0].y, q[0].w)), max(q[1].y, q[1].w));
+            count_of[st][0] = (s - sum) | ((uint32_t)__builtin_popcount(q[0].x) != q[0].y ? 1u << 31 : 0u);
+            count_of[st][1] = (s - sum + q[0].y) | ((uint32_t)__builtin_popcount(q[0].z) != q[0].w ? 1u << 31 : 0u);
+            count_of[st][2] = (s - q[1].y - q[1].w) | ((uint32_t)__builtin_popcount(q[1].x) != q[1].y ? 1u << 31 : 0u);
+            count_of[st][3] = (s - q[1].w) | ((uint32_t)__builtin_popcount(q[1].z) != q[1].w ? 1u << 31 : 0u);
+            carry = (uint32_t)__builtin_amdgcn_readlane((int)s, kWave - 1);
         }
+        if (lane == 0) bases[1][wave] = carry;
+        if (__builtin_amdgcn_ballot_w64(fullest > (ROWS > 0 ? ORDER_ROW_BUCKET_LIMIT : ORDER_BUCKET_LIMIT)) != 0 && lane == 0) overflow = 1;
         __syncthreads();
+        const bool give_up = __builtin_amdgcn_readfirstlane((int)overflow) != 0;
+        if (!give_up) {
+            uint32_t base = 0;
+#pragma unroll
+            for (int v = 0; v < WAVES; ++v)
+                if (v < wave) base += bases[1][v];
+#pragma unroll
+            for (int st = 0; st < STEPS; ++st) {
+                if (st >= steps) break;
+                const int w = ((wave * steps + st) * kWave + lane) * 4;
+                if (w < n_words)
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) words[w + t].y = count_of[st][t] + base;
+            }
+            __syncthreads();
 
-        // ---- ranks ---------------------------------------------------------------------------------------------------
-        uint32_t n_listed = 0;
+            // ---- ranks ---------------------------------------------------------------------------------------------------
+            uint32_t n_listed = 0;
 #pragma unroll
-        for (int round = 0; round < ROUNDS; ++round) {
-            if (!begun(round)) break;
-            uint2 w[4];
-            uint32_t r[4];
-            uint64_t dirty[4];
-            if (plain) {
+            for (int round = 0; round < ROUNDS; ++round) {
+                if (!begun(round)) break;
+                uint2 w[4];
+                uint32_t r[4];
+                uint64_t dirty[4];
+                if (whole) {
 #pragma unroll
-                for (int j = 0; j < 4; ++j) w[j].y = 0;
-                if (input(round, 0) < n)
+                    for (int j = 0; j < 4; ++j) w[j].y = 0;
+                    if (input(round, 0) < n)
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) w[j] = words[d[round * 4 + j] >> 20];
-            } else {
+                        for (int j = 0; j < 4; ++j) w[j] = words[d[round * 4 + j] >> 20];
+                } else {
 #pragma unroll
-                for (int j = 0; j < 4; ++j) w[j] = words[d[round * 4 + j] == kNone ? spare : d[round * 4 + j] >> 20];
-            }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                r[j] = (uint32_t)__builtin_popcount(__builtin_amdgcn_ubfe(w[j].x, 0, d[round * 4 + j] >> 15)) + (w[j].y & 0xffffu);
-                dirty[j] = __builtin_amdgcn_ballot_w64((int)w[j].y < 0);
-            }
-            if (has_last) {
-                uint64_t l[4];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) l[j] = last_of(round, j);
-                uint32_t below = 0;
-                if constexpr (VEC == 4)
-                    below = n_first + last_before[round] + lanes_below(l[0]) + lanes_below(l[1]) + lanes_below(l[2]) + lanes_below(l[3]);
+                    for (int j = 0; j < 4; ++j) w[j] = words[d[round * 4 + j] >= kFrequent ? spare : d[round * 4 + j] >> 20];
+                }
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    if constexpr (VEC == 1) below = n_first + last_before[round * 4 + j] + lanes_below(l[j]);
-                    const bool mine = __builtin_amdgcn_inverse_ballot_w64(l[j]);
-                    r[j] = mine ? below : r[j];
-                    if constexpr (VEC == 4) below += mine ? 1u : 0u;
+                    r[j] = (uint32_t)__builtin_popcount(__builtin_amdgcn_ubfe(w[j].x, 0, d[round * 4 + j] >> 15)) + (w[j].y & 0xffffu);
+                    dirty[j] = __builtin_amdgcn_ballot_w64((int)w[j].y < 0);
+                }
+                if (has_last) {
+                    uint64_t l[4];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) l[j] = last_of(round, j);
+                    uint32_t below = 0;
+                    if constexpr (VEC == 4)
+                        below = n_first + last_before[round] + lanes_below(l[0]) + lanes_below(l[1]) + lanes_below(l[2]) + lanes_below(l[3]);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        if constexpr (VEC == 1) below = n_first + last_before[round * 4 + j] + lanes_below(l[j]);
+                        const bool mine = __builtin_amdgcn_inverse_ballot_w64(l[j]);
+                        r[j] = mine ? below : r[j];
+                        if constexpr (VEC == 4) below += mine ? 1u : 0u;
+                    }
+                }
+                if constexpr (ROWS > 0)
+                    if (tied) {
+                        uint64_t f[4];
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) f[j] = __builtin_amdgcn_ballot_w64(d[round * 4 + j] == kFrequent);
+                        uint32_t below = 0;
+                        if constexpr (VEC == 4)
+                            below = frequent_before[round] + lanes_below(f[0]) + lanes_below(f[1]) + lanes_below(f[2]) + lanes_below(f[3]);
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            if constexpr (VEC == 1) below = frequent_before[round * 4 + j] + lanes_below(f[j]);
+                            const bool mine = __builtin_amdgcn_inverse_ballot_w64(f[j]);
+                            const bool above = d[round * 4 + j] < kFrequent && order_key(value[min(input(round, j), n - 1)]) > k_frequent;
+                            r[j] = mine ? below : above ? r[j] + n_frequent : r[j];
+                            if constexpr (VEC == 4) below += mine ? 1u : 0u;
+                        }
+                    }
+                if constexpr (VEC == 4) {
+                    if (input(round, 0) < n)
+                        *reinterpret_cast<uint2*>(rank + input(round, 0)) =
+                            make_uint2(pack_ranks(r[0] | r[1] << 16), pack_ranks(r[2] | r[3] << 16));
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        if (input(round, j) < n) rank[input(round, j)] = (uint16_t)pack_ranks(r[j]);
+                }
+                // inputs of words in which a bit is shared: a list per wavefront
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    if (__builtin_amdgcn_inverse_ballot_w64(dirty[j])) dirty_list[n_listed + lanes_below(dirty[j])] = (uint16_t)input(round, j);
+                    n_listed += (uint32_t)__builtin_popcountll(dirty[j]);
                 }
             }
-            if constexpr (VEC == 4) {
-                if (input(round, 0) < n)
-                    *reinterpret_cast<uint2*>(rank + input(round, 0)) =
-                        make_uint2(pack_ranks(r[0] | r[1] << 16), pack_ranks(r[2] | r[3] << 16));
-            } else {
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    if (input(round, j) < n) rank[input(round, j)] = (uint16_t)pack_ranks(r[j]);
-            }
-            // inputs of words in which a bit is shared: a list per wavefront
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                if (__builtin_amdgcn_inverse_ballot_w64(dirty[j])) dirty_list[n_listed + lanes_below(dirty[j])] = (uint16_t)input(round, j);
-                n_listed += (uint32_t)__builtin_popcountll(dirty[j]);
-            }
-        }
-        // ... which are gathered by word and counted among themselves
-        lds_order();
-        auto gather = [&](uint32_t e, uint32_t& k, uint32_t*& word) {
-            k = order_key(value[e]);
-            const uint32_t dist = min(k - k_min, d_limit);
-            word = &words[min(position(dist, coarse[dist >> sh]), kNone - 1) >> 20].y;
-        };
-        auto count = [&](uint32_t e, uint32_t k, const uint32_t* word) {
-            const uint32_t m = *word, s0 = m & 0xffffu, s1 = s0 + ((m >> 16) & 0x7fffu);
-            const uint64_t mine = (uint64_t)k << 32 | e;
-            uint32_t r = s0;
-            for (uint32_t q = s0; q < s1; q += 4) {
-                uint32_t o[4], ko[4];
-#pragma unroll
-                for (int t = 0; t < 4; ++t) o[t] = slots[min(q + t, s1 - 1)];
-#pragma unroll
-                for (int t = 0; t < 4; ++t) ko[t] = order_key(value[o[t]]);
-#pragma unroll
-                for (int t = 0; t < 4; ++t) r += (q + t < s1) & (((uint64_t)ko[t] << 32 | o[t]) < mine);
-            }
-            rank[e] = (uint16_t)pack_ranks(r);
-        };
-        auto arrive = [&](uint32_t e, uint32_t* word) {
-            const uint32_t m = atomicAdd(word, 1u << 16);
-            slots[(m & 0xffffu) + ((m >> 16) & 0x7fffu)] = (uint16_t)e;
-        };
-        uint32_t e0 = 0, k0 = 0, *word0 = nullptr;          // the first 64 of the list stay in registers, most often all
-        if (lane < (int)n_listed) {
-            e0 = dirty_list[lane];
-            gather(e0, k0, word0);
-            arrive(e0, word0);
-        }
-        for (uint32_t i = kWave + lane; i < n_listed; i += kWave) {
-            uint32_t e = dirty_list[i], k, *word;
-            gather(e, k, word);
-            arrive(e, word);
-        }
-        __syncthreads();
-        if (lane < (int)n_listed) count(e0, k0, word0);
-        for (uint32_t i = kWave + lane; i < n_listed; i += kWave) {
-            uint32_t e = dirty_list[i], k, *word;
-            gather(e, k, word);
-            count(e, k, word);
-        }
-    } else if constexpr (ROWS > 0) {
-        constexpr int EPT = ROWS / T;
-        u64 v[EPT];
-#pragma unroll
-        for (int q = 0; q < EPT; ++q) {
-            const int e = tid * EPT + q;
-            v[q] = (u64)(e < n ? order_key(value[e]) : ~0u) << 32 | (uint32_t)e;
-        }
-        bitonic_sort<EPT, T>(v, tid, reinterpret_cast<u64*>(area));
-#pragma unroll
-        for (int q = 0; q < EPT; ++q)
-            if (const uint32_t e = (uint32_t)v[q]; e < (uint32_t)n) rank[e] = (uint16_t)pack_ranks((uint32_t)(tid * EPT + q));
-    } else {
-        // a value repeats too often: stable radix sort of the inputs' indexes, eight bits of the distance from the
-        // smallest key a pass; the last pass leaves ranks.  A wavefront takes a run of inputs, 64 at a time.
-        constexpr int DIGITS = 256, PITCH = ORDER_RADIX_PITCH, GROUP = WAVES / 4;
-        const int rounds = (n + T - 1) / T, half = (g.n_cap + 3) / 4 * 4;
-        uint16_t* item = reinterpret_cast<uint16_t*>(area);                              // [2][half], from pass to pass
-        uint32_t* count = area + half;                      // [wavefront][digit]
-        uint32_t* own = count + wave * PITCH;
-        const uint32_t spread = k_max - k_min;
-        int shift = 0;
-        do {
-            const bool last_pass = spread >> shift < DIGITS;
-            const uint16_t* from = item + ((shift / 8) & 1) * half;
-            uint16_t* to = item + ((shift / 8 + 1) & 1) * half;
-            auto index_at = [&](int at) { return shift == 0 ? (uint32_t)at : (uint32_t)from[at]; };
-            auto digit_of = [&](uint32_t e) { return ((order_key(value[e]) - k_min) >> shift) & (DIGITS - 1); };
-            reinterpret_cast<uint4*>(own)[lane] = make_uint4(0, 0, 0, 0);
+            // ... which are gathered by word and counted among themselves
             lds_order();
-#pragma unroll 1
-            for (int r = 0; r < rounds; ++r) {
-                const int at = (wave * rounds + r) * kWave + lane;
-                if (at < n) atomicAdd(&own[digit_of(index_at(at))], 1u);
+            auto gather = [&](uint32_t e, uint32_t& k, uint32_t*& word) {
+                k = order_key(value[e]);
+                const uint32_t dist = min(k - k_min, d_limit);
+                word = &words[min(position(dist, coarse[dist >> sh]), kFrequent - 1) >> 20].y;
+            };
+            auto count = [&](uint32_t e, uint32_t k, const uint32_t* word) {
+                const uint32_t m = *word, s0 = m & 0xffffu, s1 = s0 + ((m >> 16) & 0x7fffu);
+                const uint64_t mine = (uint64_t)k << 32 | e;
+                uint32_t r = s0;
+                for (uint32_t q = s0; q < s1; q += 4) {
+                    uint32_t o[4], ko[4];
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) o[t] = slots[min(q + t, s1 - 1)];
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) ko[t] = order_key(value[o[t]]);
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) r += (q + t < s1) & (((uint64_t)ko[t] << 32 | o[t]) < mine);
+                }
+                if constexpr (ROWS > 0) r += tied && k > k_frequent ? n_frequent : 0;
+                rank[e] = (uint16_t)pack_ranks(r);
+            };
+            auto arrive = [&](uint32_t e, uint32_t* word) {
+                const uint32_t m = atomicAdd(word, 1u << 16);
+                slots[(m & 0xffffu) + ((m >> 16) & 0x7fffu)] = (uint16_t)e;
+            };
+            uint32_t e0 = 0, k0 = 0, *word0 = nullptr;          // the first 64 of the list stay in registers, most often all
+            if (lane < (int)n_listed) {
+                e0 = dirty_list[lane];
+                gather(e0, k0, word0);
+                arrive(e0, word0);
+            }
+            for (uint32_t i = kWave + lane; i < n_listed; i += kWave) {
+                uint32_t e = dirty_list[i], k, *word;
+                gather(e, k, word);
+                arrive(e, word);
             }
             __syncthreads();
-            // inputs before the ones of a wavefront and digit: in order of (digit, wavefront), four wavefronts per thread
-            const int digit = tid / GROUP, first = tid % GROUP * 4;
-            uint32_t c[4], sum = 0;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) sum += c[q] = count[(first + q) * PITCH + digit];
-            uint32_t at_or_below = wave_prefix(sum);
-            if (lane == kWave - 1) bases[0][wave] = at_or_below;
-            __syncthreads();
-            uint32_t start = at_or_below - sum;
-#pragma unroll 1
-            for (int v = 0; v < wave; ++v) start += bases[0][v];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                count[(first + q) * PITCH + digit] = start;
-                start += c[q];
+            if (lane < (int)n_listed) count(e0, k0, word0);
+            for (uint32_t i = kWave + lane; i < n_listed; i += kWave) {
+                uint32_t e = dirty_list[i], k, *word;
+                gather(e, k, word);
+                count(e, k, word);
             }
-            __syncthreads();
-#pragma unroll 1
-            for (int r = 0; r < rounds; ++r) {
-                const int at = (wave * rounds + r) * kWave + lane;
-                const uint32_t e = at < n ? index_at(at) : 0, dg = digit_of(e);
-                const uint64_t some = __builtin_amdgcn_ballot_w64(at < n);
-                uint32_t lo = (uint32_t)some, hi = (uint32_t)(some >> 32);               // lanes with the same digit
-#pragma unroll 4
-                for (int b = 0; b < 8; ++b) {               // (in two goes: all eight at once cost every launch 12 registers)
-                    const uint32_t unset = ((dg >> b) & 1) - 1;
-                    const uint64_t set = __builtin_amdgcn_ballot_w64(unset == 0);
-                    lo &= (uint32_t)set ^ unset;
-                    hi &= (uint32_t)(set >> 32) ^ unset;
-                }
-                const uint64_t same = (uint64_t)hi << 32 | lo;
-                if (at < n) {
-                    const uint32_t before = own[dg], place = before + lanes_below(same);
-                    if ((same >> lane) == 1) own[dg] = place + 1;                        // the last of them
-                    if (last_pass) rank[e] = (uint16_t)pack_ranks(place);
-                    else to[place] = (uint16_t)e;
-                }
+        } else if constexpr (ROWS > 0) {
+            constexpr int KEYS = ROWS / T;
+            u64 v[KEYS];
+#pragma unroll
+            for (int q = 0; q < KEYS; ++q) {
+                const int e = tid * KEYS + q;
+                v[q] = (u64)(e < n ? order_key(value[e]) : ~0u) << 32 | (uint32_t)e;
+            }
+            bitonic_sort<KEYS, T>(v, tid, reinterpret_cast<u64*>(area));
+#pragma unroll
+            for (int q = 0; q < KEYS; ++q)
+                if (const uint32_t e = (uint32_t)v[q]; e < (uint32_t)n) rank[e] = (uint16_t)pack_ranks((uint32_t)(tid * KEYS + q));
+        } else {
+            // a value repeats too often: stable radix sort of the inputs' indexes, eight bits of the distance from the
+            // smallest key a pass; the last pass leaves ranks.  A wavefront takes a run of inputs, 64 at a time.
+            constexpr int DIGITS = 256, PITCH = ORDER_RADIX_PITCH, GROUP = WAVES / 4;
+            const int rounds = (n + T - 1) / T, half = (g.n_cap + 3) / 4 * 4;
+            uint16_t* item = reinterpret_cast<uint16_t*>(area);                              // [2][half], from pass to pass
+            uint32_t* count = area + half;                      // [wavefront][digit]
+            uint32_t* own = count + wave * PITCH;
+            const uint32_t spread = k_max - k_min;
+            int shift = 0;
+            do {
+                const bool last_pass = spread >> shift < DIGITS;
+                const uint16_t* from = item + ((shift / 8) & 1) * half;
+                uint16_t* to = item + ((shift / 8 + 1) & 1) * half;
+                auto index_at = [&](int at) { return shift == 0 ? (uint32_t)at : (uint32_t)from[at]; };
+                auto digit_of = [&](uint32_t e) { return ((order_key(value[e]) - k_min) >> shift) & (DIGITS - 1); };
+                reinterpret_cast<uint4*>(own)[lane] = make_uint4(0, 0, 0, 0);
                 lds_order();
-            }
-            __syncthreads();
-            shift += 8;
-        } while (shift < 32 && spread >> shift);
+#pragma unroll 1
+                for (int r = 0; r < rounds; ++r) {
+                    const int at = (wave * rounds + r) * kWave + lane;
+                    if (at < n) atomicAdd(&own[digit_of(index_at(at))], 1u);
+                }
+                __syncthreads();
+                // inputs before the ones of a wavefront and digit: in order of (digit, wavefront), four wavefronts per thread
+                const int digit = tid / GROUP, first = tid % GROUP * 4;
+                uint32_t c[4], sum = 0;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) sum += c[q] = count[(first + q) * PITCH + digit];
+                uint32_t at_or_below = wave_prefix(sum);
+                if (lane == kWave - 1) bases[0][wave] = at_or_below;
+                __syncthreads();
+                uint32_t start = at_or_below - sum;
+#pragma unroll 1
+                for (int v = 0; v < wave; ++v) start += bases[0][v];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    count[(first + q) * PITCH + digit] = start;
+                    start += c[q];
+                }
+                __syncthreads();
+#pragma unroll 1
+                for (int r = 0; r < rounds; ++r) {
+                    const int at = (wave * rounds + r) * kWave + lane;
+                    const uint32_t e = at < n ? index_at(at) : 0, dg = digit_of(e);
+                    const uint64_t some = __builtin_amdgcn_ballot_w64(at < n);
+                    uint32_t lo = (uint32_t)some, hi = (uint32_t)(some >> 32);               // lanes with the same digit
+#pragma unroll 4
+                    for (int b = 0; b < 8; ++b) {               // (in two goes: all eight at once cost every launch 12 registers)
+                        const uint32_t unset = ((dg >> b) & 1) - 1;
+                        const uint64_t set = __builtin_amdgcn_ballot_w64(unset == 0);
+                        lo &= (uint32_t)set ^ unset;
+                        hi &= (uint32_t)(set >> 32) ^ unset;
+                    }
+                    const uint64_t same = (uint64_t)hi << 32 | lo;
+                    if (at < n) {
+                        const uint32_t before = own[dg], place = before + lanes_below(same);
+                        if ((same >> lane) == 1) own[dg] = place + 1;                        // the last of them
+                        if (last_pass) rank[e] = (uint16_t)pack_ranks(place);
+                        else to[place] = (uint16_t)e;
+                    }
+                    lds_order();
+                }
+                __syncthreads();
+                shift += 8;
+            } while (shift < 32 && spread >> shift);
+        }
     }
     __syncthreads();                                        // ranks are in place, the tables are free
 
@@ -928,27 +1082,33 @@ constexpr OrderRowsForm order_rows_form() {
     return OrderRowsForm{N, T, order_patches_kernel<T, true, 1, 0, 1, false, N>, order_patches_kernel<T, true, 1, 0, 4, false, N>};
 }
 const OrderRowsForm kOrderRowsForms[] = {order_rows_form<256, 512>(), order_rows_form<256, 1024>(), order_rows_form<256, 2048>(),
-                                         order_rows_form<512, 4096>(), order_rows_form<1024, 8192>()};
+                                         order_rows_form<512, 4096>(), order_rows_form<1024, 8192>(), order_rows_form<512, 2048>()};
+constexpr int ORDER_FEW_ROWS = 256;                         // of 1025 to 2048 inputs: a workgroup per CU or none, of twice the threads
 
 size_t order_rows_lds(int64_t I, const OrderRowsForm& form) {
     const size_t ranks = order_lds_bytes((int)I, form.threads, (int)padded_stride(I), 1, 0, 0);
     const size_t network = ((size_t)I * 6 + 15) / 16 * 16 + (size_t)form.inputs * 8;
-    return std::max(ranks, network);
+    const size_t groups = ((size_t)I * 6 + 15) / 16 * 16 + (ORDER_COARSE + kWave + (size_t)form.threads / kWave / 2 * ORDER_GROUP_PITCH) * 4;
+    return std::max({ranks, network, groups});
 }
 }  // namespace
 
-// Dense rows: against the sorting networks, us, 2 / 128 / 2048 / 8192 rows:
-//   of 300     4.5 / 4.8 / 12.4 / 35 -> - / - / 10.2 / 27       of 2048    9.5 / 12 / 45 / 129 -> 6.9 / 9.1 / 25 / 67
-//   of 784     5.8 / 6.7 / 29 / 71   -> - / 6.2 / 21 / 35       of 4096    18 / 22 / 91        -> 8.3 / 12 / 42
-//   of 1521    9.6 / 11 / 44 / 122   -> 7.0 / 9.0 / 22 / 61     of 8192    34 / 36 / 204       -> 12 / 13 / 93
-// A network's steps grow with the square of the length's logarithm, the ranking's do not; below some 300 inputs, and for few rows of
-// up to 1024, both wait for a workgroup's latency and the network is as fast.  Up to 512 inputs the network is one wavefront's and a
-// full chip of them catches up (16 384 / 65 536 rows of 300 47 / 161 -> 46 / 171), sooner where rows are read an input at a time (of
-// 499 at 2009 / 5000 / 16 384 rows 13.3 / 30 / 49 -> 13.1 / 22 / 58).  Rows whose values repeat are found out after the
-// histogram (a value of an eighth of the inputs) or in the bitmap and go to the network all the same: 4096 rows of 784 with 256 levels 41 -> 38 us,
-// mostly background 41 -> 45; of 1521 69 -> 76 and 68 -> 87.  (By radix sort, as regions are: 784 mostly background 81, 4096 454.)
+// Dense rows: the sorting networks -> ranked, us between events, values all different (as they are / a tenth silent), then with repeats
+// (8-bit levels / mostly background / background and different values), then crowded in a tenth of an octave with outliers:
+//   16 x 1521      12.0 -> 8.7 / 9.4, 10.0 / 10.8 / 11.2, 11.0          3500 x 512     26.7 -> 17.0 / 19.8, 20.5 / 23.5 / 24.5, 22.6
+//   256 x 2048     16.0 -> 12.3 / 13.1, 14.4 / 15.6 / 16.2, 14.8        5000 x 384     28.6 -> 20.6 / 23.7, 24.6 / 27.0 / 28.7, 27.7
+//   400 x 1521     20.2 -> 14.0 / 15.6, 17.0 / 18.4 / 18.4, 17.8        1024 x 784     17.2 -> 10.4 / 12.1, 12.8 / 14.6 / 15.5, 16.1
+//   512 x 4096     41.0 -> 24.3 / 25.4, 29.8 / 34.6 / 33.3, 32.6        4096 x 784     45.7 -> 21.9 / 25.4, 29.3 / 33.2 / 33.2, 30.5
+//   512 x 8192     69.0 -> 33.0 / 37.0, 47.7 / 56.4 / 54.3, 67.2        16 384 x 784    132 -> 60 / 72, 84 / 100 / 99, 90
+// A network's steps grow with the square of the length's logarithm, the ranking's do not; but up to 1024 inputs it waits for a
+// workgroup's latency until several share a CU (512 x 1024: 13.7 -> 12.0 / 12.9, 13.9 / 15.0 / 15.0, 14.5), and up to 512 the network
+// is one wavefront's, which a full chip hides (8192 x 512: 37.7 -> 29.3 / 33.8, 36.8 / 42.8 / 44.3, 40.9) and which rows that are read an input
+// at a time do not beat (5000 x 449: 30.2 -> 25.0 / 28.4, 28.5 / 31.4 / 32.3, 33.7).  The ranking stands where it is faster on all of these.
+// Rows with several values that repeat among others of their bucket go to a network after all, and are slower for it (a
+// background with most other values close to it: 4096 x 784 45 -> 41, 512 x 4096 41 -> 47, 16 x 1521 12.0 -> 14.4).
 bool order_rows_supported(int64_t S, int64_t I) {
-    return S > 0 && I <= ORDER_MAX_REGION && (I > 1024 || (I > 512 && S >= 100) || (I > 256 && S >= (I % 4 ? 2560 : 1536) && S <= 8192));
+    if (S <= 0 || I > ORDER_MAX_REGION) return false;
+    return I > 1024 || (I > 512 && S >= 1024) || (I >= 352 && I % 4 == 0 && S >= 3072 && S <= 6144);
 }
 
 int launch_order_rows(const float* x, float* sorted, int32_t* perm, int32_t* n_real, int64_t S, int64_t I, int64_t stride,
@@ -959,6 +1119,7 @@ int launch_order_rows(const float* x, float* sorted, int32_t* perm, int32_t* n_r
     if (rc) return rc;
     const OrderRowsForm* form = kOrderRowsForms;
     while (I > form->inputs) ++form;
+    if (I > 1024 && I <= 2048 && S <= ORDER_FEW_ROWS) form = std::end(kOrderRowsForms) - 1;
     OrderGeom og{};
     og.H = 1; og.W = (int)I; og.C = 1; og.Kh = 1; og.Kw = (int)I; og.Sh = 1; og.Sw = 1; og.Nh = 1; og.Nw = 1; og.P = (int)I;
     og.th = og.tw = og.tiles_y = og.tiles_x = 1;

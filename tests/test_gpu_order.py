@@ -119,3 +119,87 @@ def test_dense_rows_at_any_alignment(B, I, offset):
     out = snn.snnfc(view, torch.from_numpy(w).to(DEV), capi.fc_params(1.0))
     ref = fc_forward_dev(x, w, capi.fc_params(1.0))
     assert np.array_equal(out.cpu().numpy().view(np.uint32), (ref[0] if isinstance(ref, tuple) else ref).view(np.uint32))
+
+
+def _tied_rows(kind, rng, B, I):
+    x = np.exp(rng.random((B, I))).astype(np.float32)
+    if kind == "levels":                                    # every bucket a single value; a tenth silent, a row of one value
+        x = np.exp(rng.integers(0, 200, (B, I)) / 200.0).astype(np.float32)
+        x[rng.random((B, I)) < 0.1] = 1e5
+        x[B // 2] = 1.5
+    elif kind == "runs":                                    # the same in long runs of equal neighbours
+        x = np.exp((np.arange(I) // 37 * 11 % 50 + rng.integers(0, 3, (B, 1))) / 60.0).astype(np.float32)
+    elif kind in ("lowest", "middle", "highest"):           # one value in two inputs, the others different, on both sides or one
+        x[rng.random((B, I)) < 0.5] = {"lowest": 0.5, "middle": 1.7, "highest": 3.0}[kind]
+        x[:, ::41] = 1e5
+        x[B // 2, : I // 2] = 1e5
+    elif kind == "close":                                   # ... and next to it within its bucket
+        x[rng.random((B, I)) < 0.5] = 1.7
+        x[:, ::5] = (np.float32(1.7) + rng.integers(-9, 9, x[:, ::5].shape) * np.float32(2.0 ** -20)).astype(np.float32)
+    elif kind == "two":                                     # two values among different ones: one of them stays in the bitmap
+        x[rng.random((B, I)) < 0.4] = 1.7
+        x[rng.random((B, I)) < 0.3] = 2.1
+    elif kind == "octave":                                  # crowded, all different, with outliers
+        x = (2 + 0.2 * rng.random((B, I))).astype(np.float32)
+        far = rng.random((B, I)) < 0.03
+        x[far] = np.exp(rng.uniform(0, 11, int(far.sum())))
+    elif kind == "zeros":
+        x = np.where(rng.random((B, I)) < 0.6, rng.choice(np.array([0.0, -0.0], np.float32), (B, I)), rng.standard_normal((B, I))).astype(np.float32)
+    return x
+
+
+TIED_ROWS = [(3072, 352), (6144, 512), (1024, 513), (1024, 784), (1025, 1023), (1024, 1024),             # edges of the rule and of the forms
+             (1, 1025), (256, 1028), (257, 1025), (3, 2047), (256, 2048), (257, 2048), (2, 2049), (3, 4096), (2, 4097), (3, 8192)]
+
+
+@pytest.mark.parametrize("kind", ["levels", "runs", "lowest", "middle", "highest", "close", "two", "octave", "zeros"])
+@pytest.mark.parametrize("B,I", TIED_ROWS)
+def test_dense_rows_whose_values_repeat(B, I, kind):
+    """Counted rows, rows with one value out of the bitmap, rows ranked as they are and rows that go to a network: order, causal sets, outputs."""
+    import snntc_amd as snn
+    rng = np.random.default_rng(B * 3 + I)
+    x = _tied_rows(kind, rng, B, I)
+    w = (4.0 / I + rng.standard_normal((I + 1, 3)) / np.sqrt(I)).astype(np.float32)
+    p = capi.fc_params(1.0)
+    ref_out, ref_k, ref_sorted, ref_perm = capi.fc_forward_dev(x, w, p, want_aux=True)
+    out, sz, perm, ck = (v.cpu().numpy() for v in snn.snnfc(torch.from_numpy(x).to(DEV), torch.from_numpy(w).to(DEV), p, return_aux=True))
+    assert np.array_equal(perm, ref_perm)
+    assert np.array_equal(sz, ref_sorted)
+    assert np.array_equal(ck, ref_k)
+    assert np.array_equal(out.view(np.uint32), ref_out.view(np.uint32))
+
+
+def _odd_rows(rng, B, I):
+    x = np.exp(rng.random((B, I))).astype(np.float32)
+    pick = np.array([np.inf, -np.inf, np.nan, -np.nan, 0.0, -0.0, 1e-45, -1e-45, 3.4e38, 1e5, 1e5 - 0.1], np.float32)
+    some = rng.random((B, I)) < 0.2
+    some[: B // 2] &= rng.random((B // 2, 1)) < 0.5          # rows without any among them
+    x[some] = pick[rng.integers(0, len(pick), some.sum())]
+    return torch.from_numpy(x).to(DEV)
+
+
+@pytest.mark.parametrize("I", [513, 784, 1024])
+def test_odd_values_take_part_alike_in_ranked_and_sorted_rows(I):
+    """Infinities and NaN of both signs: which inputs a scan walks (n_real) does not depend on how its row was ordered."""
+    import snntc_amd as snn
+    rng = np.random.default_rng(I)
+    x = _odd_rows(rng, 1024, I)
+    w = torch.from_numpy((4.0 / I + rng.standard_normal((I + 1, 40)) / np.sqrt(I)).astype(np.float32)).to(DEV)
+    p = capi.fc_params(1.0)
+    out, z, perm, ck = snn.snnfc(x, w, p, return_aux=True)                               # ranked
+    few, z2, perm2, ck2 = snn.snnfc(x[:600].contiguous(), w, p, return_aux=True)         # a network
+    assert torch.equal(perm[:600], perm2) and torch.equal(ck[:600], ck2)
+    assert torch.equal(z[:600].view(torch.int32), z2.view(torch.int32))
+    assert torch.equal(out[:600].view(torch.int32), few[:600].view(torch.int32))
+    assert torch.equal(out[1024:1624].view(torch.int32), few[600:].view(torch.int32))
+
+
+@pytest.mark.parametrize("B,I,J", [(5, 784, 30), (3, 300, 16), (4, 1024, 100), (7, 129, 10)])
+def test_odd_values_take_part_alike_where_the_scan_orders_its_rows(B, I, J):
+    import snntc_amd as snn
+    rng = np.random.default_rng(I)
+    x = _odd_rows(rng, B, I)
+    w = torch.from_numpy((4.0 / I + rng.standard_normal((I + 1, J)) / np.sqrt(I)).astype(np.float32)).to(DEV)
+    p = capi.fc_params(1.0)
+    own = snn.snnfc(x, w, p)                                # (asked for the order, a launch of its own makes it)
+    assert torch.equal(own.view(torch.int32), snn.snnfc(x, w, p, return_aux=True)[0].view(torch.int32))
