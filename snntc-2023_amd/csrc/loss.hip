@@ -30,7 +30,9 @@ softmax_time_loss_kernel(const float* __restrict__ times, const float* __restric
     if (b >= B) return;
     const float* __restrict__ t = times + (size_t)b * J;
     const float* __restrict__ y = label + (size_t)b * J;
-    // BATCH values of a lane are requested together (1000 classes: three trips to memory instead of 48, 17.8 -> 7.3 us)
+    // BATCH values of a lane are requested together (1000 classes: three trips to memory instead of 48, 17.8 -> 7.3 us).  Requests past the
+    // end repeat the last value and cost as much as others.  2048 rows, us with batches of 1 / 8 / 16: 65 classes 6.1 / 6.2 / 7.0, 128
+    // 6.2 / 6.2 / 7.1, 256 6.6 / 6.5 / 7.6, 512 8.6 / 7.0 / 8.3, 700 10.3 / 9.1 / 8.9, 1000 15.8 / 10.1 / 9.8.
     auto values = [&](const float* p, int j0, float (&v)[BATCH]) {
 #pragma unroll
         for (int i = 0; i < BATCH; ++i) v[i] = p[min(j0 + i * kWave + lane, J - 1)];
@@ -83,8 +85,9 @@ int launch_softmax_time_loss(const float* times, const float* label, float* samp
     if (blocks > 0x7fffffffLL) return fail(SNNTC_ERR_TOO_LARGE, "loss: too many samples");
     {
         KernelTimerScope timer_("softmax_time_loss", stream);
-        hipLaunchKernelGGL(J <= kWave ? softmax_time_loss_kernel<1> : softmax_time_loss_kernel<16>, dim3((unsigned)blocks), dim3(256), 0, stream, times, label,
-                           sample_loss, dtimes, (int)B, (int)J, 1.0f / (float)B);
+        auto kern = J <= kWave ? softmax_time_loss_kernel<1> : J <= 8 * kWave ? softmax_time_loss_kernel<8> : softmax_time_loss_kernel<16>;
+        hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), 0, stream, times, label, sample_loss, dtimes, (int)B, (int)J,
+                           1.0f / (float)B);
     }
     SNNTC_HIP_CHECK(hipGetLastError());
     return SNNTC_OK;

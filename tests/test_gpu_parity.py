@@ -390,6 +390,21 @@ def test_loss_kernel_against_closed_form(B, J):
     assert np.all(np.abs(T.grad.cpu().numpy() - 3.0 * want_g) <= 3e-6 / B + 3e-6 * np.abs(want_g))
 
 
+@pytest.mark.parametrize("J", [64, 128, 511, 512, 513, 1025])
+def test_loss_kernel_around_a_batch(J):
+    """Classes around the rounds of 64, 512 and 1024 in which a sample's values are requested; tolerance as above."""
+    import snntc_amd as snn
+    from oracle.closed_form import softmax_time_loss
+    rng = np.random.default_rng(J)
+    times = (1.0 + 4.0 * rng.random((5, J))).astype(np.float32)
+    label = rng.random((5, J)).astype(np.float32)
+    label /= label.sum(axis=1, keepdims=True)
+    want_s, want_g = softmax_time_loss(times, label)
+    got_s, got_g = snn.softmax_time_loss(t(times), t(label))
+    assert np.all(np.abs(got_s.cpu().numpy() - want_s) <= 1e-6 * np.maximum(1.0, np.abs(want_s)))
+    assert np.all(np.abs(got_g.cpu().numpy() - want_g) <= 1e-6 / 5 + 1e-6 * np.abs(want_g))
+
+
 HEAD_CASES = [
     # seed, B, I, J, bias: classifier heads, i.e. fewer (sample group, column slice) work items than CUs
     (20, 70, 800, 10, True),       # batch not a multiple of the segments a wavefront holds
