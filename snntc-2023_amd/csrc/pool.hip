@@ -10,6 +10,8 @@
 //
 // Also here: the SAME padding of SNN_conv (SNN_TC_Modules.py:147-161, tf.pad with MAX_SPIKE_TIME) as
 // one pass that writes every element of the padded tensor once, and the matching crop of the gradient.
+#include <type_traits>
+
 #include "snntc_common.h"
 
 namespace snntc {
@@ -49,35 +51,42 @@ min_pool_forward_kernel(const float* __restrict__ x, float* __restrict__ y, int3
     int where[VEC];
 #pragma unroll
     for (int v = 0; v < VEC; ++v) { best[v] = (H <= 0 || W <= 0) && pad_value < INFINITY ? pad_value : INFINITY; where[v] = 0; }
-    // The window's positions in (kh, kw) order, BATCH requests at a time: a global pool would otherwise wait for memory once per
-    // position (7x7 of one image, 512 channels: 19.3 -> 9.2 us).  Requests outside the image go to its nearest pixel; the last position is
-    // repeated to fill the last batch, which changes nothing since only a smaller value replaces the minimum.
+    // The window's positions in (kh, kw) order, up to BATCH requests at a time: a global pool would otherwise wait for memory once per
+    // position (7x7 of one image, 512 channels: 19.3 -> 9.2 us).  Requests outside the image go to its nearest pixel.  What is left of the
+    // window goes in batches of four and one by one: positions repeated to fill a last batch cost more than they hide
+    // (1x5 windows of 32 images of 56x56x64 17.5 us one by one, 21.5 in a batch of nine, 15.2 so; 2x5 25.4, 32.7 and 20.5).
     const int total = H > 0 && W > 0 ? Kh * Kw : 0;
-    int kh = 0, kw = 0;
-    for (int p0 = 0; p0 < total; p0 += BATCH) {
-        float val[BATCH][VEC];
-        bool in[BATCH];
+    int kh = 0, kw = 0, p0 = 0;
+    auto positions = [&](auto n_c) {
+        constexpr int N = decltype(n_c)::value;
+        for (; p0 + N <= total; p0 += N) {
+            float val[N][VEC];
+            bool in[N];
 #pragma unroll
-        for (int i = 0; i < BATCH; ++i) {
-            const int h = h0 + kh, w = w0 + kw;
-            in[i] = h >= 0 && h < H && w >= 0 && w < W;
-            const float* p = img + ((size_t)min(max(h, 0), H - 1) * W + min(max(w, 0), W - 1)) * C;
-            if (VEC == 4) {
-                const float4 q = *reinterpret_cast<const float4*>(p);
-                val[i][0] = q.x; val[i][1] = q.y; val[i][2] = q.z; val[i][3] = q.w;
-            } else {
-                val[i][0] = *p;
+            for (int i = 0; i < N; ++i) {
+                const int h = h0 + kh, w = w0 + kw;
+                in[i] = h >= 0 && h < H && w >= 0 && w < W;
+                const float* p = img + ((size_t)min(max(h, 0), H - 1) * W + min(max(w, 0), W - 1)) * C;
+                if (VEC == 4) {
+                    const float4 q = *reinterpret_cast<const float4*>(p);
+                    val[i][0] = q.x; val[i][1] = q.y; val[i][2] = q.z; val[i][3] = q.w;
+                } else {
+                    val[i][0] = *p;
+                }
+                if (++kw == Kw) { kw = 0; ++kh; }
             }
-            if (p0 + i + 1 < total && ++kw == Kw) { kw = 0; ++kh; }
+#pragma unroll
+            for (int i = 0; i < N; ++i)
+#pragma unroll
+                for (int v = 0; v < VEC; ++v) {
+                    const float now = in[i] ? val[i][v] : pad_value;
+                    if (now < best[v]) { best[v] = now; where[v] = p0 + i; }
+                }
         }
-#pragma unroll
-        for (int i = 0; i < BATCH; ++i)
-#pragma unroll
-            for (int v = 0; v < VEC; ++v) {
-                const float now = in[i] ? val[i][v] : pad_value;
-                if (now < best[v]) { best[v] = now; where[v] = min(p0 + i, total - 1); }
-            }
-    }
+    };
+    positions(std::integral_constant<int, BATCH>{});
+    if constexpr (BATCH > 4) positions(std::integral_constant<int, 4>{});
+    positions(std::integral_constant<int, 1>{});
     const size_t t = (size_t)row * Nw * C + e;
     if (VEC == 4) {
         *reinterpret_cast<float4*>(y + t) = make_float4(best[0], best[1], best[2], best[3]);
@@ -237,7 +246,7 @@ int launch_min_pool_forward(const float* x, float* y, int32_t* arg, const PoolGe
     if (grid.y > 65535u) return fail(SNNTC_ERR_TOO_LARGE, "pooling: output row of %lld elements too long", (long long)per_row);
     {
         KernelTimerScope timer_("min_pool", stream);
-        auto kern = g.Kh * g.Kw <= 4 ? (vec ? min_pool_forward_kernel<4, 4> : min_pool_forward_kernel<1, 4>)
+        auto kern = g.Kh * g.Kw < 9 ? (vec ? min_pool_forward_kernel<4, 4> : min_pool_forward_kernel<1, 4>)
                                      : (vec ? min_pool_forward_kernel<4, 9> : min_pool_forward_kernel<1, 9>);
         hipLaunchKernelGGL(kern, grid, dim3(256), 0, stream, x, y, arg, (int)g.H, (int)g.W, (int)g.C, (int)g.Kh,
                            (int)g.Kw, (int)g.Sh, (int)g.Sw, (int)g.pad_top, (int)g.pad_left, (int)g.Nh, (int)g.Nw,
