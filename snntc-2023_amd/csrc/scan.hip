@@ -14,8 +14,9 @@
 //   scan_lds_split_kernel  fewer work items than CUs: one item per workgroup, its weights gathered
 //                          into LDS in scan order first, then one wavefront accumulating and the
 //                          others sharing the item's tests;
-//   scan_kernel            segments so long that not even eight weight columns fit in LDS: weight
-//                          rows streamed from memory, one wavefront per (segment, 64 neurons).
+//   scan_kernel            segments so long that not even eight weight columns fit in LDS, and small launches of
+//                          segments of less than a chunk: weight rows streamed from memory, one wavefront
+//                          per (segment, 64 neurons).
 // In all of them lanes run across neurons, so a weight row is read coalesced (or conflict-free from
 // LDS), while the sorted value and the row index of a step are the same for all lanes of a segment
 // (segment rows are padded to a multiple of 16 entries so that they are fetched eight at a time
@@ -1335,7 +1336,7 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
                 }
                 if constexpr (LONE) {
                     // Half h (four inputs) is worked on while the weights of the next three are on their way.
-                    constexpr int NH = 4, HALVES = 2 * PHASES;
+                    constexpr int NH = 4;
                     float wv[NH][CH][4];                    // [half buffer][scan][input]
                     float run_w[CH], run_y[CH], end_w_of[CH], end_y_of[CH];
                     uint64_t pass[CH];
@@ -1931,6 +1932,16 @@ bool scan_sorts_rows(int64_t S, int64_t I, int64_t stride, int64_t J, const Neur
     return cols != 0 && split_sorts(cols) && takes_split(cols, S, I, stride, J, np, cus);
 }
 
+// Rows of less than a chunk, few enough that a wavefront per 64 neurons that reads its weights from memory is through sooner than
+// a workgroup that copies a slice for them and sets the filter's loop up for nothing.  us, slices / memory: 4000 rows of 1 to
+// 61 / 261 neurons 8.0 / 13.3 -> 6.3 / 10.1, 17 472 rows of 1 / 2 / 3 / 5 to 61 12.8 / 13.1 / 13.7 / 14.4 -> 9.8 / 11.0 / 12.2 / 14.0,
+// of 1 to 261 27.9 -> 25.8; on the other side 17 472 of 2 / 5 to 128 14.5 / 17.0 -> 16.0 / 21.2, of 1 to 16 7.8 -> 8.8, where a wavefront
+// of the other kernel holds several rows.
+static bool takes_stream(int64_t S, int64_t I, int64_t J) {
+    const int64_t waves = S * ((J + kWave - 1) / kWave);
+    return I < CHUNK && (J > kWave / 2 ? waves * I <= (I == 1 ? 98304 : 53248) : waves <= 4096);
+}
+
 template <int COLS>
 int launch_scan_lds(const float* sorted, const int32_t* perm, const int32_t* n_real, const float* w, float* y,
                     float* rcp, int32_t* causal_k, int64_t S, int64_t I, int64_t stride, int64_t J,
@@ -1995,7 +2006,7 @@ int launch_scan(const float* sorted, const int32_t* perm, const int32_t* n_real,
     if (prep) return prep;
     const int cols = slice_columns(S, I, stride, J, np, cus);            // none: W is streamed from memory
     const size_t lds_bytes = ((size_t)I + np.bias) * cols * sizeof(float);
-    if (cols) {
+    if (cols && !takes_stream(S, I, J)) {
         switch (cols) {
             case 64: return launch_scan_lds<64>(sorted, perm, n_real, w, y, rcp, causal_k, S, I, stride, J, np, copy, lds_bytes, cus, stream);
             case 32: return launch_scan_lds<32>(sorted, perm, n_real, w, y, rcp, causal_k, S, I, stride, J, np, copy, lds_bytes, cus, stream);

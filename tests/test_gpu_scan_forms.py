@@ -54,6 +54,17 @@ def test_scan_forms(B, I, J, law):
     _check(x, w, p)
 
 
+@pytest.mark.parametrize("B,I,J", [(13312, 4, 64), (13313, 4, 64), (7606, 7, 40), (700, 7, 261), (1000, 6, 33), (4096, 3, 32), (4097, 3, 32), (5, 2, 10),
+                                   (49152, 1, 70), (49153, 1, 70), (1, 1, 1)])
+@pytest.mark.parametrize("bias", [True, False])
+def test_scans_of_less_than_a_chunk(B, I, J, bias):
+    """Both sides of the line between weights in LDS and weights from memory; some rows silent in part or as a whole."""
+    x, w, p, _ = dense_case(B + I + J, B, I, J, bias, "baseline")
+    x[np.random.default_rng(I).random(x.shape) < 0.1] = 1e5
+    x[::7] = 2e5
+    _check(x, w, p)
+
+
 # Launches that leave a SIMD a wavefront or two: rounds of twelve chunks (rows of sixteen lanes) and of eight (quads)
 LONE_SIZES = [
     (700, 7, 64), (700, 95, 64), (700, 96, 64), (700, 97, 64), (700, 201, 63),          # 64-column slices, one neuron per lane
