@@ -21,6 +21,7 @@
 // LDS), while the sorted value and the row index of a step are the same for all lanes of a segment
 // (segment rows are padded to a multiple of 16 entries so that they are fetched eight at a time
 // without bounds checks).
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 #include <utility>
@@ -1807,8 +1808,12 @@ constexpr int FILTER_MAX_CH = COLS == 8 ? 2 : 4;
 // 25 000 rows of 5 to 379 neurons 67 / 55 / 53.
 template <int COLS>
 int filter_neurons(int64_t S, int64_t I, int n_slices, int cus) {
-    static const int wide[3][4] = {{14, 19, 22, 32}, {20, 29, 35, 53}, {38, 52, 62, 77}};
-    static const int narrow[2][4] = {{14, 19, 22, 32}, {25, 33, 46, 58}};                         // eight-column slices
+    constexpr bool full = COLS == 64;
+    // (up to 4, 8, 12 and 16 wavefronts, then per 16; 64 columns: one neuron for thirteen to sixteen wavefronts of rows of middling length:
+    // 1024 rows of 256 to 130 / 250 neurons 20.9 / 21.4 against 25.5 / 25.2 us, of 39 to 130 12.1 against 11.6, of 576 36.1 against 34.0)
+    const int wide[3][5] = {{14, 19, 22, full && I >= 64 && I < 360 ? 29 : 32, 32},
+                            {20, 29, full ? 34 : 35, full ? 51 : 53, 53}, {38, COLS == 32 ? 54 : 52, 62, 77, 77}};
+    static const int narrow[2][5] = {{14, 19, 22, 32, 32}, {25, 33, 46, 58, 58}};                 // eight-column slices
     static const int fixed_chunks[3] = {6, 7, 9};
     // A single slice of 8 or 16 columns: rows come from HBM once, and quads hold too few bytes in flight for that (262 144
     // patches of 144 to 16 neurons 134 / 147 / 174 us).
@@ -1820,27 +1825,34 @@ int filter_neurons(int64_t S, int64_t I, int n_slices, int cus) {
         const int64_t groups = n_slices < cus ? cus / n_slices : 1;                               // workgroups per slice
         const int64_t per_group = ((S + segs - 1) / segs + groups - 1) / groups;                  // items of the fullest
         const int* chunk_time = COLS == 8 ? narrow[k % 2] : wide[k];
-        const int64_t t = (per_group < 16 ? 16 * chunk_time[(per_group + 3) / 4 - 1] : per_group * chunk_time[3]) * (I / CHUNK + fixed_chunks[k]);
+        const int64_t t = (per_group <= 16 ? 16 * chunk_time[(per_group + 3) / 4 - 1] : per_group * chunk_time[4]) * (I / CHUNK + fixed_chunks[k]);
         if (t < best_time) { best_time = t; best = ch; }
     }
     return best;
 }
-// Eight-column slices of rows shorter than this keep the loop of the full chip with one neuron per lane too: the other one
-// requests eight chunks ahead there, which such rows do not have (401 408 rows of 75 to 8 neurons 90 against 100 us).
-constexpr int FILTER_LONE_FROM = 128;
+// Which loop a launch with less than the most neurons per lane takes.  One neuron: short rows stay with the loop of the full chip --
+// below a block of four chunks the other one's set-up is all it adds (512 rows of 8 / 27 to 64 neurons 6.6 against 6.8 us, 200 of 8
+// to 1000 8.2 against 8.5); eight-column slices below 128 inputs, since it requests eight chunks ahead there, which such rows do not
+// have (401 408 rows of 75 to 8 neurons 90 against 100).  Two neurons and 64 columns: nine to sixteen wavefronts hide what the
+// lone loop saves (1536 rows of 150 to 130 neurons 18.2 against 19.8 us, 400 to 800 17.2 against 18.4; of 576 42.7 and 41.3), fewer do not (1024 of
+// 576 to 130 7 % slower), nor do turns (333 of 39 to 1500 14 % slower, 700 of 576 to 800 11 %).
+template <int COLS>
+constexpr bool filter_lone(int ch, int64_t per_group, int64_t I) {
+    if (ch == 1) return I >= (COLS == 8 ? 128 : 4 * CHUNK);
+    return ch < FILTER_MAX_CH<COLS> && (COLS != 64 || per_group <= 8 || per_group > 16);
+}
 constexpr size_t FILTER_WIDE_COPY_BYTES = 48 * 1024;        // slices from here on are copied by 16 wavefronts
 
 // The instantiation for ch neurons per lane.
 template <int COLS, bool WANT_K>
 decltype(&scan_filter_kernel<COLS, 1, true, WANT_K>) filter_kernel(int ch, bool lone) {
-    if (ch == 1) {
-        if constexpr (COLS == 8) {
-            if (!lone) return scan_filter_kernel<COLS, 1, false, WANT_K>;
-        }
-        return scan_filter_kernel<COLS, 1, true, WANT_K>;
-    }
+    if (ch == 1) return lone ? scan_filter_kernel<COLS, 1, true, WANT_K> : scan_filter_kernel<COLS, 1, false, WANT_K>;
     if constexpr (COLS == 8) return scan_filter_kernel<COLS, 2, false, WANT_K>;
-    else return ch == 2 ? scan_filter_kernel<COLS, 2, true, WANT_K> : scan_filter_kernel<COLS, 4, false, WANT_K>;
+    else if (ch == 4) return scan_filter_kernel<COLS, 4, false, WANT_K>;
+    if constexpr (COLS == 64) {
+        if (!lone) return scan_filter_kernel<COLS, 2, false, WANT_K>;
+    }
+    return scan_filter_kernel<COLS, COLS == 8 ? 1 : 2, true, WANT_K>;
 }
 
 template <int COLS>
@@ -1852,6 +1864,8 @@ int raise_scan_lds_limits() {
         reinterpret_cast<const void*>(filter_kernel<COLS, false>(1, false)),
         reinterpret_cast<const void*>(filter_kernel<COLS, true>(2, true)),
         reinterpret_cast<const void*>(filter_kernel<COLS, false>(2, true)),
+        reinterpret_cast<const void*>(filter_kernel<COLS, true>(2, false)),
+        reinterpret_cast<const void*>(filter_kernel<COLS, false>(2, false)),
         reinterpret_cast<const void*>(filter_kernel<COLS, true>(FILTER_MAX_CH<COLS>, false)),
         reinterpret_cast<const void*>(filter_kernel<COLS, false>(FILTER_MAX_CH<COLS>, false))};
     for (const void* k : whole)
@@ -1973,18 +1987,19 @@ int launch_scan_lds(const float* sorted, const int32_t* perm, const int32_t* n_r
     const int64_t items = (S + segs - 1) / segs;
     // One workgroup per CU (its 16 wavefronts take all registers; small slices let two of up to eight share a CU),
     // and as many of them as there are items for: a CU that holds few wavefronts of its own copies the slice
-    // with a full workgroup all the same.
+    // with a full workgroup all the same.  (Wavefronts by the items of a group: by those of the chip, a slice count that does not divide
+    // it left a few items for a second turn, 512 rows of 333 to 1500 neurons 57.0 -> 49.4 us, 4096 to 130 58.7 -> 52.7.)
     const int64_t per_cu = (items * n_slices + cus - 1) / cus;
     const bool shared = per_cu <= 8 && (lds_bytes + FILTER_RED_BYTES) * 2 <= (size_t)LDS_SCAN_BYTES;
     const int64_t capacity = (int64_t)cus * (shared ? 2 : 1);
-    const int64_t per_wg = (items * n_slices + capacity - 1) / capacity;
-    const int waves = (int)(per_wg >= 16 ? 16 : (per_wg + 3) / 4 * 4);
     int64_t n_groups = capacity / n_slices;
+    if (n_groups < 1) n_groups = 1;
+    const int64_t per_wg = (items + n_groups - 1) / n_groups;
+    const int waves = (int)(per_wg >= 16 ? 16 : (per_wg + 3) / 4 * 4);
     const int64_t max_groups = (items + waves - 1) / waves;
     if (n_groups > max_groups) n_groups = max_groups;
-    if (n_groups < 1) n_groups = 1;
     const int threads = lds_bytes > FILTER_WIDE_COPY_BYTES && !shared ? LDS_SCAN_THREADS : waves * kWave;
-    const bool lone = ch < FILTER_MAX_CH<COLS> && !(COLS == 8 && I < FILTER_LONE_FROM);
+    const bool lone = filter_lone<COLS>(ch, (items + std::max(cus / n_slices, 1) - 1) / std::max(cus / n_slices, 1), I);
     auto kern = causal_k ? filter_kernel<COLS, true>(ch, lone) : filter_kernel<COLS, false>(ch, lone);
     {
         KernelTimerScope timer_("scan", stream);
