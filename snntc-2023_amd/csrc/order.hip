@@ -1101,14 +1101,17 @@ size_t order_rows_lds(int64_t I, const OrderRowsForm& form) {
 //   512 x 4096     41.0 -> 24.3 / 25.4, 29.8 / 34.6 / 33.3, 32.6        4096 x 784     45.7 -> 21.9 / 25.4, 29.3 / 33.2 / 33.2, 30.5
 //   512 x 8192     69.0 -> 33.0 / 37.0, 47.7 / 56.4 / 54.3, 67.2        16 384 x 784    132 -> 60 / 72, 84 / 100 / 99, 90
 // A network's steps grow with the square of the length's logarithm, the ranking's do not; but up to 1024 inputs it waits for a
-// workgroup's latency until several share a CU (512 x 1024: 13.7 -> 12.0 / 12.9, 13.9 / 15.0 / 15.0, 14.5), and up to 512 the network
-// is one wavefront's, which a full chip hides (8192 x 512: 37.7 -> 29.3 / 33.8, 36.8 / 42.8 / 44.3, 40.9) and which rows that are read an input
-// at a time do not beat (5000 x 449: 30.2 -> 25.0 / 28.4, 28.5 / 31.4 / 32.3, 33.7).  The ranking stands where it is faster on all of these.
+// workgroup's latency until several share a CU (128 x 784: 8.8 -> 8.2 / 9.2, 9.8 / 10.3 / 10.7, 10.3; 300 x 785: 11.6 -> 10.4 / 11.1,
+// 12.0 / 12.7 / 12.8, 12.7; 512 x 1024: 13.7 -> 12.0 / 12.9, 13.9 / 15.0 / 15.0, 14.5), and up to 512 the network is one wavefront's,
+// which a full chip hides (8192 x 512: 37.7 -> 29.3 / 33.8, 36.8 / 42.8 / 44.3, 40.9) and which rows that are read an input
+// at a time hardly beat (5000 x 385: 28.9 -> 24.8 / 28.2, 27.9 / 29.7 / 31.7, 33.0; 5000 x 511: 33.4 -> 25.4 / 28.8, 28.6 / 32.3 / 33.1, 34.1;
+// in fours 2048 x 300: 13.7 -> 11.3 / 12.8, 14.4 / 13.4 / 14.7, 14.8).  Different values decide, and repeats may not cost more than those gain.
 // Rows with several values that repeat among others of their bucket go to a network after all, and are slower for it (a
 // background with most other values close to it: 4096 x 784 45 -> 41, 512 x 4096 41 -> 47, 16 x 1521 12.0 -> 14.4).
 bool order_rows_supported(int64_t S, int64_t I) {
     if (S <= 0 || I > ORDER_MAX_REGION) return false;
-    return I > 1024 || (I > 512 && S >= 1024) || (I >= 352 && I % 4 == 0 && S >= 3072 && S <= 6144);
+    if (I > 512) return I > 1024 || S >= 300;
+    return I % 4 == 0 ? I > 256 && S >= 2048 && S <= 6144 : I >= 448 && S >= 3072 && S <= 5120;
 }
 
 int launch_order_rows(const float* x, float* sorted, int32_t* perm, int32_t* n_real, int64_t S, int64_t I, int64_t stride,
