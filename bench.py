@@ -351,8 +351,21 @@ def roofline_for(name, flops, nbytes, avg_ms, launches_per_step):
             "traffic": None}
 
 
+def kernel_sources():
+    """Digest of the device sources, which ties counter readings to the kernels they were taken on."""
+    import hashlib
+    folder = os.path.join(ROOT, "snntc-2023_amd", "csrc")
+    digest = hashlib.sha256()
+    for name in sorted(os.listdir(folder)):
+        if name.endswith((".hip", ".h")):
+            with open(os.path.join(folder, name), "rb") as f:
+                digest.update(name.encode() + f.read())
+    return digest.hexdigest()[:12]
+
+
 def carried_counters(workload_key, kernel):
-    """Counter readings for (workload, kernel) from profiles/counters.json, or {}."""
+    """Counter readings for (workload, kernel) from profiles/counters.json, or {}; their source says so where they were taken
+    on other device sources than those of this tree."""
     try:
         with open(COUNTERS_FILE) as f:
             table = json.load(f)
@@ -363,6 +376,8 @@ def carried_counters(workload_key, kernel):
         entry["valu_busy"] = min(1.0, entry["valu_busy"])
     if entry:
         entry["source"] = f"profiles/counters.json at commit {table.get('commit', '?')}"
+        if table.get("sources") != kernel_sources():
+            entry["source"] += " (other kernels than these)"
     return entry
 
 

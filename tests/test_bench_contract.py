@@ -34,6 +34,18 @@ def test_carried_counters_name_their_source():
     assert bench.carried_counters("cfg3", "no_such_kernel") == {}
 
 
+def test_counters_of_other_kernels_say_so(tmp_path, monkeypatch):
+    sys.path.insert(0, ROOT)
+    import json
+    import bench
+    table = {"commit": "0123456", "sources": bench.kernel_sources(), "workloads": {"cfg3": {"scan": {"valu_busy": 0.5}}}}
+    monkeypatch.setattr(bench, "COUNTERS_FILE", str(tmp_path / "counters.json"))
+    (tmp_path / "counters.json").write_text(json.dumps(table))
+    assert bench.carried_counters("cfg3", "scan")["source"] == "profiles/counters.json at commit 0123456"
+    (tmp_path / "counters.json").write_text(json.dumps({**table, "sources": "0" * 12}))
+    assert "other kernels" in bench.carried_counters("cfg3", "scan")["source"]
+
+
 def test_roofline_picks_the_binding_side():
     sys.path.insert(0, ROOT)
     import bench
