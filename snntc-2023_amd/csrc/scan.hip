@@ -896,7 +896,7 @@ __device__ __forceinline__ void read_columns(__attribute__((address_space(3))) c
 //
 // CH (1, 2 or 4) adjacent neurons per lane: one row address, one input time and one 4-, 8- or 16-byte LDS read
 // serve CH scans, and a wavefront covers 64*CH/COLS segments.  Two loops:
-//   * the full chip (four neurons per lane; two with eight-column slices): what bounds it is vector issue (120
+//   * the full chip (four neurons per lane; two with eight-column slices): what bounds it is vector issue (117
 //     instructions per chunk of 4 x 64 neurons) and, under it, the power limit: the same instruction stream runs
 //     16 % slower on random weights than on zeros.  3x3 patches of 64 channels to 64 neurons, 65 536 segments: 310 -> 238 us;
 //     128 -> 128 channels on 28x28, 32 images: 472 -> 416; 256 -> 256 on 14x14: 555 -> 440; dense 784 -> 800 at 4096 rows: 379 -> 302,
@@ -924,7 +924,8 @@ __device__ __forceinline__ void read_columns(__attribute__((address_space(3))) c
 // bound itself; sums inside the chunk differ from the final ones by at most seven inputs).  Every t_u then
 // exceeds thr, which is the condition above.  With weight sums that stay above 4W the bound is t_7 itself;
 // below, a chunk may fail although none of its inputs closes the set, by (x_7 - x_0)*4W at most.
-// Two additions per input and seven instructions per chunk and neuron.
+// Two additions per input and seven vector instructions per chunk and neuron (two multiply-adds, a minimum, the compare and three
+// selects), five per chunk for the operands they share.
 //
 // That slack is small next to ysum - x*wsum, which starts at theta*x, where weights are small and the sum soon leaves zero;
 // under weights of a larger spread (the layers' own initialiser: mean 0, deviation sqrt(15 / inputs)) it stops most scans several
