@@ -1095,14 +1095,14 @@ size_t order_rows_lds(int64_t I, const OrderRowsForm& form) {
 
 // Dense rows: the sorting networks -> ranked, us between events, values all different (as they are / a tenth silent), then with repeats
 // (8-bit levels / mostly background / background and different values), then crowded in a tenth of an octave with outliers:
-//   16 x 1521      12.0 -> 8.7 / 9.4, 10.0 / 10.8 / 11.2, 11.0          3500 x 512     26.7 -> 17.0 / 19.8, 20.5 / 23.5 / 24.5, 22.6
+//   16 x 1521      11.9 -> 8.7 / 9.5, 10.0 / 10.8 / 11.2, 11.3          3500 x 512     26.7 -> 17.0 / 19.8, 20.5 / 23.5 / 24.5, 22.6
 //   256 x 2048     16.0 -> 12.3 / 13.1, 14.4 / 15.6 / 16.2, 14.8        5000 x 384     28.6 -> 20.6 / 23.7, 24.6 / 27.0 / 28.7, 27.7
-//   400 x 1521     20.2 -> 14.0 / 15.6, 17.0 / 18.4 / 18.4, 17.8        1024 x 784     17.2 -> 10.4 / 12.1, 12.8 / 14.6 / 15.5, 16.1
+//   400 x 1521     20.2 -> 14.0 / 15.6, 17.0 / 18.4 / 18.4, 17.8        1024 x 784     18.2 -> 13.5 / 14.4, 15.8 / 17.3 / 17.0, 16.3
 //   512 x 4096     41.0 -> 24.3 / 25.4, 29.8 / 34.6 / 33.3, 32.6        4096 x 784     45.7 -> 21.9 / 25.4, 29.3 / 33.2 / 33.2, 30.5
 //   512 x 8192     69.0 -> 33.0 / 37.0, 47.7 / 56.4 / 54.3, 67.2        16 384 x 784    132 -> 60 / 72, 84 / 100 / 99, 90
 // A network's steps grow with the square of the length's logarithm, the ranking's do not; but up to 1024 inputs it waits for a
-// workgroup's latency until several share a CU (128 x 784: 8.8 -> 8.2 / 9.2, 9.8 / 10.3 / 10.7, 10.3; 300 x 785: 11.6 -> 10.4 / 11.1,
-// 12.0 / 12.7 / 12.8, 12.7; 512 x 1024: 13.7 -> 12.0 / 12.9, 13.9 / 15.0 / 15.0, 14.5), and up to 512 the network is one wavefront's,
+// workgroup's latency until several share a CU (128 x 784: 8.8 -> 8.2 / 9.2, 9.8 / 10.3 / 10.7, 10.3; 300 x 785: 11.4 -> 10.2 / 11.2,
+// 11.9 / 12.7 / 12.7, 12.5; 512 x 1024: 13.7 -> 12.0 / 12.9, 13.9 / 15.0 / 15.0, 14.5), and up to 512 the network is one wavefront's,
 // which a full chip hides (8192 x 512: 37.7 -> 29.3 / 33.8, 36.8 / 42.8 / 44.3, 40.9) and which rows that are read an input
 // at a time hardly beat (5000 x 385: 28.9 -> 24.8 / 28.2, 27.9 / 29.7 / 31.7, 33.0; 5000 x 511: 33.4 -> 25.4 / 28.8, 28.6 / 32.3 / 33.1, 34.1;
 // in fours 2048 x 300: 13.7 -> 11.3 / 12.8, 14.4 / 13.4 / 14.7, 14.8).  Different values decide, and repeats may not cost more than those gain.
