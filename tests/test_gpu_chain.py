@@ -24,6 +24,7 @@ def t(a):
     (4, 2, 12, 12, 16, 8, 5, 1, "reftest"),        # 5x5 kernel, two pixels of padding: patch-space dX + col2im
     (5, 300, 8, 8, 32, 64, 3, 1, "baseline"),      # a launch large enough for the filtered scan
     (6, 2, 9, 70, 8, 16, 3, 1, "baseline"),        # eight channels, rows of two 64-pixel tiles
+    (7, 2, 9, 9, 5, 48, 1, 1, "baseline"),          # patches of less than a chunk: weights from memory
 ])
 def test_conv_ops_with_a_second_destination_and_a_gradient_window(seed, B, H, W, C, Kc, K, S, dist):
     import snntc_amd as snn
