@@ -150,6 +150,19 @@ constexpr int LDS_SCAN_BYTES = 160 * 1024;
 // The widest slice that fits is taken: the register budget allows one 16-wave workgroup per CU anyway,
 // and fewer slices re-read the sorted rows less often.
 constexpr int FILTER_RED_BYTES = 64;                       // behind the slice: one float per wavefront for a reduction
+constexpr int FILTER_STAGE_BYTES = 1024;                   // then, per wavefront, the row entries on their way to its lanes (STAGED)
+// Most neurons per lane: four; two with 8-column slices (the segments of a wavefront would be too many for its row entries).
+template <int COLS>
+constexpr int FILTER_MAX_CH = COLS == 8 ? 2 : 4;
+// STAGED: row entries reach the lanes of a segment through LDS instead of DPP broadcasts.  A vector instruction with a DPP operand
+// makes the plain ones around it issue at half their rate (probe kernels, four wavefronts per SIMD: multiply-adds alone 2.0 clocks
+// each, with one such move to four, sixteen, thirty-two or sixty-four of them 4.3, 3.8, 3.0 and 2.2 clocks an instruction), and an LDS read
+// costs about five plain instructions whatever its width: four reads per chunk in place of sixteen broadcasts.  us with
+// DPP / staged: 65 536 segments of 576 to 64 neurons 226 / 207, 100 352 329 / 299, 32 768 of 576 120 / 108.  Only with rows of 256 bytes: slices of 32,
+// 16 and 8 columns read their weights with bank conflicts, and four more reads make LDS the bound (4096 rows of 784
+// to 800 neurons 242 / 262, 6272 segments of 2304 to 256 365 / 405, 1568 of 4608 to 512 514 / 545).
+template <int COLS, int CH, bool LONE>
+constexpr bool filter_staged = COLS == 64 && CH == 4 && !LONE;
 constexpr int LDS_SCAN_TARGET = LDS_SCAN_BYTES - FILTER_RED_BYTES;
 
 struct Chunk {
@@ -961,6 +974,26 @@ constexpr float FILTER_END_W = 0x1p-15f;                  // 512u >= 36u + 310u,
 constexpr float FILTER_AT = 1.0f + 0x1p-18f;
 constexpr float FILTER_DX = 0x1p-16f;
 
+// The test of a round: the same bound over 32 inputs at a time.  None of 32 sums lies more than sixteen weights below both ends, so
+// with A = 16W - min(wsum_start, wsum_31, 16W) the scan passes if t' - dx' * A > 4096u * x_31 * W, t' evaluated at x_31 * (1 + 256u)
+// and dx' = x_31 - x_0 + 1024u * x_31.  What a test of the reference inside the round needs is (31 roundings of the two sums,
+// sixteen of a weight sum and six of the bound's own, sums that differ from the last ones by up to 31 inputs; compare thr above)
+//   T - dx * A > 57.6u * |ysum_31| + 53.6u * x_31 * |wsum_31| + 3665u * x_31 * W,   |ysum_31| <= T + x_31 * |wsum_31|;
+// the same two cases as above leave
+//   wsum_31 >= 0:  T - dx * A >= 500u * t' + 254u * x_31 * wsum_31 + 4090u * x_31 * W,
+//   wsum_31 < 0:   T - dx * A >= 500u * t' + 252u * x_31 * |wsum_31| + 4090u * x_31 * W.
+constexpr float ROUND_END_W = 0x1p-12f;                   // 4096u
+constexpr float ROUND_AT = 1.0f + 0x1p-16f;               // 1 + 256u
+constexpr float ROUND_DX = 0x1p-14f;                      // 1024u
+// A wavefront's scans are tested by rounds until the first of them comes close to its close, about half of a row where 64 ... 256 of
+// them share a wavefront (the first closes at 0.50 ... 0.57 of a row, the mean at 0.80): a round is 363 vector instructions
+// instead of 467.  us without / with: 4096 rows of 784 to 800 neurons 260 / 243, 25 088 segments of 1152 to 128 350 / 335, 6272 of 2304 to 256
+// 396 / 374, 65 536 of 576 to 64 (staged) 222 / 211; from 400 inputs on: 131 072 segments of 288 to 32 164 / 173, 32 768 of 288 to 64 64.7 / 67.1,
+// 2048 rows of 300 to 800 61.9 / 62.4, since a wavefront fills its pipeline a second time when it goes over to chunks.  16W * 32 / I is about
+// the slack of a round next to a threshold of one; beyond 0.6 of it rounds end early (576 inputs with deviation 3.87 / sqrt(I): at 0.15 of a row).
+constexpr float ROUNDS_UP_TO = 0.6f;
+constexpr int ROUNDS_FROM = 400;
+
 // The test of a chunk for one scan of every lane: wb, yb are the sums behind it.  Lanes in the mask `open`
 // that pass take them over; open lanes that fail keep the sums from before the chunk, take the chunk's
 // first index as kcur and leave `open`.  The arithmetic does not depend on EXEC or branches (lanes that
@@ -1195,7 +1228,7 @@ __device__ __forceinline__ void row_row_addresses(int even, int odd, unsigned ba
         : [e] "v"(even), [o] "v"(odd), [base] "v"(base), [n0] "n"(N), [n1] "n"(N + 1));
 }
 
-template <int COLS, int CH, bool LONE, bool WANT_K>
+template <int COLS, int CH, bool LONE, bool WANT_K, bool ROUNDS = false>
 __global__ void __launch_bounds__(LDS_SCAN_THREADS)
 scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__ perm,
                    const int32_t* __restrict__ n_real, const float* __restrict__ w, float* __restrict__ y_out,
@@ -1208,16 +1241,19 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
     // How a segment's (x, row) entries reach its lanes (see the fast loop): through rows of sixteen lanes where
     // a segment has at least that many, else through quads
     constexpr bool BY_ROW = LANES % 16 == 0;
+    constexpr bool STAGED = filter_staged<COLS, CH, LONE>;
     constexpr int ROUND = 4;                               // chunks per round of the fast loop
     const int block = xcd_contiguous(blockIdx.x, gridDim.x);
     const int slice = block / n_groups;
     const int group = block - slice * n_groups;
     const int j0 = slice * COLS;
-    const int rows = I + np.bias;
     // the slice, and the largest |w| in it (the threads' shares of the copy, then the workgroup's)
-    const float w_max = block_max(fill_weight_slice<COLS>(wl, w, rows, J, j0), wl + rows * COLS);
+    const float w_max = block_max(fill_weight_slice<COLS>(wl, w, I, J, j0), wl + I * COLS);
+    if constexpr (STAGED) __syncthreads();                  // (the room of the maximum is the rows' staging next)
     const float end_w = FILTER_END_W * w_max;               // margin of the fast loop
     const float w4 = 4.0f * 1.00001f * w_max;               // 4W of its bound on the weight sums
+    const float end_w_round = ROUND_END_W * w_max;
+    const bool by_rounds = __builtin_amdgcn_readfirstlane(w_max * 512.0f <= ROUNDS_UP_TO * np.theta * (float)I);
     const bool single = (S + SEGS - 1) / SEGS <= n_groups * waves;      // a wavefront has one item
     const bool tight = __builtin_amdgcn_readfirstlane(w_max > (single ? TIGHT_FROM_SINGLE : TIGHT_FROM) * np.theta);
 
@@ -1264,7 +1300,8 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
         // held: rows: block b holds the round b rounds ahead of the current one; quads: a ring of chunks.
         // The first entries are requested here, next to the two loads above and before anything waits for
         // them: practically every item starts its first pass at input 0.
-        constexpr int BLOCKS = BY_ROW ? (LONE ? 3 : 2) : LONE ? 2 * ROUND : ROUND;
+        static_assert(!STAGED || (LANES == 16 && ROUND * CHUNK == 2 * LANES), "a block is a round");
+        constexpr int BLOCKS = STAGED ? 1 : BY_ROW ? (LONE ? 3 : 2) : LONE ? 2 * ROUND : ROUND;
         constexpr int PHASES = BY_ROW ? ROUND * BLOCKS : BLOCKS;     // chunks held (the loop for one and two neurons per lane)
         constexpr int BLOCK_INPUTS = BY_ROW ? ROUND * CHUNK : CHUNK;
         u32x2 rx[BLOCKS], rp[BLOCKS];
@@ -1276,13 +1313,16 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
         const int last_block = stride - CHUNK;
         auto request_first = [&](int k) {
 #pragma unroll
-            for (int b = 0; b < BLOCKS - (LONE ? 0 : 1); ++b) request(b, LONE ? min(k + b * BLOCK_INPUTS, last_block) : k + b * BLOCK_INPUTS);
+            for (int b = 0; b < BLOCKS - (LONE || STAGED ? 0 : 1); ++b) request(b, LONE || STAGED ? min(k + b * BLOCK_INPUTS, last_block) : k + b * BLOCK_INPUTS);
         };
         request_first(0);
         const int n_full = n_seg & ~(CHUNK - 1);
-        int n_full_max = 0;                                 // of the longest of the wavefront's rows
+        int n_full_max = 0, n_full_min = NONE;              // of the longest and the shortest of the wavefront's rows
 #pragma unroll
-        for (int q = 0; q < SEGS; ++q) n_full_max = max(n_full_max, __builtin_amdgcn_readlane(n_full, q * LANES));
+        for (int q = 0; q < SEGS; ++q) {
+            n_full_max = max(n_full_max, __builtin_amdgcn_readlane(n_full, q * LANES));
+            n_full_min = min(n_full_min, __builtin_amdgcn_readlane(n_full, q * LANES));
+        }
 
         // Per scan: the running sums, the number of inputs they hold (kcur), and where it stands, as lane masks (in
         // scalar registers: per-lane flags cost four-neuron lanes the registers the fast loop needs)
@@ -1292,9 +1332,12 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
         //   fired    the fired state that goes with the sums
         float wsum[CH], ysum[CH];
         int kcur[CH];
-        uint64_t armed[CH], step[CH], fin[CH], fired[CH], any_armed = 0;
+        uint64_t armed[CH], step[CH], fin[CH], fired[CH], any_armed = 0, any_odd = 0;
         float wb[CH];
-        if (np.bias) read_columns<CH>(wcol + I * COLS, wb);
+        if (np.bias) {
+#pragma unroll
+            for (int c = 0; c < CH; ++c) wb[c] = j + c < J ? w[(size_t)I * J + j + c] : 0.0f;
+        }
 #pragma unroll
         for (int c = 0; c < CH; ++c) {
             const bool live = seg_raw < S && j + c < J;
@@ -1318,12 +1361,195 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
             armed[c] = ballot(live && n_full > 0 && plain);
             step[c] = ballot(live && n_full > 0 && !plain);
             any_armed |= armed[c];
+            any_odd |= step[c];
+        }
+        int kmin = any_armed != 0 ? 0 : NONE;               // every armed scan starts at input 0
+
+        // The loop of the full chip, in pieces.
+        //
+        // The weights of a chunk are read in two halves of four inputs.  Per half, with h the half
+        // being consumed: read the weights of half h + NH - 1, then run half h; NH = 2 keeps
+        // four-neuron lanes within the registers of a 16-wavefront workgroup, the others read
+        // a whole chunk ahead.  H counts halves from the start of the round.
+        constexpr int NH = CH == 4 || STAGED ? 2 : 4;
+        float wv[NH][CH][4];                        // [half buffer][scan][step]
+        // STAGED: the round's entries in quarters of a chunk, [quarter][segment][4], times and then row indices.  LDS serves a
+        // wavefront's requests in order: a round is written once all reads of the one before have been issued, and nothing has to wait.
+        // Per half, its times are read one half ahead and its row indices two.
+        constexpr int QUARTERS = BLOCK_INPUTS / 4;
+        constexpr int STAGE_ROWS = FILTER_STAGE_BYTES / 8;
+        float4 xh[2];
+        int4 half_rows;
+        float* const stage = wl + I * COLS + wave * (FILTER_STAGE_BYTES / 4);
+        float* const stage_in = stage + ((cg >> 1) * SEGS + sub) * 4 + (cg & 1) * 2;
+        float* const stage_out = stage + sub * 4;
+        auto stage_x = [&] {
+            *reinterpret_cast<float2*>(stage_in) = make_float2(__uint_as_float(rx[0].x), __uint_as_float(rx[0].y));
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        };
+        auto stage_rows = [&] {
+            *reinterpret_cast<int2*>(stage_in + STAGE_ROWS) = make_int2((int)rp[0].x, (int)rp[0].y);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        };
+        auto read_x = [&](int h) { xh[h % 2] = *reinterpret_cast<const float4*>(stage_out + h % QUARTERS * SEGS * 4); };
+        auto read_rows = [&](int h) { half_rows = *reinterpret_cast<const int4*>(stage_out + STAGE_ROWS + h % QUARTERS * SEGS * 4); };
+        auto read_weights = [&](int buf, const unsigned (&at)[4]) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                float wr[CH];
+                read_columns<CH>(reinterpret_cast<lds_cfloat*>((uintptr_t)at[u]), wr);
+#pragma unroll
+                for (int c = 0; c < CH; ++c) wv[buf][c][u] = wr[c];
+            }
+        };
+        auto weights = [&](auto h_c) {
+            constexpr int H = decltype(h_c)::value, P = H / 2, HH = H % 2;
+            unsigned at[4];
+            if constexpr (STAGED) {
+                const int r[4] = {half_rows.x, half_rows.y, half_rows.z, half_rows.w};
+#pragma unroll
+                for (int u = 0; u < 4; ++u) at[u] = ((unsigned)r[u] << ROW_SHIFT) + wbase;
+            } else if constexpr (BY_ROW) {
+                constexpr int b = P / ROUND;
+                row_row_addresses<(P % ROUND) * 4 + HH * 2>((int)rp[b].x << ROW_SHIFT, (int)rp[b].y << ROW_SHIFT, wbase, at);
+            } else {
+                constexpr int b = P % ROUND;
+                quad_row_addresses<HH>((int)rp[b].x << ROW_SHIFT, (int)rp[b].y << ROW_SHIFT, wbase, at);
+            }
+            read_weights(H % NH, at);
+        };
+        auto times = [&](auto h_c, float (&x)[4]) {
+            constexpr int H = decltype(h_c)::value, P = H / 2, HH = H % 2;
+            if constexpr (STAGED) {
+                const float4 v = xh[H % 2];
+                x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w;
+            } else if constexpr (BY_ROW) {
+                constexpr int N = P * 4 + HH * 2;
+                const float xe = __uint_as_float(rx[0].x), xo = __uint_as_float(rx[0].y);
+                x[0] = row_broadcast<N>(xe); x[1] = row_broadcast<N>(xo);
+                x[2] = row_broadcast<N + 1>(xe); x[3] = row_broadcast<N + 1>(xo);
+            } else {
+                const float xe = __uint_as_float(rx[P].x), xo = __uint_as_float(rx[P].y);
+                x[0] = quad_broadcast<2 * HH>(xe); x[1] = quad_broadcast<2 * HH>(xo);
+                x[2] = quad_broadcast<2 * HH + 1>(xe); x[3] = quad_broadcast<2 * HH + 1>(xo);
+            }
+        };
+        // The first weights, and what the loop expects under way, for a pass that starts at input k (its first entries are in rx, rp).
+        auto start_weights = [&](int k) {
+            if constexpr (STAGED) {
+                stage_rows();
+                stage_x();
+                request(0, min(k + BLOCK_INPUTS, last_block));
+                read_rows(0);
+                weights(std::integral_constant<int, 0>{});
+                read_rows(1);
+                read_x(0);
+            } else {
+                weights(std::integral_constant<int, 0>{});
+                if constexpr (NH == 4) {
+                    weights(std::integral_constant<int, 1>{});
+                    weights(std::integral_constant<int, 2>{});
+                }
+            }
+        };
+        // One chunk: wb / yb are the scans' sums behind its inputs.  The requests stay ahead of the
+        // arithmetic: what a half consumes was requested a half or more ago, and what it requests has the
+        // whole half to arrive.
+        float yb[CH], low[CH], x0, x7;
+        auto chunk = [&](auto ph_c, int k, auto by_round_c) {
+            constexpr int ph = decltype(ph_c)::value;
+            constexpr bool BY_ROUND = decltype(by_round_c)::value;
+            if constexpr (!BY_ROW && !STAGED) request((ph + ROUND - 1) % ROUND, k + (ROUND - 1) * CHUNK);
+            auto half = [&](auto half_c) {
+                constexpr int hh = decltype(half_c)::value, H = 2 * ph + hh;
+                weights(std::integral_constant<int, H + NH - 1>{});
+                if constexpr (STAGED) {
+                    if constexpr ((H + 2) % QUARTERS == 0) stage_rows();
+                    read_rows(H + 2);
+                    if constexpr ((H + 1) % QUARTERS == 0) {
+                        stage_x();
+                        request(0, min(k - ph * CHUNK + 2 * BLOCK_INPUTS, last_block));
+                    }
+                    read_x(H + 1);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                float x[4];
+                times(std::integral_constant<int, H>{}, x);
+                if (hh == 0) x0 = x[0];
+                else x7 = x[3];
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+#pragma unroll
+                    for (int c = 0; c < CH; ++c) {
+                        const float wc = wv[H % NH][c][u];
+                        const bool start = hh == 0 && u == 0 && (ph == 0 || !BY_ROUND);
+                        const float before = wb[c];
+                        wb[c] = (start ? wsum[c] : wb[c]) + wc;
+                        yb[c] = __fmaf_rn(x[u], wc, start ? ysum[c] : yb[c]);
+                        if (TIGHT && !BY_ROUND && u % 2 == 1) low[c] = fminf(fminf(hh == 0 && u == 1 ? 0.0f : low[c], before), wb[c]);
+                    }
+            };
+            half(std::integral_constant<int, 0>{});
+            half(std::integral_constant<int, 1>{});
+        };
+        // rows: the next round's block moves up, the one after it is requested
+        auto next_round = [&] {
+            if constexpr (BY_ROW && !STAGED) {
+#pragma unroll
+                for (int b = 0; b + 1 < BLOCKS; ++b) { rx[b] = rx[b + 1]; rp[b] = rp[b + 1]; }
+            }
+        };
+        auto start_round = [&](int k0) {
+            if constexpr (BY_ROW && !STAGED) request(BLOCKS - 1, k0 + (BLOCKS - 1) * BLOCK_INPUTS);
+        };
+        // By rounds of four chunks with one test, until the first scan of the wavefront comes close: all scans take a round over
+        // together.  (Lanes without a scan compute along.)
+        if constexpr (ROUNDS) {
+            if (by_rounds && any_odd == 0 && n_full_min >= ROUND * CHUNK) {
+                start_weights(0);
+                int k0 = 0;
+                bool more = true;
+                while (more && k0 + ROUND * CHUNK <= n_full_min) {
+                    rotate_wave_priority(k0 / (ROUND * CHUNK) + (wave >> 2));
+                    start_round(k0);
+                    float x_first;
+                    for_each_phase<ROUND>([&](auto ph_c) {
+                        chunk(ph_c, k0 + decltype(ph_c)::value * CHUNK, std::true_type{});
+                        if (decltype(ph_c)::value == 0) x_first = x0;
+                        return true;
+                    });
+                    const float dx = __fmaf_rn(x7, ROUND_DX, x7 - x_first), x7e = x7 * ROUND_AT;
+                    const float thr = __fmaf_rn(dx, 4.0f * w4, x7 * end_w_round);
+                    float at_end[CH], lowest[CH];
+                    uint64_t soon = 0;                      // not even with the fall that a round like this one brings
+#pragma unroll
+                    for (int c = 0; c < CH; ++c) {
+                        at_end[c] = __fmaf_rn(-x7e, wb[c], yb[c]);
+                        lowest[c] = fminf(fminf(wsum[c], wb[c]), 4.0f * w4);
+                        soon |= armed[c] & ~ballot(__fmaf_rn(dx, lowest[c] - fabsf(wb[c]), at_end[c]) > thr);
+                    }
+                    more = soon == 0;
+                    if (!more) {
+                        uint64_t fails = 0;
+#pragma unroll
+                        for (int c = 0; c < CH; ++c) fails |= armed[c] & ~ballot(__fmaf_rn(dx, lowest[c], at_end[c]) > thr);
+                        if (fails != 0) break;              // (the round again, chunk by chunk)
+                    }
+#pragma unroll
+                    for (int c = 0; c < CH; ++c) { wsum[c] = wb[c]; ysum[c] = yb[c]; }
+                    next_round();
+                    k0 += ROUND * CHUNK;
+                }
+                kmin = k0;
+#pragma unroll
+                for (int c = 0; c < CH; ++c) kcur[c] = k0;
+                request_first(kmin);
+            }
         }
 
         // Passes: the fast loop for the armed scans that are furthest behind, then the scans it left behind
         // step by step.  A scan that does not close there is armed again.
         // Practically every item takes one pass and a second look without work.
-        int kmin = any_armed != 0 ? 0 : NONE;               // every armed scan starts at input 0
         for (;;) {
             uint64_t ran[CH];                               // the scans that take part in this pass's fast loop
 #pragma unroll
@@ -1461,88 +1687,7 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
 #pragma unroll
                     for (int c = 0; c < CH; ++c) kcur[c] = in_mask(ran[c]) ? kmin + (int)passed[c] * CHUNK : kcur[c];
                 } else {
-                // The weights of a chunk are read in two halves of four inputs.  Per half, with h the half
-                // being consumed: read the weights of half h + NH - 1, then run half h; NH = 2 keeps
-                // four-neuron lanes within the registers of a 16-wavefront workgroup, the others read
-                // a whole chunk ahead.  H counts halves from the start of the round.
-                constexpr int NH = CH == 4 ? 2 : 4;
-                float wv[NH][CH][4];                        // [half buffer][scan][step]
-                auto weights = [&](auto h_c) {
-                    constexpr int H = decltype(h_c)::value, P = H / 2, HH = H % 2;
-                    unsigned at[4];
-                    if constexpr (BY_ROW) {
-                        constexpr int b = P / ROUND;
-                        row_row_addresses<(P % ROUND) * 4 + HH * 2>((int)rp[b].x << ROW_SHIFT, (int)rp[b].y << ROW_SHIFT, wbase, at);
-                    } else {
-                        constexpr int b = P % ROUND;
-                        quad_row_addresses<HH>((int)rp[b].x << ROW_SHIFT, (int)rp[b].y << ROW_SHIFT, wbase, at);
-                    }
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        float wr[CH];
-                        read_columns<CH>(reinterpret_cast<lds_cfloat*>((uintptr_t)at[u]), wr);
-#pragma unroll
-                        for (int c = 0; c < CH; ++c) wv[H % NH][c][u] = wr[c];
-                    }
-                };
-                auto times = [&](auto h_c, float (&x)[4]) {
-                    constexpr int H = decltype(h_c)::value, P = H / 2, HH = H % 2;
-                    if constexpr (BY_ROW) {
-                        constexpr int N = P * 4 + HH * 2;
-                        const float xe = __uint_as_float(rx[0].x), xo = __uint_as_float(rx[0].y);
-                        x[0] = row_broadcast<N>(xe); x[1] = row_broadcast<N>(xo);
-                        x[2] = row_broadcast<N + 1>(xe); x[3] = row_broadcast<N + 1>(xo);
-                    } else {
-                        const float xe = __uint_as_float(rx[P].x), xo = __uint_as_float(rx[P].y);
-                        x[0] = quad_broadcast<2 * HH>(xe); x[1] = quad_broadcast<2 * HH>(xo);
-                        x[2] = quad_broadcast<2 * HH + 1>(xe); x[3] = quad_broadcast<2 * HH + 1>(xo);
-                    }
-                };
-                weights(std::integral_constant<int, 0>{});
-                if constexpr (NH == 4) {
-                    weights(std::integral_constant<int, 1>{});
-                    weights(std::integral_constant<int, 2>{});
-                }
-                // One chunk: wb / yb are the scans' sums behind its inputs.  The requests stay ahead of the
-                // arithmetic: what a half consumes was requested a half or more ago, and what it requests has the
-                // whole half to arrive.
-                float yb[CH], low[CH], x0, x7;
-                auto chunk = [&](auto ph_c, int k) {
-                    constexpr int ph = decltype(ph_c)::value;
-                    if constexpr (!BY_ROW) request((ph + ROUND - 1) % ROUND, k + (ROUND - 1) * CHUNK);
-                    auto half = [&](auto half_c) {
-                        constexpr int hh = decltype(half_c)::value, H = 2 * ph + hh;
-                        weights(std::integral_constant<int, H + NH - 1>{});
-                        __builtin_amdgcn_sched_barrier(0);
-                        float x[4];
-                        times(std::integral_constant<int, H>{}, x);
-                        if (hh == 0) x0 = x[0];
-                        else x7 = x[3];
-#pragma unroll
-                        for (int u = 0; u < 4; ++u)
-#pragma unroll
-                            for (int c = 0; c < CH; ++c) {
-                                const float wc = wv[H % NH][c][u];
-                                const bool start = hh == 0 && u == 0;
-                                const float before = wb[c];
-                                wb[c] = (start ? wsum[c] : wb[c]) + wc;
-                                yb[c] = __fmaf_rn(x[u], wc, start ? ysum[c] : yb[c]);
-                                if (TIGHT && u % 2 == 1) low[c] = fminf(fminf(hh == 0 && u == 1 ? 0.0f : low[c], before), wb[c]);
-                            }
-                    };
-                    half(std::integral_constant<int, 0>{});
-                    half(std::integral_constant<int, 1>{});
-                };
-                // rows: the next round's block moves up, the one after it is requested
-                auto next_round = [&] {
-                    if constexpr (BY_ROW) {
-#pragma unroll
-                        for (int b = 0; b + 1 < BLOCKS; ++b) { rx[b] = rx[b + 1]; rp[b] = rp[b + 1]; }
-                    }
-                };
-                auto start_round = [&](int k0) {
-                    if constexpr (BY_ROW) request(BLOCKS - 1, k0 + (BLOCKS - 1) * BLOCK_INPUTS);
-                };
+                start_weights(kmin);
                 auto test = [&](int k) {
                     const float dx = __fmaf_rn(x7, FILTER_DX, x7 - x0), x7e = x7 * FILTER_AT;
                     const float thr = TIGHT ? x7 * end_w : __fmaf_rn(dx, w4, x7 * end_w);
@@ -1573,7 +1718,7 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
                     for_each_phase<ROUND>([&](auto ph_c) {
                         const int k = k0 + decltype(ph_c)::value * CHUNK;
                         inside(k);
-                        chunk(ph_c, k);
+                        chunk(ph_c, k, std::false_type{});
                         test(k);
                         return true;
                     });
@@ -1584,7 +1729,7 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
                     for_each_phase<ROUND>([&](auto ph_c) {
                         const int k = k0 + decltype(ph_c)::value * CHUNK;
                         if (!inside(k)) return false;
-                        chunk(ph_c, k);
+                        chunk(ph_c, k, std::false_type{});
                         test(k);
                         return true;
                     });
@@ -1794,11 +1939,6 @@ unpad_rows_kernel(const float* __restrict__ sorted, const int32_t* __restrict__ 
 }  // namespace
 
 namespace {
-// Neurons per lane of the instantiations: one, two or four; two at most with 8-column slices (a quad of lanes has
-// to stay within one segment).
-template <int COLS>
-constexpr int FILTER_MAX_CH = COLS == 8 ? 2 : 4;
-
 // How many of them a launch of S segments of I inputs uses: the form with the smallest estimated time.  A SIMD
 // works on its wavefronts four at a time; the time of a chunk with w of them at work and the fixed share of an
 // item (first requests, evaluation of the closing chunks, leftover inputs, output) in chunks are measured
@@ -1846,10 +1986,10 @@ constexpr size_t FILTER_WIDE_COPY_BYTES = 48 * 1024;        // slices from here 
 
 // The instantiation for ch neurons per lane.
 template <int COLS, bool WANT_K>
-decltype(&scan_filter_kernel<COLS, 1, true, WANT_K>) filter_kernel(int ch, bool lone) {
+decltype(&scan_filter_kernel<COLS, 1, true, WANT_K>) filter_kernel(int ch, bool lone, bool rounds) {
     if (ch == 1) return lone ? scan_filter_kernel<COLS, 1, true, WANT_K> : scan_filter_kernel<COLS, 1, false, WANT_K>;
-    if constexpr (COLS == 8) return scan_filter_kernel<COLS, 2, false, WANT_K>;
-    else if (ch == 4) return scan_filter_kernel<COLS, 4, false, WANT_K>;
+    if (ch == FILTER_MAX_CH<COLS>)
+        return rounds ? scan_filter_kernel<COLS, FILTER_MAX_CH<COLS>, false, WANT_K, true> : scan_filter_kernel<COLS, FILTER_MAX_CH<COLS>, false, WANT_K>;
     if constexpr (COLS == 64) {
         if (!lone) return scan_filter_kernel<COLS, 2, false, WANT_K>;
     }
@@ -1859,16 +1999,18 @@ decltype(&scan_filter_kernel<COLS, 1, true, WANT_K>) filter_kernel(int ch, bool 
 template <int COLS>
 int raise_scan_lds_limits() {
     const void* whole[] = {
-        reinterpret_cast<const void*>(filter_kernel<COLS, true>(1, true)),
-        reinterpret_cast<const void*>(filter_kernel<COLS, false>(1, true)),
-        reinterpret_cast<const void*>(filter_kernel<COLS, true>(1, false)),
-        reinterpret_cast<const void*>(filter_kernel<COLS, false>(1, false)),
-        reinterpret_cast<const void*>(filter_kernel<COLS, true>(2, true)),
-        reinterpret_cast<const void*>(filter_kernel<COLS, false>(2, true)),
-        reinterpret_cast<const void*>(filter_kernel<COLS, true>(2, false)),
-        reinterpret_cast<const void*>(filter_kernel<COLS, false>(2, false)),
-        reinterpret_cast<const void*>(filter_kernel<COLS, true>(FILTER_MAX_CH<COLS>, false)),
-        reinterpret_cast<const void*>(filter_kernel<COLS, false>(FILTER_MAX_CH<COLS>, false))};
+        reinterpret_cast<const void*>(filter_kernel<COLS, true>(1, true, false)),
+        reinterpret_cast<const void*>(filter_kernel<COLS, false>(1, true, false)),
+        reinterpret_cast<const void*>(filter_kernel<COLS, true>(1, false, false)),
+        reinterpret_cast<const void*>(filter_kernel<COLS, false>(1, false, false)),
+        reinterpret_cast<const void*>(filter_kernel<COLS, true>(2, true, false)),
+        reinterpret_cast<const void*>(filter_kernel<COLS, false>(2, true, false)),
+        reinterpret_cast<const void*>(filter_kernel<COLS, true>(2, false, false)),
+        reinterpret_cast<const void*>(filter_kernel<COLS, false>(2, false, false)),
+        reinterpret_cast<const void*>(filter_kernel<COLS, true>(FILTER_MAX_CH<COLS>, false, false)),
+        reinterpret_cast<const void*>(filter_kernel<COLS, false>(FILTER_MAX_CH<COLS>, false, false)),
+        reinterpret_cast<const void*>(filter_kernel<COLS, true>(FILTER_MAX_CH<COLS>, false, true)),
+        reinterpret_cast<const void*>(filter_kernel<COLS, false>(FILTER_MAX_CH<COLS>, false, true))};
     for (const void* k : whole)
         SNNTC_HIP_CHECK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_SCAN_BYTES));
     constexpr bool SORTS = split_sorts(COLS);
@@ -1983,7 +2125,12 @@ int launch_scan_lds(const float* sorted, const int32_t* perm, const int32_t* n_r
         return SNNTC_OK;
     }
 
-    const int ch = filter_neurons<COLS>(S, I, n_slices, cus);
+    int ch = filter_neurons<COLS>(S, I, n_slices, cus);
+    // Where the staging of sixteen wavefronts does not fit beside the slice, eight or four of them work on items.
+    const auto stage_bytes = [&](int w) { return COLS == 64 && ch == 4 ? (size_t)w * FILTER_STAGE_BYTES : (size_t)FILTER_RED_BYTES; };
+    int max_waves = 16;
+    while (max_waves > 4 && lds_bytes + stage_bytes(max_waves) > (size_t)LDS_SCAN_BYTES) max_waves /= 2;
+    if (lds_bytes + stage_bytes(max_waves) > (size_t)LDS_SCAN_BYTES) { ch /= 2; max_waves = 16; }
     const int segs = kWave / COLS * ch;                     // segments per wavefront
     const int64_t items = (S + segs - 1) / segs;
     // One workgroup per CU (its 16 wavefronts take all registers; small slices let two of up to eight share a CU),
@@ -1991,20 +2138,21 @@ int launch_scan_lds(const float* sorted, const int32_t* perm, const int32_t* n_r
     // with a full workgroup all the same.  (Wavefronts by the items of a group: by those of the chip, a slice count that does not divide
     // it left a few items for a second turn, 512 rows of 333 to 1500 neurons 57.0 -> 49.4 us, 4096 to 130 58.7 -> 52.7.)
     const int64_t per_cu = (items * n_slices + cus - 1) / cus;
-    const bool shared = per_cu <= 8 && (lds_bytes + FILTER_RED_BYTES) * 2 <= (size_t)LDS_SCAN_BYTES;
+    const bool shared = per_cu <= 8 && (lds_bytes + stage_bytes(8)) * 2 <= (size_t)LDS_SCAN_BYTES;
     const int64_t capacity = (int64_t)cus * (shared ? 2 : 1);
     int64_t n_groups = capacity / n_slices;
     if (n_groups < 1) n_groups = 1;
     const int64_t per_wg = (items + n_groups - 1) / n_groups;
-    const int waves = (int)(per_wg >= 16 ? 16 : (per_wg + 3) / 4 * 4);
+    const int waves = (int)(per_wg >= max_waves ? max_waves : (per_wg + 3) / 4 * 4);
     const int64_t max_groups = (items + waves - 1) / waves;
     if (n_groups > max_groups) n_groups = max_groups;
     const int threads = lds_bytes > FILTER_WIDE_COPY_BYTES && !shared ? LDS_SCAN_THREADS : waves * kWave;
     const bool lone = filter_lone<COLS>(ch, (items + std::max(cus / n_slices, 1) - 1) / std::max(cus / n_slices, 1), I);
-    auto kern = causal_k ? filter_kernel<COLS, true>(ch, lone) : filter_kernel<COLS, false>(ch, lone);
+    const bool rounds = I >= ROUNDS_FROM;
+    auto kern = causal_k ? filter_kernel<COLS, true>(ch, lone, rounds) : filter_kernel<COLS, false>(ch, lone, rounds);
     {
         KernelTimerScope timer_("scan", stream);
-        hipLaunchKernelGGL(kern, dim3((unsigned)(n_slices * n_groups)), dim3((unsigned)threads), lds_bytes + FILTER_RED_BYTES, stream,
+        hipLaunchKernelGGL(kern, dim3((unsigned)(n_slices * n_groups)), dim3((unsigned)threads), lds_bytes + stage_bytes(waves), stream,
                            sorted, perm, n_real, w, y, rcp, causal_k, (int)S, (int)I, (int)stride, (int)J, n_slices, (int)n_groups,
                            waves, np, copy);
     }
@@ -2021,7 +2169,7 @@ int launch_scan(const float* sorted, const int32_t* perm, const int32_t* n_real,
     const int prep = scan_prepare_device(dev, &cus);
     if (prep) return prep;
     const int cols = slice_columns(S, I, stride, J, np, cus);            // none: W is streamed from memory
-    const size_t lds_bytes = ((size_t)I + np.bias) * cols * sizeof(float);
+    const size_t lds_bytes = (size_t)I * cols * sizeof(float);
     if (cols && !takes_stream(S, I, J)) {
         switch (cols) {
             case 64: return launch_scan_lds<64>(sorted, perm, n_real, w, y, rcp, causal_k, S, I, stride, J, np, copy, lds_bytes, cus, stream);

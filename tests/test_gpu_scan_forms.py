@@ -90,6 +90,26 @@ def test_scan_forms_of_small_launches(B, I, J, law):
     _check(x, w, p)
 
 
+# Rows long enough to be tested a round of four chunks at a time at first, either side of that line, and slices of 64 columns that leave
+# room for the row entries of sixteen, eight, four and no wavefronts; other widths.
+LONG_SIZES = [(12003, 399, 64), (12003, 400, 64), (12003, 431, 50), (12011, 576, 64), (12011, 577, 63), (12007, 608, 64), (12007, 609, 64),
+              (12005, 624, 64), (12005, 625, 64), (12005, 638, 41), (9001, 700, 32), (5003, 1537, 16), (2603, 3001, 24), (1207, 4700, 16)]
+
+
+@pytest.mark.parametrize("law", ["spread", "jump"])
+@pytest.mark.parametrize("B,I,J", LONG_SIZES)
+def test_scans_by_rounds(B, I, J, law):
+    """`jump`: the times stand close together, then leap, so that a round fails that the one before it did not announce."""
+    x, w, p, _ = dense_case(B + I + J, B, I, J, True, "baseline")
+    rng = np.random.default_rng(I + J)
+    if law == "jump":
+        x = np.where(rng.random(x.shape) < rng.uniform(0.1, 0.9, (B, 1)), 1 + 0.3 * rng.random(x.shape), 3 + 0.2 * rng.random(x.shape)).astype(np.float32)
+    x[1::3] = np.where(rng.random(x[1::3].shape) < 0.1, np.float32(1e5), x[1::3])
+    x[::50] = 2e5
+    x[7::50, I // 2:] = 1e5
+    _check(x, w, p)
+
+
 # Launches whose workgroups order their own rows: one and two rows per item, networks of 512 and 1024, several slices
 SORTING_SIZES = [(1, 784, 800), (1, 128, 30), (1, 129, 33), (3, 300, 20), (5, 511, 16), (6, 512, 40), (7, 513, 10), (5, 1023, 16), (2, 1024, 100),
                  (255, 800, 10), (1, 512, 1000), (100, 200, 64)]
