@@ -22,62 +22,53 @@ namespace {
 // rows of the TILE + Kw - 1 patches one kernel row can touch are staged in a wavefront-private
 // piece of LDS (lane = output channel while staging) and read back as broadcasts, four output
 // channels per read.  Gather form: no atomics, fixed summation order.
-//
-// The mask x <= ym is evaluated arithmetically (dx_mac8).  That is exact while MAX_SPIKE_TIME is at
-// most 2^86 and no two unequal spike times lie closer together than 1 / dx_mask_scale (2^-109 for
-// MAX_SPIKE_TIME = 1e5): differences that small exist only between values below 2^-85.
 // ---------------------------------------------------------------------------------------------
 constexpr int DX_TILE = 8;
 constexpr int DX_WAVES3 = 4;           // wavefronts per SIMD the KW = 3 variant is compiled for
 
-// Eight masked MACs  acc += upm_k * (x <= ym_k ? w_k : 0)  without a compare or a select: with
-//   m = clamp01(x * BIG - ym_k * BIG)       (one fused multiply-add with the clamp output modifier)
-// m is exactly 1 where x > ym_k and exactly 0 where x <= ym_k: the fused operation rounds the exact
-// value of (x - ym_k) * BIG, whose sign is that of x - ym_k, and BIG (dx_mask_scale) is large enough
-// that the smallest difference two unequal spike times can have maps to at least 1 while MAX * BIG stays finite.
-// Then t = w_k - m * w_k is w_k or 0 (both exact) and acc += upm_k * t.  All three are plain
-// multiply-adds on vector registers, which this chip issues faster than compares, selects and DPP
-// operands (about 2.8 against 4.2 cycles each with several wavefronts per SIMD).  ny_k = -ym_k * BIG
-// (+inf for outputs that take no part, so m = 1) and upm_k arrive as broadcast LDS reads.  The
-// schedule keeps every result two other instructions away from its first use.
-#define SNNTC_DX_M(K, T) "v_fma_f32 %[" #T "], %[x], %[big], %[y" #K "] clamp\n"
-#define SNNTC_DX_T(K, T) "v_fma_f32 %[" #T "], -%[" #T "], %[w" #K "], %[w" #K "]\n"
+// Eight masked MACs  acc += upm_k * (x <= ym_k ? w_k : 0).  A compare and a select next to a multiply-add: both take the
+// slower of a SIMD's two pipes, but a third of such a stream leaves it enough else to do, and all three have four-byte
+// encodings (probe kernels, four wavefronts per SIMD: 2.3 clocks an instruction; the mask as two multiply-adds, m = clamp01((x - ym) * BIG) and
+// w - m * w, takes 2.9).
+#define SNNTC_DX_M(K) "v_cmp_ge_f32_e32 vcc, %[y" #K "], %[x]\n"
+#define SNNTC_DX_T(K, T) "v_cndmask_b32_e32 %[" #T "], 0, %[w" #K "], vcc\n"
 #define SNNTC_DX_F(K, T) "v_fmac_f32_e32 %[acc], %[u" #K "], %[" #T "]\n"
 
-__device__ __forceinline__ void dx_mac8(float& acc, float x, float big, const float* u, const float* y,
-                                        const float* w) {
-    float ta, tb, tc;
+__device__ __forceinline__ void dx_mac8(float& acc, float x, const float* u, const float* y, const float* w) {
+    float ta, tb;
     asm volatile(
-        SNNTC_DX_M(0, ta)
-        SNNTC_DX_M(1, tb) SNNTC_DX_T(0, ta)
-        SNNTC_DX_M(2, tc) SNNTC_DX_T(1, tb) SNNTC_DX_F(0, ta)
-        SNNTC_DX_M(3, ta) SNNTC_DX_T(2, tc) SNNTC_DX_F(1, tb)
-        SNNTC_DX_M(4, tb) SNNTC_DX_T(3, ta) SNNTC_DX_F(2, tc)
-        SNNTC_DX_M(5, tc) SNNTC_DX_T(4, tb) SNNTC_DX_F(3, ta)
-        SNNTC_DX_M(6, ta) SNNTC_DX_T(5, tc) SNNTC_DX_F(4, tb)
-        SNNTC_DX_M(7, tb) SNNTC_DX_T(6, ta) SNNTC_DX_F(5, tc)
-        SNNTC_DX_T(7, tb) SNNTC_DX_F(6, ta)
+        SNNTC_DX_M(0) SNNTC_DX_T(0, ta)
+        SNNTC_DX_M(1) SNNTC_DX_T(1, tb) SNNTC_DX_F(0, ta)
+        SNNTC_DX_M(2) SNNTC_DX_T(2, ta) SNNTC_DX_F(1, tb)
+        SNNTC_DX_M(3) SNNTC_DX_T(3, tb) SNNTC_DX_F(2, ta)
+        SNNTC_DX_M(4) SNNTC_DX_T(4, ta) SNNTC_DX_F(3, tb)
+        SNNTC_DX_M(5) SNNTC_DX_T(5, tb) SNNTC_DX_F(4, ta)
+        SNNTC_DX_M(6) SNNTC_DX_T(6, ta) SNNTC_DX_F(5, tb)
+        SNNTC_DX_M(7) SNNTC_DX_T(7, tb) SNNTC_DX_F(6, ta)
         SNNTC_DX_F(7, tb)
-        : [acc] "+v"(acc), [ta] "=&v"(ta), [tb] "=&v"(tb), [tc] "=&v"(tc)
-        : [x] "v"(x), [big] "v"(big), [y0] "v"(y[0]), [y1] "v"(y[1]), [y2] "v"(y[2]), [y3] "v"(y[3]), [y4] "v"(y[4]),
+        : [acc] "+v"(acc), [ta] "=&v"(ta), [tb] "=&v"(tb)
+        : [x] "v"(x), [y0] "v"(y[0]), [y1] "v"(y[1]), [y2] "v"(y[2]), [y3] "v"(y[3]), [y4] "v"(y[4]),
           [y5] "v"(y[5]), [y6] "v"(y[6]), [y7] "v"(y[7]), [u0] "v"(u[0]), [u1] "v"(u[1]), [u2] "v"(u[2]),
           [u3] "v"(u[3]), [u4] "v"(u[4]), [u5] "v"(u[5]), [u6] "v"(u[6]), [u7] "v"(u[7]), [w0] "v"(w[0]),
           [w1] "v"(w[1]), [w2] "v"(w[2]), [w3] "v"(w[3]), [w4] "v"(w[4]), [w5] "v"(w[5]), [w6] "v"(w[6]),
-          [w7] "v"(w[7]));
+          [w7] "v"(w[7])
+        : "vcc");
 }
 
 // MULTI is for layers with at most 32 input channels: the wavefront is cut into 2, 4, 8 or 16 parts
 // of 32, 16, 8 or 4 lanes (`1 << parts_shift` of them) that take the same channels of as many neighbouring
 // 8-pixel tiles, so few lanes idle.  Which patch lies under a tap then differs between the parts; a
-// part whose patch does not exist reads a slot that holds (ym, upm) = (-inf, 0) -- +inf in the scaled form
-// of dx_mac8 -- and so adds nothing.
+// part whose patch does not exist reads a slot that holds (ym, upm) = (-inf, 0) and so adds nothing.
 //
 // KW = 3 (the layer's kernel is three columns wide; 0: any width): the sweep is turned inside out.  A slot's
 // operands are read once per DX_GK output channels and serve the up to three (pixel, tap) pairs that meet
 // that patch, with the weights of all three taps of those channels in registers.  That takes far fewer
 // registers than a whole weight row per tap; they go into a second set of weights and of slot operands,
 // fetched while the current ones are in use, and fewer LDS reads are needed (80 instead of 192 per tile and
-// 16 output channels).
+// 16 output channels).  us, arithmetic masks, a branch per (pixel, tap) block and tiles over the whole padded row / compare and
+// select, no branches, tiles over the wanted window: 64 -> 64 at 56 x 56, 32 images 252 / 229, 128 -> 128 at 28 x 28 262 / 214, 256 -> 256 at
+// 14 x 14 238 / 217, 512 -> 512 at 7 x 7 235 / 213, 32 -> 32 at 32 x 32, 128 images 122 / 95, 64 -> 128 at 8 x 8 69 / 52; one image of 64 -> 64 at
+// 56 x 56 49 / 42.
 constexpr int DX_GK = 8;
 template <int KCB, bool MULTI, int KW>
 __global__ void __launch_bounds__(256)
@@ -86,7 +77,7 @@ cv_grad_input_chan_kernel(const float* __restrict__ xpad, const float* __restric
                           const float* __restrict__ upm, const float* __restrict__ ym,
                           float* __restrict__ dx, CropGeom crop, int H, int W, int C, int Kc, int Kh, int Kw, int Sh,
                           int Sw, int Nh, int Nw, int tiles_w, int c_blocks, int64_t n_items, int64_t lead_items,
-                          int lead_blocks, float max_cmp, int ksplit, float big, int parts_shift) {
+                          int lead_blocks, float max_cmp, int ksplit, int parts_shift) {
     extern __shared__ __align__(16) float staged[];      // per wavefront: [2][n_slots + 1][KCB]; ksplit > 1: then `partial`
     const int parts = MULTI ? 1 << parts_shift : 1;
     const int span = DX_TILE * parts;                    // pixels of one wavefront
@@ -111,31 +102,30 @@ cv_grad_input_chan_kernel(const float* __restrict__ xpad, const float* __restric
     int64_t rest = item / c_blocks;
     int tw = tiles_w - 1;
     if (lead) { tw = (int)(rest % tiles_lead); rest /= tiles_lead; }
-    const int h = (int)(rest % H);
-    const int a = (int)(rest / H);
-    const int w0 = tw * span;                            // first pixel of the wavefront
-    const int p0 = w0 + part * DX_TILE;                  // first pixel of this lane
+    const int oh = (int)(rest % crop.h);
+    const int h = crop.top + oh;
+    const int a = (int)(rest / crop.h);
     const int c = MULTI ? (lane & ((kWave >> parts_shift) - 1)) : cb * kWave + lane;
     const bool lane_ok = c < C;
     const unsigned cc = (unsigned)(lane_ok ? c : C - 1);
+    const float* __restrict__ xrow = xpad + ((size_t)(a * H + h) * W) * C + cc;
+    // A window that begins with a padded column (the whole padded image of a SAME layer): the row's tiles start behind it.
+    // (Per row and channels, so neighbouring tiles agree.  64 -> 64 at 32 x 32: four tiles a row instead of five.)
+    const int skip = KW == 3 && crop.left == 0 && !__any(xrow[0] <= max_cmp) ? 1 : 0;
+    const int w0 = crop.left + skip + tw * span;         // first pixel of the wavefront
+    const int p0 = w0 + part * DX_TILE;                  // first pixel of this lane
     const int n_slots = span + Kw - 1;                   // slot d: the patch whose left column is w0-Kw+1+d
     float* __restrict__ ys = staged + (size_t)wave * 2 * (n_slots + 1) * KCB;
     float* __restrict__ us = ys + (n_slots + 1) * KCB;
     if (lane < KCB) {                                    // the spare slot
-        ys[n_slots * KCB + lane] = INFINITY;             // in the scaled form the loop below produces
+        ys[n_slots * KCB + lane] = -INFINITY;
         us[n_slots * KCB + lane] = 0.0f;
     }
 
-    // Pixels that need no work: those outside the window of the gradient the caller wants (with the
-    // window of the un-padded image that is the whole SAME border: 11 % of a 34 x 34 padded image, 40 %
-    // of a 9 x 9 one) and padded pixels anywhere (x > MAX-0.1 can never satisfy x <= ym).  `live` has
-    // bit t set when pixel t of some lane's tile has work; a wavefront whose row lies outside the
-    // window has none at all (with ksplit > 1 that holds for the whole workgroup).
-    const int oh = h - crop.top;
-    if (oh < 0 || oh >= crop.h) return;
+    // Tiles cover the window of the gradient that the caller wants.  Pixels that need no work: those behind its last column and
+    // padded ones (x > MAX-0.1 can never satisfy x <= ym).  `live` has bit t set when pixel t of some lane's tile has work.
     float xv[DX_TILE], acc[DX_TILE];
     unsigned live = 0;
-    const float* __restrict__ xrow = xpad + ((size_t)(a * H + h) * W) * C + cc;
 #pragma unroll
     for (int t = 0; t < DX_TILE; ++t) {
         const int wx = min(p0 + t, W - 1);
@@ -144,10 +134,11 @@ cv_grad_input_chan_kernel(const float* __restrict__ xpad, const float* __restric
         const int ow = p0 + t - crop.left;
         if (__any(xv[t] <= max_cmp && ow >= 0 && ow < crop.w)) live |= 1u << t;
     }
-    // KW = 3: slots that hold no patch are filled with (+inf, 0), a term that adds nothing, so a lane may read
-    // any slot.  With a column stride of 1 those are the slots outside [slot_lo, slot_hi): they are filled once and
-    // left alone by the rescaling pass of every staging round; otherwise they are filled again after every round.
-    // Bit 3 * d + kw of `work` says that the d-th slot of a part and tap kw meet a pixel with work (for some lane).
+    // KW = 3: slots that hold no patch are filled with (-inf, 0), a term that adds nothing, so a lane may read
+    // any slot.  (No staging round loads them: filled once.)
+    // Nearly all of the 24 (pixel, tap) blocks of a sweep have work, so it takes them all, without a branch: a test, a jump and a
+    // wait per 24 vector instructions cost more than the blocks they leave out (every instruction takes an issue slot, scalar ones
+    // too).  It ends early, in four places, where the last slots meet no pixel with work or hold no patch.
     auto slot_exists = [&](int sl) {
         const int ww = w0 - Kw + 1 + sl;
         if (ww < 0) return false;
@@ -155,25 +146,10 @@ cv_grad_input_chan_kernel(const float* __restrict__ xpad, const float* __restric
     };
     auto fill_empty_slots = [&]() {
         for (int sl = 0; sl < n_slots; ++sl)
-            if (!slot_exists(sl) && lane < KCB) { ys[sl * KCB + lane] = INFINITY; us[sl * KCB + lane] = 0.0f; }
+            if (!slot_exists(sl) && lane < KCB) { ys[sl * KCB + lane] = -INFINITY; us[sl * KCB + lane] = 0.0f; }
     };
-    const int slot_lo = max(0, Kw - 1 - w0), slot_hi = min(n_slots, Nw + Kw - 1 - w0);
-    unsigned work = 0;
-    float bigv = big;
-    if constexpr (KW == 3) {
-#pragma unroll
-        for (int d = 0; d < DX_TILE + 2; ++d) {
-            bool any_patch = false;
-            for (int pt = 0; pt < parts; ++pt) any_patch = any_patch || slot_exists(d + pt * DX_TILE);
-#pragma unroll
-            for (int kw = 0; kw < 3; ++kw) {
-                const int t = d - 2 + kw;                                 // the pixel that meets it under tap kw
-                if (t >= 0 && t < DX_TILE && any_patch && (live >> t & 1u)) work |= 1u << (3 * d + kw);
-            }
-        }
-        if (Sw == 1) fill_empty_slots();
-    }
-    asm volatile("v_mov_b32 %0, %1" : "=v"(bigv) : "s"(big));             // one register for all the blocks below
+    if constexpr (KW == 3) fill_empty_slots();
+    const int slots_end = min(live != 0 ? 32 - __builtin_clz(live) + 2 : 0, (Nw - 1) * Sw + Kw - w0);
     if (live != 0) {
         for (int kh = 0; kh < Kh; ++kh) {
             const int hh = h - kh;
@@ -211,32 +187,24 @@ cv_grad_input_chan_kernel(const float* __restrict__ xpad, const float* __restric
                 asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                 __builtin_amdgcn_wave_barrier();
-                // ym -> -ym * BIG, the operand of dx_mac8 (-inf, an output that takes no part, becomes +inf).
-                // Slots that were not loaded: the tap-major sweep never reads them (it reads the spare slot
-                // instead), the slot-major one reads them as (+inf, 0), see fill_empty_slots
-                for (int i = lane; i < n_slots * (KCB / 4); i += kWave) {
-                    if (KW == 3 && Sw == 1 && (i / (KCB / 4) < slot_lo || i / (KCB / 4) >= slot_hi)) continue;
-                    float4 v4 = reinterpret_cast<float4*>(ys)[i];
-                    v4.x *= -big; v4.y *= -big; v4.z *= -big; v4.w *= -big;
-                    reinterpret_cast<float4*>(ys)[i] = v4;
-                }
-                if (KW == 3 && Sw != 1) fill_empty_slots();
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                __builtin_amdgcn_wave_barrier();
                 if constexpr (KW == 3) {
                     // wq[tap][kc / 4][c][kc % 4]: the 16-byte pieces the lanes fetch together are neighbours
                     // in memory.  Two register sets: the weights of the next DX_GK output channels are
                     // fetched while the current ones are in use.
-                    const float4* __restrict__ wbase =
-                        reinterpret_cast<const float4*>(wq) + ((size_t)(kh * 3) * (Kc / 4) + kc0 / 4) * C + cc;
-                    const size_t tap_stride = (size_t)(Kc / 4) * C;
+                    // (Through a buffer descriptor: scalar offsets, one vector register of address for all of them.)
+                    const int tap_bytes = Kc * C * (int)sizeof(float);
+                    const __amdgpu_buffer_rsrc_t wbuf = __builtin_amdgcn_make_buffer_rsrc(
+                        const_cast<float*>(wq + ((size_t)(kh * 3) * Kc + kc0) * C), 0, 3 * tap_bytes, 0x00020000);
+                    typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
                     auto load_w = [&](float (&wr)[3][DX_GK], int g) {
 #pragma unroll
                         for (int kw = 0; kw < 3; ++kw)
 #pragma unroll
                             for (int q = 0; q < DX_GK; q += 4) {
-                                const float4 v4 = wbase[kw * tap_stride + (size_t)(g * (DX_GK / 4) + q / 4) * C];
-                                wr[kw][q] = v4.x; wr[kw][q + 1] = v4.y; wr[kw][q + 2] = v4.z; wr[kw][q + 3] = v4.w;
+                                const u32x4 v4 = __builtin_amdgcn_raw_buffer_load_b128(
+                                    wbuf, (int)cc * 16, kw * tap_bytes + (g * DX_GK + q) * C * (int)sizeof(float), 0);
+#pragma unroll
+                                for (int e = 0; e < 4; ++e) wr[kw][q + e] = __uint_as_float(v4[e]);
                             }
                     };
                     const float* __restrict__ ybase = ys + part * DX_TILE * KCB;
@@ -252,22 +220,18 @@ cv_grad_input_chan_kernel(const float* __restrict__ xpad, const float* __restric
                     };
                     // all slots of a half against the three taps of DX_GK output channels; the operands of the
                     // next slot are read while the current one computes
-                    auto sweep = [&](const float (&wr)[3][DX_GK], const float* __restrict__ yg) {
+                    auto sweep = [&](const float (&wr)[3][DX_GK], const float* __restrict__ yg) __attribute__((always_inline)) {
                         float yq[2][DX_GK], uq[2][DX_GK];
-                        // the bits are tested where they are used: as thirty loop-invariant conditions they would
-                        // take sixty scalar registers
-                        unsigned wk = work;
-                        asm volatile("" : "+s"(wk));
                         read_slot(yg, 0, yq[0], uq[0]);
 #pragma unroll
                         for (int d = 0; d < DX_TILE + 2; ++d) {
+                            if ((d == 3 || d == 5 || d == 7 || d == 8) && d >= slots_end) break;
                             if (d + 1 < DX_TILE + 2) read_slot(yg, d + 1, yq[(d + 1) & 1], uq[(d + 1) & 1]);
                             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                             for (int kw = 0; kw < 3; ++kw) {
                                 const int t = d - 2 + kw;
-                                if (t < 0 || t >= DX_TILE) continue;
-                                if (wk >> (3 * d + kw) & 1u) dx_mac8(acc[t], xv[t], bigv, uq[d & 1], yq[d & 1], wr[kw]);
+                                if (t >= 0 && t < DX_TILE) dx_mac8(acc[t], xv[t], uq[d & 1], yq[d & 1], wr[kw]);
                             }
                             __builtin_amdgcn_sched_barrier(0);
                         }
@@ -316,8 +280,8 @@ cv_grad_input_chan_kernel(const float* __restrict__ xpad, const float* __restric
                                 uq[v] = u4.x; uq[v + 1] = u4.y; uq[v + 2] = u4.z; uq[v + 3] = u4.w;
                             }
                             __builtin_amdgcn_sched_barrier(0);
-                            dx_mac8(acc[t], xv[t], bigv, &uq[0], &yq[0], &wreg[g * 16]);
-                            dx_mac8(acc[t], xv[t], bigv, &uq[8], &yq[8], &wreg[g * 16 + 8]);
+                            dx_mac8(acc[t], xv[t], &uq[0], &yq[0], &wreg[g * 16]);
+                            dx_mac8(acc[t], xv[t], &uq[8], &yq[8], &wreg[g * 16 + 8]);
                         }
                     }
                 }
@@ -341,6 +305,7 @@ cv_grad_input_chan_kernel(const float* __restrict__ xpad, const float* __restric
     // only the pixels inside the caller's window of the padded image are stored
     if (lane_ok) {
         float* __restrict__ orow = dx + ((size_t)(a * crop.h + oh) * crop.w) * C + c;
+        if (skip && tw == 0 && part == 0) orow[0] = 0.0f;
 #pragma unroll
         for (int t = 0; t < DX_TILE; ++t) {
             const int ow = p0 + t - crop.left;
@@ -599,6 +564,7 @@ static DxPlan dx_plan(const ConvGeom& g) {
     // input channels do not cover (7x7/2 on 3 channels at 224 x 224, B = 32: 2.8 ms against 2.2 ms through
     // patch space).
     if (g.C < 32 && g.Kw != 3) return p;
+    if (g.Kw == 3 && 12 * g.Kc * g.C >= 0x7fffffffLL) return p;         // (three taps of weights behind one)
     // parts of a wavefront: as many as the channels leave room for, but no wider a tile than the row needs
     int parts = g.C > 32 ? 1 : g.C > 16 ? 2 : g.C > 8 ? 4 : g.C > 4 ? 8 : 16;
     while (parts > 2 && DX_TILE * (parts / 2) >= g.W) parts /= 2;
@@ -632,41 +598,32 @@ static DxPlan dx_plan(const ConvGeom& g) {
 
 bool cv_grad_input_chan_supported(const ConvGeom& g) { return dx_plan(g).ok; }
 
-// The factor BIG of dx_mac8: the largest power of two with MAX_SPIKE_TIME * BIG <= 2^126.
-static float dx_mask_scale(float max_time) {
-    int e = 0;
-    if (max_time > 1.0f) {
-        if (max_time < 0x1p86f) frexpf(max_time, &e);     // max_time < 2^e
-        else e = 86;
-    }
-    return ldexpf(1.0f, 126 - e);
-}
-
 // wq: the weights regrouped by launch_backward_prologue
 int launch_cv_grad_input_chan(const float* xpad, const float* wq, const float* upm, const float* ym,
                               float* dx, const CropGeom& crop, const ConvGeom& g, const NeuronParams& np,
                               hipStream_t stream) {
+    if (crop.h <= 0 || crop.w <= 0) return SNNTC_OK;
     const DxPlan pl = dx_plan(g);
     if (!pl.ok) return fail(SNNTC_ERR_UNSUPPORTED, "conv backward: no channel-lane launch shape for this layer");
-    const int span = pl.span, tiles_w = pl.tiles_w, c_blocks = pl.c_blocks, kcb = pl.kcb, ksplit = pl.ksplit;
+    const int span = pl.span, c_blocks = pl.c_blocks, kcb = pl.kcb, ksplit = pl.ksplit;
+    const int tiles_w = (int)((crop.w + span - 1) / span);
     const bool multi = pl.parts_shift > 0;
-    const int64_t n_items = g.B * g.H * tiles_w * c_blocks;
+    const int64_t n_items = g.B * crop.h * tiles_w * c_blocks;
     // One item per workgroup.  Without the split a workgroup is a single wavefront: the
     // wavefronts do not cooperate, their running times differ (border tiles, rows outside the window),
     // and a CU takes a new workgroup only when a whole one has left, so in larger workgroups the slots
     // of the early finishers would idle.
     const int wg_waves = ksplit;
     // a last tile with at most half its pixels inside the row goes to the end of the launch
-    const bool partial_last = tiles_w > 1 && (g.W - (int64_t)(tiles_w - 1) * span) * 2 <= span;
-    const int64_t lead_items = partial_last ? g.B * g.H * (tiles_w - 1) * c_blocks : n_items;
+    const bool partial_last = tiles_w > 1 && (crop.w - (int64_t)(tiles_w - 1) * span) * 2 <= span;
+    const int64_t lead_items = partial_last ? g.B * crop.h * (tiles_w - 1) * c_blocks : n_items;
     int64_t lead_blocks = lead_items;
     if (partial_last) lead_blocks = (lead_blocks + kXcds - 1) / kXcds * kXcds;
     const int64_t blocks = lead_blocks + (n_items - lead_items);
     if (blocks > 0x7fffffffLL) return fail(SNNTC_ERR_TOO_LARGE, "conv backward: grid too large");
     dim3 grid((unsigned)blocks), block(wg_waves * kWave);
     const size_t lds = pl.lds;
-    void (*kern)(const float*, const float*, const float*, const float*, float*, CropGeom, int, int, int, int, int, int,
-                 int, int, int, int, int, int, int64_t, int64_t, int, float, int, float, int);
+    decltype(&cv_grad_input_chan_kernel<64, false, 3>) kern;
     if (g.Kw == 3) {
         if (multi)
             kern = kcb == 64 ? cv_grad_input_chan_kernel<64, true, 3> : kcb == 32 ? cv_grad_input_chan_kernel<32, true, 3>
@@ -685,7 +642,7 @@ int launch_cv_grad_input_chan(const float* xpad, const float* wq, const float* u
         KernelTimerScope timer_("cv_grad_input", stream);
         hipLaunchKernelGGL(kern, grid, block, lds, stream, xpad, wq, upm, ym, dx, crop, (int)g.H, (int)g.W, (int)g.C,
                            (int)g.Kc, (int)g.Kh, (int)g.Kw, (int)g.Sh, (int)g.Sw, (int)g.Nh, (int)g.Nw, tiles_w,
-                           c_blocks, n_items, lead_items, (int)lead_blocks, np.max_cmp, ksplit, dx_mask_scale(np.max_time),
+                           c_blocks, n_items, lead_items, (int)lead_blocks, np.max_cmp, ksplit,
                            pl.parts_shift);
     }
     SNNTC_HIP_CHECK(hipGetLastError());

@@ -75,3 +75,38 @@ def test_dense_gradients_in_one_launch(B, I, J, bias):
     adx, adw, _ = capi.fc_backward_dev(np.abs(g), x, np.abs(w), p, out, wide=True)
     assert np.all(np.abs(dx - rdx) <= 1e-6 * np.abs(adx) + 1e-30)
     assert np.all(np.abs(dw - rdw) <= 1e-6 * np.abs(adw) + 1e-30)
+
+
+@pytest.mark.parametrize("B,H,W,C,Kc,S", [
+    (2, 5, 9, 64, 64, 1), (2, 4, 10, 64, 128, 1), (1, 3, 11, 65, 16, 1), (1, 5, 16, 32, 64, 1), (2, 3, 18, 20, 32, 1),      # tiles of 8 to 128 pixels
+    (1, 4, 19, 3, 64, 1), (1, 3, 30, 7, 48, 1), (2, 3, 31, 64, 80, 2), (1, 7, 34, 33, 64, 1), (3, 9, 8, 64, 256, 1), (1, 3, 3, 4, 16, 1),
+])
+def test_conv_input_gradients_at_the_edges_of_tiles(B, H, W, C, Kc, S):
+    """Three-column kernels: rows that begin or end with a padded column, or have none, in one image; the whole gradient and windows of it."""
+    import snntc_amd as snn
+    from snntc_amd import ops
+    rng = np.random.default_rng(B + H + W + C + Kc)
+    xpad = np.exp(rng.random((B, H, W, C))).astype(np.float32)
+    xpad[rng.random(xpad.shape) < 0.1] = 1e5
+    first, last = rng.random((B, H)) < 0.5, rng.random((B, H)) < 0.5
+    xpad[:, :, 0][first] = 1e5
+    xpad[:, :, -1][last] = 1e5
+    p = capi.cv_params(3, 3, S, S, same=True, biasvolt=1.0)
+    Nh, Nw, _ = capi.cv_dims(xpad.shape, p)
+    w = rng.standard_normal((9 * C + 1, Kc)).astype(np.float32)
+    out = np.concatenate([np.exp(1.2 * rng.random((B, Nh, Nw, Kc))), rng.standard_normal((B, Nh, Nw, Kc))]).astype(np.float32)
+    dead = rng.random((B, Nh, Nw, Kc)) < 0.1
+    out[:B][dead] = 1e5
+    out[B:][dead] = 0.0
+    g = np.zeros((2 * B, Nh, Nw, Kc), np.float32)
+    g[:B] = rng.standard_normal((B, Nh, Nw, Kc))
+    dx = snn.snncv_grad(t(g), t(xpad), t(w), p, t(out))[0].cpu().numpy()
+    rdx, _, _ = capi.cv_backward_dev(g, xpad, w, p, out, wide=True)
+    ao = out.copy()
+    ao[B:] = np.abs(ao[B:])
+    adx, _, _ = capi.cv_backward_dev(np.abs(g), xpad, np.abs(w), p, ao, wide=True)
+    # (up to 2304 terms of either sign: partial sums stay near their square root, so the error stays near one rounding of |terms|)
+    assert np.all(np.abs(dx - rdx) <= 2e-6 * np.abs(adx) + 1e-30)
+    for h, wd, top, left in [(H - 2, W - 2, 1, 1), (1, W // 2 + 1, H // 2, 1), (H, W - 1, 0, 0), (2, 2, 0, W - 2)]:
+        part = ops.snncv_grad(t(g), t(xpad), t(w), p, t(out), crop=(h, wd, top, left))[0].cpu().numpy()
+        assert np.array_equal(part, dx[:, top:top + h, left:left + wd])
