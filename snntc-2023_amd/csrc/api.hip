@@ -5,6 +5,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <string>
@@ -168,27 +169,28 @@ int forward_chain(const SegmentSource& src, const FcFwdWs& ws, const float* w, f
 // Backward scratch.  `rows` is the weight row count including a possible bias row; the partial-sum
 // area is sized for the worst case of 256 slices only when slicing can happen at all.
 struct BwdWs { float* upm; float* wt; float* dxp; float* partial; int max_split; size_t bytes; };
-// patch_scratch: elements of the per-patch gradient of conv layers whose dX goes through patch space
-// dense_split: slices of a dense layer's dW (0: a conv layer)
-BwdWs bwd_ws(void* ws, int64_t S, int64_t rows, int64_t J, int64_t min_base_blocks, int64_t patch_scratch = 0,
-             int dense_split = 0) {
+// patch_scratch: elements of the per-patch gradient of conv layers whose dX goes through patch space; max_split: slices of dW
+BwdWs bwd_ws(void* ws, int64_t S, int64_t rows, int64_t J, int64_t patch_scratch, int max_split) {
     Carver c(ws);
     BwdWs r;
     r.upm = c.take<float>(S * J);
     r.wt = c.take<float>(rows * J);                        // (only conv layers use it; the size callers may rely on has room for it)
     r.dxp = c.take<float>(patch_scratch);
-    r.max_split = dense_split > 0 ? dense_split : weight_grad_splits(S, min_base_blocks);
+    r.max_split = max_split;
     r.partial = c.take<float>(r.max_split > 1 ? (int64_t)r.max_split * rows * J : 0);
     r.bytes = c.used;
     return r;
 }
 
-// Smallest block count the weight-gradient launch of a conv layer can have (it decides how far the
-// patch range may be sliced): the wide kernel covers 32 rows per block, the generic one 8.
-int64_t cv_weight_base_blocks(const ConvGeom& g) {
-    const int64_t generic = grad_weight_blocks(g.P + 1, g.Kc);
-    const int64_t wide = cv_grad_weight_wide_supported(g) ? cv_grad_weight_wide_blocks(g) : generic;
-    return wide < generic ? wide : generic;
+// Slices of a conv layer's dW, and its backward scratch.  Where the caller's workspace has no room for all of them there are fewer, down to
+// the count of the kernels for any shape; less is refused.
+BwdWs cv_bwd_ws(void* ws, size_t room, const ConvGeom& g) {
+    const int64_t patch_scratch = cv_grad_input_chan_supported(g) ? 0 : g.S * g.P;
+    const int generic = grad_weight_blocks(g.P + 1, g.Kc);
+    const bool wide = cv_grad_weight_wide_supported(g);
+    const int least = weight_grad_splits(g.S, wide ? std::min(generic, cv_grad_weight_row32_blocks(g)) : generic);
+    const BwdWs full = bwd_ws(ws, g.S, g.P + 1, g.Kc, patch_scratch, wide ? std::max(least, cv_grad_weight_splits(g)) : least);
+    return full.bytes <= room ? full : bwd_ws(ws, g.S, g.P + 1, g.Kc, patch_scratch, least);
 }
 
 int fc_forward_impl(const float* x, const float* w, const float* params, float* out, float* sorted_z,
@@ -602,7 +604,7 @@ static int fc_splits(int64_t B, int64_t I, int64_t J) {
 int snntc_fc_backward_workspace_bytes(int64_t B, int64_t I, int64_t J, size_t* bytes) {
     if (!bytes || B < 0 || I < 0 || J < 0)
         return fail(SNNTC_ERR_BAD_ARGUMENT, "snntc_fc_backward_workspace_bytes: bad argument");
-    *bytes = bwd_ws(nullptr, B, I + 1, J, 0, 0, fc_splits(B, I, J)).bytes;
+    *bytes = bwd_ws(nullptr, B, I + 1, J, 0, fc_splits(B, I, J)).bytes;
     return SNNTC_OK;
 }
 
@@ -672,7 +674,7 @@ int snntc_fc_backward(const float* grad, const float* x, const float* w, const f
     }
     if (!grad || !x || !w || !oldout) return fail(SNNTC_ERR_BAD_ARGUMENT, "snntc_fc_backward: NULL tensor pointer");
     const int narrow = fc_narrow_split(B, I, J);
-    BwdWs ws = bwd_ws(workspace, B, I + 1, J, 0, 0, fc_splits(B, I, J));
+    BwdWs ws = bwd_ws(workspace, B, I + 1, J, 0, fc_splits(B, I, J));
     rc = check_workspace(workspace, workspace_bytes, ws.bytes);
     if (rc) return rc;
     const NeuronParams np = neuron_params(params_host[0], params_host[2], params_host[5]);
@@ -721,8 +723,7 @@ int snntc_cv_backward_workspace_bytes(int64_t B, int64_t H, int64_t W, int64_t C
     int rc = cv_geom(B, H, W, C, Kc, 0, params_host, false, "snntc_cv_backward_workspace_bytes", &g);
     if (rc) return rc;
     if (!bytes) return fail(SNNTC_ERR_BAD_ARGUMENT, "snntc_cv_backward_workspace_bytes: bytes is NULL");
-    *bytes = bwd_ws(nullptr, g.S, g.P + 1, Kc, cv_weight_base_blocks(g),
-                    cv_grad_input_chan_supported(g) ? 0 : g.S * g.P).bytes;
+    *bytes = cv_bwd_ws(nullptr, SIZE_MAX, g).bytes;
     return SNNTC_OK;
 }
 
@@ -769,8 +770,7 @@ static int cv_backward_impl(const float* grad, const float* xpad, const float* w
         return dw ? launch_fill_zero(dw, w_rows * Kc, st) : SNNTC_OK;
     }
     if (!grad || !xpad || !w || !oldout) return fail(SNNTC_ERR_BAD_ARGUMENT, "snntc_cv_backward: NULL tensor pointer");
-    BwdWs ws = bwd_ws(workspace, g.S, g.P + 1, Kc, cv_weight_base_blocks(g),
-                      cv_grad_input_chan_supported(g) ? 0 : g.S * g.P);
+    BwdWs ws = cv_bwd_ws(workspace, workspace_bytes, g);
     rc = check_workspace(workspace, workspace_bytes, ws.bytes);
     if (rc) return rc;
     const NeuronParams np = neuron_params(params_host[0], params_host[4], params_host[11]);
@@ -789,7 +789,7 @@ static int cv_backward_impl(const float* grad, const float* xpad, const float* w
     }
     if (!dw) return SNNTC_OK;
     const bool wide = cv_grad_weight_wide_supported(g);
-    int nsplit = weight_grad_splits(g.S, wide ? cv_grad_weight_wide_blocks(g) : grad_weight_blocks(w_rows, Kc));
+    int nsplit = wide ? cv_grad_weight_splits(g) : weight_grad_splits(g.S, grad_weight_blocks(w_rows, Kc));
     if (nsplit > ws.max_split) nsplit = ws.max_split;
     float* dst = nsplit > 1 ? ws.partial : dw;
     const SegmentSource src = conv_source(xpad, g);

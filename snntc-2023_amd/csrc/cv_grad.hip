@@ -7,6 +7,7 @@
 // Both kernels put the channel (dX) or the output channel (dW) on the lanes, so everything that
 // depends only on the patch is wave-uniform and is fetched through the scalar path.
 #include "snntc_common.h"
+#include <algorithm>
 #include <type_traits>
 
 namespace snntc {
@@ -429,6 +430,163 @@ cv_grad_weight_wide_kernel(const float* __restrict__ xpad, const float* __restri
 }
 
 // ---------------------------------------------------------------------------------------------
+// dW of three-column kernels of stride one whose channels come in thirty-twos.  A pixel is an input of up to three patches of an
+// output row, one per kernel column: a wavefront owns 32 channels of one kernel row, all three columns (96 accumulators a
+// lane), and walks over the pixels of its patches' image rows; the spike times and upstream values of the last three patches stay in
+// registers.  Next to a block of 32 weight rows that is a third of the fetches for the same arithmetic and fewer instructions
+// around it (an issue slot each, whatever they are): 192 vector instructions per pixel instead of three times 64.
+// A wait for one scalar load is a wait for all: a pixel's inputs are fetched in two halves, each while the other is worked on.
+// Terms are added in the order of the patches, then wavefronts, then slices.  us, blocks of 32 rows / this, the slices' sum included: 64 -> 64 at
+// 32 x 32, 64 images 131 / 115, at 56 x 56, 32 images 187 / 162, 128 -> 128 at 28 x 28 191 / 160, 256 -> 256 at 14 x 14 222 / 161,
+// 256 -> 512 at 7 x 7 129 / 95, 512 -> 512 198 / 168.  (Without any fetch it takes 103 of 108: what bounds it is the issue rate.)
+// ---------------------------------------------------------------------------------------------
+constexpr int DWT_KW = 3, DWT_WAVES = 8;
+// (read by scalar loads where the address is uniform)
+typedef __attribute__((address_space(4))) const float scalar_cfloat;
+
+template <int CB>
+__global__ void __launch_bounds__(DWT_WAVES * kWave, CB == 32 ? 4 : 6)
+cv_grad_weight_taps_kernel(const float* __restrict__ xpad, const float* __restrict__ upm, const float* __restrict__ ym,
+                           float* __restrict__ dst, int S, int Kc, int rows, int seg_per_slice, int H, int W, int C, int Sh, int Nh,
+                           int Nw, int blocks_j, int blocks_rows, int bias_row, float biasvolt, float neg_s, float post) {
+    constexpr int HALF = CB / 2;
+    __shared__ float red[DWT_WAVES - 1][CB + 1][kWave];
+    const int lane = threadIdx.x % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    // (the workgroups of a slice on one XCD, whose L2 then holds its ym, upm and image rows)
+    const int block = xcd_contiguous(blockIdx.x, gridDim.x);
+    const int slice = block / (blocks_j * blocks_rows), in_slice = block - slice * (blocks_j * blocks_rows);
+    const int rows_block = in_slice / blocks_j;
+    const int j = (in_slice - rows_block * blocks_j) * kWave + lane;
+    const int blocks_c = C / CB;
+    const int kh = rows_block / blocks_c;
+    const int c0 = (rows_block - kh * blocks_c) * CB;
+
+    const int s_begin = slice * seg_per_slice;
+    const int s_end = min(S, s_begin + seg_per_slice);
+    const int per_wave = (s_end - s_begin + DWT_WAVES - 1) / DWT_WAVES;
+    const int s_lo = s_begin + wave * per_wave;
+    const int s_hi = min(s_end, s_lo + per_wave);
+
+    float acc[DWT_KW][CB];
+#pragma unroll
+    for (int t = 0; t < DWT_KW; ++t)
+#pragma unroll
+        for (int r = 0; r < CB; ++r) acc[t][r] = 0.0f;
+    const bool with_bias = bias_row >= 0 && rows_block == 0;
+    float acc_bias = 0.0f;
+
+    if (s_lo < s_hi) {
+        const int per_img = Nh * Nw;
+        const int a = s_lo / per_img;
+        const int r2 = s_lo - a * per_img;
+        int nh = r2 / Nw, nw = r2 - nh * Nw;
+        scalar_cfloat* x_at = (scalar_cfloat*)(uintptr_t)(xpad + ((size_t)(a * H + nh * Sh + kh) * W + nw) * C + c0);
+        const ptrdiff_t next_row = (ptrdiff_t)Sh * W * C, next_image = (ptrdiff_t)(H - Nh * Sh) * W * C;
+        // Rows of ym and upm: buffer descriptors of the wavefront's patches, a scalar running offset (held at the last patch: it is
+        // not bounds-checked) and the lane's column.  Requested a patch ahead.
+        const int range_bytes = (int)min((int64_t)(s_hi - s_lo) * Kc * (int64_t)sizeof(float), (int64_t)0x7ffffffc);
+        const __amdgpu_buffer_rsrc_t ybuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(ym + (size_t)s_lo * Kc), 0, range_bytes, 0x00020000);
+        const __amdgpu_buffer_rsrc_t ubuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(upm + (size_t)s_lo * Kc), 0, range_bytes, 0x00020000);
+        const int col_bytes = min(j, Kc - 1) * (int)sizeof(float), patch_bytes = Kc * (int)sizeof(float), last_bytes = (s_hi - 1 - s_lo) * patch_bytes;
+        int ahead_bytes = 0;
+        float y_next, u_next;
+        auto request = [&] {
+            y_next = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ybuf, col_bytes, ahead_bytes, 0));
+            u_next = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ubuf, col_bytes, ahead_bytes, 0));
+            ahead_bytes = min(ahead_bytes + patch_bytes, last_bytes);
+        };
+        request();
+        float y0 = 0.0f, y1 = 0.0f, y2 = 0.0f, u0 = 0.0f, u1 = 0.0f, u2 = 0.0f;      // of the patches under columns 0, 1, 2
+        float xa[HALF], xb[HALF];
+#pragma unroll
+        for (int r = 0; r < HALF; ++r) xa[r] = x_at[r];
+        // One pixel, of the columns T0, T1, T2 it has patches under; then x_next is the pixel at work.
+        auto pixel = [&](auto t0_c, auto t1_c, auto t2_c, scalar_cfloat* x_next) __attribute__((always_inline)) {
+            constexpr bool T0 = decltype(t0_c)::value, T1 = decltype(t1_c)::value, T2 = decltype(t2_c)::value;
+            y2 = y1; u2 = u1; y1 = y0; u1 = u0;
+            if (T0) {
+                y0 = y_next * -neg_s; u0 = u_next;
+                request();
+            } else {
+                u0 = 0.0f;
+            }
+            auto half = [&](const float (&x)[HALF], auto first_c) __attribute__((always_inline)) {
+                constexpr int FIRST = decltype(first_c)::value;
+#pragma unroll
+                for (int r = 0; r < HALF; ++r) {
+                    if (T0) acc[0][FIRST + r] = __fmaf_rn(scaled_lead(x[r], neg_s, y0), u0, acc[0][FIRST + r]);
+                    if (T1) acc[1][FIRST + r] = __fmaf_rn(scaled_lead(x[r], neg_s, y1), u1, acc[1][FIRST + r]);
+                    if (T2) acc[2][FIRST + r] = __fmaf_rn(scaled_lead(x[r], neg_s, y2), u2, acc[2][FIRST + r]);
+                }
+            };
+            asm volatile("" :: "s"(xa[0]), "s"(xa[HALF - 1]));              // (waits for this half)
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int r = 0; r < HALF; ++r) xb[r] = x_at[HALF + r];
+            __builtin_amdgcn_sched_barrier(0);
+            half(xa, std::integral_constant<int, 0>{});
+            if (T0 && with_bias) {                                          // block-uniform: a branch, not a select
+                asm volatile("");
+                acc_bias = __fmaf_rn(scaled_lead(biasvolt, neg_s, y0), u0, acc_bias);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            asm volatile("" :: "s"(xb[0]), "s"(xb[HALF - 1]));
+            __builtin_amdgcn_sched_barrier(0);
+            x_at = x_next;
+#pragma unroll
+            for (int r = 0; r < HALF; ++r) xa[r] = x_at[r];
+            __builtin_amdgcn_sched_barrier(0);
+            half(xb, std::integral_constant<int, HALF>{});
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        constexpr std::true_type yes;
+        constexpr std::false_type no;
+        for (int s = s_lo; s < s_hi;) {                                     // s: first patch of a run that shares an image row
+            const int run = min(Nw - nw, s_hi - s);
+            s += run;
+            // the first pixel of the next run (behind the last one: this run's, requested for nothing)
+            scalar_cfloat* x_run = x_at + next_row - (ptrdiff_t)nw * C;
+            nw = 0;
+            if (++nh == Nh) { nh = 0; x_run += next_image; }
+            if (s >= s_hi) x_run = x_at;
+            u0 = u1 = 0.0f;
+            pixel(yes, no, no, x_at + C);
+            if (run > 1) {
+                pixel(yes, yes, no, x_at + C);
+#pragma clang loop unroll(disable)
+                for (int t = 2; t < run; ++t) pixel(yes, yes, yes, x_at + C);
+            }
+            pixel(no, yes, yes, x_at + C);
+            pixel(no, no, yes, x_run);
+        }
+    }
+    // the wavefronts' sums, one kernel column at a time
+    float* out = dst + (size_t)slice * rows * Kc;
+#pragma unroll
+    for (int t = 0; t < DWT_KW; ++t) {
+        if (t > 0) __syncthreads();
+        if (wave > 0) {
+#pragma unroll
+            for (int r = 0; r < CB; ++r) red[wave - 1][r][lane] = acc[t][r];
+            if (t == 0) red[wave - 1][CB][lane] = acc_bias;
+        }
+        __syncthreads();
+        if (wave == 0 && j < Kc) {
+            const size_t row0 = (size_t)(kh * DWT_KW + t) * C + c0;
+            auto total = [&](float sum, int r) {
+#pragma unroll
+                for (int v = 0; v < DWT_WAVES - 1; ++v) sum += red[v][r][lane];
+                return sum * post;
+            };
+#pragma unroll
+            for (int r = 0; r < CB; ++r) out[(row0 + r) * Kc + j] = total(acc[t][r], r);
+            if (t == 0 && with_bias) out[(size_t)bias_row * Kc + j] = total(acc_bias, CB);
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------------------------
 // dW for layers with at most 32 output channels.  Lane = (half, kc): the two halves of a wavefront
 // take alternate patches, so no lane idles.  The 32 inputs of a patch that a block's rows need are
 // fetched two per lane (lane r of the first 16 lanes of a half fetches inputs r and 16 + r of the half's own
@@ -656,16 +814,44 @@ static int64_t cv_grad_weight_row_blocks(const ConvGeom& g) {
     return g.Kh * ((g.Kw * g.C + DWW_RI - 1) / DWW_RI);
 }
 
-int cv_grad_weight_wide_blocks(const ConvGeom& g) {
-    return (int)(((g.Kc + kWave - 1) / kWave) * cv_grad_weight_row_blocks(g));
+// Channels a wavefront of cv_grad_weight_taps_kernel owns, 0: the layer goes to the kernels for any shape.  Thirty-two where that makes
+// workgroups enough; launches that do not fill the chip keep the blocks of 32 weight rows, of which there are three times as many (3136 patches of
+// 64 channels to 64: 15.2 us against 18 – 20, 784 of 128 to 100 16.2 against 18 – 20); 32 channels to 64 are three workgroups a slice, or six of sixteen
+// channels (32 768 patches 40 / 38 us).  Channels in sixteens otherwise (100 352 patches of 16 to 48 38 -> 30 us, 784 of 112 to 48
+// 14.6 -> 13.0; 1200 of 16 to 128, too few for it, 11.3 against 13.0).
+static int cv_grad_weight_taps_channels(const ConvGeom& g) {
+    if (g.Kw != DWT_KW || g.Sw != 1 || g.C % 16 != 0 || g.Kc <= 32 || g.S * g.Kc * 4 >= 0x7fffffffLL) return 0;
+    const int64_t blocks16 = (g.Kc + kWave - 1) / kWave * g.Kh * (g.C / 16);
+    if (g.C % 32 != 0) return blocks16 * std::min<int64_t>(g.S / 128, 128) >= 100 ? 16 : 0;
+    if (blocks16 * std::min<int64_t>(g.S / 128, 128) < 700) return 0;
+    return blocks16 >= 12 ? 32 : 16;
+}
+
+// Workgroups per slice of the kernels for any shape, and slices that the patch range is cut into (cv_grad_weight_taps_kernel: its
+// workgroups have twice as many wavefronts).
+int cv_grad_weight_row32_blocks(const ConvGeom& g) { return (int)(((g.Kc + kWave - 1) / kWave) * cv_grad_weight_row_blocks(g)); }
+int cv_grad_weight_splits(const ConvGeom& g) {
+    const int cb = cv_grad_weight_taps_channels(g);
+    return cb ? weight_grad_splits(g.S / 2, (g.Kc + kWave - 1) / kWave * g.Kh * (g.C / cb) * 2)
+              : weight_grad_splits(g.S, cv_grad_weight_row32_blocks(g));
 }
 
 // All rows of dW, bias row included (or of every partial-sum slice when nsplit > 1).
 int launch_cv_grad_weight_wide(const float* xpad, const float* upm, const float* ym, float* dst, int nsplit,
                                const ConvGeom& g, int64_t rows, const NeuronParams& np, hipStream_t stream) {
     const int seg_per_slice = (int)((g.S + nsplit - 1) / nsplit);
-    dim3 grid((unsigned)((g.Kc + kWave - 1) / kWave), (unsigned)cv_grad_weight_row_blocks(g), (unsigned)nsplit);
+    const int taps = cv_grad_weight_taps_channels(g);
+    dim3 grid((unsigned)((g.Kc + kWave - 1) / kWave), (unsigned)(taps ? g.Kh * (g.C / taps) : cv_grad_weight_row_blocks(g)), (unsigned)nsplit);
     if (grid.y > 65535u) return fail(SNNTC_ERR_TOO_LARGE, "weight gradient: too many weight rows");
+    if (taps) {
+        KernelTimerScope timer_("grad_weight", stream);
+        const LeadScale ls = lead_scale(np.max_time);
+        hipLaunchKernelGGL(taps == 32 ? cv_grad_weight_taps_kernel<32> : cv_grad_weight_taps_kernel<16>, dim3(grid.x * grid.y * grid.z), dim3(DWT_WAVES * kWave), 0, stream, xpad, upm, ym, dst, (int)g.S, (int)g.Kc, (int)rows,
+                           seg_per_slice, (int)g.H, (int)g.W, (int)g.C, (int)g.Sh, (int)g.Nh, (int)g.Nw, (int)grid.x, (int)grid.y, np.bias ? (int)g.P : -1,
+                           np.biasvolt, ls.neg_s, ls.post);
+        SNNTC_HIP_CHECK(hipGetLastError());
+        return SNNTC_OK;
+    }
     // patches before s_safe can fetch DWW_RI floats from any of their kernel-row starts without leaving
     // the image tensor (only the last few patches of the last image cannot)
     const int64_t n_x = g.B * g.H * g.W * g.C;

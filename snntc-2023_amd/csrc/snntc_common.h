@@ -222,7 +222,8 @@ int launch_cv_grad_input_chan(const float* xpad, const float* wq, const float* u
                               float* dx, const CropGeom& crop, const ConvGeom& g, const NeuronParams& np,
                               hipStream_t stream);
 bool cv_grad_weight_wide_supported(const ConvGeom& g);
-int cv_grad_weight_wide_blocks(const ConvGeom& g);
+int cv_grad_weight_row32_blocks(const ConvGeom& g);
+int cv_grad_weight_splits(const ConvGeom& g);
 int launch_cv_grad_weight_wide(const float* xpad, const float* upm, const float* ym, float* dst, int nsplit,
                                const ConvGeom& g, int64_t rows, const NeuronParams& np, hipStream_t stream);
 

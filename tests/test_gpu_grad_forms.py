@@ -110,3 +110,55 @@ def test_conv_input_gradients_at_the_edges_of_tiles(B, H, W, C, Kc, S):
     for h, wd, top, left in [(H - 2, W - 2, 1, 1), (1, W // 2 + 1, H // 2, 1), (H, W - 1, 0, 0), (2, 2, 0, W - 2)]:
         part = ops.snncv_grad(t(g), t(xpad), t(w), p, t(out), crop=(h, wd, top, left))[0].cpu().numpy()
         assert np.array_equal(part, dx[:, top:top + h, left:left + wd])
+
+
+@pytest.mark.parametrize("bias", [True, False])
+@pytest.mark.parametrize("B,H,W,C,Kc,Kh,Sh", [
+    (40, 8, 9, 32, 64, 3, 1), (9, 21, 23, 64, 65, 3, 1), (30, 12, 5, 64, 128, 3, 2), (60, 9, 4, 64, 64, 2, 1),       # 32 channels a wavefront; rows of 7, 21, 3 and 2 patches
+    (130, 6, 3, 96, 64, 3, 1), (7, 40, 12, 16, 40, 3, 1), (20, 9, 19, 48, 130, 3, 1), (6, 22, 22, 80, 33, 1, 1),     # one patch a row; sixteen channels
+])
+def test_conv_weight_gradients_by_pixels(B, H, W, C, Kc, Kh, Sh, bias):
+    """Three-column kernels: runs of patches that begin and end within rows and images, the last slices without a patch for some wavefronts."""
+    import ctypes
+    import snntc_amd as snn
+    from snntc_amd import _lib
+    rng = np.random.default_rng(B + H + W + C + Kc)
+    x = np.exp(rng.random((B, H, W, C))).astype(np.float32)
+    x[rng.random(x.shape) < 0.1] = 1e5
+    p = capi.cv_params(Kh, 3, Sh, 1, same=False, biasvolt=1.0 if bias else 0.0)
+    Nh, Nw, _ = capi.cv_dims(x.shape, p)
+    w = rng.standard_normal((Kh * 3 * C + int(bias), Kc)).astype(np.float32)
+    out = np.concatenate([np.exp(1.2 * rng.random((B, Nh, Nw, Kc))), rng.standard_normal((B, Nh, Nw, Kc))]).astype(np.float32)
+    dead = rng.random((B, Nh, Nw, Kc)) < 0.1
+    out[:B][dead] = 1e5
+    out[B:][dead] = 0.0
+    g = np.zeros((2 * B, Nh, Nw, Kc), np.float32)
+    g[:B] = rng.standard_normal((B, Nh, Nw, Kc))
+    dw = snn.snncv_grad(t(g), t(x), t(w), p, t(out))[1]
+    _, rdw, _ = capi.cv_backward_dev(g, x, w, p, out, wide=True)
+    ao = out.copy()
+    ao[B:] = np.abs(ao[B:])
+    _, adw, _ = capi.cv_backward_dev(np.abs(g), x, w, p, ao, wide=True)
+    # (a few thousand terms of either sign, 2e-7 of |terms| as for the dense gradients' partial sums, and a margin)
+    assert np.all(np.abs(dw.cpu().numpy() - rdw) <= 2e-6 * np.abs(adw) + 1e-30)
+    # with the room that the kernels for any shape ask for there are fewer slices, and with less the call is refused
+    lib = _lib.load()
+    need = ctypes.c_size_t()
+    fp = np.ascontiguousarray(p, np.float32).ctypes.data_as(ctypes.POINTER(ctypes.c_float))
+    _lib.check(lib.snntc_cv_backward_workspace_bytes(B, H, W, C, Kc, fp, ctypes.byref(need)))
+    args = [t(g), t(x), t(w), t(out)]
+    again = torch.empty_like(dw)
+    stream = torch.cuda.current_stream().cuda_stream
+    ws = torch.empty(need.value, dtype=torch.uint8, device=DEV)
+    ptr = lambda a: a.data_ptr() if a is not None else None                      # noqa: E731
+    call = lambda n: lib.snntc_cv_backward(ptr(args[0]), ptr(args[1]), ptr(args[2]), fp, ptr(args[3]), None, ptr(again), None, B, H, W, C, Kc,   # noqa: E731
+                                           w.shape[0], 2 * B, ptr(ws), n, stream)
+    assert call(need.value) == _lib.OK
+    assert torch.equal(again, dw)
+    for room in range(need.value - 256, 0, -max(256, need.value // 40 // 256 * 256)):
+        if call(room) != _lib.OK:
+            break
+        err = np.abs(again.cpu().numpy() - rdw)
+        assert np.all(err <= 2e-6 * np.abs(adw) + 1e-30)
+    else:
+        raise AssertionError("no workspace was refused")
