@@ -28,26 +28,28 @@ constexpr int DX_TILE = 8;
 constexpr int DX_WAVES3 = 4;           // wavefronts per SIMD the KW = 3 variant is compiled for
 
 // Eight masked MACs  acc += upm_k * (x <= ym_k ? w_k : 0).  A compare and a select next to a multiply-add: both take the
-// slower of a SIMD's two pipes, but a third of such a stream leaves it enough else to do, and all three have four-byte
-// encodings (probe kernels, four wavefronts per SIMD: 2.3 clocks an instruction; the mask as two multiply-adds, m = clamp01((x - ym) * BIG) and
-// w - m * w, takes 2.9).
-#define SNNTC_DX_M(K) "v_cmp_ge_f32_e32 vcc, %[y" #K "], %[x]\n"
-#define SNNTC_DX_T(K, T) "v_cndmask_b32_e32 %[" #T "], 0, %[w" #K "], vcc\n"
+// slower of a SIMD's two pipes, but a third of such a stream leaves it enough else to do (probe kernels, four wavefronts per
+// SIMD: 2.3 clocks an instruction; the mask as two multiply-adds, m = clamp01((x - ym) * BIG) and w - m * w, takes 2.9).  A
+// mask is read two instructions after the compare that writes it, at the earliest: three are under way at the start, then two, one in
+// vcc, the others in registers.
+#define SNNTC_DX_MV(K) "v_cmp_ge_f32_e32 vcc, %[y" #K "], %[x]\n"
+#define SNNTC_DX_MS(K, S) "v_cmp_ge_f32_e64 %[" #S "], %[y" #K "], %[x]\n"
+#define SNNTC_DX_TV(K, T) "v_cndmask_b32_e32 %[" #T "], 0, %[w" #K "], vcc\n"
+#define SNNTC_DX_TS(K, T, S) "v_cndmask_b32_e64 %[" #T "], 0, %[w" #K "], %[" #S "]\n"
 #define SNNTC_DX_F(K, T) "v_fmac_f32_e32 %[acc], %[u" #K "], %[" #T "]\n"
 
 __device__ __forceinline__ void dx_mac8(float& acc, float x, const float* u, const float* y, const float* w) {
     float ta, tb;
+    uint64_t m, n;
     asm volatile(
-        SNNTC_DX_M(0) SNNTC_DX_T(0, ta)
-        SNNTC_DX_M(1) SNNTC_DX_T(1, tb) SNNTC_DX_F(0, ta)
-        SNNTC_DX_M(2) SNNTC_DX_T(2, ta) SNNTC_DX_F(1, tb)
-        SNNTC_DX_M(3) SNNTC_DX_T(3, tb) SNNTC_DX_F(2, ta)
-        SNNTC_DX_M(4) SNNTC_DX_T(4, ta) SNNTC_DX_F(3, tb)
-        SNNTC_DX_M(5) SNNTC_DX_T(5, tb) SNNTC_DX_F(4, ta)
-        SNNTC_DX_M(6) SNNTC_DX_T(6, ta) SNNTC_DX_F(5, tb)
-        SNNTC_DX_M(7) SNNTC_DX_T(7, tb) SNNTC_DX_F(6, ta)
-        SNNTC_DX_F(7, tb)
-        : [acc] "+v"(acc), [ta] "=&v"(ta), [tb] "=&v"(tb)
+        SNNTC_DX_MV(0) SNNTC_DX_MS(1, m) SNNTC_DX_MS(2, n) SNNTC_DX_TV(0, ta) SNNTC_DX_TS(1, tb, m)
+        SNNTC_DX_MV(3) SNNTC_DX_F(0, ta) SNNTC_DX_TS(2, ta, n)
+        SNNTC_DX_MS(4, m) SNNTC_DX_F(1, tb) SNNTC_DX_TV(3, tb)
+        SNNTC_DX_MV(5) SNNTC_DX_F(2, ta) SNNTC_DX_TS(4, ta, m)
+        SNNTC_DX_MS(6, m) SNNTC_DX_F(3, tb) SNNTC_DX_TV(5, tb)
+        SNNTC_DX_MV(7) SNNTC_DX_F(4, ta) SNNTC_DX_TS(6, ta, m)
+        SNNTC_DX_F(5, tb) SNNTC_DX_F(6, ta) SNNTC_DX_TV(7, tb) SNNTC_DX_F(7, tb)
+        : [acc] "+v"(acc), [ta] "=&v"(ta), [tb] "=&v"(tb), [m] "=&s"(m), [n] "=&s"(n)
         : [x] "v"(x), [y0] "v"(y[0]), [y1] "v"(y[1]), [y2] "v"(y[2]), [y3] "v"(y[3]), [y4] "v"(y[4]),
           [y5] "v"(y[5]), [y6] "v"(y[6]), [y7] "v"(y[7]), [u0] "v"(u[0]), [u1] "v"(u[1]), [u2] "v"(u[2]),
           [u3] "v"(u[3]), [u4] "v"(u[4]), [u5] "v"(u[5]), [u6] "v"(u[6]), [u7] "v"(u[7]), [w0] "v"(w[0]),
