@@ -105,7 +105,7 @@ __device__ __forceinline__ void wave_lds_order() {
 // at 333.)
 // ---------------------------------------------------------------------------------------------
 constexpr int DX_A = 2, DX_S = 8 * DX_A, DX_I = 32, DX_JC = 16, DX_PITCH = 36;         // (pitch: the transposing writes of the pieces spread over the banks)
-constexpr int dx_threads(int split) { return (split == 1 ? 4 : split) * kWave; }
+constexpr int dx_threads(int split) { return (split == 1 ? 4 : split) * kWave; }     // (single-wavefront tiles of a joint launch: eight wavefronts)
 constexpr int dx_lds_bytes(int split) { return dx_threads(split) / kWave * 3 * DX_JC * DX_PITCH * 4; }
 
 // Upstream values of a backward pass: the prologue's, or (RAW) formed where they are staged, which saves small batches a launch.
@@ -137,7 +137,7 @@ fc_grad_input_tile(const SegmentSource& src, const float* __restrict__ w, const 
     const int lane = threadIdx.x % kWave;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int block = xcd_contiguous(block_index, blocks);
-    const int tile_raw = SPLIT == 1 ? block * 4 + wave : block;
+    const int tile_raw = SPLIT == 1 ? block * (int)(blockDim.x / kWave) + wave : block;
     const int tile = min(tile_raw, n_tiles - 1);
     const int ts = tile / tiles_i, s0 = ts * TS, i0 = (tile - ts * tiles_i) * DX_I;
     const int sg = lane / 8, ig = lane % 8;
@@ -396,7 +396,7 @@ grad_weight_kernel(SegmentSource src, const float* __restrict__ upm, const float
 // dW of a dense layer.  A workgroup owns 64 weight rows x 64 outputs, its wavefronts take the slice's samples eight at a
 // time in turn, a lane 8 x 8 of the tile: a sample's 64 inputs, output times and upstream values are three coalesced loads, a
 // batch ahead, go to a piece of LDS of the wavefront's own and come back as six 16-byte reads for 128 vector instructions.
-// Rows past the inputs read biasvolt, so the bias row needs no code of its own.  The wavefronts' sums are added in order
+// Rows past the inputs read biasvolt, so the bias row needs no code of its own.  The wavefronts' sums are added in a tree
 // through LDS.
 // What bounds it: the addition and the multiply-add of a term (3.3 clocks each at 4096 samples).  Before, eight rows and one
 // output per lane: two LDS reads of 8 clocks and 512 bytes of y / up per 16 instructions.  us: 4096 x 784 -> 800 254 -> 158,
@@ -492,10 +492,14 @@ grad_weight_dense_tile(const float* __restrict__ x, const Upstream& upstream, co
         __syncthreads();
         for (int e = threadIdx.x; e < SUMS; e += WAVES * kWave) {
             const int tr = e / DWD_T, i = i0 + tr / 4 * 8 + 4 * half + tr % 4, j = j0 + e % DWD_T;
-            float sum = lds[e];
+            float sum[WAVES];
 #pragma unroll
-            for (int v = 1; v < WAVES; ++v) sum += lds[v * SUMS + e];
-            if (i < rows && j < J) out[(size_t)i * J + j] = sum * post;
+            for (int v = 0; v < WAVES; ++v) sum[v] = lds[v * SUMS + e];
+#pragma unroll
+            for (int h = WAVES / 2; h > 0; h /= 2)
+#pragma unroll
+                for (int v = 0; v < h; ++v) sum[v] += sum[v + h];
+            if (i < rows && j < J) out[(size_t)i * J + j] = sum[0] * post;
         }
     }
 }
@@ -510,25 +514,27 @@ grad_weight_dense_kernel(const float* __restrict__ x, const float* __restrict__ 
                                          blockIdx.x, blockIdx.y, blockIdx.z, lds);
 }
 
-// The whole backward pass of a dense layer on a small batch in one launch: the first dx_blocks workgroups take dX tiles, the others
-// dW tiles, and both form the upstream values as they stage them.  Each part alone leaves the chip half empty and waits for its first
-// loads.  us, prologue, dX and dW / together, 784 -> 800: 1 row 18.5 / 14.0, 64 rows 22 / 16, 128 27 / 19.5, 256 41.5 / 38, 400 57 / 58,
-// 512 70 / 56; 128 rows of 2048 -> 512 35 / 30, of 128 -> 128 16.5 / 10.6.
+// The whole backward pass of a dense layer on a small batch in one launch: dX tiles of eight wavefronts (below 64 outputs, SPLIT 1, eight
+// tiles of one) and dW tiles, which both form the upstream values as they stage them.  Each part alone leaves the chip half empty and waits
+// for its first loads.  us, prologue, dX and dW (and the sum of its slices) / together, 784 -> 800: 1 row 18.5 / 14.0, 64 rows 22 / 16, 128
+// 27 / 19.5, 256 41.5 / 35, 400 57 / 49; 128 rows of 2048 -> 512 35 / 30, of 128 -> 128 16.5 / 10.6, of 784 -> 100 26.4 / 12.6, of 500 -> 50 29.5 / 12.8.
+template <int SPLIT>
 __global__ void __launch_bounds__(8 * kWave, 4)
 fc_backward_kernel(const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ grad, const float* __restrict__ y,
                    const float* __restrict__ rcp, float* __restrict__ dx, float* __restrict__ dw, float* __restrict__ zeros, int n_zeros,
-                   int B, int I, int J, int rows, int tiles_i, int dx_blocks, int dw_cols, float max_cmp, float biasvolt, float neg_s,
+                   int B, int I, int J, int rows, int tiles_i, int dx_tiles, int dx_blocks, int dx_first, int dw_cols, float max_cmp, float biasvolt, float neg_s,
                    float post) {
     constexpr int FLOATS = dwd_lds_floats(8) > dx_lds_bytes(8) / 4 ? dwd_lds_floats(8) : dx_lds_bytes(8) / 4;
     __shared__ __align__(16) float lds[FLOATS];
     const Upstream upstream{grad, rcp, max_cmp};
     if (blockIdx.x == 0 && (int)threadIdx.x < n_zeros) zeros[threadIdx.x] = 0.0f;          // the dParams output
-    if ((int)blockIdx.x < dx_blocks) {
+    const int dx_block = (int)blockIdx.x - dx_first;
+    if (dx_block >= 0 && dx_block < dx_blocks) {
         SegmentSource src{};
         src.base = x; src.conv = 0; src.I = I;
-        fc_grad_input_tile<8, false, true>(src, w, upstream, y, dx, B, I, J, tiles_i, dx_blocks, blockIdx.x, dx_blocks, lds);
+        fc_grad_input_tile<SPLIT, false, true>(src, w, upstream, y, dx, B, I, J, tiles_i, dx_tiles, dx_block, dx_blocks, lds);
     } else {
-        const int tile = (int)blockIdx.x - dx_blocks, by = tile / dw_cols;
+        const int tile = dx_block < 0 ? (int)blockIdx.x : dx_block - dx_blocks, by = tile / dw_cols;
         grad_weight_dense_tile<8, true>(x, upstream, y, dw, B, I, J, rows, B, biasvolt, neg_s, post, tile - by * dw_cols, by, 0, lds);
     }
 }
@@ -916,24 +922,45 @@ int launch_reduce_partials(const float* partial, float* dw, int64_t n, int nspli
     return SNNTC_OK;
 }
 
-// dX and dW of a dense layer in one launch (dX == NULL: dW alone), where its workgroups, of which a CU holds two, come in at most
-// two turns: beyond, the parts alone fill the chip, with tiles of their own.  (Eight wavefronts share a dX tile's outputs, sixteen each.)
-bool fc_backward_joint_supported(int64_t B, int64_t I, int64_t J, bool dx) {
-    const int64_t dx_tiles = dx ? (B + DX_S - 1) / DX_S * ((I + DX_I - 1) / DX_I) : 0;
-    const int64_t dw_tiles = ((J + DWD_T - 1) / DWD_T) * ((I + 1 + DWD_T - 1) / DWD_T);
-    return J >= DX_JC * 8 && dx_tiles + dw_tiles <= 1024;
+// Workgroups of a joint launch: dX tiles (below 64 outputs, eight of them) and dW tiles.
+struct JointGrid { int64_t dx_tiles, dx_blocks, dw_blocks; };
+static JointGrid joint_grid(int64_t B, int64_t I, int64_t rows, int64_t J, bool dx) {
+    JointGrid g{};
+    g.dx_tiles = dx ? (B + DX_S - 1) / DX_S * ((I + DX_I - 1) / DX_I) : 0;
+    g.dx_blocks = J < 64 ? (g.dx_tiles + 7) / 8 : g.dx_tiles;
+    g.dw_blocks = (J + DWD_T - 1) / DWD_T * ((rows + DWD_T - 1) / DWD_T);
+    return g;
+}
+
+// dX and dW of a dense layer in one launch (dX == NULL: dW alone).  `slices`: what the samples would be cut into for dW alone.
+// The parts of a launch with more workgroups fill the chip by themselves, with tiles of their own (us, apart / together: 200 x 2048 ->
+// 512, 1096 workgroups, 61 / 42; 333 x 1521 -> 777, 1320, 87 / 73; 400 x 3000 -> 512, 2726, 116 / 99; 512 x 3000 -> 512, 3384, 140 / 126; 300 x
+// 4096 -> 1000, 3472, 211 / 214; 400 x 10 000 -> 200, 8453, 171 / 179).  A tile of dW goes over all samples here, which up to some
+// hundred of them takes less than the launches that slices need (200 x 128 -> 128 29 / 15.4, 333 x 333 -> 333 34 / 23, 400 x 500 -> 50 34 / 24.5,
+// 512 x 128 -> 128 28.4 / 30.3; dW alone, 333 x 128 -> 128 22.4 / 21.3, 400 rows 22.3 / 24.2).
+bool fc_backward_joint_supported(int64_t B, int64_t I, int64_t J, bool dx, int slices) {
+    const JointGrid g = joint_grid(B, I, I + 1, J, dx);
+    return g.dx_blocks + g.dw_blocks <= 3072 && (slices == 1 || B <= (dx ? 448 : 352));
 }
 
 int launch_fc_backward_joint(const float* x, const float* w, const float* grad, const float* y, const float* rcp, float* dx, float* dw,
                              float* zeros, int n_zeros, int64_t B, int64_t I, int64_t J, const NeuronParams& np, hipStream_t stream) {
-    const int64_t rows = I + np.bias, tiles_i = (I + DX_I - 1) / DX_I, dx_blocks = dx ? (B + DX_S - 1) / DX_S * tiles_i : 0;
-    const int64_t dw_cols = (J + DWD_T - 1) / DWD_T, dw_blocks = dw_cols * ((rows + DWD_T - 1) / DWD_T);
+    const int64_t rows = I + np.bias;
+    const JointGrid g = joint_grid(B, I, rows, J, dx != nullptr);
+    // The longer tiles come first, so that the shorter ones fill the end: dW takes 8192 terms a sample, dX 512 an output, of which it
+    // does a third as many a clock.  (us, dX / dW first: 256 x 784 -> 800 41 / 35, 400 rows 62 / 49, 300 x 1521 -> 777 64 / 59; 256 x 300 -> 2048
+    // 38 / 46, 32 x 3000 -> 512 15.3 / 20.7.)  Where all workgroups, of which a CU holds two, are there at once, only much longer ones
+    // (128 x 1000 -> 130 15 / 13, but 333 x 512 -> 1000 35.5 / 37), and not where the dW tiles behind the first turn are many and have a CU
+    // each (333 x 784 -> 800 43 / 46.5, 128 x 1521 -> 777 33 / 34).
+    const int64_t behind = g.dx_blocks + g.dw_blocks - 512;
+    const bool dw_first = behind <= 0 ? 2 * B > J : 4 * B > J && !(behind >= 128 && behind <= 256);
     const LeadScale ls = lead_scale(np.max_time);
     {
         KernelTimerScope timer_("fc_backward", stream);
-        hipLaunchKernelGGL(fc_backward_kernel, dim3((unsigned)(dx_blocks + dw_blocks)), dim3(8 * kWave), 0, stream, x, w, grad, y, rcp, dx,
-                           dw, zeros, zeros ? n_zeros : 0, (int)B, (int)I, (int)J, (int)rows, (int)tiles_i, (int)dx_blocks, (int)dw_cols,
-                           np.max_cmp, np.biasvolt, ls.neg_s, ls.post);
+        auto kern = J < 64 ? fc_backward_kernel<1> : fc_backward_kernel<8>;
+        hipLaunchKernelGGL(kern, dim3((unsigned)(g.dx_blocks + g.dw_blocks)), dim3(8 * kWave), 0, stream, x, w, grad, y, rcp, dx, dw, zeros,
+                           zeros ? n_zeros : 0, (int)B, (int)I, (int)J, (int)rows, (int)((I + DX_I - 1) / DX_I), (int)g.dx_tiles, (int)g.dx_blocks,
+                           (int)(dw_first ? g.dw_blocks : 0), (int)((J + DWD_T - 1) / DWD_T), np.max_cmp, np.biasvolt, ls.neg_s, ls.post);
     }
     SNNTC_HIP_CHECK(hipGetLastError());
     return SNNTC_OK;

@@ -189,7 +189,7 @@ int order_prepare_device();
 int launch_backward_prologue(const float* grad, const float* y, const float* rcp, float* upm, int64_t n, const NeuronParams& np, const float* w, float* wt, int64_t rows,
                              int64_t cols, int64_t chan, float* zeros, int n_zeros, hipStream_t stream);
 
-bool fc_backward_joint_supported(int64_t B, int64_t I, int64_t J, bool dx);
+bool fc_backward_joint_supported(int64_t B, int64_t I, int64_t J, bool dx, int slices);
 int launch_fc_backward_joint(const float* x, const float* w, const float* grad, const float* y, const float* rcp, float* dx, float* dw,
                              float* zeros, int n_zeros, int64_t B, int64_t I, int64_t J, const NeuronParams& np, hipStream_t stream);
 int launch_fc_grad_input(const float* x, const float* w, const float* upm, const float* ym, float* dx,

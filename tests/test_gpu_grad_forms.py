@@ -77,6 +77,39 @@ def test_dense_gradients_in_one_launch(B, I, J, bias):
     assert np.all(np.abs(dw - rdw) <= 1e-6 * np.abs(adw) + 1e-30)
 
 
+@pytest.mark.parametrize("B,I,J", [
+    (1, 1, 17), (129, 255, 17), (33, 64, 63), (40, 65, 64), (17, 31, 127),                    # dX tiles of one wavefront, of eight
+    (352, 70, 130), (353, 70, 130), (448, 40, 50), (449, 40, 50),                             # slices alone up to here, behind it
+    (130, 100, 260), (131, 100, 260), (256, 784, 700), (300, 784, 770),                       # dX tiles first, dW tiles first
+    (370, 2048, 1000), (430, 3000, 500), (446, 3300, 500),                                    # up to 3072 workgroups, and more
+])
+def test_dense_gradients_whole_or_in_parts(B, I, J):
+    """Both sides of the rules that choose one launch, the order of its tiles and their form, within the band of the fp64 sums."""
+    import snntc_amd as snn
+    rng = np.random.default_rng(B + I + J)
+    x = np.exp(rng.random((B, I))).astype(np.float32)
+    x[rng.random((B, I)) < 0.1] = 1e5
+    y = np.exp(1.2 * rng.random((B, J))).astype(np.float32)
+    y[rng.random((B, J)) < 0.1] = 1e5
+    x[0, : min(I, J)] = y[0, : min(I, J)]
+    w = rng.standard_normal((I + 1, J)).astype(np.float32)
+    out = np.concatenate([y, rng.random((B, J)).astype(np.float32)])
+    g = np.zeros((2 * B, J), np.float32)
+    g[:B] = rng.standard_normal((B, J))
+    p = capi.fc_params(1.0)
+    args = (t(g), t(x), t(w), p, t(out))
+    dx, dw, _ = snn.snnfc_grad(*args)
+    alone = snn.snnfc_grad(*args, want_dx=False)[1].cpu().numpy()
+    assert torch.equal(dx, snn.snnfc_grad(*args, want_dw=False)[0])                           # a sample's sums depend on J alone
+    dx, dw = dx.cpu().numpy(), dw.cpu().numpy()
+    rdx, rdw, _ = capi.fc_backward_dev(g, x, w, p, out, wide=True)
+    adx, adw, _ = capi.fc_backward_dev(np.abs(g), x, np.abs(w), p, out, wide=True)
+    # (a sum's partial sums of either sign stay well below its terms' absolute sum: a few roundings of that, as above)
+    assert np.all(np.abs(dx - rdx) <= 1e-6 * np.abs(adx) + 1e-30)
+    for got in (dw, alone):
+        assert np.all(np.abs(got - rdw) <= 1e-6 * np.abs(adw) + 1e-30)
+
+
 @pytest.mark.parametrize("B,H,W,C,Kc,S", [
     (2, 5, 9, 64, 64, 1), (2, 4, 10, 64, 128, 1), (1, 3, 11, 65, 16, 1), (1, 5, 16, 32, 64, 1), (2, 3, 18, 20, 32, 1),      # tiles of 8 to 128 pixels
     (1, 4, 19, 3, 64, 1), (1, 3, 30, 7, 48, 1), (2, 3, 31, 64, 80, 2), (1, 7, 34, 33, 64, 1), (3, 9, 8, 64, 256, 1), (1, 3, 3, 4, 16, 1),
