@@ -993,6 +993,12 @@ constexpr float ROUND_DX = 0x1p-14f;                      // 1024u
 // the slack of a round next to a threshold of one; beyond 0.6 of it rounds end early (576 inputs with deviation 3.87 / sqrt(I): at 0.15 of a row).
 constexpr float ROUNDS_UP_TO = 0.6f;
 constexpr int ROUNDS_FROM = 400;
+// Few wavefronts (LONE): 41 instructions a chunk instead of 51, with the decision once per turn of the entries' ring, whose requests and
+// weights go on into the chunks behind.  A wavefront fetches a second loop of some 3 KB of code for it, so only the rows of slices of
+// eight columns are long enough (us without / with: 49 segments of 4608 to 512 86 / 78, 100 of 4096 to 256 77 / 70, 200 of 3000 to 300 74 / 69,
+// deviation 3.87 / sqrt(I) 109 / 102, 87 / 80, 136 / 134; sixteen columns, 16 of 2048 to 512 33.9 / 35.0, 100 of 2400 to 64 38.6 / 40.4, 128 of
+// 1521 to 500 32.1 / 33.0).
+constexpr int LONE_ROUNDS_FROM = 1280;
 
 // The test of a chunk for one scan of every lane: wb, yb are the sums behind it.  Lanes in the mask `open`
 // that pass take them over; open lanes that fail keep the sums from before the chunk, take the chunk's
@@ -1504,7 +1510,7 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
         };
         // By rounds of four chunks with one test, until the first scan of the wavefront comes close: all scans take a round over
         // together.  (Lanes without a scan compute along.)
-        if constexpr (ROUNDS) {
+        if constexpr (ROUNDS && !LONE) {
             if (by_rounds && any_odd == 0 && n_full_min >= ROUND * CHUNK) {
                 start_weights(0);
                 int k0 = 0;
@@ -1547,6 +1553,7 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
             }
         }
 
+        bool first_pass = true;                             // (LONE: every armed scan takes part and starts at input 0)
         // Passes: the fast loop for the armed scans that are furthest behind, then the scans it left behind
         // step by step.  A scan that does not close there is armed again.
         // Practically every item takes one pass and a second look without work.
@@ -1612,14 +1619,27 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
                                 : [open] "s"(open[c]), [wb] "v"(end_w_of[c]), [yb] "v"(end_y_of[c]) : "vcc");
                         }
                     };
-                    auto chunk = [&](auto ph_c, int k) {
+                    // BY_ROUND: tested with the other chunks of its round, behind the last of them.
+                    float round_start[CH], x_first;
+                    uint64_t soon = 0, fails = 0;
+                    auto chunk = [&](auto ph_c, int k, auto by_round_c) {
                         constexpr int ph = decltype(ph_c)::value, R = BY_ROW ? ph / ROUND : ph;
+                        constexpr bool BY_ROUND = decltype(by_round_c)::value;
                         // The next entry (block of four chunks, chunk) whose weights will be read, and the test's operands
                         if constexpr (!BY_ROW || ph % ROUND == 0) {
                             constexpr int B = BY_ROW ? (R + 1) % BLOCKS : (ph + 2) % BLOCKS;
                             at[B] = shifted(rp[B]);
-                            test_operands(R, k);
-                            asm volatile("s_nop 1" : "+v"(rx[R].x), "+v"(rx[R].y), "+v"(at[B].x), "+v"(at[B].y), "+v"(nx), "+v"(dx), "+v"(thr));
+                            if constexpr (BY_ROUND) {
+                                asm volatile("s_nop 1" : "+v"(rx[R].x), "+v"(rx[R].y), "+v"(at[B].x), "+v"(at[B].y));
+                            } else {
+                                test_operands(R, k);
+                                asm volatile("s_nop 1" : "+v"(rx[R].x), "+v"(rx[R].y), "+v"(at[B].x), "+v"(at[B].y), "+v"(nx), "+v"(dx), "+v"(thr));
+                            }
+                        }
+                        if constexpr (BY_ROUND && ph % ROUND == 0) {
+                            x_first = BY_ROW ? row_broadcast<0>(__uint_as_float(rx[R].x)) : quad_broadcast<0>(__uint_as_float(rx[R].x));
+#pragma unroll
+                            for (int c = 0; c < CH; ++c) round_start[c] = run_w[c];
                         }
                         float start[CH], low[CH];
                         auto half = [&](auto half_c) {
@@ -1632,16 +1652,29 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
                                 if (hh == 0) start[c] = run_w[c];
                                 accumulate_half<BY_ROW, N>(run_w[c], sums, run_y[c], __uint_as_float(rx[R].x), __uint_as_float(rx[R].y), wv[H % NH][c]);
                                 run_w[c] = sums[3];
-                                if (TIGHT)
+                                if (TIGHT && !BY_ROUND)
                                     low[c] = fminf(fminf(fminf(fminf(hh == 0 ? 0.0f : low[c], sums[0]), sums[1]), sums[2]), sums[3]);
                             }
                             __builtin_amdgcn_sched_barrier(0);
                         };
                         half(std::integral_constant<int, 0>{});
-                        decide();
+                        if constexpr (!BY_ROUND) decide();
                         half(std::integral_constant<int, 1>{});
+                        if constexpr (BY_ROUND && ph % ROUND == ROUND - 1) {
+                            const float x7 = BY_ROW ? row_broadcast<15>(__uint_as_float(rx[R].y)) : quad_broadcast<3>(__uint_as_float(rx[R].y));
+                            const float dx = __fmaf_rn(x7, ROUND_DX, x7 - x_first), x7e = x7 * ROUND_AT;
+                            const float thr = __fmaf_rn(dx, 4.0f * w4, x7 * end_w_round);
 #pragma unroll
-                        for (int c = 0; c < CH; ++c) {
+                            for (int c = 0; c < CH; ++c) {
+                                const float at_end = __fmaf_rn(-x7e, run_w[c], run_y[c]), lowest = fminf(fminf(round_start[c], run_w[c]), 4.0f * w4);
+                                fails |= ran[c] & ~ballot(__fmaf_rn(dx, lowest, at_end) > thr);
+                                // not even with the fall that the rounds up to the next decision bring
+                                if constexpr (ph == PHASES - 1)
+                                    soon |= ran[c] & ~ballot(__fmaf_rn(dx, __fmaf_rn(-(float)(PHASES / ROUND), fabsf(run_w[c]), lowest), at_end) > thr);
+                            }
+                        }
+#pragma unroll
+                        for (int c = 0; c < (BY_ROUND ? 0 : CH); ++c) {
                             if (!TIGHT) low[c] = fminf(fminf(start[c], run_w[c]), w4);
                             pass[c] = chunk_passes<BY_ROW, BY_ROW ? ph % ROUND : 0>(run_w[c], run_y[c], nx, dx, thr, low[c]);
                             end_w_of[c] = run_w[c];
@@ -1650,25 +1683,49 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
                         if constexpr (!BY_ROW) request(ph, min(k + BLOCKS * CHUNK, last_block));
                         else if constexpr (ph % ROUND == ROUND - 1) request(R, min(k - (ROUND - 1) * CHUNK + BLOCKS * BLOCK_INPUTS, last_block));
                     };
-                    // the first weights
-                    at[0] = shifted(rp[0]);
-                    asm volatile("s_nop 1" : "+v"(at[0].x), "+v"(at[0].y));
-                    if constexpr (!BY_ROW) {
-                        at[1] = shifted(rp[1]);
-                        asm volatile("s_nop 1" : "+v"(at[1].x), "+v"(at[1].y));
-                    }
-                    weights(std::integral_constant<int, 0>{});
-                    weights(std::integral_constant<int, 1>{});
-                    weights(std::integral_constant<int, 2>{});
+                    auto first_weights = [&] {
+                        at[0] = shifted(rp[0]);
+                        asm volatile("s_nop 1" : "+v"(at[0].x), "+v"(at[0].y));
+                        if constexpr (!BY_ROW) {
+                            at[1] = shifted(rp[1]);
+                            asm volatile("s_nop 1" : "+v"(at[1].x), "+v"(at[1].y));
+                        }
+                        weights(std::integral_constant<int, 0>{});
+                        weights(std::integral_constant<int, 1>{});
+                        weights(std::integral_constant<int, 2>{});
+                    };
+                    first_weights();
                     int k0 = kmin;
                     bool more = true;
+                    const bool rotate = waves > 4;          // (more than a wavefront per SIMD)
+                    if (ROUNDS && by_rounds && first_pass && any_odd == 0) {
+                        while (soon == 0 && k0 + PHASES * CHUNK <= n_full_min) {
+                            if (rotate) rotate_wave_priority(k0 / (PHASES * CHUNK) + (wave >> 2));
+                            for_each_phase<PHASES>([&](auto ph_c) {
+                                chunk(ph_c, k0 + decltype(ph_c)::value * CHUNK, std::true_type{});
+                                return true;
+                            });
+                            if (fails != 0) break;          // (its rounds again, chunk by chunk)
+#pragma unroll
+                            for (int c = 0; c < CH; ++c) { wsum[c] = run_w[c]; ysum[c] = run_y[c]; }
+                            k0 += PHASES * CHUNK;
+                        }
+#pragma unroll
+                        for (int c = 0; c < CH; ++c) { end_w_of[c] = wsum[c]; end_y_of[c] = ysum[c]; passed[c] = k0 / CHUNK - 1; }
+                        if (fails != 0) {
+                            request_first(k0);
+#pragma unroll
+                            for (int c = 0; c < CH; ++c) { run_w[c] = wsum[c]; run_y[c] = ysum[c]; }
+                            first_weights();
+                        }
+                    }
+                    first_pass = false;
                     // Whole rounds as long as the longest row has one left, without an exit inside (behind an exit between a request
                     // and its use the compiler would move the request to the use), then its last chunks one by one.
-                    const bool rotate = waves > 4;          // (more than a wavefront per SIMD)
                     for (; k0 + PHASES * CHUNK <= n_full_max && more; k0 += PHASES * CHUNK) {
                         if (rotate) rotate_wave_priority(k0 / (PHASES * CHUNK) + (wave >> 2));
                         for_each_phase<PHASES>([&](auto ph_c) {
-                            chunk(ph_c, k0 + decltype(ph_c)::value * CHUNK);
+                            chunk(ph_c, k0 + decltype(ph_c)::value * CHUNK, std::false_type{});
                             return true;
                         });
                         uint64_t any = 0;
@@ -1680,7 +1737,7 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
                         for_each_phase<PHASES>([&](auto ph_c) {
                             const int k = k0 + decltype(ph_c)::value * CHUNK;
                             if (k >= n_full_max) return false;
-                            chunk(ph_c, k);
+                            chunk(ph_c, k, std::false_type{});
                             return true;
                         });
                     decide();
@@ -1987,7 +2044,9 @@ constexpr size_t FILTER_WIDE_COPY_BYTES = 48 * 1024;        // slices from here 
 // The instantiation for ch neurons per lane.
 template <int COLS, bool WANT_K>
 decltype(&scan_filter_kernel<COLS, 1, true, WANT_K>) filter_kernel(int ch, bool lone, bool rounds) {
-    if (ch == 1) return lone ? scan_filter_kernel<COLS, 1, true, WANT_K> : scan_filter_kernel<COLS, 1, false, WANT_K>;
+    constexpr bool LONG_ROWS = COLS == 8;
+    if (ch == 1 && lone) return rounds ? scan_filter_kernel<COLS, 1, true, WANT_K, LONG_ROWS> : scan_filter_kernel<COLS, 1, true, WANT_K>;
+    if (ch == 1) return scan_filter_kernel<COLS, 1, false, WANT_K>;
     if (ch == FILTER_MAX_CH<COLS>)
         return rounds ? scan_filter_kernel<COLS, FILTER_MAX_CH<COLS>, false, WANT_K, true> : scan_filter_kernel<COLS, FILTER_MAX_CH<COLS>, false, WANT_K>;
     if constexpr (COLS == 64) {
@@ -2001,6 +2060,8 @@ int raise_scan_lds_limits() {
     const void* whole[] = {
         reinterpret_cast<const void*>(filter_kernel<COLS, true>(1, true, false)),
         reinterpret_cast<const void*>(filter_kernel<COLS, false>(1, true, false)),
+        reinterpret_cast<const void*>(filter_kernel<COLS, true>(1, true, true)),
+        reinterpret_cast<const void*>(filter_kernel<COLS, false>(1, true, true)),
         reinterpret_cast<const void*>(filter_kernel<COLS, true>(1, false, false)),
         reinterpret_cast<const void*>(filter_kernel<COLS, false>(1, false, false)),
         reinterpret_cast<const void*>(filter_kernel<COLS, true>(2, true, false)),
@@ -2148,7 +2209,7 @@ int launch_scan_lds(const float* sorted, const int32_t* perm, const int32_t* n_r
     if (n_groups > max_groups) n_groups = max_groups;
     const int threads = lds_bytes > FILTER_WIDE_COPY_BYTES && !shared ? LDS_SCAN_THREADS : waves * kWave;
     const bool lone = filter_lone<COLS>(ch, (items + std::max(cus / n_slices, 1) - 1) / std::max(cus / n_slices, 1), I);
-    const bool rounds = I >= ROUNDS_FROM;
+    const bool rounds = I >= (lone ? LONE_ROUNDS_FROM : ROUNDS_FROM);
     auto kern = causal_k ? filter_kernel<COLS, true>(ch, lone, rounds) : filter_kernel<COLS, false>(ch, lone, rounds);
     {
         KernelTimerScope timer_("scan", stream);

@@ -110,6 +110,20 @@ def test_scans_by_rounds(B, I, J, law):
     _check(x, w, p)
 
 
+# Few wavefronts with rows of slices of eight columns: whole turns of eight chunks and a chunk, an input more or less, and rows that end early.
+@pytest.mark.parametrize("law", ["spread", "jump"])
+@pytest.mark.parametrize("B,I,J", [(9, 2496, 64), (17, 2559, 40), (24, 2561, 64), (49, 3001, 70), (20, 4607, 33), (100, 4608, 200)])
+def test_long_rows_of_few_wavefronts(B, I, J, law):
+    x, w, p, _ = dense_case(B + I + J, B, I, J, True, "baseline")
+    rng = np.random.default_rng(I + J)
+    if law == "jump":
+        x = np.where(rng.random(x.shape) < rng.uniform(0.1, 0.9, (B, 1)), 1 + 0.3 * rng.random(x.shape), 3 + 0.2 * rng.random(x.shape)).astype(np.float32)
+    x[1::3] = np.where(rng.random(x[1::3].shape) < 0.1, np.float32(1e5), x[1::3])
+    x[-2, I // 2:] = 1e5
+    x[-1] = 2e5
+    _check(x, w, p)
+
+
 # Launches whose workgroups order their own rows: one and two rows per item, networks of 512 and 1024, several slices
 SORTING_SIZES = [(1, 784, 800), (1, 128, 30), (1, 129, 33), (3, 300, 20), (5, 511, 16), (6, 512, 40), (7, 513, 10), (5, 1023, 16), (2, 1024, 100),
                  (255, 800, 10), (1, 512, 1000), (100, 200, 64)]
