@@ -69,8 +69,8 @@ __device__ __forceinline__ void dx_mac8(float& acc, float x, const float* u, con
 // registers than a whole weight row per tap; they go into a second set of weights and of slot operands,
 // fetched while the current ones are in use, and fewer LDS reads are needed (80 instead of 192 per tile and
 // 16 output channels).  us, arithmetic masks, a branch per (pixel, tap) block and tiles over the whole padded row / compare and
-// select, no branches, tiles over the wanted window: 64 -> 64 at 56 x 56, 32 images 252 / 229, 128 -> 128 at 28 x 28 262 / 214, 256 -> 256 at
-// 14 x 14 238 / 217, 512 -> 512 at 7 x 7 235 / 213, 32 -> 32 at 32 x 32, 128 images 122 / 95, 64 -> 128 at 8 x 8 69 / 52; one image of 64 -> 64 at
+// select, no branches, tiles over the wanted window: 64 -> 64 at 56 x 56, 32 images 252 / 233, 128 -> 128 at 28 x 28 262 / 223, 256 -> 256 at
+// 14 x 14 238 / 224, 512 -> 512 at 7 x 7 235 / 219, 32 -> 32 at 32 x 32, 128 images 122 / 99, 64 -> 128 at 8 x 8 69 / 53; one image of 64 -> 64 at
 // 56 x 56 49 / 42.
 constexpr int DX_GK = 8;
 template <int KCB, bool MULTI, int KW>
