@@ -212,17 +212,27 @@ __device__ __forceinline__ void load_chunk_flat(Chunk& c, const float* __restric
 //     EXEC &= yg > x*|wsum|                       (a closing lane keeps its sums)
 //     wsum  += w ; ysum = fma(x, w, ysum) ; ya = wsum < 0 ? -ysum : ysum
 //     yg     = ya > x*|wsum| ? ya : +inf
-// No vector -> scalar -> EXEC round trips, so a step of a lone wavefront takes few cycles.
-#define SNNTC_VSCAN_STEP(U)                                                  \
-    "v_mul_f32_e64 %[t], %[x" #U "], |%[wsum]|\n"                            \
+// No vector -> scalar -> EXEC round trips, so a step of a lone wavefront takes few cycles.  A select that reads a lane mask needs two
+// wait states behind the compare that writes it: the first has the steps in between, the second AHEAD, two instructions, which
+// are the next step's product x*|wsum| where there is one, the count where one is wanted, and waits.
+#define SNNTC_VSCAN_PRODUCT(U) "v_mul_f32_e64 %[t], %[x" #U "], |%[wsum]|\n"
+#define SNNTC_VSCAN_STEP(U, AHEAD)                                           \
     "v_cmpx_gt_f32_e32 vcc, %[yg], %[t]\n"                                   \
     "v_add_f32_e32 %[wsum], %[wsum], %[w" #U "]\n"                           \
-    "v_fmac_f32_e32 %[ysum], %[x" #U "], %[w" #U "]\n"                       \
     "v_cmp_gt_f32_e32 vcc, 0, %[wsum]\n"                                     \
+    "v_fmac_f32_e32 %[ysum], %[x" #U "], %[w" #U "]\n"                       \
+    SNNTC_VSCAN_PRODUCT(U)                                                   \
     "v_cndmask_b32_e64 %[ya], %[ysum], -%[ysum], vcc\n"                      \
-    "v_mul_f32_e64 %[t], %[x" #U "], |%[wsum]|\n"                            \
     "v_cmp_gt_f32_e32 vcc, %[ya], %[t]\n"                                    \
+    AHEAD                                                                    \
     "v_cndmask_b32_e32 %[yg], %[inf], %[ya], vcc\n"
+// the steps of a chunk: FILL is the instruction next to the product, LAST what the last step has instead of both
+#define SNNTC_VSCAN_CHUNK(FILL, LAST)                                                                                   \
+    SNNTC_VSCAN_PRODUCT(0)                                                                                              \
+    SNNTC_VSCAN_STEP(0, SNNTC_VSCAN_PRODUCT(1) FILL) SNNTC_VSCAN_STEP(1, SNNTC_VSCAN_PRODUCT(2) FILL)                   \
+    SNNTC_VSCAN_STEP(2, SNNTC_VSCAN_PRODUCT(3) FILL) SNNTC_VSCAN_STEP(3, SNNTC_VSCAN_PRODUCT(4) FILL)                   \
+    SNNTC_VSCAN_STEP(4, SNNTC_VSCAN_PRODUCT(5) FILL) SNNTC_VSCAN_STEP(5, SNNTC_VSCAN_PRODUCT(6) FILL)                   \
+    SNNTC_VSCAN_STEP(6, SNNTC_VSCAN_PRODUCT(7) FILL) SNNTC_VSCAN_STEP(7, LAST)
 #define SNNTC_VSCAN_PROLOGUE                        \
     "s_mov_b64 %[save], exec\n"                     \
     "s_mov_b64 exec, %[run]\n"
@@ -246,15 +256,10 @@ __device__ __forceinline__ void scan_chunk_vector(float& wsum, float& ysum, floa
     float t;
     const float inf = INFINITY;
     if (WANT_K)
-        asm volatile(SNNTC_VSCAN_PROLOGUE SNNTC_VSCAN_STEP(0) SNNTC_SCAN_COUNT SNNTC_VSCAN_STEP(1) SNNTC_SCAN_COUNT
-                     SNNTC_VSCAN_STEP(2) SNNTC_SCAN_COUNT SNNTC_VSCAN_STEP(3) SNNTC_SCAN_COUNT SNNTC_VSCAN_STEP(4)
-                     SNNTC_SCAN_COUNT SNNTC_VSCAN_STEP(5) SNNTC_SCAN_COUNT SNNTC_VSCAN_STEP(6) SNNTC_SCAN_COUNT
-                     SNNTC_VSCAN_STEP(7) SNNTC_SCAN_COUNT SNNTC_VSCAN_EPILOGUE
+        asm volatile(SNNTC_VSCAN_PROLOGUE SNNTC_VSCAN_CHUNK(SNNTC_SCAN_COUNT, SNNTC_SCAN_COUNT "s_nop 0\n") SNNTC_VSCAN_EPILOGUE
                      : SNNTC_VSCAN_STATE : SNNTC_VSCAN_INPUTS : "vcc", "scc");
     else
-        asm volatile(SNNTC_VSCAN_PROLOGUE SNNTC_VSCAN_STEP(0) SNNTC_VSCAN_STEP(1) SNNTC_VSCAN_STEP(2)
-                     SNNTC_VSCAN_STEP(3) SNNTC_VSCAN_STEP(4) SNNTC_VSCAN_STEP(5) SNNTC_VSCAN_STEP(6)
-                     SNNTC_VSCAN_STEP(7) SNNTC_VSCAN_EPILOGUE
+        asm volatile(SNNTC_VSCAN_PROLOGUE SNNTC_VSCAN_CHUNK("s_nop 0\n", "s_nop 1\n") SNNTC_VSCAN_EPILOGUE
                      : SNNTC_VSCAN_STATE : SNNTC_VSCAN_INPUTS : "vcc", "scc");
 }
 
@@ -305,7 +310,7 @@ __device__ __forceinline__ void scan_step_vector(float& wsum, float& ysum, float
     uint64_t saved_exec;
     float t;
     const float inf = INFINITY;
-    asm volatile(SNNTC_VSCAN_PROLOGUE SNNTC_VSCAN_STEP(0) SNNTC_SCAN_COUNT "s_mov_b64 exec, %[save]\n"
+    asm volatile(SNNTC_VSCAN_PROLOGUE SNNTC_VSCAN_PRODUCT(0) SNNTC_VSCAN_STEP(0, SNNTC_SCAN_COUNT "s_nop 0\n") "s_mov_b64 exec, %[save]\n"
                  : [wsum] "+v"(wsum), [ysum] "+v"(ysum), [ya] "+v"(ya), [yg] "+v"(yg), [kcnt] "+v"(kcnt),
                    [save] "=&s"(saved_exec), [t] "=&v"(t)
                  : [run] "s"(run), [inf] "v"(inf), [x0] "v"(x), [w0] "v"(w) : "vcc", "scc");

@@ -1,8 +1,10 @@
-"""The device code of the built library: lane-crossing operands (DPP) wait as the hardware asks.
+"""The device code of the built library: lane-crossing operands (DPP) and lane masks wait as the hardware asks.
 
 A DPP operand needs two wait states behind the vector instruction that wrote its register, and five behind one that
 wrote EXEC.  The compiler keeps both where it sees the instructions; the scan's inline assembly keeps the first by `s_nop`
-statements of its own, which hold only while no copy of an operand lands between them and the read."""
+statements of its own, which hold only while no copy of an operand lands between them and the read.
+
+A scalar register (a lane mask, vcc) that a vector instruction wrote needs two wait states before another reads it."""
 import os
 import re
 import shutil
@@ -109,6 +111,76 @@ def test_dpp_operands_of_the_library_wait(tmp_path):
     for part in sorted(p for p in os.listdir(tmp_path) if "gfx950" in p):
         text = subprocess.run([OBJDUMP, "-d", part], cwd=tmp_path, check=True, capture_output=True, text=True).stdout
         n, b = short_waits(text)
+        seen += n
+        bad += b
+    assert seen > 10000
+    assert not bad, "\n".join(bad[:20])
+
+
+# vector instructions with a second result, the carry
+CARRIES = re.compile(r"v_(add|sub|subrev|addc|subb|subbrev)_co_|v_div_scale|v_mad_[ui]64")
+
+
+def _scalars(operand):
+    """The scalar registers an operand names."""
+    operand = operand.strip("-|")
+    if operand.startswith("vcc"):
+        return {"vcc"}
+    m = re.fullmatch(r"s(\d+)", operand) or re.fullmatch(r"s\[(\d+):(\d+)\]", operand)
+    return set(range(int(m.group(1)), int(m.groups()[-1]) + 1)) if m else set()
+
+
+def short_mask_waits(text):
+    """(reads of scalar registers by vector instructions seen, lines that come too soon behind a vector instruction's write)."""
+    code, before = _parse(text)
+    seen, bad = 0, []
+
+    def registers(entry):
+        operands = [_scalars(o.split(" ")[0]) for o in entry[2]]
+        results = 2 if CARRIES.match(entry[1]) else 1
+        return set().union(*operands[:results]), set().union(*operands[results:])
+
+    for entry in code:
+        if not entry or not entry[1].startswith("v_"):
+            continue
+        read = registers(entry)[1]
+        if not read:
+            continue
+        seen += 1
+        todo = [(i, 0) for i in before.get(entry[0], [])]
+        while todo:
+            index, waited = todo.pop()
+            address, mnemonic, operands, rest = code[index]
+            if mnemonic.startswith("v_") and registers(code[index])[0] & read:
+                bad.append(f"{address:x} {mnemonic} {rest} -> {entry[0]:x} {entry[1]} {entry[3]}")
+                break
+            waited += int(rest) + 1 if mnemonic == "s_nop" else 1
+            if waited < 2:
+                todo += [(i, waited) for i in before.get(address, [])]
+    return seen, bad
+
+
+@pytest.mark.parametrize("write,read,other", [
+    ("v_cmp_gt_f32_e32 vcc, 0, v59", "v_cndmask_b32_e64 v56, v55, -v55, vcc", "v_cndmask_b32_e64 v56, v55, -v55, s[2:3]"),
+    ("v_cmp_gt_f32_e64 s[4:5], 0, v59", "v_cndmask_b32_e64 v56, v55, v54, s[4:5]", "v_cndmask_b32_e32 v56, v55, v54, vcc"),
+    ("v_addc_co_u32_e64 v1, vcc, 0, v1, s[6:7]", "v_cndmask_b32_e32 v56, v55, v54, vcc", "v_mul_f32_e32 v2, s9, v2"),
+    ("v_readfirstlane_b32 s9, v3", "v_mul_f32_e32 v2, s9, v2", "v_mul_f32_e32 v2, s8, v2"),
+])
+def test_the_check_sees_masks(write, read, other):
+    for between, ok in [([], False), (["s_nop 0"], False), (["s_nop 1"], True), (["v_mov_b32_e32 v6, 0", "s_waitcnt lgkmcnt(0)"], True)]:
+        assert bool(short_mask_waits(_listing(write, *between, read))[1]) != ok
+    assert not short_mask_waits(_listing(write, other))[1]
+
+
+def test_lane_masks_of_the_library_wait(tmp_path):
+    if not os.path.exists(LIBRARY) or not os.path.exists(OBJDUMP):
+        pytest.skip("needs the built library and llvm-objdump")
+    shutil.copy(LIBRARY, tmp_path / "lib.so")
+    subprocess.run([OBJDUMP, "--offloading", "lib.so"], cwd=tmp_path, check=True, stdout=subprocess.DEVNULL)
+    seen, bad = 0, []
+    for part in sorted(p for p in os.listdir(tmp_path) if "gfx950" in p):
+        text = subprocess.run([OBJDUMP, "-d", part], cwd=tmp_path, check=True, capture_output=True, text=True).stdout
+        n, b = short_mask_waits(text)
         seen += n
         bad += b
     assert seen > 10000
