@@ -160,9 +160,10 @@ constexpr int FILTER_MAX_CH = COLS == 8 ? 2 : 4;
 // costs about five plain instructions whatever its width: four reads per chunk in place of sixteen broadcasts.  us with
 // DPP / staged: 65 536 segments of 576 to 64 neurons 226 / 207, 100 352 329 / 299, 32 768 of 576 120 / 108.  Only with rows of 256 bytes: slices of 32,
 // 16 and 8 columns read their weights with bank conflicts, and four more reads make LDS the bound (4096 rows of 784
-// to 800 neurons 242 / 262, 6272 segments of 2304 to 256 365 / 405, 1568 of 4608 to 512 514 / 545).
-template <int COLS, int CH, bool LONE>
-constexpr bool filter_staged = COLS == 64 && CH == 4 && !LONE;
+// to 800 neurons 242 / 262, 6272 segments of 2304 to 256 365 / 405, 1568 of 4608 to 512 514 / 545), and only where the entries of all
+// wavefronts fit beside the slice (launch_scan_lds): rows of up to 576 inputs.
+template <int COLS>
+constexpr bool FILTER_STAGES = COLS == 64;
 constexpr int LDS_SCAN_TARGET = LDS_SCAN_BYTES - FILTER_RED_BYTES;
 
 struct Chunk {
@@ -1239,7 +1240,7 @@ __device__ __forceinline__ void row_row_addresses(int even, int odd, unsigned ba
         : [e] "v"(even), [o] "v"(odd), [base] "v"(base), [n0] "n"(N), [n1] "n"(N + 1));
 }
 
-template <int COLS, int CH, bool LONE, bool WANT_K, bool ROUNDS = false>
+template <int COLS, int CH, bool LONE, bool WANT_K, bool ROUNDS = false, bool STAGED = false>
 __global__ void __launch_bounds__(LDS_SCAN_THREADS)
 scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__ perm,
                    const int32_t* __restrict__ n_real, const float* __restrict__ w, float* __restrict__ y_out,
@@ -1252,7 +1253,6 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
     // How a segment's (x, row) entries reach its lanes (see the fast loop): through rows of sixteen lanes where
     // a segment has at least that many, else through quads
     constexpr bool BY_ROW = LANES % 16 == 0;
-    constexpr bool STAGED = filter_staged<COLS, CH, LONE>;
     constexpr int ROUND = 4;                               // chunks per round of the fast loop
     const int block = xcd_contiguous(blockIdx.x, gridDim.x);
     const int slice = block / n_groups;
@@ -2048,12 +2048,14 @@ constexpr size_t FILTER_WIDE_COPY_BYTES = 48 * 1024;        // slices from here 
 
 // The instantiation for ch neurons per lane.
 template <int COLS, bool WANT_K>
-decltype(&scan_filter_kernel<COLS, 1, true, WANT_K>) filter_kernel(int ch, bool lone, bool rounds) {
-    constexpr bool LONG_ROWS = COLS == 8;
+decltype(&scan_filter_kernel<COLS, 1, true, WANT_K>) filter_kernel(int ch, bool lone, bool rounds, bool staged) {
+    constexpr bool LONG_ROWS = COLS == 8, STAGES = FILTER_STAGES<COLS>;
+    constexpr int MOST = FILTER_MAX_CH<COLS>;
     if (ch == 1 && lone) return rounds ? scan_filter_kernel<COLS, 1, true, WANT_K, LONG_ROWS> : scan_filter_kernel<COLS, 1, true, WANT_K>;
     if (ch == 1) return scan_filter_kernel<COLS, 1, false, WANT_K>;
-    if (ch == FILTER_MAX_CH<COLS>)
-        return rounds ? scan_filter_kernel<COLS, FILTER_MAX_CH<COLS>, false, WANT_K, true> : scan_filter_kernel<COLS, FILTER_MAX_CH<COLS>, false, WANT_K>;
+    if (ch == MOST && staged)
+        return rounds ? scan_filter_kernel<COLS, MOST, false, WANT_K, true, STAGES> : scan_filter_kernel<COLS, MOST, false, WANT_K, false, STAGES>;
+    if (ch == MOST) return rounds ? scan_filter_kernel<COLS, MOST, false, WANT_K, true> : scan_filter_kernel<COLS, MOST, false, WANT_K>;
     if constexpr (COLS == 64) {
         if (!lone) return scan_filter_kernel<COLS, 2, false, WANT_K>;
     }
@@ -2062,23 +2064,14 @@ decltype(&scan_filter_kernel<COLS, 1, true, WANT_K>) filter_kernel(int ch, bool 
 
 template <int COLS>
 int raise_scan_lds_limits() {
-    const void* whole[] = {
-        reinterpret_cast<const void*>(filter_kernel<COLS, true>(1, true, false)),
-        reinterpret_cast<const void*>(filter_kernel<COLS, false>(1, true, false)),
-        reinterpret_cast<const void*>(filter_kernel<COLS, true>(1, true, true)),
-        reinterpret_cast<const void*>(filter_kernel<COLS, false>(1, true, true)),
-        reinterpret_cast<const void*>(filter_kernel<COLS, true>(1, false, false)),
-        reinterpret_cast<const void*>(filter_kernel<COLS, false>(1, false, false)),
-        reinterpret_cast<const void*>(filter_kernel<COLS, true>(2, true, false)),
-        reinterpret_cast<const void*>(filter_kernel<COLS, false>(2, true, false)),
-        reinterpret_cast<const void*>(filter_kernel<COLS, true>(2, false, false)),
-        reinterpret_cast<const void*>(filter_kernel<COLS, false>(2, false, false)),
-        reinterpret_cast<const void*>(filter_kernel<COLS, true>(FILTER_MAX_CH<COLS>, false, false)),
-        reinterpret_cast<const void*>(filter_kernel<COLS, false>(FILTER_MAX_CH<COLS>, false, false)),
-        reinterpret_cast<const void*>(filter_kernel<COLS, true>(FILTER_MAX_CH<COLS>, false, true)),
-        reinterpret_cast<const void*>(filter_kernel<COLS, false>(FILTER_MAX_CH<COLS>, false, true))};
-    for (const void* k : whole)
-        SNNTC_HIP_CHECK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_SCAN_BYTES));
+    for (int ch = 1; ch <= FILTER_MAX_CH<COLS>; ch *= 2)
+        for (int form = 0; form < 8; ++form) {
+            const bool lone = form & 1, rounds = form & 2, staged = form & 4;
+            if (lone && ch == 4) continue;
+            for (const void* k : {reinterpret_cast<const void*>(filter_kernel<COLS, true>(ch, lone, rounds, staged)),
+                                  reinterpret_cast<const void*>(filter_kernel<COLS, false>(ch, lone, rounds, staged))})
+                SNNTC_HIP_CHECK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_SCAN_BYTES));
+        }
     constexpr bool SORTS = split_sorts(COLS);
     const void* split[] = {reinterpret_cast<const void*>(scan_lds_split_kernel<COLS, 0, true>),
                            reinterpret_cast<const void*>(scan_lds_split_kernel<COLS, 0, false>),
@@ -2191,12 +2184,7 @@ int launch_scan_lds(const float* sorted, const int32_t* perm, const int32_t* n_r
         return SNNTC_OK;
     }
 
-    int ch = filter_neurons<COLS>(S, I, n_slices, cus);
-    // Where the staging of sixteen wavefronts does not fit beside the slice, eight or four of them work on items.
-    const auto stage_bytes = [&](int w) { return COLS == 64 && ch == 4 ? (size_t)w * FILTER_STAGE_BYTES : (size_t)FILTER_RED_BYTES; };
-    int max_waves = 16;
-    while (max_waves > 4 && lds_bytes + stage_bytes(max_waves) > (size_t)LDS_SCAN_BYTES) max_waves /= 2;
-    if (lds_bytes + stage_bytes(max_waves) > (size_t)LDS_SCAN_BYTES) { ch /= 2; max_waves = 16; }
+    const int ch = filter_neurons<COLS>(S, I, n_slices, cus);
     const int segs = kWave / COLS * ch;                     // segments per wavefront
     const int64_t items = (S + segs - 1) / segs;
     // One workgroup per CU (its 16 wavefronts take all registers; small slices let two of up to eight share a CU),
@@ -2204,21 +2192,27 @@ int launch_scan_lds(const float* sorted, const int32_t* perm, const int32_t* n_r
     // with a full workgroup all the same.  (Wavefronts by the items of a group: by those of the chip, a slice count that does not divide
     // it left a few items for a second turn, 512 rows of 333 to 1500 neurons 57.0 -> 49.4 us, 4096 to 130 58.7 -> 52.7.)
     const int64_t per_cu = (items * n_slices + cus - 1) / cus;
-    const bool shared = per_cu <= 8 && (lds_bytes + stage_bytes(8)) * 2 <= (size_t)LDS_SCAN_BYTES;
+    const bool shared = per_cu <= 8 && (lds_bytes + FILTER_RED_BYTES) * 2 <= (size_t)LDS_SCAN_BYTES;
     const int64_t capacity = (int64_t)cus * (shared ? 2 : 1);
     int64_t n_groups = capacity / n_slices;
     if (n_groups < 1) n_groups = 1;
     const int64_t per_wg = (items + n_groups - 1) / n_groups;
-    const int waves = (int)(per_wg >= max_waves ? max_waves : (per_wg + 3) / 4 * 4);
+    const int waves = (int)(per_wg >= 16 ? 16 : (per_wg + 3) / 4 * 4);
     const int64_t max_groups = (items + waves - 1) / waves;
     if (n_groups > max_groups) n_groups = max_groups;
     const int threads = lds_bytes > FILTER_WIDE_COPY_BYTES && !shared ? LDS_SCAN_THREADS : waves * kWave;
     const bool lone = filter_lone<COLS>(ch, (items + std::max(cus / n_slices, 1) - 1) / std::max(cus / n_slices, 1), I);
     const bool rounds = I >= (lone ? LONE_ROUNDS_FROM : ROUNDS_FROM);
-    auto kern = causal_k ? filter_kernel<COLS, true>(ch, lone, rounds) : filter_kernel<COLS, false>(ch, lone, rounds);
+    // Staged where the row entries of all its wavefronts fit beside the slice, broadcasts elsewhere: fewer wavefronts lose more than the
+    // broadcasts cost.  us of the layer, its order included, fewer staged wavefronts (eight up to 608 inputs, four up to 624, then two
+    // neurons per lane) / broadcasts: 65 536 segments of 600, 616 and 638 to 64 neurons 446 / 415, 643 / 417, 553 / 452, 4096 of 620 to 800 408 / 210,
+    // 1024 of 600 to 800 78 / 71.
+    const size_t staged_lds = lds_bytes + (size_t)waves * FILTER_STAGE_BYTES;
+    const bool staged = FILTER_STAGES<COLS> && ch == FILTER_MAX_CH<COLS> && staged_lds * (shared ? 2 : 1) <= (size_t)LDS_SCAN_BYTES;
+    auto kern = causal_k ? filter_kernel<COLS, true>(ch, lone, rounds, staged) : filter_kernel<COLS, false>(ch, lone, rounds, staged);
     {
         KernelTimerScope timer_("scan", stream);
-        hipLaunchKernelGGL(kern, dim3((unsigned)(n_slices * n_groups)), dim3((unsigned)threads), lds_bytes + stage_bytes(waves), stream,
+        hipLaunchKernelGGL(kern, dim3((unsigned)(n_slices * n_groups)), dim3((unsigned)threads), staged ? staged_lds : lds_bytes + FILTER_RED_BYTES, stream,
                            sorted, perm, n_real, w, y, rcp, causal_k, (int)S, (int)I, (int)stride, (int)J, n_slices, (int)n_groups,
                            waves, np, copy);
     }

@@ -91,13 +91,17 @@ def test_scan_forms_of_small_launches(B, I, J, law):
 
 
 # Rows long enough to be tested a round of four chunks at a time at first, either side of that line, and slices of 64 columns that leave
-# room for the row entries of sixteen, eight, four and no wavefronts; other widths.
+# room for the row entries of sixteen wavefronts (up to 576 inputs) and that do not; other widths.
 LONG_SIZES = [(12003, 399, 64), (12003, 400, 64), (12003, 431, 50), (12011, 576, 64), (12011, 577, 63), (12007, 608, 64), (12007, 609, 64),
               (12005, 624, 64), (12005, 625, 64), (12005, 638, 41), (9001, 700, 32), (5003, 1537, 16), (2603, 3001, 24), (1207, 4700, 16)]
 
 
+# Two workgroups of four wavefronts to a CU, four neurons per lane: room for row entries in both (up to 304 inputs), and none
+SHARED_SIZES = [(80, 289, 6400), (80, 304, 6400), (80, 305, 6400), (80, 319, 6400)]
+
+
 @pytest.mark.parametrize("law", ["spread", "jump"])
-@pytest.mark.parametrize("B,I,J", LONG_SIZES)
+@pytest.mark.parametrize("B,I,J", LONG_SIZES + SHARED_SIZES)
 def test_scans_by_rounds(B, I, J, law):
     """`jump`: the times stand close together, then leap, so that a round fails that the one before it did not announce."""
     x, w, p, _ = dense_case(B + I + J, B, I, J, True, "baseline")
