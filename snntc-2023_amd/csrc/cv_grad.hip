@@ -73,7 +73,7 @@ __device__ __forceinline__ void dx_mac8(float& acc, float x, const float* u, con
 // 14 x 14 238 / 224, 512 -> 512 at 7 x 7 235 / 219, 32 -> 32 at 32 x 32, 128 images 122 / 99, 64 -> 128 at 8 x 8 69 / 53; one image of 64 -> 64 at
 // 56 x 56 49 / 42.
 constexpr int DX_GK = 8;
-template <int KCB, bool MULTI, int KW>
+template <int KCB, bool MULTI, int KW, bool STRIDED = false>
 __global__ void __launch_bounds__(256)
     __attribute__((amdgpu_waves_per_eu(KW == 3 ? DX_WAVES3 : KCB == 64 && MULTI ? 3 : 4)))
 cv_grad_input_chan_kernel(const float* __restrict__ xpad, const float* __restrict__ wq,
@@ -139,9 +139,12 @@ cv_grad_input_chan_kernel(const float* __restrict__ xpad, const float* __restric
     }
     // KW = 3: slots that hold no patch are filled with (-inf, 0), a term that adds nothing, so a lane may read
     // any slot.  (No staging round loads them: filled once.)
-    // Nearly all of the 24 (pixel, tap) blocks of a sweep have work, so it takes them all, without a branch: a test, a jump and a
-    // wait per 24 vector instructions cost more than the blocks they leave out (every instruction takes an issue slot, scalar ones
-    // too).  It ends early, in four places, where the last slots meet no pixel with work or hold no patch.
+    // With a column stride of one nearly all of the 24 (pixel, tap) blocks of a sweep have work, so it takes them all, without a branch: a
+    // test, a jump and a wait per 24 vector instructions cost more than the blocks they leave out (every instruction takes an issue slot,
+    // scalar ones too).  It ends early, in four places, where the last slots meet no pixel with work or hold no patch.
+    // STRIDED: at most every second slot holds a patch, and the sweep steps over the others.  us, all slots / this: 64 -> 128 at 56 x 56, 3x3/2, 32 images
+    // 281 / 193, 128 -> 256 at 28 x 28 276 / 187, 32 -> 64 at 32 x 32, 64 images 93 / 84, 64 -> 128 at 56 x 56, 3x3/3 178 / 122.  (The slots of
+    // one parity with their operands read ahead: 240, 220, 104 and 153, with spilled registers.)
     auto slot_exists = [&](int sl) {
         const int ww = w0 - Kw + 1 + sl;
         if (ww < 0) return false;
@@ -152,6 +155,14 @@ cv_grad_input_chan_kernel(const float* __restrict__ xpad, const float* __restric
             if (!slot_exists(sl) && lane < KCB) { ys[sl * KCB + lane] = -INFINITY; us[sl * KCB + lane] = 0.0f; }
     };
     if constexpr (KW == 3) fill_empty_slots();
+    unsigned patch_slots = 0;                            // STRIDED: bit d is set where the d-th slot of a part holds a patch
+    if constexpr (STRIDED)
+        for (int sl = 0; sl < n_slots; ++sl)             // (a part's last two slots are the first two of the next)
+            if (slot_exists(sl)) {
+                const int d = sl % DX_TILE;
+                if (sl < span) patch_slots |= 1u << d;
+                if (sl >= DX_TILE && d < 2) patch_slots |= 1u << (d + DX_TILE);
+            }
     const int slots_end = min(live != 0 ? 32 - __builtin_clz(live) + 2 : 0, (Nw - 1) * Sw + Kw - w0);
     if (live != 0) {
         for (int kh = 0; kh < Kh; ++kh) {
@@ -222,9 +233,22 @@ cv_grad_input_chan_kernel(const float* __restrict__ xpad, const float* __restric
                         }
                     };
                     // all slots of a half against the three taps of DX_GK output channels; the operands of the
-                    // next slot are read while the current one computes
+                    // next slot are read while the current one computes (STRIDED: read where they are used)
                     auto sweep = [&](const float (&wr)[3][DX_GK], const float* __restrict__ yg) __attribute__((always_inline)) {
                         float yq[2][DX_GK], uq[2][DX_GK];
+                        if constexpr (STRIDED) {
+#pragma unroll
+                            for (int d = 0; d < DX_TILE + 2; ++d) {
+                                if (!(patch_slots >> d & 1u)) continue;
+                                read_slot(yg, d, yq[0], uq[0]);
+#pragma unroll
+                                for (int kw = 0; kw < 3; ++kw) {
+                                    const int t = d - 2 + kw;
+                                    if (t >= 0 && t < DX_TILE) dx_mac8(acc[t], xv[t], uq[0], yq[0], wr[kw]);
+                                }
+                            }
+                            return;
+                        }
                         read_slot(yg, 0, yq[0], uq[0]);
 #pragma unroll
                         for (int d = 0; d < DX_TILE + 2; ++d) {
@@ -783,21 +807,16 @@ int launch_cv_grad_input_chan(const float* xpad, const float* wq, const float* u
     if (blocks > 0x7fffffffLL) return fail(SNNTC_ERR_TOO_LARGE, "conv backward: grid too large");
     dim3 grid((unsigned)blocks), block(wg_waves * kWave);
     const size_t lds = pl.lds;
-    decltype(&cv_grad_input_chan_kernel<64, false, 3>) kern;
-    if (g.Kw == 3) {
-        if (multi)
-            kern = kcb == 64 ? cv_grad_input_chan_kernel<64, true, 3> : kcb == 32 ? cv_grad_input_chan_kernel<32, true, 3>
-                                                                                   : cv_grad_input_chan_kernel<16, true, 3>;
-        else
-            kern = kcb == 64 ? cv_grad_input_chan_kernel<64, false, 3> : kcb == 32 ? cv_grad_input_chan_kernel<32, false, 3>
-                                                                                    : cv_grad_input_chan_kernel<16, false, 3>;
-    } else if (multi) {
-        kern = kcb == 64 ? cv_grad_input_chan_kernel<64, true, 0> : kcb == 32 ? cv_grad_input_chan_kernel<32, true, 0>
-                                                                               : cv_grad_input_chan_kernel<16, true, 0>;
-    } else {
-        kern = kcb == 64 ? cv_grad_input_chan_kernel<64, false, 0> : kcb == 32 ? cv_grad_input_chan_kernel<32, false, 0>
-                                                                                : cv_grad_input_chan_kernel<16, false, 0>;
-    }
+    const auto chosen = [&](auto kcb_c) {
+        constexpr int KCB = decltype(kcb_c)::value;
+        if (g.Kw != 3) return multi ? cv_grad_input_chan_kernel<KCB, true, 0> : cv_grad_input_chan_kernel<KCB, false, 0>;
+        // (the parts of a wavefront begin eight columns apart: with an odd stride their patches lie under other slots, nearly all between them.
+        // 3x3/3, 32 -> 64 at 32 x 32, 64 images 62.8 us against 65.6, 16 -> 32, 128 images 56 against 65, 3 -> 32 33 against 40)
+        if (multi ? g.Sw % 2 == 0 : g.Sw != 1) return multi ? cv_grad_input_chan_kernel<KCB, true, 3, true> : cv_grad_input_chan_kernel<KCB, false, 3, true>;
+        return multi ? cv_grad_input_chan_kernel<KCB, true, 3> : cv_grad_input_chan_kernel<KCB, false, 3>;
+    };
+    const auto kern = kcb == 64 ? chosen(std::integral_constant<int, 64>{}) : kcb == 32 ? chosen(std::integral_constant<int, 32>{})
+                                                                                        : chosen(std::integral_constant<int, 16>{});
     {
         KernelTimerScope timer_("cv_grad_input", stream);
         hipLaunchKernelGGL(kern, grid, block, lds, stream, xpad, wq, upm, ym, dx, crop, (int)g.H, (int)g.W, (int)g.C,

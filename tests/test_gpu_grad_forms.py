@@ -113,6 +113,10 @@ def test_dense_gradients_whole_or_in_parts(B, I, J):
 @pytest.mark.parametrize("B,H,W,C,Kc,S", [
     (2, 5, 9, 64, 64, 1), (2, 4, 10, 64, 128, 1), (1, 3, 11, 65, 16, 1), (1, 5, 16, 32, 64, 1), (2, 3, 18, 20, 32, 1),      # tiles of 8 to 128 pixels
     (1, 4, 19, 3, 64, 1), (1, 3, 30, 7, 48, 1), (2, 3, 31, 64, 80, 2), (1, 7, 34, 33, 64, 1), (3, 9, 8, 64, 256, 1), (1, 3, 3, 4, 16, 1),
+    # strides that leave out slots: tiles of 8 pixels, of 16 to 128 with even strides, and odd strides that leave out none there
+    (2, 7, 21, 64, 64, 2), (1, 5, 34, 64, 128, 2), (1, 7, 30, 64, 64, 3), (1, 9, 28, 65, 16, 4), (1, 6, 23, 128, 256, 5),
+    (2, 6, 25, 32, 64, 2), (1, 5, 40, 16, 32, 2), (2, 4, 33, 7, 48, 2), (1, 6, 140, 3, 64, 2), (1, 5, 39, 16, 64, 4), (1, 7, 37, 30, 32, 6),
+    (2, 5, 37, 32, 64, 3), (1, 4, 44, 9, 16, 3),
 ])
 def test_conv_input_gradients_at_the_edges_of_tiles(B, H, W, C, Kc, S):
     """Three-column kernels: rows that begin or end with a padded column, or have none, in one image; the whole gradient and windows of it."""
