@@ -682,7 +682,7 @@ int snntc_fc_backward(const float* grad, const float* x, const float* w, const f
         return launch_fc_backward_narrow(x, w, grad, oldout, oldout + B * J, dx, dw, ws.partial, dparams, 6, B, I, J,
                                          np, st);
     if (dw && fc_backward_joint_supported(B, I, J, dx != nullptr, ws.max_split))
-        return launch_fc_backward_joint(x, w, grad, oldout, oldout + B * J, dx, dw, dparams, 6, B, I, J, np, st);
+        return launch_fc_backward_joint(x, w, grad, oldout, oldout + B * J, dx, dw, dparams, 6, B, I, J, ws.max_split, np, st);
     rc = launch_backward_prologue(grad, oldout, oldout + B * J, ws.upm, B * J, np, w, nullptr, I, J, 0, dparams, 6, st);
     if (rc) return rc;
     if (dx) {

@@ -397,24 +397,24 @@ grad_weight_kernel(SegmentSource src, const float* __restrict__ upm, const float
 // time in turn, a lane 8 x 8 of the tile: a sample's 64 inputs, output times and upstream values are three coalesced loads, a
 // batch ahead, go to a piece of LDS of the wavefront's own and come back as six 16-byte reads for 128 vector instructions.
 // Rows past the inputs read biasvolt, so the bias row needs no code of its own.  The wavefronts' sums are added in a tree
-// through LDS.
+// through LDS.  FOLDS: and begun anew every `fold` turns (a batch per wavefront each), so that no chain of additions is long.
 // What bounds it: the addition and the multiply-add of a term (3.3 clocks each at 4096 samples).  Before, eight rows and one
 // output per lane: two LDS reads of 8 clocks and 512 bytes of y / up per 16 instructions.  us: 4096 x 784 -> 800 254 -> 158,
 // 1024 rows 69 -> 47 (both + 6 for adding up slices), 333 x 1521 -> 777 48 -> 40, 128 x 784 -> 800 15 -> 13.  (The times are scaled as they
 // are staged: a sum of two registers issues faster than a multiply-add of three, 225 us.)
 // ---------------------------------------------------------------------------------------------
-constexpr int DWD_T = 64, DWD_BATCH = 4;
+constexpr int DWD_T = 64, DWD_BATCH = 4, DWD_TURN = 8 * DWD_BATCH;       // (a turn: samples that eight wavefronts take together)
 
 // staging: [wave][sample][x 64 | y 64 | up 64]; sums: [wave][row 32][output 64], half a tile at a time
 constexpr int DWD_STAGE = DWD_BATCH * 3 * DWD_T, DWD_SUMS = DWD_T / 2 * DWD_T;
 constexpr int dwd_lds_floats(int waves) { return waves * (DWD_STAGE > DWD_SUMS ? DWD_STAGE : DWD_SUMS); }
 
-template <int WAVES, bool RAW>
+template <int WAVES, bool RAW, bool FOLDS>
 __device__ __forceinline__ void
 grad_weight_dense_tile(const float* __restrict__ x, const Upstream& upstream, const float* __restrict__ ym, float* __restrict__ dst,
-                       int S, int I, int J, int rows, int seg_per_slice, float biasvolt, float neg_s, float post, int bx, int by,
+                       int S, int I, int J, int rows, int seg_per_slice, int fold, float biasvolt, float neg_s, float post, int bx, int by,
                        int bz, float* lds) {
-    constexpr int STAGE = DWD_STAGE, SUMS = DWD_SUMS;
+    constexpr int STAGE = DWD_STAGE, SUMS = DWD_SUMS, MINE = SUMS / (WAVES * kWave);
     typedef float f4 __attribute__((ext_vector_type(4)));
     const int lane = threadIdx.x % kWave;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -447,9 +447,49 @@ grad_weight_dense_tile(const float* __restrict__ x, const Upstream& upstream, co
             if constexpr (RAW) rv[q] = rcol[(size_t)s * J];
         }
     };
-    int sb = s_begin + wave * DWD_BATCH;
+    float total[FOLDS ? 2 * MINE : 1];                      // of the thread's elements of a tile
+    // Adds up the wavefronts' sums, half a tile at a time: f(half, n, sum) for the thread's n-th element of it.
+    auto add_up = [&](auto&& f) __attribute__((always_inline)) {
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            __syncthreads();                                // (the staging, or the first half, has been read)
+            float* mine = lds + wave * SUMS;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    *reinterpret_cast<f4*>(mine + (rg * 4 + r) * DWD_T + cg * 8 + 4 * h) =
+                        f4{acc[4 * half + r][4 * h], acc[4 * half + r][4 * h + 1], acc[4 * half + r][4 * h + 2], acc[4 * half + r][4 * h + 3]};
+            __syncthreads();
+#pragma unroll
+            for (int n = 0; n < MINE; ++n) {
+                float sum[WAVES];
+#pragma unroll
+                for (int v = 0; v < WAVES; ++v) sum[v] = lds[v * SUMS + n * WAVES * kWave + threadIdx.x];
+#pragma unroll
+                for (int h = WAVES / 2; h > 0; h /= 2)
+#pragma unroll
+                    for (int v = 0; v < h; ++v) sum[v] += sum[v + h];
+                f(half, n, sum[0]);
+            }
+        }
+    };
+    if constexpr (FOLDS)
+#pragma unroll
+        for (int n = 0; n < 2 * MINE; ++n) total[n] = 0.0f;
+    int sb = s_begin + wave * DWD_BATCH, fold_at = s_begin + fold * WAVES * DWD_BATCH;
     if (sb < s_end) request(sb);
     for (; sb < s_end; sb += WAVES * DWD_BATCH) {
+        if constexpr (FOLDS)
+            if (sb - wave * DWD_BATCH == fold_at && fold_at + (WAVES - 1) * DWD_BATCH < s_end) {      // (all wavefronts or none: each has a batch in this turn)
+                add_up([&](int half, int n, float sum) __attribute__((always_inline)) { total[half * MINE + n] += sum; });
+#pragma unroll
+                for (int r = 0; r < 8; ++r)
+#pragma unroll
+                    for (int c = 0; c < 8; ++c) acc[r][c] = 0.0f;
+                fold_at += fold * WAVES * DWD_BATCH;
+                __syncthreads();
+            }
 #pragma unroll
         for (int q = 0; q < DWD_BATCH; ++q) {
             stage[q * 3 * DWD_T + lane] = (is_input ? xv[q] : biasvolt) * neg_s;
@@ -479,29 +519,12 @@ grad_weight_dense_tile(const float* __restrict__ x, const Upstream& upstream, co
         wave_lds_order();
     }
     float* out = dst + (size_t)bz * rows * J;
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-        __syncthreads();                                    // (the staging, or the first half, has been read)
-        float* mine = lds + wave * SUMS;
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-                *reinterpret_cast<f4*>(mine + (rg * 4 + r) * DWD_T + cg * 8 + 4 * h) =
-                    f4{acc[4 * half + r][4 * h], acc[4 * half + r][4 * h + 1], acc[4 * half + r][4 * h + 2], acc[4 * half + r][4 * h + 3]};
-        __syncthreads();
-        for (int e = threadIdx.x; e < SUMS; e += WAVES * kWave) {
-            const int tr = e / DWD_T, i = i0 + tr / 4 * 8 + 4 * half + tr % 4, j = j0 + e % DWD_T;
-            float sum[WAVES];
-#pragma unroll
-            for (int v = 0; v < WAVES; ++v) sum[v] = lds[v * SUMS + e];
-#pragma unroll
-            for (int h = WAVES / 2; h > 0; h /= 2)
-#pragma unroll
-                for (int v = 0; v < h; ++v) sum[v] += sum[v + h];
-            if (i < rows && j < J) out[(size_t)i * J + j] = sum[0] * post;
-        }
-    }
+    add_up([&](int half, int n, float sum) __attribute__((always_inline)) {
+        const int e = n * WAVES * kWave + threadIdx.x;
+        const int tr = e / DWD_T, i = i0 + tr / 4 * 8 + 4 * half + tr % 4, j = j0 + e % DWD_T;
+        if constexpr (FOLDS) sum = total[half * MINE + n] + sum;
+        if (i < rows && j < J) out[(size_t)i * J + j] = sum * post;
+    });
 }
 
 template <int WAVES>
@@ -510,19 +533,19 @@ grad_weight_dense_kernel(const float* __restrict__ x, const float* __restrict__ 
                          float* __restrict__ dst, int S, int I, int J, int rows, int seg_per_slice, float biasvolt,
                          float neg_s, float post) {
     __shared__ __align__(16) float lds[dwd_lds_floats(WAVES)];
-    grad_weight_dense_tile<WAVES, false>(x, Upstream{upm, nullptr, 0.0f}, ym, dst, S, I, J, rows, seg_per_slice, biasvolt, neg_s, post,
-                                         blockIdx.x, blockIdx.y, blockIdx.z, lds);
+    grad_weight_dense_tile<WAVES, false, false>(x, Upstream{upm, nullptr, 0.0f}, ym, dst, S, I, J, rows, seg_per_slice, 0, biasvolt, neg_s, post,
+                                                blockIdx.x, blockIdx.y, blockIdx.z, lds);
 }
 
 // The whole backward pass of a dense layer on a small batch in one launch: dX tiles of eight wavefronts (below 64 outputs, SPLIT 1, eight
 // tiles of one) and dW tiles, which both form the upstream values as they stage them.  Each part alone leaves the chip half empty and waits
 // for its first loads.  us, prologue, dX and dW (and the sum of its slices) / together, 784 -> 800: 1 row 18.5 / 14.0, 64 rows 22 / 16, 128
 // 27 / 19.5, 256 41.5 / 35, 400 57 / 49; 128 rows of 2048 -> 512 35 / 30, of 128 -> 128 16.5 / 10.6, of 784 -> 100 26.4 / 12.6, of 500 -> 50 29.5 / 12.8.
-template <int SPLIT>
+template <int SPLIT, bool FOLDS>
 __global__ void __launch_bounds__(8 * kWave, 4)
 fc_backward_kernel(const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ grad, const float* __restrict__ y,
                    const float* __restrict__ rcp, float* __restrict__ dx, float* __restrict__ dw, float* __restrict__ zeros, int n_zeros,
-                   int B, int I, int J, int rows, int tiles_i, int dx_tiles, int dx_blocks, int dx_first, int dw_cols, float max_cmp, float biasvolt, float neg_s,
+                   int B, int I, int J, int rows, int tiles_i, int dx_tiles, int dx_blocks, int dx_first, int dw_cols, int fold, float max_cmp, float biasvolt, float neg_s,
                    float post) {
     constexpr int FLOATS = dwd_lds_floats(8) > dx_lds_bytes(8) / 4 ? dwd_lds_floats(8) : dx_lds_bytes(8) / 4;
     __shared__ __align__(16) float lds[FLOATS];
@@ -535,7 +558,7 @@ fc_backward_kernel(const float* __restrict__ x, const float* __restrict__ w, con
         fc_grad_input_tile<SPLIT, false, true>(src, w, upstream, y, dx, B, I, J, tiles_i, dx_tiles, dx_block, dx_blocks, lds);
     } else {
         const int tile = dx_block < 0 ? (int)blockIdx.x : dx_block - dx_blocks, by = tile / dw_cols;
-        grad_weight_dense_tile<8, true>(x, upstream, y, dw, B, I, J, rows, B, biasvolt, neg_s, post, tile - by * dw_cols, by, 0, lds);
+        grad_weight_dense_tile<8, true, FOLDS>(x, upstream, y, dw, B, I, J, rows, B, fold, biasvolt, neg_s, post, tile - by * dw_cols, by, 0, lds);
     }
 }
 
@@ -935,16 +958,26 @@ static JointGrid joint_grid(int64_t B, int64_t I, int64_t rows, int64_t J, bool 
 // dX and dW of a dense layer in one launch (dX == NULL: dW alone).  `slices`: what the samples would be cut into for dW alone.
 // The parts of a launch with more workgroups fill the chip by themselves, with tiles of their own (us, apart / together: 200 x 2048 ->
 // 512, 1096 workgroups, 61 / 42; 333 x 1521 -> 777, 1320, 87 / 73; 400 x 3000 -> 512, 2726, 116 / 99; 512 x 3000 -> 512, 3384, 140 / 126; 300 x
-// 4096 -> 1000, 3472, 211 / 214; 400 x 10 000 -> 200, 8453, 171 / 179).  A tile of dW goes over all samples here, which up to some
-// hundred of them takes less than the launches that slices need (200 x 128 -> 128 29 / 15.4, 333 x 333 -> 333 34 / 23, 400 x 500 -> 50 34 / 24.5,
-// 512 x 128 -> 128 28.4 / 30.3; dW alone, 333 x 128 -> 128 22.4 / 21.3, 400 rows 22.3 / 24.2).
+// 4096 -> 1000, 3472, 211 / 214; 400 x 10 000 -> 200, 8453, 171 / 179).
+// Where dW alone would be cut into slices, a tile goes over all samples here and folds its sums (joint_folds): less than the launches that
+// slices need where tiles are many, or samples few (us, slices / together: 512 -> 512, 72 tiles, 270, 333, 448 rows 30 / 23, 31 / 26, 33.5 / 31,
+// 480 37 / 34 but 300 -> 300, 25 tiles, 270 and 333 rows 20.6 / 22, 21 / 27; 500 -> 50, eight tiles, 200, 240, 256 rows 21 / 16.5, 21 / 18,
+// 20 / 20; 128 -> 128, six tiles, 200 rows 16.1 / 16.4), and not for dW alone (256 x 300 -> 300 13 / 20, 512 -> 512 17 / 19).
+constexpr int64_t JOINT_FEW_ROWS = 240;
 bool fc_backward_joint_supported(int64_t B, int64_t I, int64_t J, bool dx, int slices) {
     const JointGrid g = joint_grid(B, I, I + 1, J, dx);
-    return g.dx_blocks + g.dw_blocks <= 3072 && (slices == 1 || B <= (dx ? 448 : 352));
+    if (g.dx_blocks + g.dw_blocks > 3072) return false;
+    return slices == 1 || (dx && B <= 448 && (g.dw_blocks >= 64 || (g.dw_blocks >= 8 && B <= JOINT_FEW_ROWS)));
 }
+// How often a tile's sums are folded: as often as there would be slices, which keeps its error against 64 bits at or below that of the slices (rms, in
+// units of the terms' absolute sum and 1e-9, slices / one chain per wavefront / folded: 256 x 512 -> 512 8.8 / 10.3 / 8.2, 333 rows 8.1 / 10.1 / 7.6,
+// 448 7.4 / 9.7 / 7.0, 448 x 333 -> 1000 8.0 / 9.7 / 7.7).  Up to 240 rows half as often does that, since a tree adds its wavefronts and slices add
+// theirs one after the other (230 x 300 -> 300 9.1 / 10.5 / 8.9).  A fold costs about 1.3 us.
+static int joint_folds(int64_t B, int slices) { return slices == 1 ? 1 : B <= JOINT_FEW_ROWS ? slices / 2 + 1 : slices; }
 
 int launch_fc_backward_joint(const float* x, const float* w, const float* grad, const float* y, const float* rcp, float* dx, float* dw,
-                             float* zeros, int n_zeros, int64_t B, int64_t I, int64_t J, const NeuronParams& np, hipStream_t stream) {
+                             float* zeros, int n_zeros, int64_t B, int64_t I, int64_t J, int slices, const NeuronParams& np, hipStream_t stream) {
+    const int turns = (int)((B + DWD_TURN - 1) / DWD_TURN), folds = joint_folds(B, slices);
     const int64_t rows = I + np.bias;
     const JointGrid g = joint_grid(B, I, rows, J, dx != nullptr);
     // The longer tiles come first, so that the shorter ones fill the end: dW takes 8192 terms a sample, dX 512 an output, of which it
@@ -957,10 +990,11 @@ int launch_fc_backward_joint(const float* x, const float* w, const float* grad, 
     const LeadScale ls = lead_scale(np.max_time);
     {
         KernelTimerScope timer_("fc_backward", stream);
-        auto kern = J < 64 ? fc_backward_kernel<1> : fc_backward_kernel<8>;
+        auto kern = J < 64 ? (folds > 1 ? fc_backward_kernel<1, true> : fc_backward_kernel<1, false>)
+                           : (folds > 1 ? fc_backward_kernel<8, true> : fc_backward_kernel<8, false>);
         hipLaunchKernelGGL(kern, dim3((unsigned)(g.dx_blocks + g.dw_blocks)), dim3(8 * kWave), 0, stream, x, w, grad, y, rcp, dx, dw, zeros,
                            zeros ? n_zeros : 0, (int)B, (int)I, (int)J, (int)rows, (int)((I + DX_I - 1) / DX_I), (int)g.dx_tiles, (int)g.dx_blocks,
-                           (int)(dw_first ? g.dw_blocks : 0), (int)((J + DWD_T - 1) / DWD_T), np.max_cmp, np.biasvolt, ls.neg_s, ls.post);
+                           (int)(dw_first ? g.dw_blocks : 0), (int)((J + DWD_T - 1) / DWD_T), (turns + folds - 1) / folds, np.max_cmp, np.biasvolt, ls.neg_s, ls.post);
     }
     SNNTC_HIP_CHECK(hipGetLastError());
     return SNNTC_OK;

@@ -191,7 +191,7 @@ int launch_backward_prologue(const float* grad, const float* y, const float* rcp
 
 bool fc_backward_joint_supported(int64_t B, int64_t I, int64_t J, bool dx, int slices);
 int launch_fc_backward_joint(const float* x, const float* w, const float* grad, const float* y, const float* rcp, float* dx, float* dw,
-                             float* zeros, int n_zeros, int64_t B, int64_t I, int64_t J, const NeuronParams& np, hipStream_t stream);
+                             float* zeros, int n_zeros, int64_t B, int64_t I, int64_t J, int slices, const NeuronParams& np, hipStream_t stream);
 int launch_fc_grad_input(const float* x, const float* w, const float* upm, const float* ym, float* dx,
                          int64_t B, int64_t I, int64_t J, hipStream_t stream);
 int grad_prepare_device();

@@ -19,7 +19,7 @@ def t(a):
     (33, 40, 255), (20, 63, 257),                                         # eight and sixteen wavefronts
     (260, 520, 130), (700, 500, 40), (1100, 1000, 101),                   # many tiles: eight, one, four
     (129, 64, 300), (515, 127, 64), (1030, 300, 257),                     # slices of the samples
-    (300, 1500, 1299),                                                    # four wavefronts per tile of dW
+    (300, 1500, 1299), (512, 1300, 900),                                  # many tiles in one launch, and in parts: four wavefronts per tile of dW
     (2200, 63, 33), (4200, 64, 65),                                       # one and four tiles: more slices than sixteen
 ])
 def test_dense_gradients(B, I, J):
@@ -47,7 +47,7 @@ def test_dense_gradients(B, I, J):
 @pytest.mark.parametrize("bias", [True, False])
 @pytest.mark.parametrize("B,I,J", [
     (1, 1, 128), (16, 32, 128), (17, 33, 129), (15, 64, 191), (33, 63, 320),                  # less than a tile, one, a bit more
-    (63, 191, 1000), (208, 2000, 130), (240, 2000, 130),                                    # both sides of the line to separate launches
+    (63, 191, 1000), (208, 2000, 130), (240, 2000, 130),                                    # tiles of a turn of the chip, and of more
 ])
 def test_dense_gradients_in_one_launch(B, I, J, bias):
     """dX and dW together, dW alone and dX alone: the same bits, and within the band of the fp64 sums."""
@@ -79,9 +79,12 @@ def test_dense_gradients_in_one_launch(B, I, J, bias):
 
 @pytest.mark.parametrize("B,I,J", [
     (1, 1, 17), (129, 255, 17), (33, 64, 63), (40, 65, 64), (17, 31, 127),                    # dX tiles of one wavefront, of eight
-    (352, 70, 130), (353, 70, 130), (448, 40, 50), (449, 40, 50),                             # slices alone up to here, behind it
+    (352, 70, 130), (353, 70, 130), (448, 40, 50), (449, 40, 50),                             # slices, and few tiles
+    (128, 200, 100), (240, 500, 50), (241, 500, 50), (240, 500, 33), (240, 447, 64), (240, 448, 64),   # eight tiles up to 240 rows and beyond, seven tiles
+    (257, 300, 1000), (385, 511, 512), (412, 511, 512), (413, 511, 512), (448, 511, 512), (449, 511, 512), (448, 447, 512),    # 64 tiles up to 448 rows and beyond, 56
     (130, 100, 260), (131, 100, 260), (256, 784, 700), (300, 784, 770),                       # dX tiles first, dW tiles first
-    (370, 2048, 1000), (430, 3000, 500), (446, 3300, 500),                                    # up to 3072 workgroups, and more
+    (370, 2048, 1000), (430, 3000, 500), (446, 3300, 500), (100, 13000, 64), (100, 13100, 64),      # up to 3072 workgroups, and more
+    (16, 8000, 1536), (16, 8000, 1559),                                                       # dW alone
 ])
 def test_dense_gradients_whole_or_in_parts(B, I, J):
     """Both sides of the rules that choose one launch, the order of its tiles and their form, within the band of the fp64 sums."""
@@ -108,6 +111,27 @@ def test_dense_gradients_whole_or_in_parts(B, I, J):
     assert np.all(np.abs(dx - rdx) <= 1e-6 * np.abs(adx) + 1e-30)
     for got in (dw, alone):
         assert np.all(np.abs(got - rdw) <= 1e-6 * np.abs(adw) + 1e-30)
+
+
+@pytest.mark.parametrize("B,I,J,slices", [(230, 300, 300, 13.55), (256, 512, 512, 12.88), (300, 128, 128, 12.04), (333, 512, 512, 11.69), (400, 500, 50, 10.89),
+                                          (448, 200, 100, 10.17), (448, 300, 700, 10.30)])
+def test_dense_weight_gradients_are_as_exact_in_one_launch(B, I, J, slices):
+    """Samples that would be cut into slices (of 64 or more) are not summed in longer chains where one launch takes them."""
+    import snntc_amd as snn
+    rng = np.random.default_rng(B + I + J)
+    x = np.exp(1.0 - rng.random((B, I))).astype(np.float32)
+    y = np.exp(1.2 * rng.random((B, J))).astype(np.float32)
+    w = rng.standard_normal((I + 1, J)).astype(np.float32)
+    out = np.concatenate([y, rng.random((B, J)).astype(np.float32)])
+    g = np.zeros((2 * B, J), np.float32)
+    g[:B] = rng.standard_normal((B, J))
+    p = capi.fc_params(1.0)
+    dw = snn.snnfc_grad(t(g), t(x), t(w), p, t(out))[1].cpu().numpy()
+    rdw, adw = (capi.fc_backward_dev(q, x, w, p, out, wide=True)[1] for q in (g, np.abs(g)))
+    # `slices`: what the sum of slices of 64 samples and more shows on these inputs, in 1e-9 of the terms' absolute sum (the rounding of the
+    # reference's results among it); one chain of additions per wavefront shows 13.0 to 14.7.  The margin is for another order of additions.
+    error = (dw.astype(np.float64) - rdw)[adw != 0] / adw[adw != 0]
+    assert np.sqrt(np.mean(error ** 2)) <= 1.03e-9 * slices
 
 
 @pytest.mark.parametrize("B,H,W,C,Kc,S", [
