@@ -981,12 +981,14 @@ int launch_fc_backward_joint(const float* x, const float* w, const float* grad, 
     const int64_t rows = I + np.bias;
     const JointGrid g = joint_grid(B, I, rows, J, dx != nullptr);
     // The longer tiles come first, so that the shorter ones fill the end: dW takes 8192 terms a sample, dX 512 an output, of which it
-    // does a third as many a clock.  (us, dX / dW first: 256 x 784 -> 800 41 / 35, 400 rows 62 / 49, 300 x 1521 -> 777 64 / 59; 256 x 300 -> 2048
+    // does a third as many a clock.  (us, dX / dW first: 256 x 784 -> 800 38 / 33, 400 rows 59 / 49, 300 x 1000 -> 200 30 / 25; 256 x 300 -> 2048
     // 38 / 46, 32 x 3000 -> 512 15.3 / 20.7.)  Where all workgroups, of which a CU holds two, are there at once, only much longer ones
-    // (128 x 1000 -> 130 15 / 13, but 333 x 512 -> 1000 35.5 / 37), and not where the dW tiles behind the first turn are many and have a CU
-    // each (333 x 784 -> 800 43 / 46.5, 128 x 1521 -> 777 33 / 34).
+    // (364 x 407 -> 812 35 / 31, 253 x 720 -> 557 25 / 23, 128 x 1000 -> 130 13 / 11, but 333 x 512 -> 1000 33 / 34, 121 x 1032 -> 717 23 / 22.5).  Over
+    // 230 shapes of 48 to 740 rows the other order was never more than 4 % ahead, but for one case: dX tiles that are a little more than the
+    // first turn, and dW tiles behind them with a CU each (dX first 0 to 7 % ahead in 20 of 27: 333 x 784 -> 800 43 / 45, 586 x 460 -> 1412 68 / 74).
     const int64_t behind = g.dx_blocks + g.dw_blocks - 512;
-    const bool dw_first = behind <= 0 ? 2 * B > J : 4 * B > J && !(behind >= 128 && behind <= 256);
+    const bool just_over = behind >= 128 && behind <= 256 && g.dx_blocks > 512 && g.dx_blocks <= 600;
+    const bool dw_first = behind <= 0 ? 8 * B > 3 * J : 4 * B > J && !just_over;
     const LeadScale ls = lead_scale(np.max_time);
     {
         KernelTimerScope timer_("fc_backward", stream);
