@@ -721,7 +721,10 @@ reduce_partials_kernel(const float* __restrict__ partial, float* __restrict__ ou
 }
 
 // Up to eight slices of whole float4s: an element is added up by one thread, four at a time, in the same order (a slice is a group of
-// its own there).  Wide layers have few slices of many elements: 4 of 2.4 M 27 -> 14 us.
+// its own there).  Wide layers have few slices of many elements: 4 of 2.4 M 27 -> 14 us, 3 of 1 M 67 -> 59 with the launch before it.  With too few
+// for the chip a thread's chain of slices takes longer than the sums of eight groups: the line lies at about 25 600 elements for each
+// slice (3 of 69 and 114 K 12.6 -> 12.4 and 13.7 -> 13.4, 5 of 98 and 175 K 14.7 -> 14.9 and 16.8 -> 16.0, 8 of 60 and 119 K 13.4 -> 14.5 and 21.7 -> 23.0).
+constexpr int64_t RED_FEW_FROM = 25600;
 __global__ void __launch_bounds__(256)
 reduce_few_kernel(const float4* __restrict__ partial, float4* __restrict__ out, int64_t n4, int nsplit) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -933,7 +936,7 @@ int launch_reduce_partials(const float* partial, float* dw, int64_t n, int nspli
     if (n <= 0 || nsplit <= 1) return SNNTC_OK;
     {
         KernelTimerScope timer_("reduce_partials", stream);
-        const bool few = nsplit <= RED_GROUPS && n % 4 == 0 &&
+        const bool few = nsplit <= RED_GROUPS && n >= RED_FEW_FROM * nsplit && n % 4 == 0 &&
                          ((reinterpret_cast<uintptr_t>(partial) | reinterpret_cast<uintptr_t>(dw)) & 15) == 0;
         if (few)
             hipLaunchKernelGGL(reduce_few_kernel, dim3(blocks_for(n / 4, 256)), dim3(256), 0, stream,
