@@ -835,33 +835,44 @@ static int64_t cv_grad_weight_row_blocks(const ConvGeom& g) {
     return g.Kh * ((g.Kw * g.C + DWW_RI - 1) / DWW_RI);
 }
 
-// Channels a wavefront of cv_grad_weight_taps_kernel owns, 0: the layer goes to the kernels for any shape.  Thirty-two where that makes
-// workgroups enough; launches that do not fill the chip keep the blocks of 32 weight rows, of which there are three times as many (3136 patches of
-// 64 channels to 64: 15.2 us against 18 – 20, 784 of 128 to 100 16.2 against 18 – 20); 32 channels to 64 are three workgroups a slice, or six of sixteen
-// channels (32 768 patches 40 / 38 us).  Channels in sixteens otherwise (100 352 patches of 16 to 48 38 -> 30 us, 784 of 112 to 48
-// 14.6 -> 13.0; 1200 of 16 to 128, too few for it, 11.3 against 13.0).
-static int cv_grad_weight_taps_channels(const ConvGeom& g) {
-    if (g.Kw != DWT_KW || g.Sw != 1 || g.C % 16 != 0 || g.Kc <= 32 || g.S * g.Kc * 4 >= 0x7fffffffLL) return 0;
-    const int64_t blocks16 = (g.Kc + kWave - 1) / kWave * g.Kh * (g.C / 16);
-    if (g.C % 32 != 0) return blocks16 * std::min<int64_t>(g.S / 128, 128) >= 100 ? 16 : 0;
-    if (blocks16 * std::min<int64_t>(g.S / 128, 128) < 700) return 0;
-    return blocks16 >= 12 ? 32 : 16;
+// Whether a layer's dW goes to cv_grad_weight_taps_kernel, the channels a wavefront owns there, and into how many slices its patches are cut.
+// Lines from some 400 shapes, each in all forms (us; blocks of 32 rows / sixteen channels / thirty-two).  `terms`: 64 outputs of sixteen channels of a
+// kernel row times runs of 128 patches.
+//   Channels in thirty-twos: the blocks of 32 rows, of which there are three times as many, below 700 terms (784 patches of 512 to 48 23.7 / 25.4 / 24.4,
+//   1568 of 96 to 64 17.1 / 18.8 / 21.1); sixteen channels up to 3000 in as many slices as thirty-two would have, so that sums are no longer
+//   (3136 of 128 to 128 38.4 / 34.9 / 40.0, 1568 of 256 to 256 65.7 / 58.7 / 58.7, 12 544 of 64 to 64 37.4 / 38.5 / 39.5); then thirty-two (12 544 of 128 to
+//   128 100 / 93 / 89, 100 352 of 64 to 64 194 / 183 / 166, 61 440 of 32 to 64 under five rows 107 / 115 / 97).
+//   Others, whose rows the blocks do not divide: from 100 terms up to 48 channels, else 200 (784 of 144 to 64 15.3 / 16.1, 784 of 112 to 128 18.4 / 17.3,
+//   6272 of 16 to 64 19.4 / 17.2).
+struct TapsPlan { int channels, slices; };               // channels == 0: the kernels for any shape
+static TapsPlan cv_grad_weight_taps_plan(const ConvGeom& g) {
+    if (g.Kw != DWT_KW || g.Sw != 1 || g.C % 16 != 0 || g.Kc <= 32 || g.S * g.Kc * 4 >= 0x7fffffffLL) return {};
+    const int64_t blocks = (g.Kc + kWave - 1) / kWave * g.Kh * (g.C / 16);
+    const int64_t terms = blocks * (g.S / 128), capped = blocks * std::min<int64_t>(g.S / 128, 128);
+    // slices of launches of so many workgroups, which have twice as many wavefronts as the line's others
+    const auto slices = [&](int64_t workgroups) { return weight_grad_splits(g.S / 2, workgroups * 2); };
+    if (g.C % 32 != 0) {
+        if (capped < (g.C <= 48 ? 100 : 200)) return {};
+        // (small launches in more of them: 1568 of 80 to 64 18.0 -> 15.9, 1568 of 144 to 100 29.0 -> 26.5; but 25 088 of 16 to 100 41.4 -> 43.4)
+        return {16, capped < 700 ? weight_grad_splits(g.S / 2, blocks) : slices(blocks)};
+    }
+    if (capped < 700) return {};
+    if (terms >= 3000) return {32, slices(blocks / 2)};
+    return {16, slices(blocks >= 12 ? blocks / 2 : blocks)};
 }
 
-// Workgroups per slice of the kernels for any shape, and slices that the patch range is cut into (cv_grad_weight_taps_kernel: its
-// workgroups have twice as many wavefronts).
+// Workgroups per slice of the blocks of 32 rows, and slices that the patch range is cut into.
 int cv_grad_weight_row32_blocks(const ConvGeom& g) { return (int)(((g.Kc + kWave - 1) / kWave) * cv_grad_weight_row_blocks(g)); }
 int cv_grad_weight_splits(const ConvGeom& g) {
-    const int cb = cv_grad_weight_taps_channels(g);
-    return cb ? weight_grad_splits(g.S / 2, (g.Kc + kWave - 1) / kWave * g.Kh * (g.C / cb) * 2)
-              : weight_grad_splits(g.S, cv_grad_weight_row32_blocks(g));
+    const TapsPlan taps = cv_grad_weight_taps_plan(g);
+    return taps.channels ? taps.slices : weight_grad_splits(g.S, cv_grad_weight_row32_blocks(g));
 }
 
 // All rows of dW, bias row included (or of every partial-sum slice when nsplit > 1).
 int launch_cv_grad_weight_wide(const float* xpad, const float* upm, const float* ym, float* dst, int nsplit,
                                const ConvGeom& g, int64_t rows, const NeuronParams& np, hipStream_t stream) {
     const int seg_per_slice = (int)((g.S + nsplit - 1) / nsplit);
-    const int taps = cv_grad_weight_taps_channels(g);
+    const int taps = cv_grad_weight_taps_plan(g).channels;
     dim3 grid((unsigned)((g.Kc + kWave - 1) / kWave), (unsigned)(taps ? g.Kh * (g.C / taps) : cv_grad_weight_row_blocks(g)), (unsigned)nsplit);
     if (grid.y > 65535u) return fail(SNNTC_ERR_TOO_LARGE, "weight gradient: too many weight rows");
     if (taps) {

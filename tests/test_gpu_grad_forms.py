@@ -173,13 +173,32 @@ def test_conv_input_gradients_at_the_edges_of_tiles(B, H, W, C, Kc, S):
         assert np.array_equal(part, dx[:, top:top + h, left:left + wd])
 
 
+# Three-column kernels.  `slices`: what the form that the layer takes asks for, `least`: what a smaller workspace may come down to (the count of the
+# blocks of 32 weight rows; where it is the larger one the workspace has room for it).  A layer that changes its form changes these.
 @pytest.mark.parametrize("bias", [True, False])
-@pytest.mark.parametrize("B,H,W,C,Kc,Kh,Sh", [
-    (40, 8, 9, 32, 64, 3, 1), (9, 21, 23, 64, 65, 3, 1), (30, 12, 5, 64, 128, 3, 2), (60, 9, 4, 64, 64, 2, 1),       # 32 channels a wavefront; rows of 7, 21, 3 and 2 patches
-    (130, 6, 3, 96, 64, 3, 1), (7, 40, 12, 16, 40, 3, 1), (20, 9, 19, 48, 130, 3, 1), (6, 22, 22, 80, 33, 1, 1),     # one patch a row; sixteen channels
+@pytest.mark.parametrize("B,H,W,C,Kc,Kh,Sh,slices,least", [
+    # blocks of 32 rows
+    (40, 8, 9, 32, 64, 3, 1, 26, 26), (9, 21, 23, 64, 65, 3, 1, 42, 42), (30, 12, 5, 64, 128, 3, 2, 7, 7), (60, 9, 4, 64, 64, 2, 1, 15, 15),
+    (130, 6, 3, 96, 64, 3, 1, 8, 8), (7, 40, 12, 16, 40, 3, 1, 41, 41), (6, 22, 22, 80, 33, 1, 1, 32, 32),
+    # sixteen channels a wavefront: rows of 17, 7, 1, 2 and 7 patches; 80 channels, two kernel rows
+    (20, 9, 19, 48, 130, 3, 1, 18, 34), (25, 10, 9, 256, 65, 3, 1, 8, 7), (120, 21, 3, 256, 66, 3, 2, 8, 7), (60, 21, 4, 256, 66, 3, 2, 8, 7),
+    (40, 8, 9, 256, 70, 3, 1, 8, 7), (30, 12, 12, 80, 70, 2, 1, 25, 48),
 ])
-def test_conv_weight_gradients_by_pixels(B, H, W, C, Kc, Kh, Sh, bias):
-    """Three-column kernels: runs of patches that begin and end within rows and images, the last slices without a patch for some wavefronts."""
+def test_conv_weight_gradients_by_pixels(B, H, W, C, Kc, Kh, Sh, slices, least, bias):
+    """Runs of patches that begin and end within rows and images, the last slices without a patch for some wavefronts."""
+    _check_weight_gradients(B, H, W, C, Kc, Kh, Sh, slices, least, bias)
+
+
+@pytest.mark.parametrize("B,H,W,C,Kc,Kh,Sh,slices,least,bias", [
+    (75, 10, 9, 256, 65, 3, 1, 16, 7, True), (205, 21, 3, 512, 65, 3, 2, 8, 6, True), (103, 21, 4, 512, 65, 3, 2, 8, 6, False), (192, 9, 4, 512, 65, 2, 1, 12, 8, True),
+    (60, 30, 30, 64, 33, 2, 1, 192, 128, False),
+])
+def test_conv_weight_gradients_by_pixels_of_32_channels(B, H, W, C, Kc, Kh, Sh, slices, least, bias):
+    """The launches that fill the chip: rows of 7, 1, 2, 2 and 28 patches, row strides of two, two kernel rows, outputs that are no multiple of 64."""
+    _check_weight_gradients(B, H, W, C, Kc, Kh, Sh, slices, least, bias)
+
+
+def _check_weight_gradients(B, H, W, C, Kc, Kh, Sh, slices, least, bias):
     import ctypes
     import snntc_amd as snn
     from snntc_amd import _lib
@@ -214,12 +233,21 @@ def test_conv_weight_gradients_by_pixels(B, H, W, C, Kc, Kh, Sh, bias):
     ptr = lambda a: a.data_ptr() if a is not None else None                      # noqa: E731
     call = lambda n: lib.snntc_cv_backward(ptr(args[0]), ptr(args[1]), ptr(args[2]), fp, ptr(args[3]), None, ptr(again), None, B, H, W, C, Kc,   # noqa: E731
                                            w.shape[0], 2 * B, ptr(ws), n, stream)
+    align = lambda floats: -(-4 * floats // 256) * 256                           # noqa: E731
+    P, S = Kh * 3 * C, B * Nh * Nw
+    others = align(S * Kc) + align((P + 1) * Kc) + (align(S * P) if Kc % 16 else 0)          # (the last for dX of such layers)
+    partial = lambda n: others + (align(n * (P + 1) * Kc) if n > 1 else 0)                   # noqa: E731
+    assert need.value == partial(max(slices, least))
     assert call(need.value) == _lib.OK
     assert torch.equal(again, dw)
+    fewer = 0
     for room in range(need.value - 256, 0, -max(256, need.value // 40 // 256 * 256)):
         if call(room) != _lib.OK:
             break
         err = np.abs(again.cpu().numpy() - rdw)
         assert np.all(err <= 2e-6 * np.abs(adw) + 1e-30)
+        fewer += 1
     else:
         raise AssertionError("no workspace was refused")
+    assert (fewer > 0) == (slices > least)
+    assert call(partial(least)) == _lib.OK and call(partial(least) - 256) != _lib.OK
