@@ -2130,10 +2130,10 @@ static bool takes_split(int cols, int64_t S, int64_t I, int64_t stride, int64_t 
            I + np.bias < (1 << 24) && J < (1 << 22) && (I + np.bias) * J * 4 < 0x7fffffffLL;
 }
 
-// Widest column slice (8..64) whose I + bias rows fit in LDS; 0: none does.  (The split kernel's items are 32 lanes: where such
+// Widest column slice (8..64) whose I rows fit in LDS (the bias row is read from memory); 0: none does.  (The split kernel's items are 32 lanes: where such
 // slices are few enough for it they are taken: 512 -> 1000 of one row 4.2 + 13 -> 11.8 us with the order.)
 static int slice_columns(int64_t S, int64_t I, int64_t stride, int64_t J, const NeuronParams& np, int cus) {
-    const size_t rows = (size_t)I + np.bias;
+    const size_t rows = (size_t)I;
     int cols = 64;
     while (cols > 8 && (rows * cols * sizeof(float) > (size_t)LDS_SCAN_TARGET || cols / 2 >= J)) cols >>= 1;
     if (rows * cols * sizeof(float) > (size_t)LDS_SCAN_TARGET) return 0;

@@ -114,6 +114,15 @@ def test_scans_by_rounds(B, I, J, law):
     _check(x, w, p)
 
 
+# The most inputs whose slice of 64, 32, 16 and 8 columns fits in LDS, with the bias row in memory, and one more
+@pytest.mark.parametrize("bias", [True, False])
+@pytest.mark.parametrize("B,I,J", [(5003, 639, 64), (40, 639, 200), (2603, 1279, 40), (33, 1279, 100), (1207, 2559, 24), (49, 2559, 40), (605, 5118, 9), (9, 5118, 20), (9, 5119, 20)])
+def test_widest_slices(B, I, J, bias):
+    x, w, p, _ = dense_case(B + I + J, B, I, J, bias, "baseline")
+    x[1::3] = np.where(np.random.default_rng(I).random(x[1::3].shape) < 0.1, np.float32(1e5), x[1::3])
+    _check(x, w, p)
+
+
 # Few wavefronts with rows of slices of eight columns: whole turns of eight chunks and a chunk, an input more or less, and rows that end early.
 @pytest.mark.parametrize("law", ["spread", "jump"])
 @pytest.mark.parametrize("B,I,J", [(9, 2496, 64), (17, 2559, 40), (24, 2561, 64), (49, 3001, 70), (20, 4607, 33), (100, 4608, 200)])
