@@ -139,7 +139,7 @@ scan_kernel(const float* __restrict__ sorted, const int32_t* __restrict__ perm,
 //
 // Walking W rows in sorted order from memory re-reads the whole matrix once per segment (8 GB of
 // cache traffic for 65 536 patches of a 3x3x64 -> 64 layer).  Here a workgroup copies the COLS
-// columns it owns -- all I(+1) rows, at most 160 KB -- into LDS once and then scans many segments
+// columns it owns -- all I rows, at most 160 KB -- into LDS once and then scans many segments
 // against it.  A wavefront covers 64/COLS segments at a time (lanes = segment x column), so narrow
 // layers (J = 10, Kc = 32) and long segments (COLS = 8 for 4608 inputs) use the same kernel.
 // Sorted values and row indices are fetched per lane (all lanes of a segment read the same
@@ -999,11 +999,12 @@ constexpr float ROUND_DX = 0x1p-14f;                      // 1024u
 // the slack of a round next to a threshold of one; beyond 0.6 of it rounds end early (576 inputs with deviation 3.87 / sqrt(I): at 0.15 of a row).
 constexpr float ROUNDS_UP_TO = 0.6f;
 constexpr int ROUNDS_FROM = 400;
-// Few wavefronts (LONE): 41 instructions a chunk instead of 51, with the decision once per turn of the entries' ring, whose requests and
-// weights go on into the chunks behind.  A wavefront fetches a second loop of some 3 KB of code for it, so only the rows of slices of
-// eight columns are long enough (us without / with: 49 segments of 4608 to 512 86 / 78, 100 of 4096 to 256 77 / 70, 200 of 3000 to 300 74 / 69,
-// deviation 3.87 / sqrt(I) 109 / 102, 87 / 80, 136 / 134; sixteen columns, 16 of 2048 to 512 33.9 / 35.0, 100 of 2400 to 64 38.6 / 40.4, 128 of
-// 1521 to 500 32.1 / 33.0).
+// Few wavefronts (LONE): 53 instructions a chunk instead of 64, 37 of them vector and LDS ones instead of 51, with the decision once per turn of
+// the entries' ring, whose requests and weights go on into the chunks behind.  A wavefront fetches a second loop of some 3 KB of code for it, so only the rows of slices of
+// eight columns are long enough: 2560 inputs and more, or from here on layers of at most eight neurons (us of the layer without / with: 49 segments of
+// 4608 to 512 95 / 86, 49 of 2560 to 512 60 / 55, 200 of 3000 to 300 87 / 80, 300 of 1280 to 8 35 / 33, 1000 of 1280 to 8 36.4 / 34.9, 600 of 1400 to 5 38 / 36,
+// 3000 of 2300 to 8 86 / 82; of the scan, deviation 3.87 / sqrt(I), 49 of 4608 to 512 109 / 102, 100 of 4096 to 256 87 / 80, 200 of 3000 to 300
+// 136 / 134; sixteen columns, 16 of 2048 to 512 33.9 / 35.0, 100 of 2400 to 64 38.6 / 40.4, 128 of 1521 to 500 32.1 / 33.0).
 constexpr int LONE_ROUNDS_FROM = 1280;
 
 // The test of a chunk for one scan of every lane: wb, yb are the sums behind it.  Lanes in the mask `open`
@@ -1246,7 +1247,7 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
                    const int32_t* __restrict__ n_real, const float* __restrict__ w, float* __restrict__ y_out,
                    float* __restrict__ rcp_out, int32_t* __restrict__ k_out, int S, int I, int stride, int J,
                    int n_slices, int n_groups, int waves, NeuronParams np, TimeCopy copy) {
-    extern __shared__ __align__(16) float wl[];                          // [I + bias][COLS], then `red`
+    extern __shared__ __align__(16) float wl[];                          // [I][COLS], then block_max's room, which the rows' staging reuses
     constexpr int LANES = COLS / CH;                       // lanes per segment
     constexpr int SEGS = kWave / LANES;                    // segments per wavefront
     static_assert(LANES % 4 == 0, "the four lanes of a quad belong to one segment");
@@ -1625,6 +1626,7 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
                         }
                     };
                     // BY_ROUND: tested with the other chunks of its round, behind the last of them.
+                    static_assert(!ROUNDS || !BY_ROW, "eight-column slices alone have rows long enough");
                     float round_start[CH], x_first;
                     uint64_t soon = 0, fails = 0;
                     auto chunk = [&](auto ph_c, int k, auto by_round_c) {
@@ -1642,7 +1644,7 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
                             }
                         }
                         if constexpr (BY_ROUND && ph % ROUND == 0) {
-                            x_first = BY_ROW ? row_broadcast<0>(__uint_as_float(rx[R].x)) : quad_broadcast<0>(__uint_as_float(rx[R].x));
+                            x_first = quad_broadcast<0>(__uint_as_float(rx[R].x));
 #pragma unroll
                             for (int c = 0; c < CH; ++c) round_start[c] = run_w[c];
                         }
@@ -1666,7 +1668,7 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
                         if constexpr (!BY_ROUND) decide();
                         half(std::integral_constant<int, 1>{});
                         if constexpr (BY_ROUND && ph % ROUND == ROUND - 1) {
-                            const float x7 = BY_ROW ? row_broadcast<15>(__uint_as_float(rx[R].y)) : quad_broadcast<3>(__uint_as_float(rx[R].y));
+                            const float x7 = quad_broadcast<3>(__uint_as_float(rx[R].y));
                             const float dx = __fmaf_rn(x7, ROUND_DX, x7 - x_first), x7e = x7 * ROUND_AT;
                             const float thr = __fmaf_rn(dx, 4.0f * w4, x7 * end_w_round);
 #pragma unroll
@@ -1703,7 +1705,7 @@ scan_filter_kernel(const float* __restrict__ sorted, const int32_t* __restrict__
                     int k0 = kmin;
                     bool more = true;
                     const bool rotate = waves > 4;          // (more than a wavefront per SIMD)
-                    if (ROUNDS && by_rounds && first_pass && any_odd == 0) {
+                    if constexpr (ROUNDS) if (by_rounds && first_pass && any_odd == 0) {
                         while (soon == 0 && k0 + PHASES * CHUNK <= n_full_min) {
                             if (rotate) rotate_wave_priority(k0 / (PHASES * CHUNK) + (wave >> 2));
                             for_each_phase<PHASES>([&](auto ph_c) {

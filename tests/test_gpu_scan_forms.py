@@ -123,9 +123,11 @@ def test_widest_slices(B, I, J, bias):
     _check(x, w, p)
 
 
-# Few wavefronts with rows of slices of eight columns: whole turns of eight chunks and a chunk, an input more or less, and rows that end early.
+# Few wavefronts with rows of slices of eight columns, long ones and those of up to eight neurons from 1280 inputs on: whole turns of eight chunks
+# and a chunk, an input more or less, and rows that end early.
 @pytest.mark.parametrize("law", ["spread", "jump"])
-@pytest.mark.parametrize("B,I,J", [(9, 2496, 64), (17, 2559, 40), (24, 2561, 64), (49, 3001, 70), (20, 4607, 33), (100, 4608, 200)])
+@pytest.mark.parametrize("B,I,J", [(9, 2560, 64), (17, 2623, 40), (24, 2561, 64), (49, 3001, 70), (20, 4607, 33), (100, 4608, 200),
+                                   (600, 1279, 8), (600, 1280, 8), (1000, 1343, 5), (300, 1345, 7), (700, 2047, 6)])
 def test_long_rows_of_few_wavefronts(B, I, J, law):
     x, w, p, _ = dense_case(B + I + J, B, I, J, True, "baseline")
     rng = np.random.default_rng(I + J)
