@@ -29,7 +29,8 @@ constexpr int DX_WAVES3 = 4;           // wavefronts per SIMD the KW = 3 variant
 
 // Eight masked MACs  acc += upm_k * (x <= ym_k ? w_k : 0).  A compare and a select next to a multiply-add: both take the
 // slower of a SIMD's two pipes, but a third of such a stream leaves it enough else to do (probe kernels, four wavefronts per
-// SIMD: 2.3 clocks an instruction; the mask as two multiply-adds, m = clamp01((x - ym) * BIG) and w - m * w, takes 2.9).  A
+// SIMD, all masks in vcc: 2.3 clocks an instruction; the mask as two multiply-adds, m = clamp01((x - ym) * BIG) and w - m * w, takes
+// 2.9.  In kernels of other than three columns, where one wavefront waits for more, they differ by 2 % either way).  A
 // mask is read two instructions after the compare that writes it, at the earliest: three are under way at the start, then two, one in
 // vcc, the others in registers.
 #define SNNTC_DX_MV(K) "v_cmp_ge_f32_e32 vcc, %[y" #K "], %[x]\n"
@@ -810,9 +811,12 @@ int launch_cv_grad_input_chan(const float* xpad, const float* wq, const float* u
     const auto chosen = [&](auto kcb_c) {
         constexpr int KCB = decltype(kcb_c)::value;
         if (g.Kw != 3) return multi ? cv_grad_input_chan_kernel<KCB, true, 0> : cv_grad_input_chan_kernel<KCB, false, 0>;
-        // (the parts of a wavefront begin eight columns apart: with an odd stride their patches lie under other slots, nearly all between them.
-        // 3x3/3, 32 -> 64 at 32 x 32, 64 images 62.8 us against 65.6, 16 -> 32, 128 images 56 against 65, 3 -> 32 33 against 40)
-        if (multi ? g.Sw % 2 == 0 : g.Sw != 1) return multi ? cv_grad_input_chan_kernel<KCB, true, 3, true> : cv_grad_input_chan_kernel<KCB, false, 3, true>;
+        // The parts of a wavefront begin eight columns apart: with an odd stride their patches lie under other slots, nearly all between them (3x3/3,
+        // 32 -> 64 at 32 x 32, 64 images 62.8 us against 65.6).  Wavefronts of eight and more parts, whose operands are as many reads, and
+        // layers of sixteen outputs lose more by waiting for them than the slots left out save (3x3/2, 4 images and more, all slots / some: 3 -> 64 at 64 x 64
+        // 296 / 360, 7 -> 32 138 / 188, 3 -> 16 at 30 x 30 24.2 / 25.9, but 3 -> 128 89 / 75, 16 -> 64 29.4 / 28.5, 32 -> 128 50.9 / 43.2).
+        const bool strided = multi ? g.Sw % 2 == 0 && pl.parts_shift <= 2 && g.Kc >= 32 : g.Sw != 1;
+        if (strided) return multi ? cv_grad_input_chan_kernel<KCB, true, 3, true> : cv_grad_input_chan_kernel<KCB, false, 3, true>;
         return multi ? cv_grad_input_chan_kernel<KCB, true, 3> : cv_grad_input_chan_kernel<KCB, false, 3>;
     };
     const auto kern = kcb == 64 ? chosen(std::integral_constant<int, 64>{}) : kcb == 32 ? chosen(std::integral_constant<int, 32>{})
