@@ -195,10 +195,38 @@ def test_conv_weight_gradients_by_pixels(B, H, W, C, Kc, Kh, Sh, slices, least, 
 ])
 def test_conv_weight_gradients_by_pixels_of_32_channels(B, H, W, C, Kc, Kh, Sh, slices, least, bias):
     """The launches that fill the chip: rows of 7, 1, 2, 2 and 28 patches, row strides of two, two kernel rows, outputs that are no multiple of 64."""
-    _check_weight_gradients(B, H, W, C, Kc, Kh, Sh, slices, least, bias)
+    _check_weight_gradients(B, H, W, C, Kc, Kh, Sh, slices, least, bias, _weight_gradients_64)
 
 
-def _check_weight_gradients(B, H, W, C, Kc, Kh, Sh, slices, least, bias):
+def _weight_gradients_oracle(g, x, w, p, out):
+    """dW and the sums of its terms' sizes."""
+    sizes = out.copy()
+    sizes[len(x):] = np.abs(sizes[len(x):])
+    return capi.cv_backward_dev(g, x, w, p, out, wide=True)[1], np.abs(capi.cv_backward_dev(np.abs(g), x, w, p, sizes, wide=True)[1])
+
+
+def _weight_gradients_64(g, x, w, p, out):
+    """The same in plain 64-bit arithmetic on the GPU, tap by tap (hundreds of millions of terms)."""
+    B, _, _, C = x.shape
+    Nh, Nw, Kc = out.shape[1:]
+    Kh, Sh, biasvolt = int(p[6]), int(p[8]), float(p[11])
+    upstream = (t(g[:B]).double() * t(out[B:]).double()).reshape(-1, Kc)
+    times = t(out[:B]).double().reshape(-1, Kc)
+    xd = t(x).double()
+    sums, sizes = (torch.zeros(w.shape, dtype=torch.float64, device=DEV) for _ in range(2))
+    taps = [xd[:, kh:kh + (Nh - 1) * Sh + 1:Sh, kw:kw + Nw].reshape(-1, C) for kh in range(Kh) for kw in range(3)]
+    if len(w) > 3 * Kh * C:
+        taps.append(torch.full((B * Nh * Nw, 1), biasvolt, dtype=torch.float64, device=DEV))
+    for tap, inputs in enumerate(taps):
+        rows = slice(tap * C, tap * C + inputs.shape[1])
+        for s in range(0, len(inputs), 512):
+            terms = (inputs[s:s + 512, :, None] - times[s:s + 512, None]).clamp(max=0) * upstream[s:s + 512, None]
+            sums[rows] += terms.sum(0)
+            sizes[rows] += terms.abs().sum(0)
+    return sums.cpu().numpy(), sizes.cpu().numpy()
+
+
+def _check_weight_gradients(B, H, W, C, Kc, Kh, Sh, slices, least, bias, reference=_weight_gradients_oracle):
     import ctypes
     import snntc_amd as snn
     from snntc_amd import _lib
@@ -215,12 +243,9 @@ def _check_weight_gradients(B, H, W, C, Kc, Kh, Sh, slices, least, bias):
     g = np.zeros((2 * B, Nh, Nw, Kc), np.float32)
     g[:B] = rng.standard_normal((B, Nh, Nw, Kc))
     dw = snn.snncv_grad(t(g), t(x), t(w), p, t(out))[1]
-    _, rdw, _ = capi.cv_backward_dev(g, x, w, p, out, wide=True)
-    ao = out.copy()
-    ao[B:] = np.abs(ao[B:])
-    _, adw, _ = capi.cv_backward_dev(np.abs(g), x, w, p, ao, wide=True)
-    # (a few thousand terms of either sign, 2e-7 of |terms| as for the dense gradients' partial sums, and a margin)
-    assert np.all(np.abs(dw.cpu().numpy() - rdw) <= 2e-6 * np.abs(adw) + 1e-30)
+    rdw, adw = reference(g, x, w, p, out)
+    # (some thousand terms of either sign, 2e-7 of |terms| as for the dense gradients' partial sums, and a margin)
+    assert np.all(np.abs(dw.cpu().numpy() - rdw) <= 2e-6 * adw + 1e-30)
     # with the room that the kernels for any shape ask for there are fewer slices, and with less the call is refused
     lib = _lib.load()
     need = ctypes.c_size_t()
@@ -245,7 +270,7 @@ def _check_weight_gradients(B, H, W, C, Kc, Kh, Sh, slices, least, bias):
         if call(room) != _lib.OK:
             break
         err = np.abs(again.cpu().numpy() - rdw)
-        assert np.all(err <= 2e-6 * np.abs(adw) + 1e-30)
+        assert np.all(err <= 2e-6 * adw + 1e-30)
         fewer += 1
     else:
         raise AssertionError("no workspace was refused")
