@@ -30,7 +30,9 @@ constexpr int DX_WAVES3 = 4;           // wavefronts per SIMD the KW = 3 variant
 // Eight masked MACs  acc += upm_k * (x <= ym_k ? w_k : 0).  A compare and a select next to a multiply-add: both take the
 // slower of a SIMD's two pipes, but a third of such a stream leaves it enough else to do (probe kernels, four wavefronts per
 // SIMD, all masks in vcc: 2.3 clocks an instruction; the mask as two multiply-adds, m = clamp01((x - ym) * BIG) and w - m * w, takes
-// 2.9.  In kernels of other than three columns, where one wavefront waits for more, they differ by 2 % either way).  A
+// 2.9.  In kernels of other than three columns, where one wavefront waits for more, they differ by 2 % either way.  In the sweep
+// of three-column kernels a vector instruction takes 3.5 clocks, since there are 80 LDS reads to 1152 of them, half of the masks in eight-byte
+// encodings, and waits for weights.)  A
 // mask is read two instructions after the compare that writes it, at the earliest: three are under way at the start, then two, one in
 // vcc, the others in registers.
 #define SNNTC_DX_MV(K) "v_cmp_ge_f32_e32 vcc, %[y" #K "], %[x]\n"
@@ -465,7 +467,8 @@ cv_grad_weight_wide_kernel(const float* __restrict__ xpad, const float* __restri
 // A wait for one scalar load is a wait for all: a pixel's inputs are fetched in two halves, each while the other is worked on.
 // Terms are added in the order of the patches, then wavefronts, then slices.  us, blocks of 32 rows / this, the slices' sum included: 64 -> 64 at
 // 32 x 32, 64 images 131 / 115, at 56 x 56, 32 images 187 / 162, 128 -> 128 at 28 x 28 191 / 160, 256 -> 256 at 14 x 14 222 / 161,
-// 256 -> 512 at 7 x 7 129 / 95, 512 -> 512 198 / 168.  (Without any fetch it takes 103 of 108: what bounds it is the issue rate.)
+// 256 -> 512 at 7 x 7 129 / 95, 512 -> 512 198 / 168.  (Without any fetch it takes 103 of 108: what bounds it
+// are its vector instructions, 3.1 clocks each, every second of which has a scalar operand.)
 // ---------------------------------------------------------------------------------------------
 constexpr int DWT_KW = 3, DWT_WAVES = 8;
 // (read by scalar loads where the address is uniform)
