@@ -465,7 +465,7 @@ cv_grad_weight_wide_kernel(const float* __restrict__ xpad, const float* __restri
 // registers.  Next to a block of 32 weight rows that is a third of the fetches for the same arithmetic and fewer instructions
 // around it (an issue slot each, whatever they are): 192 vector instructions per pixel instead of three times 64.
 // A wait for one scalar load is a wait for all: a pixel's inputs are fetched in two halves, each while the other is worked on.
-// Terms are added in the order of the patches, then wavefronts, then slices.  us, blocks of 32 rows / this, the slices' sum included: 64 -> 64 at
+// Terms are added in the order of the patches, then wavefronts in a tree, then slices.  us, blocks of 32 rows / this, the slices' sum included: 64 -> 64 at
 // 32 x 32, 64 images 131 / 115, at 56 x 56, 32 images 187 / 162, 128 -> 128 at 28 x 28 191 / 160, 256 -> 256 at 14 x 14 222 / 161,
 // 256 -> 512 at 7 x 7 129 / 95, 512 -> 512 198 / 168.  (Without any fetch it takes 103 of 108: what bounds it
 // are its vector instructions, 3.1 clocks each, every second of which has a scalar operand.)
@@ -604,10 +604,16 @@ cv_grad_weight_taps_kernel(const float* __restrict__ xpad, const float* __restri
         __syncthreads();
         if (wave == 0 && j < Kc) {
             const size_t row0 = (size_t)(kh * DWT_KW + t) * C + c0;
-            auto total = [&](float sum, int r) {
+            auto total = [&](float own, int r) {                            // (in a tree: three roundings, not seven)
+                float sum[DWT_WAVES];
+                sum[0] = own;
 #pragma unroll
-                for (int v = 0; v < DWT_WAVES - 1; ++v) sum += red[v][r][lane];
-                return sum * post;
+                for (int v = 1; v < DWT_WAVES; ++v) sum[v] = red[v - 1][r][lane];
+#pragma unroll
+                for (int h = DWT_WAVES / 2; h > 0; h /= 2)
+#pragma unroll
+                    for (int v = 0; v < h; ++v) sum[v] += sum[v + h];
+                return sum[0] * post;
             };
 #pragma unroll
             for (int r = 0; r < CB; ++r) out[(row0 + r) * Kc + j] = total(acc[t][r], r);
@@ -842,6 +848,9 @@ static int64_t cv_grad_weight_row_blocks(const ConvGeom& g) {
     return g.Kh * ((g.Kw * g.C + DWW_RI - 1) / DWW_RI);
 }
 
+// Workgroups per slice of the blocks of 32 rows.
+int cv_grad_weight_row32_blocks(const ConvGeom& g) { return (int)(((g.Kc + kWave - 1) / kWave) * cv_grad_weight_row_blocks(g)); }
+
 // Whether a layer's dW goes to cv_grad_weight_taps_kernel, the channels a wavefront owns there, and into how many slices its patches are cut.
 // Lines from some 400 shapes, each in all forms (us; blocks of 32 rows / sixteen channels / thirty-two).  `terms`: 64 outputs of sixteen channels of a
 // kernel row times runs of 128 patches.
@@ -856,20 +865,26 @@ static TapsPlan cv_grad_weight_taps_plan(const ConvGeom& g) {
     if (g.Kw != DWT_KW || g.Sw != 1 || g.C % 16 != 0 || g.Kc <= 32 || g.S * g.Kc * 4 >= 0x7fffffffLL) return {};
     const int64_t blocks = (g.Kc + kWave - 1) / kWave * g.Kh * (g.C / 16);
     const int64_t terms = blocks * (g.S / 128), capped = blocks * std::min<int64_t>(g.S / 128, 128);
+    // At least half as many as the blocks of 32 rows get, whose workgroups have half as many wavefronts: no chain of additions is longer than theirs, and
+    // neither is the error against 64 bits (rms at 1.06 to 1.3 times their chain up to 1.05 of theirs, at the same chain 0.95 to 1.00).
+    const int least = (weight_grad_splits(g.S, cv_grad_weight_row32_blocks(g)) + 1) / 2;
     // slices of launches of so many workgroups, which have twice as many wavefronts as the line's others
-    const auto slices = [&](int64_t workgroups) { return weight_grad_splits(g.S / 2, workgroups * 2); };
+    const auto slices = [&](int64_t workgroups) { return std::max(least, weight_grad_splits(g.S / 2, workgroups * 2)); };
     if (g.C % 32 != 0) {
         if (capped < (g.C <= 48 ? 100 : 200)) return {};
         // (small launches in more of them: 1568 of 80 to 64 18.0 -> 15.9, 1568 of 144 to 100 29.0 -> 26.5; but 25 088 of 16 to 100 41.4 -> 43.4)
-        return {16, capped < 700 ? weight_grad_splits(g.S / 2, blocks) : slices(blocks)};
+        const int n = capped < 700 ? weight_grad_splits(g.S / 2, blocks) : slices(blocks);
+        // (more than that only within the same turns of the chip, rows / this: 1725 of 144 to 96, seven slices, now nine, 29.6 / 26.9; but 2376 of 48 to 100,
+        // fourteen slices 18.6, fifteen 22.4, rows 22.4, 1620 of 144 to 48, nine 18.6, eleven 21.7, rows 20.9)
+        if (n < least && (blocks * least + 255) / 256 > (blocks * n + 255) / 256) return {};
+        return {16, std::max(n, least)};
     }
     if (capped < 700) return {};
     if (terms >= 3000) return {32, slices(blocks / 2)};
     return {16, slices(blocks >= 12 ? blocks / 2 : blocks)};
 }
 
-// Workgroups per slice of the blocks of 32 rows, and slices that the patch range is cut into.
-int cv_grad_weight_row32_blocks(const ConvGeom& g) { return (int)(((g.Kc + kWave - 1) / kWave) * cv_grad_weight_row_blocks(g)); }
+// Slices that the patch range is cut into.
 int cv_grad_weight_splits(const ConvGeom& g) {
     const TapsPlan taps = cv_grad_weight_taps_plan(g);
     return taps.channels ? taps.slices : weight_grad_splits(g.S, cv_grad_weight_row32_blocks(g));

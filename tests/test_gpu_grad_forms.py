@@ -226,6 +226,32 @@ def _weight_gradients_64(g, x, w, p, out):
     return sums.cpu().numpy(), sizes.cpu().numpy()
 
 
+# (`blocks`: the error of the blocks of 32 weight rows on these inputs)
+@pytest.mark.parametrize("B,H,W,C,Kc,blocks", [
+    (32, 9, 9, 144, 100, 5.096), (16, 9, 9, 112, 128, 6.743), (7, 40, 12, 48, 40, 3.902), (15, 7, 25, 144, 96, 4.964), (18, 20, 7, 144, 48, 4.783),
+    (11, 20, 14, 48, 100, 4.122), (65, 9, 9, 96, 100, 3.873), (4, 16, 16, 512, 512, 13.979),
+])
+def test_conv_weight_gradients_are_as_exact_by_pixels(B, H, W, C, Kc, blocks):
+    """A wavefront that walks over pixels, eight to a workgroup, rounds no more than the blocks of 32 weight rows do."""
+    assert _conv_weight_gradient_error(B, H, W, C, Kc) <= 1.005 * blocks
+
+
+def _conv_weight_gradient_error(B, H, W, C, Kc):
+    """rms error of dW, in 1e-9 of the terms' absolute sum."""
+    import snntc_amd as snn
+    rng = np.random.default_rng(B + H + W + C + Kc)
+    x = np.exp(1.0 - rng.random((B, H, W, C))).astype(np.float32)
+    p = capi.cv_params(3, 3, 1, 1, same=False, biasvolt=1.0)
+    w = rng.standard_normal((9 * C + 1, Kc)).astype(np.float32)
+    y = np.exp(1.2 * rng.random((B, H - 2, W - 2, Kc))).astype(np.float32)
+    g = np.zeros((2 * B, H - 2, W - 2, Kc), np.float32)
+    g[:B] = rng.standard_normal(y.shape)
+    out = np.concatenate([y, np.ones_like(y)])                # (upstream values without a rounding of their own)
+    dw = snn.snncv_grad(t(g), t(x), t(w), p, t(out))[1].cpu().numpy().astype(np.float64)
+    rdw, adw = _weight_gradients_64(g, x, w, p, out)
+    return 1e9 * np.sqrt(np.mean(((dw - rdw) / adw) ** 2))
+
+
 def _check_weight_gradients(B, H, W, C, Kc, Kh, Sh, slices, least, bias, reference=_weight_gradients_oracle):
     import ctypes
     import snntc_amd as snn
